@@ -124,6 +124,68 @@ int bwd_f64(const char *fn, const BwdArgs &a, size_t ws_floats, hipStream_t st) 
     return launch_bwd_f64(a, st);
 }
 
+// a square, centred, undilated window: the kernel family that serves the call
+int run_fwd(const FwdArgs &a, int dtype, hipStream_t st) {
+    const int D = a.s.D, ks = a.s.kh;
+    if (dtype == ENATTEN_F64) return launch_fwd_f64(a, st);
+    if (use_mfma(D, ks, dtype)) return launch_fwd_mfma(a, dtype, st);
+    if (use_mfma_f32(D, ks, dtype)) return launch_fwd_mfma_f32(a, st);
+    return launch_fwd_simt(a, dtype, st);
+}
+int run_bwd(const char *fn, const BwdArgs &a, int dtype, size_t ws_floats, hipStream_t st) {
+    const int D = a.s.D, ks = a.s.kh;
+    if (dtype == ENATTEN_F64) return bwd_f64(fn, a, ws_floats, st);
+    if (use_mfma(D, ks, dtype)) return launch_bwd_mfma(a, dtype, g_path.load(), st);
+    // the float32 matrix-core backward where the workspace at hand holds its P and dS (it
+    // writes contiguous gradients only)
+    if (use_mfma_f32(D, ks, dtype) && a.grads_contiguous() &&
+        ws_floats >= (size_t)a.s.B * a.s.N * a.s.H * a.s.W * mfma_f32_workspace_floats(ks))
+        return launch_bwd_mfma_f32(a, st);
+    return launch_bwd_simt(a, dtype, st);
+}
+
+// The sub-grids of a dilated call (pixels of one residue class modulo the dilation on each
+// axis) are images of at most two sizes per axis: H = dil * h + r gives r classes of h + 1 rows
+// and dil - r of h.  One axis of one such group: the classes from `first` on, `count` of them,
+// `extent` positions each.
+struct SubAxis {
+    int first, count, extent;
+};
+int split_axis(int L, int dil, SubAxis (&out)[2]) {
+    const int r = L % dil, h = L / dil;
+    int n = 0;
+    if (r) out[n++] = SubAxis{0, r, h + 1};
+    out[n++] = SubAxis{r, dil - r, h};
+    return n;
+}
+// the same tensor from the group's first pixel on
+View group_view(const View &v, int es, const SubAxis &r, const SubAxis &c) {
+    View o = v;
+    o.ptr = static_cast<const char *>(v.ptr) + (r.first * v.sh + c.first * v.sw) * es;
+    return o;
+}
+// sub-grid (i, j) of a group as an image of its own
+View one_sub(const View &v, int es, int dil, int i, int j) {
+    View o = v;
+    o.ptr = static_cast<const char *>(v.ptr) + (i * v.sh + j * v.sw) * es;
+    o.sh = v.sh * dil; o.sw = v.sw * dil;
+    return o;
+}
+void *offset(void *p, int64_t elements, int es) { return static_cast<char *>(p) + elements * es; }
+
+int check_dilation(const char *fn, int H, int W, int ks, int dil) {
+    if (dil < 1) {
+        set_error("%s: dilation must be >= 1, got %d", fn, dil);
+        return ENATTEN_EINVAL;
+    }
+    if (H / dil < ks || W / dil < ks) {
+        set_error("%s: image %dx%d is smaller than kernel_size * dilation = %lld", fn, H, W,
+                  (long long)ks * dil);
+        return ENATTEN_EINVAL;
+    }
+    return ENATTEN_OK;
+}
+
 }  // namespace
 }  // namespace enatten
 
@@ -164,11 +226,7 @@ int enatten2d_fwd(const void *q, const void *k, const void *v, void *o, float *l
     if ((rc = make_view(fn, "o", o, o_strides, heads, H, W, D, &a.o))) return rc;
     a.lse = lse;
     a.s = Shape{B, heads, H, W, D, kernel_size, kernel_size, scale};
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (dtype == ENATTEN_F64) return launch_fwd_f64(a, st);
-    if (use_mfma(D, kernel_size, dtype)) return launch_fwd_mfma(a, dtype, st);
-    if (use_mfma_f32(D, kernel_size, dtype)) return launch_fwd_mfma_f32(a, st);
-    return launch_fwd_simt(a, dtype, st);
+    return run_fwd(a, dtype, static_cast<hipStream_t>(stream));
 }
 
 size_t enatten2d_bwd_workspace_bytes(int B, int heads, int H, int W, int D, int kernel_size,
@@ -201,15 +259,7 @@ static int bwd2d(const char *fn, const void *q, const void *k, const void *v, co
     a.zinv = a.delta + (size_t)B * heads * H * W;
     a.s = Shape{B, heads, H, W, D, kernel_size, kernel_size, scale};
     if ((rc = set_grad_layout(fn, &a, grad_strides))) return rc;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (dtype == ENATTEN_F64) return bwd_f64(fn, a, ws_floats, st);
-    if (use_mfma(D, kernel_size, dtype)) return launch_bwd_mfma(a, dtype, g_path.load(), st);
-    // the float32 matrix-core backward where the workspace at hand holds its P and dS (it
-    // writes contiguous gradients only)
-    if (use_mfma_f32(D, kernel_size, dtype) && a.grads_contiguous() &&
-        ws_floats >= (size_t)B * heads * H * W * mfma_f32_workspace_floats(kernel_size))
-        return launch_bwd_mfma_f32(a, st);
-    return launch_bwd_simt(a, dtype, st);
+    return run_bwd(fn, a, dtype, ws_floats, static_cast<hipStream_t>(stream));
 }
 
 int enatten2d_bwd(const void *q, const void *k, const void *v, const void *o, const void *d_o,
@@ -306,6 +356,137 @@ int enatten2d_bwd_static(const void *q, const void *k, const void *v, const void
     return bwd2d(fn, q, k, v, o, d_o, lse, dq, dk, dv, ws,
                  (size_t)2 * ENATTEN_STATIC_BWD_MAX_QUERIES, B, heads, H, W, D, kernel_size, dtype,
                  q_strides, k_strides, v_strides, o_strides, do_strides, scale, stream);
+}
+
+// ---- dilated neighborhoods --------------------------------------------------
+// Sub-grids of one size run as one batch on the matrix-core kernels (up to four groups, one if
+// the dilation divides both sides), and one after the other on the other kernels.  The
+// log-sum-exp and the workspace are laid out by group, within a group one [B, heads, h, w]
+// block per sub-grid, whichever kernels serve the call, so that a backward that is routed
+// differently from its forward (a misaligned upstream gradient) finds what it needs.
+int enatten2d_fwd_dilated(const void *q, const void *k, const void *v, void *o, float *lse, int B,
+                          int heads, int H, int W, int D, int kernel_size, int dilation, int dtype,
+                          const int64_t *q_strides, const int64_t *k_strides,
+                          const int64_t *v_strides, const int64_t *o_strides, float scale,
+                          void *stream) {
+    const char *fn = "enatten2d_fwd_dilated";
+    int rc = check_shape(fn, B, heads, H, W, D, kernel_size, dtype);
+    if (rc || (rc = check_dilation(fn, H, W, kernel_size, dilation))) return rc;
+    FwdArgs full;
+    if ((rc = make_view(fn, "q", q, q_strides, heads, H, W, D, &full.q))) return rc;
+    if ((rc = make_view(fn, "k", k, k_strides, heads, H, W, D, &full.k))) return rc;
+    if ((rc = make_view(fn, "v", v, v_strides, heads, H, W, D, &full.v))) return rc;
+    if ((rc = make_view(fn, "o", o, o_strides, heads, H, W, D, &full.o))) return rc;
+    const int es = elem_size(dtype);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    SubAxis rows[2], cols[2];
+    const int nr = split_axis(H, dilation, rows), nc = split_axis(W, dilation, cols);
+    for (int gi = 0; gi < nr; gi++)
+        for (int gj = 0; gj < nc; gj++) {
+            const SubAxis &r = rows[gi], &c = cols[gj];
+            FwdArgsSub a;
+            a.q = group_view(full.q, es, r, c);
+            a.k = group_view(full.k, es, r, c);
+            a.v = group_view(full.v, es, r, c);
+            a.o = group_view(full.o, es, r, c);
+            a.lse = lse;
+            a.s = Shape{B, heads, r.extent, c.extent, D, kernel_size, kernel_size, scale};
+            a.sub_r = r.count; a.sub_c = c.count; a.dil = dilation;
+            const int64_t per_sub = (int64_t)B * heads * r.extent * c.extent;
+            if (use_mfma(D, kernel_size, dtype) && sub_layout_ok(a)) {
+                if ((rc = launch_fwd_mfma_sub(a, dtype, st))) return rc;
+            } else {
+                for (int i = 0; i < r.count; i++)
+                    for (int j = 0; j < c.count; j++) {
+                        FwdArgs b = a;
+                        b.q = one_sub(a.q, es, dilation, i, j);
+                        b.k = one_sub(a.k, es, dilation, i, j);
+                        b.v = one_sub(a.v, es, dilation, i, j);
+                        b.o = one_sub(a.o, es, dilation, i, j);
+                        if (lse) b.lse = lse + (i * c.count + j) * per_sub;
+                        if ((rc = run_fwd(b, dtype, st))) return rc;
+                    }
+            }
+            if (lse) lse += r.count * c.count * per_sub;
+        }
+    return ENATTEN_OK;
+}
+
+size_t enatten2d_bwd_dilated_workspace_bytes(int B, int heads, int H, int W, int dtype) {
+    if (B < 1 || heads < 1 || H < 1 || W < 1) return 0;
+    // two floats per query, four for float64; sub-grids that run one after the other share them
+    return (size_t)B * heads * H * W * (dtype == ENATTEN_F64 ? 4 : 2) * sizeof(float);
+}
+
+int enatten2d_bwd_dilated(const void *q, const void *k, const void *v, const void *o,
+                          const void *d_o, const float *lse, void *dq, void *dk, void *dv,
+                          void *workspace, int B, int heads, int H, int W, int D, int kernel_size,
+                          int dilation, int dtype, const int64_t *q_strides,
+                          const int64_t *k_strides, const int64_t *v_strides,
+                          const int64_t *o_strides, const int64_t *do_strides, float scale,
+                          void *stream) {
+    const char *fn = "enatten2d_bwd_dilated";
+    int rc = check_shape(fn, B, heads, H, W, D, kernel_size, dtype);
+    if (rc || (rc = check_dilation(fn, H, W, kernel_size, dilation))) return rc;
+    BwdArgs full;
+    if ((rc = make_view(fn, "q", q, q_strides, heads, H, W, D, &full.q))) return rc;
+    if ((rc = make_view(fn, "k", k, k_strides, heads, H, W, D, &full.k))) return rc;
+    if ((rc = make_view(fn, "v", v, v_strides, heads, H, W, D, &full.v))) return rc;
+    if ((rc = make_view(fn, "o", o, o_strides, heads, H, W, D, &full.o))) return rc;
+    if ((rc = make_view(fn, "d_o", d_o, do_strides, heads, H, W, D, &full.d_o))) return rc;
+    if (!lse || !dq || !dk || !dv || !workspace) {
+        set_error("%s: lse, dq, dk, dv and workspace must all be non-NULL", fn);
+        return ENATTEN_EINVAL;
+    }
+    const int es = elem_size(dtype);
+    const size_t ws_floats = (size_t)B * heads * H * W * (dtype == ENATTEN_F64 ? 4 : 2);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    SubAxis rows[2], cols[2];
+    const int nr = split_axis(H, dilation, rows), nc = split_axis(W, dilation, cols);
+    for (int gi = 0; gi < nr; gi++)
+        for (int gj = 0; gj < nc; gj++) {
+            const SubAxis &r = rows[gi], &c = cols[gj];
+            BwdArgsSub a;
+            a.q = group_view(full.q, es, r, c);
+            a.k = group_view(full.k, es, r, c);
+            a.v = group_view(full.v, es, r, c);
+            a.o = group_view(full.o, es, r, c);
+            a.d_o = group_view(full.d_o, es, r, c);
+            a.lse = lse;
+            a.s = Shape{B, heads, r.extent, c.extent, D, kernel_size, kernel_size, scale};
+            // contiguous [B, heads, H, W, D] gradients
+            const int64_t first = ((int64_t)r.first * W + c.first) * D;
+            a.dq = offset(dq, first, es); a.dk = offset(dk, first, es); a.dv = offset(dv, first, es);
+            a.gsw = D;
+            a.gsh = (int64_t)W * D;
+            a.gsn = (int64_t)H * W * D;
+            a.gsb = (int64_t)heads * H * W * D;
+            a.sub_r = r.count; a.sub_c = c.count; a.dil = dilation;
+            const int64_t per_sub = (int64_t)B * heads * r.extent * c.extent;
+            a.delta = static_cast<float *>(workspace);
+            if (use_mfma(D, kernel_size, dtype) && sub_layout_ok(a)) {
+                a.zinv = a.delta + r.count * c.count * per_sub;
+                if ((rc = launch_bwd_mfma_sub(a, dtype, st))) return rc;
+            } else {
+                for (int i = 0; i < r.count; i++)
+                    for (int j = 0; j < c.count; j++) {
+                        BwdArgs b = a;
+                        b.q = one_sub(a.q, es, dilation, i, j);
+                        b.k = one_sub(a.k, es, dilation, i, j);
+                        b.v = one_sub(a.v, es, dilation, i, j);
+                        b.o = one_sub(a.o, es, dilation, i, j);
+                        b.d_o = one_sub(a.d_o, es, dilation, i, j);
+                        const int64_t at = i * a.gsh + j * a.gsw;
+                        b.dq = offset(a.dq, at, es); b.dk = offset(a.dk, at, es); b.dv = offset(a.dv, at, es);
+                        b.gsh = a.gsh * dilation; b.gsw = a.gsw * dilation;
+                        b.lse = lse + (i * c.count + j) * per_sub;
+                        b.zinv = b.delta + per_sub;
+                        if ((rc = run_bwd(fn, b, dtype, ws_floats, st))) return rc;
+                    }
+            }
+            lse += r.count * c.count * per_sub;
+        }
+    return ENATTEN_OK;
 }
 
 // ---- rectangular and causal windows ----------------------------------------

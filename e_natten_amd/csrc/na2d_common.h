@@ -54,6 +54,18 @@ struct BwdArgs {
                                 // from which d_rpb is summed in a fixed order
 };
 
+// A dilated call as a batch of undilated ones: sub_r x sub_c sub-grids of s.H x s.W pixels each,
+// whose neighbouring pixels are `dil` rows / columns of the tensors apart.  The strides of the
+// views (and of the gradients) are those of the tensors, their pointers those of the first
+// sub-grid.  Types of their own, so that the undilated kernels' arguments stay what they are
+// (longer arguments changed their scalar loads, and with them B2 N8 128x128 d64 k13 by 2%).
+struct FwdArgsSub : FwdArgs {
+    int sub_r, sub_c, dil;
+};
+struct BwdArgsSub : BwdArgs {
+    int sub_r, sub_c, dil;
+};
+
 // NATTEN window start on an axis of length L: centred, shifted to stay inside
 // (e_natten/pytorch.py:7-11, e_natten/triton.py:7-12).
 __host__ __device__ inline int win_start(int i, int L, int k) {
@@ -138,6 +150,13 @@ int launch_bwd_mfma(const BwdArgs &a, int dtype, int path, hipStream_t st);
 // the same kernels built for head dims that are multiples of 8 below the next of 32, 64, 128
 int launch_fwd_mfma_narrow(const FwdArgs &a, int dtype, hipStream_t st);
 int launch_bwd_mfma_narrow(const BwdArgs &a, int dtype, int path, hipStream_t st);
+// the same kernels on all sub-grids of a dilated call at once, any head dim mfma_supported takes;
+// the log-sum-exp and the workspace hold one [B, N, H, W] block per sub-grid.  The caller has
+// asked sub_layout_ok: tensors whose rows the 16-byte loads cannot take run otherwise.
+bool sub_layout_ok(const FwdArgsSub &a);
+bool sub_layout_ok(const BwdArgsSub &a);
+int launch_fwd_mfma_sub(const FwdArgsSub &a, int dtype, hipStream_t st);
+int launch_bwd_mfma_sub(const BwdArgsSub &a, int dtype, hipStream_t st);
 // matrix-core kernels of the 1D operator (a.s: H = 1, W = T, kh = 1, kw = kernel_size):
 // bf16 / f16, D in {32, 64, 128}, odd kernel_size 3 .. 49
 bool mfma1d_supported(int D, int ks, int dtype);

@@ -6,6 +6,7 @@
 namespace enatten {
 namespace {
 constexpr bool kNarrow = false;
+constexpr bool kSub = false;
 }
 }  // namespace enatten
 

@@ -33,6 +33,13 @@
 // stores (zero_row, HaloPlan::on, load_row_chunks, store_token in na2d_mfma.h).  One
 // build serving both was measured 5-40% slower on the exact head dims (the predicates
 // cost the large-halo kernels the registers they do not have).
+//
+// na2d_mfma_dilated.hip compiles it a third time with `kSub` true: the images are then the
+// sub-grids of a dilated call (pixels of one residue class modulo the dilation on each axis,
+// between which no query sees a key), all of one size, numbered batch, sub-grid row, sub-grid
+// column, head.  The heads are innermost because in the layout of a projection they lie side by
+// side in memory: a workgroup and its neighbours then read the same lines.  `kSub` false folds
+// every one of these helpers to what it is without sub-grids.
 
 #include <algorithm>
 
@@ -57,6 +64,71 @@ constexpr bool kInnerLines = (D == 128 || D == 64) && !kNarrow;
 template <int D, int KS, int WGS>
 constexpr bool kLineStores = (D == 128 || D == 64) && !kNarrow && WGS >= 2;
 
+// ------------------------------------------------------------------ images
+using FArgs = std::conditional_t<kSub, FwdArgsSub, FwdArgs>;
+using BArgs = std::conditional_t<kSub, BwdArgsSub, BwdArgs>;
+struct SubTile : Tile {
+    int ri, rj;  // sub-grid
+};
+using ATile = std::conditional_t<kSub, SubTile, Tile>;
+
+// Images (one batch entry, head and sub-grid each) of a launch
+template <typename ARGS>
+int64_t images_of(const ARGS &a) {
+    if constexpr (kSub) return (int64_t)a.s.B * a.s.N * a.sub_r * a.sub_c;
+    else return (int64_t)a.s.B * a.s.N;
+}
+// tile_of and its like split an image number into (what is before the heads, head); with
+// sub-grids the former is (batch, sub-grid row, sub-grid column)
+template <typename ARGS, typename TL>
+__device__ __forceinline__ void sub_grid(TL &tl, const ARGS &a) {
+    tl.rj = tl.bb % a.sub_c; tl.bb /= a.sub_c;
+    tl.ri = tl.bb % a.sub_r; tl.bb /= a.sub_r;
+}
+template <typename ARGS>
+__device__ __forceinline__ ATile in_sub(Tile t, const ARGS &a) {
+    ATile tl;
+    static_cast<Tile &>(tl) = t;
+    if constexpr (kSub) sub_grid(tl, a);
+    return tl;
+}
+template <typename ARGS, typename TL>
+__device__ __forceinline__ const short *image_at(const ARGS &a, const View &v, const TL &tl) {
+    const short *p = image<short>(v, tl);
+    if constexpr (kSub) p += tl.ri * v.sh + tl.rj * v.sw;
+    return p;
+}
+// elements between pixels of an image that are one row / one column apart
+template <typename ARGS>
+__device__ __forceinline__ int64_t row_step(const ARGS &a, const View &v) {
+    if constexpr (kSub) return v.sh * a.dil;
+    else return v.sh;
+}
+template <typename ARGS>
+__device__ __forceinline__ int64_t col_step(const ARGS &a, const View &v) {
+    if constexpr (kSub) return v.sw * a.dil;
+    else return v.sw;
+}
+template <typename ARGS, typename TL>
+__device__ __forceinline__ int64_t grad_of(const ARGS &a, const TL &tl, int y, int x) {
+    if constexpr (kSub) return a.grad_at(tl.bb, tl.nn, tl.ri + y * a.dil, tl.rj + x * a.dil);
+    else return a.grad_at(tl.bb, tl.nn, y, x);
+}
+// place of an image's first query in the log-sum-exp and in the workspace
+template <typename ARGS, typename TL>
+__device__ __forceinline__ int64_t image_token(const ARGS &a, const TL &tl) {
+    const Shape &s = a.s;
+    int64_t b = tl.bb;
+    if constexpr (kSub) b += (int64_t)(tl.ri * a.sub_c + tl.rj) * s.B;
+    return (b * s.N + tl.nn) * s.H * (int64_t)s.W;
+}
+template <int KS, typename ARGS, typename TL>
+__device__ __forceinline__ LaneQ lane_at(const ARGS &a, const TL &tl, int wave, int n) {
+    LaneQ q = lane_query<KS>(tl, a.s, wave, n);
+    if constexpr (kSub) q.tok = image_token(a, tl) + (int64_t)q.qr * a.s.W + q.qc;
+    return q;
+}
+
 // ------------------------------------------------------------------ forward
 // ROLL: walk down the columns of an image and keep the halo rows that consecutive
 // tiles share in LDS (see make_runs); otherwise a strided walk over row-major tiles
@@ -68,7 +140,7 @@ constexpr bool kLineStores = (D == 128 || D == 64) && !kNarrow && WGS >= 2;
 // an explicit wait on its other side, it falls back to waiting for everything outstanding
 // (B4 N4 128x128 d128 k5: 58.8 -> 56.7 us, 256x256: 198.2 -> 189.3, d64 k5: 60.4 -> 58.5).
 template <bool BF, int D, int KS, bool ROLL, int NW = 4, bool FULL = false>
-__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void fwd_mfma(FwdArgs a, int tiles_r, int tiles_c, int ntiles, Runs rp) {
+__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void fwd_mfma(FArgs a, int tiles_r, int tiles_c, int ntiles, Runs rp) {
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_k[G::ROWS * G::PITCH];
     __shared__ __attribute__((aligned(16))) short lds_v[G::ROWS * G::PITCH];
@@ -89,22 +161,22 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void
     HaloRegs<D, KS, NW> kst, vst;
     s16x8 qnext[G::DS];
     // rows [y0, y0 + nr) of the halo are what LDS does not hold yet
-    auto prefetch = [&](const Tile &tl, const LaneQ &lq, int y0, int nr) __attribute__((always_inline)) {
+    auto prefetch = [&](const ATile &tl, const LaneQ &lq, int y0, int nr) __attribute__((always_inline)) {
         if constexpr (ROLL) {
-            halo_fetch_rows<D, KS>(kst, plan, image<short>(a.k, tl), a.k.sh, a.k.sw, y0, lq.hc0, nr, s.H, s.W);
-            halo_fetch_rows<D, KS>(vst, plan, image<short>(a.v, tl), a.v.sh, a.v.sw, y0, lq.hc0, nr, s.H, s.W);
+            halo_fetch_rows<D, KS>(kst, plan, image_at(a, a.k, tl), row_step(a, a.k), col_step(a, a.k), y0, lq.hc0, nr, s.H, s.W);
+            halo_fetch_rows<D, KS>(vst, plan, image_at(a, a.v, tl), row_step(a, a.v), col_step(a, a.v), y0, lq.hc0, nr, s.H, s.W);
         } else {
-            halo_fetch<D, KS>(kst, plan, image<short>(a.k, tl), a.k.sh, a.k.sw, lq.hr0, lq.hc0, s.H, s.W);
-            halo_fetch<D, KS>(vst, plan, image<short>(a.v, tl), a.v.sh, a.v.sw, lq.hr0, lq.hc0, s.H, s.W);
+            halo_fetch<D, KS>(kst, plan, image_at(a, a.k, tl), row_step(a, a.k), col_step(a, a.k), lq.hr0, lq.hc0, s.H, s.W);
+            halo_fetch<D, KS>(vst, plan, image_at(a, a.v, tl), row_step(a, a.v), col_step(a, a.v), lq.hr0, lq.hc0, s.H, s.W);
         }
-        load_row_chunks(qnext, image<short>(a.q, tl) + lq.qr * a.q.sh + lq.qc * a.q.sw, g, dlim);
+        load_row_chunks(qnext, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
     };
 
     auto pick = [&](int t) __attribute__((always_inline)) {
-        return ROLL ? tile_of_cm(t, tiles_r, tiles_c, s.N) : tile_of(t, tiles_r, tiles_c, s.N, G::TH);
+        return in_sub(ROLL ? tile_of_cm(t, tiles_r, tiles_c, s.N) : tile_of(t, tiles_r, tiles_c, s.N, G::TH), a);
     };
-    Tile cur = pick(sc.t);
-    LaneQ lq = lane_query<KS>(cur, s, wave, n);
+    ATile cur = pick(sc.t);
+    LaneQ lq = lane_at<KS>(a, cur, wave, n);
     int y0 = lq.hr0, nr = G::HR;
     prefetch(cur, lq, y0, nr);
     s16x8 qreg[G::DS];
@@ -130,11 +202,11 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void
 
         const int tn = sched_peek(sc);
         const bool more = tn < sc.t_end;
-        Tile nxt = cur;
+        ATile nxt = cur;
         LaneQ lqn = lq;
         if (more) {
             nxt = pick(tn);
-            lqn = lane_query<KS>(nxt, s, wave, n);
+            lqn = lane_at<KS>(a, nxt, wave, n);
             // the tile below in the same image keeps the rows the two halos share
             const bool below = ROLL && nxt.bb == cur.bb && nxt.nn == cur.nn && nxt.c0 == cur.c0 &&
                                nxt.r0 > cur.r0 && lqn.hr0 < lq.hr0 + G::HR;
@@ -201,7 +273,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void
                         o[mt]);
             }
 
-            store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(const_cast<short *>(image<short>(a.o, cur)) + lq.qr * a.o.sh + lq.qc * a.o.sw,
+            store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(const_cast<short *>(image_at(a, a.o, cur)) + lq.qr * row_step(a, a.o) + lq.qc * col_step(a, a.o),
                                g, o, 1.f / sum, lq.live, dlim);
             // (FULL: all four lanes of a token write its log-sum-exp, the same value, so that
             // this store is not predicated either)
@@ -243,7 +315,7 @@ constexpr bool kOneHaloFits = Geo<D, KS>::ROWS * Geo<D, KS>::PITCH * 2 + 1024 <=
 // tiles, no column walk.
 // FULL: as in fwd_mfma.
 template <bool BF, int D, int KS, int NW = 4, bool FULL = false>
-__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS> : 1)) void fwd2_mfma(FwdArgs a, int tiles_r, int tiles_c, int ntiles) {
+__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS> : 1)) void fwd2_mfma(FArgs a, int tiles_r, int tiles_c, int ntiles) {
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_x[G::ROWS * G::PITCH];
     const Shape &s = a.s;
@@ -258,14 +330,14 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim);
     HaloRegs<D, KS, NW> st;
     s16x8 qnext[G::DS];
-    auto fetch_rows = [&](const View &vw, const Tile &tl, const LaneQ &lq) __attribute__((always_inline)) {
-        halo_fetch<D, KS>(st, plan, image<short>(vw, tl), vw.sh, vw.sw, lq.hr0, lq.hc0, s.H, s.W);
+    auto fetch_rows = [&](const View &vw, const ATile &tl, const LaneQ &lq) __attribute__((always_inline)) {
+        halo_fetch<D, KS>(st, plan, image_at(a, vw, tl), row_step(a, vw), col_step(a, vw), lq.hr0, lq.hc0, s.H, s.W);
     };
-    auto fetch_q = [&](const Tile &tl, const LaneQ &lq) __attribute__((always_inline)) {
-        load_row_chunks(qnext, image<short>(a.q, tl) + lq.qr * a.q.sh + lq.qc * a.q.sw, g, dlim);
+    auto fetch_q = [&](const ATile &tl, const LaneQ &lq) __attribute__((always_inline)) {
+        load_row_chunks(qnext, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
     };
-    Tile cur = tile_of(sc.t, tiles_r, tiles_c, s.N, G::TH);
-    LaneQ lq = lane_query<KS>(cur, s, wave, n);
+    ATile cur = in_sub(tile_of(sc.t, tiles_r, tiles_c, s.N, G::TH), a);
+    LaneQ lq = lane_at<KS>(a, cur, wave, n);
     fetch_rows(a.k, cur, lq);
     fetch_q(cur, lq);
     s16x8 qreg[G::DS];
@@ -318,11 +390,11 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
 
         const int tn = sched_peek(sc);
         const bool more = tn < sc.t_end;
-        Tile nxt = cur;
+        ATile nxt = cur;
         LaneQ lqn = lq;
         if (more) {
-            nxt = tile_of(tn, tiles_r, tiles_c, s.N, G::TH);
-            lqn = lane_query<KS>(nxt, s, wave, n);
+            nxt = in_sub(tile_of(tn, tiles_r, tiles_c, s.N, G::TH), a);
+            lqn = lane_at<KS>(a, nxt, wave, n);
             fetch_rows(a.k, nxt, lqn);
             fetch_q(nxt, lqn);
         } else {
@@ -344,7 +416,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                         cat(lds_read_tr(G::t_at(vp[0], mt)), lds_read_tr(G::t_at(vp[1], mt))), pb[ks],
                         o[mt]);
             }
-            store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(const_cast<short *>(image<short>(a.o, cur)) + lq.qr * a.o.sh + lq.qc * a.o.sw,
+            store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(const_cast<short *>(image_at(a, a.o, cur)) + lq.qr * row_step(a, a.o) + lq.qc * col_step(a, a.o),
                                g, o, 1.f / sum, lq.live, dlim);
             if (a.lse && (FULL || (lq.live && g == 0)))
                 a.lse[lq.tok] = (mx + __builtin_amdgcn_logf(sum)) * kLn2;
@@ -378,7 +450,7 @@ constexpr int kDqWaves = D == 32 && (KS == 7 || KS == 9) && NW == 4 ? 3 : Geo<D,
 // FULL: as in fwd_mfma (no wave switched off, no store predicated, the staged rows go to LDS at
 // the end of a tile's pass through the loop).
 template <bool BF, int D, int KS, bool FRAME, bool ROLL, int NW = 4, bool FULL = false>
-__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void bwd_dq_mfma(BwdArgs a, TileSet ts, int ntiles, Runs rp) {
+__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void bwd_dq_mfma(BArgs a, TileSet ts, int ntiles, Runs rp) {
     // (the dK/dV pass that follows on the stream counts its frame tiles here, from zero)
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv) *reinterpret_cast<int *>(a.zinv) = 0;
     using G = Geo<D, KS, NW>;
@@ -397,9 +469,9 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
     const int l = threadIdx.x & 63, n = l & 15, g = l >> 4;
     const float sc2 = s.scale * kLog2e;
     auto pick = [&](int t) __attribute__((always_inline)) {
-        if constexpr (FRAME) return frame_tile(t, ts, s.N);
-        else if constexpr (ROLL) return tile_of_cm(t, ts.tiles_r, ts.tiles_c, s.N);
-        else return tile_of(t, ts.tiles_r, ts.tiles_c, s.N, G::TH);
+        if constexpr (FRAME) return in_sub(frame_tile(t, ts, s.N), a);
+        else if constexpr (ROLL) return in_sub(tile_of_cm(t, ts.tiles_r, ts.tiles_c, s.N), a);
+        else return in_sub(tile_of(t, ts.tiles_r, ts.tiles_c, s.N, G::TH), a);
     };
 
     const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim);
@@ -407,21 +479,21 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
     s16x8 qnext[G::DS], gnext[G::DS];
     float lse_next = 0.f;
     // rows [y0, y0 + nr) of the halo are what LDS does not hold yet
-    auto prefetch = [&](const Tile &tl, const LaneQ &lq, int y0, int nr) __attribute__((always_inline)) {
+    auto prefetch = [&](const ATile &tl, const LaneQ &lq, int y0, int nr) __attribute__((always_inline)) {
         if constexpr (ROLL) {
-            halo_fetch_rows<D, KS>(kst, plan, image<short>(a.k, tl), a.k.sh, a.k.sw, y0, lq.hc0, nr, s.H, s.W);
-            halo_fetch_rows<D, KS>(vst, plan, image<short>(a.v, tl), a.v.sh, a.v.sw, y0, lq.hc0, nr, s.H, s.W);
+            halo_fetch_rows<D, KS>(kst, plan, image_at(a, a.k, tl), row_step(a, a.k), col_step(a, a.k), y0, lq.hc0, nr, s.H, s.W);
+            halo_fetch_rows<D, KS>(vst, plan, image_at(a, a.v, tl), row_step(a, a.v), col_step(a, a.v), y0, lq.hc0, nr, s.H, s.W);
         } else {
-            halo_fetch<D, KS>(kst, plan, image<short>(a.k, tl), a.k.sh, a.k.sw, lq.hr0, lq.hc0, s.H, s.W);
-            halo_fetch<D, KS>(vst, plan, image<short>(a.v, tl), a.v.sh, a.v.sw, lq.hr0, lq.hc0, s.H, s.W);
+            halo_fetch<D, KS>(kst, plan, image_at(a, a.k, tl), row_step(a, a.k), col_step(a, a.k), lq.hr0, lq.hc0, s.H, s.W);
+            halo_fetch<D, KS>(vst, plan, image_at(a, a.v, tl), row_step(a, a.v), col_step(a, a.v), lq.hr0, lq.hc0, s.H, s.W);
         }
-        load_row_chunks(qnext, image<short>(a.q, tl) + lq.qr * a.q.sh + lq.qc * a.q.sw, g, dlim);
-        load_row_chunks(gnext, image<short>(a.d_o, tl) + lq.qr * a.d_o.sh + lq.qc * a.d_o.sw, g, dlim);
+        load_row_chunks(qnext, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
+        load_row_chunks(gnext, image_at(a, a.d_o, tl) + lq.qr * row_step(a, a.d_o) + lq.qc * col_step(a, a.d_o), g, dlim);
         lse_next = a.lse[lq.tok];
     };
 
-    Tile cur = pick(sc.t);
-    LaneQ lq = lane_query<KS>(cur, s, wave, n);
+    ATile cur = pick(sc.t);
+    LaneQ lq = lane_at<KS>(a, cur, wave, n);
     int y0 = lq.hr0, nr = G::HR;
     prefetch(cur, lq, y0, nr);
     s16x8 qreg[G::DS], greg[G::DS];
@@ -449,11 +521,11 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
 
         const int tn = sched_peek(sc);
         const bool more = tn < sc.t_end;
-        Tile nxt = cur;
+        ATile nxt = cur;
         LaneQ lqn = lq;
         if (more) {
             nxt = pick(tn);
-            lqn = lane_query<KS>(nxt, s, wave, n);
+            lqn = lane_at<KS>(a, nxt, wave, n);
             // the tile below in the same image keeps the rows the two halos share
             const bool below = ROLL && nxt.bb == cur.bb && nxt.nn == cur.nn && nxt.c0 == cur.c0 &&
                                nxt.r0 > cur.r0 && lqn.hr0 < lq.hr0 + G::HR;
@@ -535,7 +607,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                         dq[mt]);
             }
 
-            store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(static_cast<short *>(a.dq) + a.grad_at(cur.bb, cur.nn, lq.qr, lq.qc), g, dq, s.scale, lq.live, dlim);
+            store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale, lq.live, dlim);
             if (FULL || (lq.live && g == 0)) a.delta[lq.tok] = delta;
         }
 
@@ -570,7 +642,7 @@ template <int D, int KS, int NW>
 constexpr int kDq2Tail = D == 128 && NW == 8 ? (KS == 13 ? 15 : KS == 11 ? 13 : 0) : 0;
 // FULL: as in fwd_mfma.
 template <bool BF, int D, int KS, int NW = 4, bool FULL = false>
-__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS> : 1)) void bwd_dq2_mfma(BwdArgs a, TileSet ts, int ntiles) {
+__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS> : 1)) void bwd_dq2_mfma(BArgs a, TileSet ts, int ntiles) {
     // (the dK/dV pass that follows on the stream counts its frame tiles here, from zero)
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv) *reinterpret_cast<int *>(a.zinv) = 0;
     using G = Geo<D, KS, NW>;
@@ -593,23 +665,23 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     // The last TAIL chunks of a halo are loaded when the arithmetic of the phase is over
     // (fetch_tail): where the registers do not hold a whole halo beside it.
     constexpr int TAIL = kDq2Tail<D, KS, NW>, HEAD = G::NL - TAIL;
-    auto fetch_rows = [&](const View &vw, const Tile &tl, const LaneQ &lq) __attribute__((always_inline)) {
-        halo_fetch<D, KS, NW, 1, 0, HEAD>(st, plan, image<short>(vw, tl), vw.sh, vw.sw, lq.hr0, lq.hc0, s.H, s.W);
+    auto fetch_rows = [&](const View &vw, const ATile &tl, const LaneQ &lq) __attribute__((always_inline)) {
+        halo_fetch<D, KS, NW, 1, 0, HEAD>(st, plan, image_at(a, vw, tl), row_step(a, vw), col_step(a, vw), lq.hr0, lq.hc0, s.H, s.W);
     };
-    auto fetch_tail = [&](const View &vw, const Tile &tl, const LaneQ &lq) __attribute__((always_inline)) {
+    auto fetch_tail = [&](const View &vw, const ATile &tl, const LaneQ &lq) __attribute__((always_inline)) {
         if constexpr (TAIL > 0)
-            halo_fetch<D, KS, NW, 1, HEAD, G::NL>(st, plan, image<short>(vw, tl), vw.sh, vw.sw, lq.hr0, lq.hc0, s.H, s.W);
+            halo_fetch<D, KS, NW, 1, HEAD, G::NL>(st, plan, image_at(a, vw, tl), row_step(a, vw), col_step(a, vw), lq.hr0, lq.hc0, s.H, s.W);
     };
-    auto fetch_do = [&](const Tile &tl, const LaneQ &lq) __attribute__((always_inline)) {
-        load_row_chunks(gnext, image<short>(a.d_o, tl) + lq.qr * a.d_o.sh + lq.qc * a.d_o.sw, g, dlim);
+    auto fetch_do = [&](const ATile &tl, const LaneQ &lq) __attribute__((always_inline)) {
+        load_row_chunks(gnext, image_at(a, a.d_o, tl) + lq.qr * row_step(a, a.d_o) + lq.qc * col_step(a, a.d_o), g, dlim);
     };
-    auto fetch_q = [&](const Tile &tl, const LaneQ &lq) __attribute__((always_inline)) {
-        load_row_chunks(qreg, image<short>(a.q, tl) + lq.qr * a.q.sh + lq.qc * a.q.sw, g, dlim);
+    auto fetch_q = [&](const ATile &tl, const LaneQ &lq) __attribute__((always_inline)) {
+        load_row_chunks(qreg, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
         lse_cur = a.lse[lq.tok];
     };
 
-    Tile cur = tile_of(sc.t, ts.tiles_r, ts.tiles_c, s.N, G::TH);
-    LaneQ lq = lane_query<KS>(cur, s, wave, n);
+    ATile cur = in_sub(tile_of(sc.t, ts.tiles_r, ts.tiles_c, s.N, G::TH), a);
+    LaneQ lq = lane_at<KS>(a, cur, wave, n);
     fetch_rows(a.v, cur, lq);
     fetch_tail(a.v, cur, lq);
     fetch_do(cur, lq);
@@ -648,11 +720,11 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
 
         const int tn = sched_peek(sc);
         const bool more = tn < sc.t_end;
-        Tile nxt = cur;
+        ATile nxt = cur;
         LaneQ lqn = lq;
         if (more) {
-            nxt = tile_of(tn, ts.tiles_r, ts.tiles_c, s.N, G::TH);
-            lqn = lane_query<KS>(nxt, s, wave, n);
+            nxt = in_sub(tile_of(tn, ts.tiles_r, ts.tiles_c, s.N, G::TH), a);
+            lqn = lane_at<KS>(a, nxt, wave, n);
             fetch_rows(a.v, nxt, lqn);
             fetch_do(nxt, lqn);
         } else {
@@ -700,7 +772,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                         cat(lds_read_tr(G::t_at(kp[0], mt)), lds_read_tr(G::t_at(kp[1], mt))), dsb[ks],
                         dq[mt]);
             }
-            store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(static_cast<short *>(a.dq) + a.grad_at(cur.bb, cur.nn, lq.qr, lq.qc), g, dq, s.scale, lq.live, dlim);
+            store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale, lq.live, dlim);
             if (FULL || (lq.live && g == 0)) a.delta[lq.tok] = delta;
         }
         if (more) fetch_tail(a.v, nxt, lqn);
@@ -730,7 +802,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
 //   dV^T += dO^T P, dK^T += Q^T dS    (dO, Q read back from LDS transposed)
 struct KeyBlock {
     int t;                // tile
-    Tile tl;
+    ATile tl;
     int qa, qb, ca, cb;   // queries that attend to any key of the tile
     int br, bc;           // origin of the staged block of queries
     bool first, last;     // first / last block of its tile
@@ -756,7 +828,7 @@ __device__ __forceinline__ bool next_block(KeyBlock &b) {
 // queries, a wave's queries are the (4+k-1)^2 halo of its 4x4 keys at a fixed
 // place in it, and the mask depends on the lane only.
 template <bool BF, int D, int KS, bool ROLL, int SP, int PART>
-__device__ __forceinline__ void dkdv_inner(const BwdArgs &a, const TileSet &ts, int ntiles, Runs rp,
+__device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, int ntiles, Runs rp,
                                            int block, int nblocks, short *lds_q, short *lds_g,
                                            float2 *lds_stat, f32x4 *lds_red) {
     using G = Geo<D, KS, 4, SP>;
@@ -783,22 +855,22 @@ __device__ __forceinline__ void dkdv_inner(const BwdArgs &a, const TileSet &ts, 
         return ROLL ? G::token_row_rot(tile, x, orow, ocol, rot) : G::token_row(tile, x, orow, ocol);
     };
     auto pick = [&](int t) __attribute__((always_inline)) {
-        return ROLL ? inner_tile_cm(t, ts, s.N) : inner_tile(t, ts, s.N);
+        return in_sub(ROLL ? inner_tile_cm(t, ts, s.N) : inner_tile(t, ts, s.N), a);
     };
 
     const HaloPlan<D, KS, 4, SP> plan = make_plan<D, KS, 4, SP>(dlim);
     HaloRegs<D, KS, 4, SP> qst, gst;
     float2 sst[G::NST];
     // ROLL: rows [y0, y0 + nr) of the block are what LDS does not hold yet
-    auto prefetch = [&](const Tile &tl, int y0, int nr) __attribute__((always_inline)) {
-        const int64_t img_tok = ((int64_t)tl.bb * s.N + tl.nn) * s.H * (int64_t)s.W;
+    auto prefetch = [&](const ATile &tl, int y0, int nr) __attribute__((always_inline)) {
+        const int64_t img_tok = image_token(a, tl);
         const int br = tl.r0 - KS / 2, bc = tl.c0 - KS / 2;
         if constexpr (ROLL) {
-            halo_fetch_rows<D, KS>(qst, plan, image<short>(a.q, tl), a.q.sh, a.q.sw, y0, bc, nr, s.H, s.W);
-            halo_fetch_rows<D, KS>(gst, plan, image<short>(a.d_o, tl), a.d_o.sh, a.d_o.sw, y0, bc, nr, s.H, s.W);
+            halo_fetch_rows<D, KS>(qst, plan, image_at(a, a.q, tl), row_step(a, a.q), col_step(a, a.q), y0, bc, nr, s.H, s.W);
+            halo_fetch_rows<D, KS>(gst, plan, image_at(a, a.d_o, tl), row_step(a, a.d_o), col_step(a, a.d_o), y0, bc, nr, s.H, s.W);
         } else {
-            halo_fetch<D, KS>(qst, plan, image<short>(a.q, tl), a.q.sh, a.q.sw, br, bc, s.H, s.W);
-            halo_fetch<D, KS>(gst, plan, image<short>(a.d_o, tl), a.d_o.sh, a.d_o.sw, br, bc, s.H, s.W);
+            halo_fetch<D, KS>(qst, plan, image_at(a, a.q, tl), row_step(a, a.q), col_step(a, a.q), br, bc, s.H, s.W);
+            halo_fetch<D, KS>(gst, plan, image_at(a, a.d_o, tl), row_step(a, a.d_o), col_step(a, a.d_o), br, bc, s.H, s.W);
         }
 #pragma unroll
         for (int i = 0; i < G::NST; i++) {
@@ -839,13 +911,13 @@ __device__ __forceinline__ void dkdv_inner(const BwdArgs &a, const TileSet &ts, 
     // the previous tile's math is over (they would not fit beside it) and complete
     // before the barrier below, i.e. before any newer load is in flight.
     s16x8 kreg[G::DS], vreg[G::DS];
-    auto load_keys = [&](const Tile &tl) __attribute__((always_inline)) {
+    auto load_keys = [&](const ATile &tl) __attribute__((always_inline)) {
         const int kr = tl.r0 + orow + (n >> 2), kc = tl.c0 + ocol + (n & 3);
-        load_row_chunks(kreg, image<short>(a.k, tl) + kr * a.k.sh + kc * a.k.sw, g, dlim);
-        load_row_chunks(vreg, image<short>(a.v, tl) + kr * a.v.sh + kc * a.v.sw, g, dlim);
+        load_row_chunks(kreg, image_at(a, a.k, tl) + kr * row_step(a, a.k) + kc * col_step(a, a.k), g, dlim);
+        load_row_chunks(vreg, image_at(a, a.v, tl) + kr * row_step(a, a.v) + kc * col_step(a, a.v), g, dlim);
     };
 
-    Tile cur = pick(sc.t);
+    ATile cur = pick(sc.t);
     int y0 = cur.r0 - KS / 2, nr = G::HR;
     prefetch(cur, y0, nr);
     load_keys(cur);
@@ -857,7 +929,7 @@ __device__ __forceinline__ void dkdv_inner(const BwdArgs &a, const TileSet &ts, 
 
         const int tn = sched_peek(sc);
         const bool more = tn < sc.t_end;
-        Tile nxt = cur;
+        ATile nxt = cur;
         if (ROLL) rot = (cur.r0 - KS / 2) % G::HR;
         if (more) {
             nxt = pick(tn);
@@ -915,7 +987,7 @@ __device__ __forceinline__ void dkdv_inner(const BwdArgs &a, const TileSet &ts, 
         }
 
         const int kr = cur.r0 + orow + (n >> 2), kc = cur.c0 + ocol + (n & 3);
-        const int64_t goff = a.grad_at(cur.bb, cur.nn, kr, kc);
+        const int64_t goff = grad_of(a, cur, kr, kc);
         if constexpr (SP == 1) {
             store_token<BF, D, kInnerLines<D>, true>(static_cast<short *>(a.dk) + goff, g, dk, s.scale, true, dlim);
             store_token<BF, D, kInnerLines<D>, true>(static_cast<short *>(a.dv) + goff, g, dv, 1.f, true, dlim);
@@ -959,7 +1031,7 @@ __device__ __forceinline__ void dkdv_inner(const BwdArgs &a, const TileSet &ts, 
 // one block instead of up to four.  `lds_red` then lies over the staged rows (RED_OVER):
 // the partial sums are exchanged when a tile's last block has been read by every wave.
 template <bool BF, int D, int KS, int SP, int KSG, bool RED_OVER>
-__device__ __forceinline__ void dkdv_frame(const BwdArgs &a, const TileSet &ts, int ntiles,
+__device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, int ntiles,
                                            int block, int nblocks, short *lds_q, short *lds_g,
                                            float4 *lds_stat, f32x4 *lds_red, int *tile_ctr, int *lds_tile) {
     using G = Geo<D, KSG, 4, SP>;
@@ -995,14 +1067,14 @@ __device__ __forceinline__ void dkdv_frame(const BwdArgs &a, const TileSet &ts, 
     HaloRegs<D, KSG, 4, SP> qst, gst;
     float2 sst[G::NST];
     // the wave's 4x4 keys of a tile: this lane's key pixel (clamped into the image)
-    auto key_of = [&](const Tile &tl, int &kr, int &kc) __attribute__((always_inline)) {
+    auto key_of = [&](const ATile &tl, int &kr, int &kc) __attribute__((always_inline)) {
         kr = min(tl.r0 + (wave >> 1) * 4 + (n >> 2), s.H - 1);
         kc = min(tl.c0 + (wave & 1) * 4 + (n & 3), s.W - 1);
     };
     auto stage = [&](const KeyBlock &b) __attribute__((always_inline)) {
-        const int64_t img_tok = ((int64_t)b.tl.bb * s.N + b.tl.nn) * s.H * (int64_t)s.W;
-        halo_fetch<D, KSG>(qst, plan, image<short>(a.q, b.tl), a.q.sh, a.q.sw, b.br, b.bc, b.qb, b.cb);
-        halo_fetch<D, KSG>(gst, plan, image<short>(a.d_o, b.tl), a.d_o.sh, a.d_o.sw, b.br, b.bc, b.qb, b.cb);
+        const int64_t img_tok = image_token(a, b.tl);
+        halo_fetch<D, KSG>(qst, plan, image_at(a, a.q, b.tl), row_step(a, a.q), col_step(a, a.q), b.br, b.bc, b.qb, b.cb);
+        halo_fetch<D, KSG>(gst, plan, image_at(a, a.d_o, b.tl), row_step(a, a.d_o), col_step(a, a.d_o), b.br, b.bc, b.qb, b.cb);
 #pragma unroll
         for (int i = 0; i < G::NST; i++) {
             const int id = threadIdx.x + i * G::NT;
@@ -1013,16 +1085,16 @@ __device__ __forceinline__ void dkdv_frame(const BwdArgs &a, const TileSet &ts, 
     };
     // B operands of the tile: this lane's key, channels ds*32 + g*8 ..
     s16x8 kreg[G::DS], vreg[G::DS];
-    auto load_keys = [&](const Tile &tl) __attribute__((always_inline)) {
+    auto load_keys = [&](const ATile &tl) __attribute__((always_inline)) {
         int kr, kc;
         key_of(tl, kr, kc);
-        load_row_chunks(kreg, image<short>(a.k, tl) + kr * a.k.sh + kc * a.k.sw, g, dlim);
-        load_row_chunks(vreg, image<short>(a.v, tl) + kr * a.v.sh + kc * a.v.sw, g, dlim);
+        load_row_chunks(kreg, image_at(a, a.k, tl) + kr * row_step(a, a.k) + kc * col_step(a, a.k), g, dlim);
+        load_row_chunks(vreg, image_at(a, a.v, tl) + kr * row_step(a, a.v) + kc * col_step(a, a.v), g, dlim);
     };
     auto first_of = [&](int t) __attribute__((always_inline)) {
         KeyBlock b;
         b.t = t;
-        b.tl = frame_tile(t, ts, s.N);
+        b.tl = in_sub(frame_tile(t, ts, s.N), a);
         b.qa = inv_lo(b.tl.r0, KS);
         b.qb = inv_hi(min(b.tl.r0 + 8, s.H) - 1, s.H, KS);
         b.ca = inv_lo(b.tl.c0, KS);
@@ -1145,7 +1217,7 @@ __device__ __forceinline__ void dkdv_frame(const BwdArgs &a, const TileSet &ts, 
         if (dyn && cur.first && threadIdx.x == 0) lds_tile[0] = fetched;
         const bool live = (wr0 + (n >> 2) < s.H) && (wc0 + (n & 3) < s.W);
         auto store = [&]() __attribute__((always_inline)) {
-            const int64_t goff = a.grad_at(cur.tl.bb, cur.tl.nn, kr, kc);
+            const int64_t goff = grad_of(a, cur.tl, kr, kc);
             store_token<BF, D, kLineStores<D, KS, fits<D, KS>() ? Geo<D, KS, 4, SP>::WAVES : 1>>(static_cast<short *>(a.dk) + goff, g, dk, s.scale, live, dlim);
             store_token<BF, D, kLineStores<D, KS, fits<D, KS>() ? Geo<D, KS, 4, SP>::WAVES : 1>>(static_cast<short *>(a.dv) + goff, g, dv, 1.f, live, dlim);
         };
@@ -1208,7 +1280,7 @@ constexpr int kDkdvWaves =
     SP == 1 && D <= 64 && 3 * (Geo<D, KS>::LDS_BYTES + 2048) <= 160 * 1024 ? 3 : Geo<D, KS, 4, SP>::WAVES;
 template <bool BF, int D, int KS, bool ROLL, int SP = 1>
 __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) void bwd_dkdv_mfma(
-    BwdArgs a, TileSet ts, int n_inner, int n_frame, int inner_blocks, Runs rp, int dyn) {
+    BArgs a, TileSet ts, int n_inner, int n_frame, int inner_blocks, Runs rp, int dyn) {
     using G = Geo<D, KS, 4, SP>;
     using FG = Geo<D, kFrameKS<D, KS, SP>, 4, SP>;  // blocks of the frame body
     // One LDS buffer, laid out by each body for itself: staged Q rows, staged dO rows,
@@ -1338,15 +1410,15 @@ template <int D, int KS>
 constexpr int kDkdvSplit = D == 64 && Geo<D, KS>::WAVES == 1 ? 2 : 1;
 
 template <bool BF, int D, int KS>
-int fwd_launch(const FwdArgs &a, hipStream_t st) {
+int fwd_launch(const FArgs &a, hipStream_t st) {
     if constexpr (kBuilt<D, KS>) {
         using G = Geo<D, KS>;
         const int tiles_r = (a.s.H + G::TH - 1) / G::TH, tiles_c = (a.s.W + G::TW - 1) / G::TW;
-        const int64_t nb = (int64_t)a.s.B * a.s.N * tiles_r * tiles_c;
+        const int64_t nb = images_of(a) * tiles_r * tiles_c;
         if constexpr (kTallBuilt<D, KS>) {
             using G8 = Geo<D, KS, 8>;
             const int tall_r = (a.s.H + G8::TH - 1) / G8::TH;
-            const int64_t nb8 = (int64_t)a.s.B * a.s.N * tall_r * tiles_c;
+            const int64_t nb8 = images_of(a) * tall_r * tiles_c;
             if (nb8 >= 512) {  // enough tall tiles for every CU to have a few
                 const int grid = persistent_grid<fwd_mfma<BF, D, KS, false, 8>>(nb8, G8::NT);
                 ProfScope prof(ENATTEN_KERNEL_FWD, "fwd_mfma", st);
@@ -1362,7 +1434,7 @@ int fwd_launch(const FwdArgs &a, hipStream_t st) {
         if constexpr (kFwd2TallBuilt<D, KS>) {
             using G8 = Geo<D, KS, 8>;
             const int tall_r = (a.s.H + G8::TH - 1) / G8::TH;
-            const int64_t nb8 = (int64_t)a.s.B * a.s.N * tall_r * tiles_c;
+            const int64_t nb8 = images_of(a) * tall_r * tiles_c;
             if (nb8 >= 256) {  // a tile for every CU
                 const int grid = persistent_grid<fwd2_mfma<BF, D, KS, 8>>(nb8, G8::NT);
                 ProfScope prof(ENATTEN_KERNEL_FWD, "fwd2_mfma", st);
@@ -1422,11 +1494,11 @@ template <int D, int KS>
 constexpr bool kDq2Full = !kNarrow && (D != 128 || KS == 7 || KS == 11);
 
 template <bool BF, int D, int KS>
-int bwd_launch(const BwdArgs &a, int path, hipStream_t st) {
+int bwd_launch(const BArgs &a, int path, hipStream_t st) {
     if constexpr (kBuilt<D, KS>) {
         using G = Geo<D, KS>;
         const int tiles_r = (a.s.H + G::TH - 1) / G::TH, tiles_c = (a.s.W + G::TW - 1) / G::TW;
-        const int64_t nb = (int64_t)a.s.B * a.s.N * tiles_r * tiles_c;
+        const int64_t nb = images_of(a) * tiles_r * tiles_c;
         // inner tiles (no key or query within reach of the border) and frame
         TileSet ts;
         ts.tiles_r = tiles_r; ts.tiles_c = tiles_c;
@@ -1438,13 +1510,13 @@ int bwd_launch(const BwdArgs &a, int path, hipStream_t st) {
         if (ts.ni_r <= 0 || ts.ni_c <= 0 || kDkdvFrameOnly<D, KS>) {
             ts.ir0 = tiles_r; ts.ic0 = 0; ts.ni_r = 0; ts.ni_c = 0;
         }
-        const int64_t slabs = (int64_t)a.s.B * a.s.N;
+        const int64_t slabs = images_of(a);
         const int64_t n_inner = slabs * ts.ni_r * ts.ni_c, n_frame = nb - n_inner;
 
         // The fused backward wherever it is built (fused_bwd_supported): 5-25% faster than the
         // two passes at every size measured, from B64 N16 8x8 (45.7 against 47.3 us) and B4 N4
         // 32x32 (14.8 against 24.1) to B16 N8 128x128 (938 against 1174).
-        if (!split_forced(path) && fused_bwd_supported(a)) {
+        if (!kSub && !split_forced(path) && fused_bwd_supported(a)) {
             const int rc = launch_bwd_fused(a, BF, ts, nb, st);
             return rc ? rc : check_launch("enatten2d_bwd");
         }
@@ -1461,7 +1533,7 @@ int bwd_launch(const BwdArgs &a, int path, hipStream_t st) {
         // 56x56 52.7 vs 49.0.  So it is the default only where at most one tile in eight is an
         // inner tile (level with the two passes there, one launch less);
         // ENATTEN_PATH_MFMA_FUSED forces it wherever it is built.
-        if (!split_forced(path) && onepass_bwd_supported(a) &&
+        if (!kSub && !split_forced(path) && onepass_bwd_supported(a) &&
             (path == ENATTEN_PATH_MFMA_FUSED || 8 * n_inner <= nb)) {
             const int rc = launch_bwd_onepass(a, BF, ts, nb, st);
             return rc ? rc : check_launch("enatten2d_bwd");
@@ -1650,7 +1722,7 @@ bool fits_rt(int D, int ks) {
 
 // The launchers' common body: tensors whose rows the 16-byte loads cannot take go to the
 // general kernels, everything else to the kernel built for its head dim and kernel size.
-int fwd_dispatch(const FwdArgs &a, int dtype, hipStream_t st) {
+int fwd_dispatch(const FArgs &a, int dtype, hipStream_t st) {
     if (!layout_ok(a.q) || !layout_ok(a.k) || !layout_ok(a.v) || !layout_ok(a.o))
         return launch_fwd_simt(a, dtype, st);  // 16-byte loads need aligned rows
     if (dtype == ENATTEN_BF16) {
@@ -1662,7 +1734,7 @@ int fwd_dispatch(const FwdArgs &a, int dtype, hipStream_t st) {
     return ENATTEN_EUNSUPPORTED;
 }
 
-int bwd_dispatch(const BwdArgs &a, int dtype, int path, hipStream_t st) {
+int bwd_dispatch(const BArgs &a, int dtype, int path, hipStream_t st) {
     auto al = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
     const bool grads_ok = a.gsb % 8 == 0 && a.gsn % 8 == 0 && a.gsh % 8 == 0 && a.gsw % 8 == 0;
     if (!layout_ok(a.q) || !layout_ok(a.k) || !layout_ok(a.v) || !layout_ok(a.o) ||

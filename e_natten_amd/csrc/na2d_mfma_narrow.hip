@@ -8,6 +8,7 @@
 namespace enatten {
 namespace {
 constexpr bool kNarrow = true;
+constexpr bool kSub = false;
 }
 }  // namespace enatten
 

@@ -228,6 +228,70 @@ struct NattenFn : public torch::autograd::Function<NattenFn<TWO_D>> {
     }
 };
 
+// Dilated neighborhoods: the contract of enatten2d_fwd_dilated, with an autograd node of its own.
+// The output is contiguous.
+void validate_dilation(const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks, int64_t dil) {
+    validate("enatten::natten2d_dilated", q, k, v, ks, 5);
+    TORCH_CHECK_VALUE(dil >= 1, "enatten::natten2d_dilated: dilation must be >= 1, got ", dil);
+    TORCH_CHECK(q.is_cuda(), "enatten::natten2d_dilated: tensors must be on the GPU; this build has no CPU path");
+}
+std::tuple<Tensor, Tensor> dilated_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, int64_t ks,
+                                       double scale, int64_t dil) {
+    validate_dilation(q_, k_, v_, ks, dil);
+    const c10::DeviceGuard guard(q_.device());
+    const Tensor q = kernel_layout(q_), k = kernel_layout(k_), v = kernel_layout(v_);
+    const int B = q.size(0), N = q.size(1), H = q.size(2), W = q.size(3), D = q.size(4);
+    Tensor o = at::empty(q.sizes(), q.options());
+    Tensor lse = at::empty({B, N, H, W}, q.options().dtype(at::kFloat));
+    check_rc(enatten2d_fwd_dilated(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+                                   lse.data_ptr<float>(), B, N, H, W, D, (int)ks, (int)dil, dtype_code(q),
+                                   q.strides().data(), k.strides().data(), v.strides().data(), nullptr,
+                                   (float)scale, c10::hip::getCurrentHIPStream().stream()));
+    return {o, lse};
+}
+struct DilatedFn : public torch::autograd::Function<DilatedFn> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v,
+                          int64_t ks, double scale, int64_t dil) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        Tensor o, lse;
+        std::tie(o, lse) = dilated_fwd(q, k, v, ks, scale, dil);
+        ctx->save_for_backward({q, k, v, o, lse});
+        ctx->saved_data["kernel_size"] = ks;
+        ctx->saved_data["scale"] = scale;
+        ctx->saved_data["dilation"] = dil;
+        return o;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const int64_t ks = ctx->saved_data["kernel_size"].toInt(), dil = ctx->saved_data["dilation"].toInt();
+        const double scale = ctx->saved_data["scale"].toDouble();
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::DeviceGuard guard(s[0].device());
+        check_bwd_extras("enatten::natten2d_dilated", s[0], s[3], grads[0]);
+        const Tensor q = kernel_layout(s[0]), k = kernel_layout(s[1]), v = kernel_layout(s[2]);
+        const Tensor &o = s[3], &lse = s[4], d_o = kernel_layout(grads[0]);
+        const int B = q.size(0), N = q.size(1), H = q.size(2), W = q.size(3), D = q.size(4);
+        Tensor dq = at::empty(q.sizes(), q.options());
+        Tensor dk = at::empty_like(dq), dv = at::empty_like(dq);
+        Tensor ws = at::empty({(int64_t)enatten2d_bwd_dilated_workspace_bytes(B, N, H, W, dtype_code(q))},
+                              q.options().dtype(at::kByte));
+        check_rc(enatten2d_bwd_dilated(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr<float>(),
+            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), B, N, H, W, D, (int)ks, (int)dil,
+            dtype_code(q), q.strides().data(), k.strides().data(), v.strides().data(), o.strides().data(),
+            d_o.strides().data(), (float)scale, c10::hip::getCurrentHIPStream().stream()));
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor()};
+    }
+};
+Tensor natten2d_dilated_autograd(const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks,
+                                 double scale, int64_t dil) {
+    return DilatedFn::apply(q, k, v, ks, scale, dil);
+}
+Tensor natten2d_dilated_plain(const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks,
+                              double scale, int64_t dil) {
+    return std::get<0>(dilated_fwd(q, k, v, ks, scale, dil));
+}
+
 Tensor natten2d_autograd(const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks,
                          double scale) {
     return NattenFn<true>::apply(q, k, v, ks, scale);
@@ -253,6 +317,7 @@ TORCH_LIBRARY(enatten, m) {
     m.def("na1d_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor d_o, "
           "int kernel_size, float scale) -> (Tensor, Tensor, Tensor)");
     m.def("natten2d(Tensor q, Tensor k, Tensor v, int kernel_size=7, float scale=1.0) -> Tensor");
+    m.def("natten2d_dilated(Tensor q, Tensor k, Tensor v, int kernel_size, float scale, int dilation) -> Tensor");
     m.def("natten1d(Tensor q, Tensor k, Tensor v, int kernel_size=7, float scale=1.0) -> Tensor");
 }
 
@@ -262,10 +327,12 @@ TORCH_LIBRARY_IMPL(enatten, CompositeExplicitAutograd, m) {
     m.impl("na1d_fwd", &na1d_fwd);
     m.impl("na1d_bwd", &na1d_bwd);
     m.impl("natten2d", &natten2d_plain);
+    m.impl("natten2d_dilated", &natten2d_dilated_plain);
     m.impl("natten1d", &natten1d_plain);
 }
 
 TORCH_LIBRARY_IMPL(enatten, Autograd, m) {
     m.impl("natten2d", &natten2d_autograd);
+    m.impl("natten2d_dilated", &natten2d_dilated_autograd);
     m.impl("natten1d", &natten1d_autograd);
 }

@@ -85,9 +85,7 @@ def _check(rc: int) -> None:
         raise (ValueError if rc == 1 else RuntimeError)(msg)
 
 
-def _fwd_impl(q, k, v, kernel_size: int, scale: float, out=None):
-    """`out`: a view of the shape of q with unit stride on the channels that the kernels
-    write in place (the strided sub-grid of a dilated call); None allocates the output."""
+def _fwd_impl(q, k, v, kernel_size: int, scale: float):
     _validate(q, k, v, kernel_size)
     _require_gpu(q, "enatten::na2d_fwd")
     lib = _lib.load()
@@ -97,7 +95,7 @@ def _fwd_impl(q, k, v, kernel_size: int, scale: float, out=None):
         # like the reference's zeros_like(Q) (e_natten/triton.py:502), the output takes
         # the memory order of q: for q sliced out of a [B, H, W, 3, heads, d] projection
         # that is [B, H, W, heads, d], which the following merge of heads needs
-        o = _kernel_layout(torch.empty_like(q)) if out is None else out
+        o = _kernel_layout(torch.empty_like(q))
         lse = torch.empty((B, N, H, W), dtype=torch.float32, device=q.device)
         _check(lib.enatten2d_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                                  lse.data_ptr(), B, N, H, W, D, kernel_size, _DTYPES[q.dtype],
@@ -106,9 +104,7 @@ def _fwd_impl(q, k, v, kernel_size: int, scale: float, out=None):
     return o, lse
 
 
-def _bwd_impl(q, k, v, o, lse, d_o, kernel_size: int, scale: float, out=None):
-    """`out`: (dq, dk, dv) views of one layout (unit stride on the channels) that the kernels
-    write in place (the strided sub-grids of a dilated call); None allocates them."""
+def _bwd_impl(q, k, v, o, lse, d_o, kernel_size: int, scale: float):
     _validate(q, k, v, kernel_size)
     _require_gpu(q, "enatten::na2d_bwd")
     if d_o.shape != q.shape or o.shape != q.shape:
@@ -120,22 +116,17 @@ def _bwd_impl(q, k, v, o, lse, d_o, kernel_size: int, scale: float, out=None):
     lse = lse.contiguous()
     B, N, H, W, D = q.shape
     with torch.cuda.device(q.device):
-        if out is None:
-            dq = torch.empty((B, N, H, W, D), dtype=q.dtype, device=q.device)
-            dk, dv = torch.empty_like(dq), torch.empty_like(dq)
-        else:
-            dq, dk, dv = out
-            assert dq.stride() == dk.stride() == dv.stride() and dq.stride(-1) == 1
+        dq = torch.empty((B, N, H, W, D), dtype=q.dtype, device=q.device)
+        dk, dv = torch.empty_like(dq), torch.empty_like(dq)
         ws = torch.empty(lib.enatten2d_bwd_workspace_bytes(B, N, H, W, D, kernel_size,
                                                             _DTYPES[q.dtype]),
                          dtype=torch.uint8, device=q.device)
-        _check(lib.enatten2d_bwd_into(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                                      d_o.data_ptr(), lse.data_ptr(), dq.data_ptr(), dk.data_ptr(),
-                                      dv.data_ptr(), ws.data_ptr(), B, N, H, W, D, kernel_size,
-                                      _DTYPES[q.dtype], _lib.strides4(q), _lib.strides4(k),
-                                      _lib.strides4(v), _lib.strides4(o), _lib.strides4(d_o),
-                                      None if out is None else _lib.strides4(dq),
-                                      float(scale), _stream_of(q)))
+        _check(lib.enatten2d_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+                                 d_o.data_ptr(), lse.data_ptr(), dq.data_ptr(), dk.data_ptr(),
+                                 dv.data_ptr(), ws.data_ptr(), B, N, H, W, D, kernel_size,
+                                 _DTYPES[q.dtype], _lib.strides4(q), _lib.strides4(k),
+                                 _lib.strides4(v), _lib.strides4(o), _lib.strides4(d_o),
+                                 float(scale), _stream_of(q)))
     return dq, dk, dv
 
 
@@ -261,34 +252,44 @@ class Natten2dDilated(torch.autograd.Function):
     has no dilation and always passes 1 to its comparator, test.py:17).  Pixels with
     equal (x mod dilation, y mod dilation) only ever see each other, and inside such
     a sub-grid the rule is the plain one, so the operator is the undilated kernels run
-    on the dilation^2 strided sub-grids of q, k, v (the C ABI takes strides), each
-    writing its own pixels of the output in place (the C ABI takes the strides of o)."""
+    on the dilation^2 strided sub-grids, in place, all sub-grids of one size in one launch
+    (enatten2d_fwd_dilated / enatten2d_bwd_dilated).  ``natten2d`` reaches the same calls
+    through the native binding where that is built."""
 
     @staticmethod
     def forward(ctx, Q, K, V, kernel_size, scale, dilation):
-        o = torch.empty(Q.shape, dtype=Q.dtype, device=Q.device)
-        lses = []
-        for i in range(dilation):
-            for j in range(dilation):
-                sub = (slice(None), slice(None), slice(i, None, dilation), slice(j, None, dilation))
-                _, lse_s = _fwd_impl(Q[sub], K[sub], V[sub], kernel_size, scale, out=o[sub])
-                lses.append(lse_s)
-        ctx.save_for_backward(Q, K, V, o, *lses)
+        lib = _lib.load()
+        q, k, v = (_kernel_layout(t) for t in (Q, K, V))
+        B, N, H, W, D = q.shape
+        with torch.cuda.device(q.device):
+            o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+            lse = torch.empty((B, N, H, W), dtype=torch.float32, device=q.device)
+            _check(lib.enatten2d_fwd_dilated(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), B, N, H, W, D,
+                kernel_size, dilation, _DTYPES[q.dtype], _lib.strides4(q), _lib.strides4(k),
+                _lib.strides4(v), None, scale, _stream_of(q)))
+        ctx.save_for_backward(Q, K, V, o, lse)
         ctx.args = (kernel_size, scale, dilation)
         return o
 
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, grad_output):
-        Q, K, V, o, *lses = ctx.saved_tensors
+        Q, K, V, o, lse = ctx.saved_tensors
         kernel_size, scale, dilation = ctx.args
-        dQ, dK, dV = (torch.empty(Q.shape, dtype=Q.dtype, device=Q.device) for _ in range(3))
-        for i in range(dilation):
-            for j in range(dilation):
-                sub = (slice(None), slice(None), slice(i, None, dilation), slice(j, None, dilation))
-                _bwd_impl(Q[sub], K[sub], V[sub], o[sub], lses[i * dilation + j], grad_output[sub],
-                          kernel_size, scale, out=(dQ[sub], dK[sub], dV[sub]))
-        return dQ, dK, dV, None, None, None
+        lib = _lib.load()
+        q, k, v, o, d_o = (_kernel_layout(t) for t in (Q, K, V, o, grad_output))
+        B, N, H, W, D = q.shape
+        with torch.cuda.device(q.device):
+            dq, dk, dv = (torch.empty(q.shape, dtype=q.dtype, device=q.device) for _ in range(3))
+            ws = torch.empty(lib.enatten2d_bwd_dilated_workspace_bytes(B, N, H, W, _DTYPES[q.dtype]),
+                             dtype=torch.uint8, device=q.device)
+            _check(lib.enatten2d_bwd_dilated(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr(),
+                dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), B, N, H, W, D, kernel_size,
+                dilation, _DTYPES[q.dtype], _lib.strides4(q), _lib.strides4(k), _lib.strides4(v),
+                _lib.strides4(o), _lib.strides4(d_o), scale, _stream_of(q)))
+        return dq, dk, dv, None, None, None
 
 
 def _pair(x, what, kind):
@@ -447,7 +448,9 @@ def natten2d(q, k, v, kernel_size=7, scale=1.0, dilation=1, is_causal=False, rpb
         if min(q.shape[2], q.shape[3]) < kernel_size * dilation:
             raise ValueError("input of extent %dx%d is smaller than kernel_size * dilation = %d"
                              % (q.shape[2], q.shape[3], kernel_size * dilation))
-        return Natten2dDilated.apply(q, k, v, kernel_size, float(scale), dilation)
+        if not NATIVE_BINDING:
+            return Natten2dDilated.apply(q, k, v, kernel_size, float(scale), dilation)
+        return torch.ops.enatten.natten2d_dilated(q, k, v, kernel_size, float(scale), dilation)
     if not NATIVE_BINDING:
         return Natten2d.apply(q, k, v, kernel_size, scale)
     # the native operator checks shapes, dtypes, devices and the kernel size itself and raises

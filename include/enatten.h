@@ -145,6 +145,31 @@ int enatten2d_bwd_into(const void *q, const void *k, const void *v, const void *
                        const int64_t *grad_strides, float scale, void *stream);
 
 /*
+ * Dilated neighborhoods: query (y, x) attends the kernel_size^2 keys `dilation` apart around
+ * it, shifted at the borders as NATTEN does (the reference has no dilation and passes 1 to its
+ * comparator, test.py:17).  Arguments as in enatten2d_fwd / enatten2d_bwd; H and W must be at
+ * least kernel_size * dilation.  Pixels of one residue class modulo the dilation on each axis
+ * form a sub-grid on which the undilated rule holds; all sub-grids of one size run as one
+ * batch of images on the matrix-core kernels, read and written in place.
+ *   lse         float32 [B * heads * H * W], in an order of the library's own: pass it on to
+ *               enatten2d_bwd_dilated
+ *   workspace   enatten2d_bwd_dilated_workspace_bytes() bytes of device memory
+ */
+int enatten2d_fwd_dilated(const void *q, const void *k, const void *v, void *o, float *lse,
+                          int B, int heads, int H, int W, int D, int kernel_size, int dilation,
+                          int dtype, const int64_t *q_strides, const int64_t *k_strides,
+                          const int64_t *v_strides, const int64_t *o_strides, float scale,
+                          void *stream);
+size_t enatten2d_bwd_dilated_workspace_bytes(int B, int heads, int H, int W, int dtype);
+int enatten2d_bwd_dilated(const void *q, const void *k, const void *v, const void *o,
+                          const void *d_o, const float *lse, void *dq, void *dk, void *dv,
+                          void *workspace, int B, int heads, int H, int W, int D,
+                          int kernel_size, int dilation, int dtype, const int64_t *q_strides,
+                          const int64_t *k_strides, const int64_t *v_strides,
+                          const int64_t *o_strides, const int64_t *do_strides, float scale,
+                          void *stream);
+
+/*
  * enatten2d_bwd for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no
  * counterpart in the reference.  Same arguments and results as enatten2d_bwd without
