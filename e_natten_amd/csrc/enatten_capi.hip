@@ -90,6 +90,12 @@ bool use_mfma(int D, int ks, int dtype) {
 bool use_mfma_f32(int D, int ks, int dtype) {
     return g_path.load() != ENATTEN_PATH_SIMT && mfma_f32_supported(D, ks, dtype);
 }
+// 1D windows of any length (H = 1): causal ones, and centred ones beyond what mfma1d_supported
+// takes
+template <typename ARGS>
+bool use_band(const ARGS &a, int dtype) {
+    return g_path.load() != ENATTEN_PATH_SIMT && band_supported(a, dtype);
+}
 // float32 per query of backward workspace: two for the general and the 16-bit kernels
 // (delta and 1/Z), 2 * ks * ks for the float32 matrix-core kernels (P and dS), four for
 // float64 tensors (two doubles: the log-sum-exp in double and delta)
@@ -532,6 +538,7 @@ int enatten2d_fwd_window(const void *q, const void *k, const void *v, const void
     a.s = Shape{B, heads, H, W, D, kernel_h, kernel_w, scale, causal_h ? 1 : 0, causal_w ? 1 : 0};
     a.rpb = rpb;
     if (dtype == ENATTEN_F64) return launch_fwd_f64(a, static_cast<hipStream_t>(stream));
+    if (use_band(a, dtype)) return launch_fwd_band(a, dtype, static_cast<hipStream_t>(stream));
     return launch_fwd_simt(a, dtype, static_cast<hipStream_t>(stream));
 }
 
@@ -593,6 +600,7 @@ int enatten2d_bwd_window(const void *q, const void *k, const void *v, const void
     a.d_rpb = d_rpb;
     a.ds_pairs = rpb ? a.delta + (size_t)4 * B * heads * H * W : nullptr;
     if (dtype == ENATTEN_F64) return bwd_f64(fn, a, ws_floats, static_cast<hipStream_t>(stream));
+    if (use_band(a, dtype)) return launch_bwd_band(a, dtype, static_cast<hipStream_t>(stream));
     return launch_bwd_simt(a, dtype, static_cast<hipStream_t>(stream));
 }
 
@@ -646,6 +654,7 @@ int enatten1d_fwd(const void *q, const void *k, const void *v, void *o, float *l
     if (dtype == ENATTEN_F64) return launch_fwd_f64(a, static_cast<hipStream_t>(stream));
     if (g_path.load() != ENATTEN_PATH_SIMT && mfma1d_supported(D, kernel_size, dtype))
         return launch_fwd1d_mfma(a, dtype, static_cast<hipStream_t>(stream));
+    if (use_band(a, dtype)) return launch_fwd_band(a, dtype, static_cast<hipStream_t>(stream));
     return launch_fwd_simt(a, dtype, static_cast<hipStream_t>(stream));
 }
 
@@ -698,6 +707,7 @@ int enatten1d_bwd_into(const void *q, const void *k, const void *v, const void *
         return bwd_f64(fn, a, (size_t)4 * B * heads * T, static_cast<hipStream_t>(stream));
     if (g_path.load() != ENATTEN_PATH_SIMT && mfma1d_supported(D, kernel_size, dtype))
         return launch_bwd1d_mfma(a, dtype, g_path.load(), static_cast<hipStream_t>(stream));
+    if (use_band(a, dtype)) return launch_bwd_band(a, dtype, static_cast<hipStream_t>(stream));
     return launch_bwd_simt(a, dtype, static_cast<hipStream_t>(stream));
 }
 

@@ -1,0 +1,607 @@
+// Matrix-core kernels for 1D windows of any length, centred or causal (sliding-window causal
+// attention), bf16 / fp16, head dims that are multiples of 8 up to 128.
+//
+// The kernels of na1d_mfma_kernels.h stage all keys of a tile at once, which ends at a
+// kernel_size of 49.  Here a workgroup of four waves owns a tile of queries and walks the keys
+// that any of them sees, 64 at a time, with an online softmax: K and V rows of a block are in
+// LDS, the next block's are in flight into registers and go into a second buffer, one barrier
+// per block.  A wave owns NQ groups of 16 queries (the columns of v_mfma_f32_16x16x32); with two
+// groups every operand that comes out of LDS feeds two or four matrix instructions.  It takes the
+// keys 32 at a time, skips the steps its own queries do not reach, and masks only the steps that
+// the band's edges cut.  Operand layouts are those of na2d_mfma_kernels.h (tokens as MFMA rows,
+// the second product's other operand through the transposing LDS read).
+//
+// The running maximum is only raised when a logit exceeds it by more than 8 (in units of log2):
+// until then the probabilities are at most 2^8 times what they would be, which neither float32
+// sums nor 16-bit operands lose anything by, and no cross-lane maximum is formed.
+//
+// Probabilities and dS enter the second products as the sum of two 16-bit terms (the value
+// rounded, and what the rounding left): the products are exact to 16 (bf16) or 22 (fp16)
+// bits of them, as close as the results' own type can show to the float32 probabilities of the
+// general kernels, which served these calls before.
+//
+// What bounds it: at k = 128 the bytes (each key row is read by two or three workgroups of one
+// XCD, out of its L2); from k of about 512 the matrix pipe and the LDS reads that feed it.
+//
+// Per-query math: e_natten/triton.py:65-222; the causal rule is not in the reference.
+
+#include "na2d_mfma.h"
+
+namespace enatten {
+namespace {
+
+// Rows of a staged block: keys in the forward and the dQ pass, queries in the dK/dV pass.  64, and
+// 32 for the dK/dV pass at head_dim 64, where the smaller buffers let a third workgroup share the CU
+// (B4 N16 T8192 k32 causal 101 -> 86 us); not for its forward (54.6 -> 57.1), and not at head_dim
+// 128, where the registers leave room for two (dK/dV B1 N16 T8192 k128 62 -> 68), nor at 32, where
+// 32 rows are fewer than the 64 that a pass of all threads moves.
+constexpr int kRowsQ = 64;
+template <int D>
+constexpr int kRowsK = D == 64 ? 32 : 64;
+
+template <int D, int KB>
+struct BGeo {
+    static constexpr int PITCH = D + 8, CPR = D / 8, RPP = 256 / CPR, NL = KB / RPP;
+    static_assert(KB % RPP == 0, "every thread moves the same number of chunks");
+    static constexpr int DS = D / 32, DT = D / 16;
+};
+
+// KB rows of a sequence from p0 on, clamped to its last position (such rows only meet zero
+// probabilities); channels at or beyond dlim are zero.
+template <int D, int KB, bool NARROW>
+struct Block {
+    using G = BGeo<D, KB>;
+    u32x4 v[G::NL];
+    __device__ __forceinline__ void fetch(const short *sq, int64_t sw, int p0, int T, int dlim) {
+        const int c = (int)threadIdx.x % G::CPR;
+        if (NARROW && c * 8 >= dlim) {
+#pragma unroll
+            for (int i = 0; i < G::NL; i++) v[i] = u32x4{0u, 0u, 0u, 0u};
+            return;
+        }
+        const int pb = min(p0, T - 1), rmax = T - 1 - pb;
+        const char *base = reinterpret_cast<const char *>(sq + pb * sw);
+        const unsigned sw2 = (unsigned)sw * 2u;
+#pragma unroll
+        for (int i = 0; i < G::NL; i++) {
+            const int r = min((int)threadIdx.x / G::CPR + i * G::RPP, rmax);
+            v[i] = *reinterpret_cast<const u32x4 *>(base + __umul24((unsigned)r, sw2) + (unsigned)c * 16u);
+        }
+    }
+    __device__ __forceinline__ void commit(short *lds) const {
+#pragma unroll
+        for (int i = 0; i < G::NL; i++)
+            *reinterpret_cast<u32x4 *>(lds + ((int)threadIdx.x / G::CPR + i * G::RPP) * G::PITCH +
+                                       ((int)threadIdx.x % G::CPR) * 8) = v[i];
+    }
+};
+
+struct BTile {
+    int bb, nn, t0;
+};
+// Consecutive workgroup ids go round-robin to the 8 XCDs: each XCD gets one contiguous run of
+// tiles, so that the tiles that share key rows meet in one L2.  false: no such tile.
+__device__ __forceinline__ bool btile(int block, int nblocks, int ntiles, int tiles_t, int size, int N, BTile &tl) {
+    const int t = (block & 7) * (nblocks >> 3) + (block >> 3);
+    if (t >= ntiles) return false;
+    tl.t0 = (t % tiles_t) * size;
+    const int slab = t / tiles_t;
+    tl.bb = slab / N;
+    tl.nn = slab % N;
+    return true;
+}
+__device__ __forceinline__ const short *bseq(const View &v, const BTile &tl) {
+    return static_cast<const short *>(v.ptr) + tl.bb * v.sb + tl.nn * v.sn;
+}
+// window of position t: keys [band_lo, band_hi)
+__device__ __forceinline__ int band_lo(int t, int T, int k, int causal) { return axis_start(t, T, k, causal); }
+__device__ __forceinline__ int band_hi(int t, int T, int k, int causal) {
+    return causal ? t + 1 : win_start(t, T, k) + k;
+}
+__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+// eight float32 values as the sum of two vectors of 16-bit ones
+template <bool BF>
+__device__ __forceinline__ void split16(const float (&x)[8], s16x8 &hi, s16x8 &lo) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        hi[e] = cvt16<BF>(x[e]);
+        lo[e] = cvt16<BF>(x[e] - cvt32<BF>(hi[e]));
+    }
+}
+// rows of an operand straight from global memory
+template <int DS, bool NARROW>
+__device__ __forceinline__ void load_row(s16x8 (&reg)[DS], const short *row, int g, int dlim) {
+    if constexpr (NARROW) {
+        load_row_chunks(reg, row, g, dlim);
+    } else {
+#pragma unroll
+        for (int ds = 0; ds < DS; ds++) reg[ds] = *reinterpret_cast<const s16x8 *>(row + ds * 32 + g * 8);
+    }
+}
+
+// ------------------------------------------------------------------ forward
+template <bool BF, int D, int NQ, bool NARROW>
+__global__ __launch_bounds__(256, 2) void fwd_band_mfma(FwdArgs a, int tiles_t, int ntiles) {
+    constexpr int KB = kRowsQ;
+    using G = BGeo<D, KB>;
+    __shared__ __attribute__((aligned(16))) short lds_k[2][KB * G::PITCH];
+    __shared__ __attribute__((aligned(16))) short lds_v[2][KB * G::PITCH];
+    const Shape &s = a.s;
+    const int T = s.W, k = s.kw, causal = s.cw, dlim = NARROW ? s.D : D;
+    BTile tl;
+    if (!btile(blockIdx.x, gridDim.x, ntiles, tiles_t, 64 * NQ, s.N, tl)) return;
+    const int wave = uni(threadIdx.x >> 6), l = threadIdx.x & 63, n = l & 15, g = l >> 4;
+    const float sc2 = s.scale * kLog2e;
+
+    const short *kseq = bseq(a.k, tl), *vseq = bseq(a.v, tl), *qseq = bseq(a.q, tl);
+    const int ka = band_lo(tl.t0, T, k, causal), kb = band_hi(min(tl.t0 + 64 * NQ, T) - 1, T, k, causal);
+    Block<D, KB, NARROW> kst, vst;
+    kst.fetch(kseq, a.k.sw, ka, T, dlim);
+    vst.fetch(vseq, a.v.sw, ka, T, dlim);
+
+    // this wave's queries and the keys they see between them
+    const int w0 = tl.t0 + wave * 16 * NQ;
+    const bool on = w0 < T;
+    const int wa = band_lo(min(w0, T - 1), T, k, causal), wb = band_hi(min(w0 + 16 * NQ, T) - 1, T, k, causal);
+    s16x8 qreg[NQ][G::DS];
+    int lo[NQ], cnt[NQ], in_lo[NQ], in_hi[NQ];  // this lane's window; the keys that all 16 queries see
+    f32x4 o[NQ][G::DT];
+    float m[NQ], sum[NQ];
+#pragma unroll
+    for (int u = 0; u < NQ; u++) {
+        const int qt = min(w0 + u * 16 + n, T - 1);
+        load_row<G::DS, NARROW>(qreg[u], qseq + qt * a.q.sw, g, dlim);
+        lo[u] = band_lo(qt, T, k, causal);
+        cnt[u] = band_hi(qt, T, k, causal) - lo[u];
+        in_lo[u] = band_lo(min(w0 + u * 16 + 15, T - 1), T, k, causal);
+        in_hi[u] = band_hi(min(w0 + u * 16, T - 1), T, k, causal);
+#pragma unroll
+        for (int t = 0; t < G::DT; t++) o[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        m[u] = -1e30f;
+        sum[u] = 0.f;
+    }
+    kst.commit(lds_k[0]);
+    vst.commit(lds_v[0]);
+    __syncthreads();
+
+    for (int k0 = ka, buf = 0; k0 < kb; k0 += KB, buf ^= 1) {
+        const bool more = k0 + KB < kb;
+        if (more) {
+            kst.fetch(kseq, a.k.sw, k0 + KB, T, dlim);
+            vst.fetch(vseq, a.v.sw, k0 + KB, T, dlim);
+        }
+        const short *lk = lds_k[buf], *lv = lds_v[buf];
+#pragma unroll
+        for (int st = 0; st < KB / 32; st++) {
+            const int kk = k0 + st * 32;
+            if (!on || kk >= wb || kk + 32 <= wa) continue;  // (the same for the whole wave)
+            f32x4 c[NQ][2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const short *kp = lk + (st * 32 + h * 16 + n) * G::PITCH + g * 8;
+#pragma unroll
+                for (int u = 0; u < NQ; u++) c[u][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ds = 0; ds < G::DS; ds++) {
+                    const s16x8 kr = *reinterpret_cast<const s16x8 *>(kp + ds * 32);
+#pragma unroll
+                    for (int u = 0; u < NQ; u++) c[u][h] = mfma16<BF>(kr, qreg[u][ds], c[u][h]);
+                }
+            }
+            s16x8 ph[NQ], pl[NQ];
+#pragma unroll
+            for (int u = 0; u < NQ; u++) {
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) x[e] = c[u][e >> 2][e & 3] * sc2;
+                if (kk < in_lo[u] || kk + 32 > in_hi[u]) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const int key = kk + (e >> 2) * 16 + g * 4 + (e & 3);
+                        x[e] = (unsigned)(key - lo[u]) < (unsigned)cnt[u] ? x[e] : -INFINITY;
+                    }
+                }
+                const float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
+                                       fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+                if (__any(mx > m[u] + 8.f)) {
+                    const float mn = fmaxf(m[u], col_max(mx)), corr = __builtin_amdgcn_exp2f(m[u] - mn);
+                    m[u] = mn;
+                    sum[u] *= corr;
+#pragma unroll
+                    for (int t = 0; t < G::DT; t++) o[u][t] *= corr;
+                }
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    x[e] = __builtin_amdgcn_exp2f(x[e] - m[u]);
+                    sum[u] += x[e];
+                }
+                split16<BF>(x, ph[u], pl[u]);
+            }
+            const short *vp[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                vp[h] = lv + (st * 32 + h * 16 + g * 4 + (n >> 2)) * G::PITCH + (n & 3) * (D / 4);
+#pragma unroll
+            for (int t = 0; t < G::DT; t++) {
+                const s16x8 vt = cat(lds_read_tr(vp[0] + t * 4), lds_read_tr(vp[1] + t * 4));
+#pragma unroll
+                for (int u = 0; u < NQ; u++) {
+                    o[u][t] = mfma16<BF>(vt, ph[u], o[u][t]);
+                    o[u][t] = mfma16<BF>(vt, pl[u], o[u][t]);
+                }
+            }
+        }
+        if (more) {
+            kst.commit(lds_k[buf ^ 1]);
+            vst.commit(lds_v[buf ^ 1]);
+        }
+        __syncthreads();
+    }
+    if (!on) return;
+    short *oseq = const_cast<short *>(bseq(a.o, tl));
+#pragma unroll
+    for (int u = 0; u < NQ; u++) {
+        const int q0 = w0 + u * 16 + n, qt = min(q0, T - 1);
+        const bool live = q0 < T;
+        const float total = col_sum(sum[u]);
+        store_token<BF, D, (D >= 64 && !NARROW)>(oseq + qt * a.o.sw, g, o[u], 1.f / total, live, dlim);
+        if (a.lse && live && g == 0)
+            a.lse[((int64_t)tl.bb * s.N + tl.nn) * T + qt] = (m[u] + __builtin_amdgcn_logf(total)) * kLn2;
+    }
+}
+
+// ------------------------------------------------------------------ dQ
+// The forward's walk with P from the saved log-sum-exp, dP^T = V dO^T, dS = P (dP - delta),
+// dQ^T += K^T dS^T.  delta = dO . O of the tile's queries is formed first and left for the
+// dK/dV pass.
+template <bool BF, int D, int NQ, bool NARROW>
+__global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_t, int ntiles) {
+    constexpr int KB = kRowsQ;
+    using G = BGeo<D, KB>;
+    __shared__ __attribute__((aligned(16))) short lds_k[2][KB * G::PITCH];
+    __shared__ __attribute__((aligned(16))) short lds_v[2][KB * G::PITCH];
+    const Shape &s = a.s;
+    const int T = s.W, k = s.kw, causal = s.cw, dlim = NARROW ? s.D : D;
+    BTile tl;
+    if (!btile(blockIdx.x, gridDim.x, ntiles, tiles_t, 64 * NQ, s.N, tl)) return;
+    const int wave = uni(threadIdx.x >> 6), l = threadIdx.x & 63, n = l & 15, g = l >> 4;
+    const float sc2 = s.scale * kLog2e;
+
+    const short *kseq = bseq(a.k, tl), *vseq = bseq(a.v, tl);
+    const int ka = band_lo(tl.t0, T, k, causal), kb = band_hi(min(tl.t0 + 64 * NQ, T) - 1, T, k, causal);
+    Block<D, KB, NARROW> kst, vst;
+    kst.fetch(kseq, a.k.sw, ka, T, dlim);
+    vst.fetch(vseq, a.v.sw, ka, T, dlim);
+
+    const int w0 = tl.t0 + wave * 16 * NQ;
+    const bool on = w0 < T;
+    const int wa = band_lo(min(w0, T - 1), T, k, causal), wb = band_hi(min(w0 + 16 * NQ, T) - 1, T, k, causal);
+    const int64_t tok0 = ((int64_t)tl.bb * s.N + tl.nn) * T;
+    s16x8 qreg[NQ][G::DS], greg[NQ][G::DS];
+    int lo[NQ], cnt[NQ], in_lo[NQ], in_hi[NQ];
+    f32x4 dq[NQ][G::DT];
+    float lse2[NQ], delta[NQ];
+#pragma unroll
+    for (int u = 0; u < NQ; u++) {
+        const int qt = min(w0 + u * 16 + n, T - 1);
+        load_row<G::DS, NARROW>(qreg[u], bseq(a.q, tl) + qt * a.q.sw, g, dlim);
+        load_row<G::DS, NARROW>(greg[u], bseq(a.d_o, tl) + qt * a.d_o.sw, g, dlim);
+        s16x8 orow[G::DS];
+        load_row<G::DS, NARROW>(orow, bseq(a.o, tl) + qt * a.o.sw, g, dlim);
+        lse2[u] = a.lse[tok0 + qt] * kLog2e;
+        lo[u] = band_lo(qt, T, k, causal);
+        cnt[u] = band_hi(qt, T, k, causal) - lo[u];
+        in_lo[u] = band_lo(min(w0 + u * 16 + 15, T - 1), T, k, causal);
+        in_hi[u] = band_hi(min(w0 + u * 16, T - 1), T, k, causal);
+        float d = 0.f;
+#pragma unroll
+        for (int ds = 0; ds < G::DS; ds++)
+            d += dot8<BF>(__builtin_bit_cast(u32x4, greg[u][ds]), __builtin_bit_cast(u32x4, orow[ds]));
+        delta[u] = col_sum(d);
+        if (w0 + u * 16 + n < T && g == 0) a.delta[tok0 + qt] = delta[u];
+#pragma unroll
+        for (int t = 0; t < G::DT; t++) dq[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    kst.commit(lds_k[0]);
+    vst.commit(lds_v[0]);
+    __syncthreads();
+
+    for (int k0 = ka, buf = 0; k0 < kb; k0 += KB, buf ^= 1) {
+        const bool more = k0 + KB < kb;
+        if (more) {
+            kst.fetch(kseq, a.k.sw, k0 + KB, T, dlim);
+            vst.fetch(vseq, a.v.sw, k0 + KB, T, dlim);
+        }
+        const short *lk = lds_k[buf], *lv = lds_v[buf];
+#pragma unroll
+        for (int st = 0; st < KB / 32; st++) {
+            const int kk = k0 + st * 32;
+            if (!on || kk >= wb || kk + 32 <= wa) continue;
+            f32x4 c[NQ][2], cp[NQ][2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int row = (st * 32 + h * 16 + n) * G::PITCH + g * 8;
+#pragma unroll
+                for (int u = 0; u < NQ; u++) {
+                    c[u][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    cp[u][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+#pragma unroll
+                for (int ds = 0; ds < G::DS; ds++) {
+                    const s16x8 kr = *reinterpret_cast<const s16x8 *>(lk + row + ds * 32);
+                    const s16x8 vr = *reinterpret_cast<const s16x8 *>(lv + row + ds * 32);
+#pragma unroll
+                    for (int u = 0; u < NQ; u++) {
+                        c[u][h] = mfma16<BF>(kr, qreg[u][ds], c[u][h]);
+                        cp[u][h] = mfma16<BF>(vr, greg[u][ds], cp[u][h]);
+                    }
+                }
+            }
+            s16x8 sh[NQ], sl[NQ];
+#pragma unroll
+            for (int u = 0; u < NQ; u++) {
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) x[e] = c[u][e >> 2][e & 3] * sc2 - lse2[u];
+                if (kk < in_lo[u] || kk + 32 > in_hi[u]) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const int key = kk + (e >> 2) * 16 + g * 4 + (e & 3);
+                        x[e] = (unsigned)(key - lo[u]) < (unsigned)cnt[u] ? x[e] : -INFINITY;
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    x[e] = __builtin_amdgcn_exp2f(x[e]) * (cp[u][e >> 2][e & 3] - delta[u]);
+                split16<BF>(x, sh[u], sl[u]);
+            }
+            const short *kp[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                kp[h] = lk + (st * 32 + h * 16 + g * 4 + (n >> 2)) * G::PITCH + (n & 3) * (D / 4);
+#pragma unroll
+            for (int t = 0; t < G::DT; t++) {
+                const s16x8 kt = cat(lds_read_tr(kp[0] + t * 4), lds_read_tr(kp[1] + t * 4));
+#pragma unroll
+                for (int u = 0; u < NQ; u++) {
+                    dq[u][t] = mfma16<BF>(kt, sh[u], dq[u][t]);
+                    dq[u][t] = mfma16<BF>(kt, sl[u], dq[u][t]);
+                }
+            }
+        }
+        if (more) {
+            kst.commit(lds_k[buf ^ 1]);
+            vst.commit(lds_v[buf ^ 1]);
+        }
+        __syncthreads();
+    }
+    if (!on) return;
+#pragma unroll
+    for (int u = 0; u < NQ; u++) {
+        const int q0 = w0 + u * 16 + n, qt = min(q0, T - 1);
+        store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dq) + a.grad_at(tl.bb, tl.nn, 0, qt), g,
+                                                 dq[u], s.scale, q0 < T, dlim);
+    }
+}
+
+// ------------------------------------------------------------------ dK, dV
+// The tile is 64 keys, 16 per wave (columns), and the walk is over the queries
+// that see any of them, the inverse neighbourhood (e_natten/pytorch.py:13-23), a block at a time: Q
+// and dO rows, the log-sum-exp and delta of a block in LDS.  dV^T += dO^T P, dK^T += Q^T dS.
+template <bool BF, int D, bool NARROW>
+__global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tiles_t, int ntiles) {
+    constexpr int KB = kRowsK<D>;
+    using G = BGeo<D, KB>;
+    __shared__ __attribute__((aligned(16))) short lds_q[2][KB * G::PITCH];
+    __shared__ __attribute__((aligned(16))) short lds_g[2][KB * G::PITCH];
+    __shared__ __attribute__((aligned(16))) float2 lds_stat[2][KB];  // (lse * log2e, delta)
+    const Shape &s = a.s;
+    const int T = s.W, k = s.kw, causal = s.cw, dlim = NARROW ? s.D : D;
+    BTile tl;
+    if (!btile(blockIdx.x, gridDim.x, ntiles, tiles_t, 64, s.N, tl)) return;
+    const int wave = uni(threadIdx.x >> 6), l = threadIdx.x & 63, n = l & 15, g = l >> 4;
+    const float sc2 = s.scale * kLog2e;
+
+    const short *qseq = bseq(a.q, tl), *gseq = bseq(a.d_o, tl);
+    const int64_t tok0 = ((int64_t)tl.bb * s.N + tl.nn) * T;
+    const int qa = axis_inv_lo(tl.t0, k, causal), qb = axis_inv_hi(min(tl.t0 + 64, T) - 1, T, k, causal);
+    Block<D, KB, NARROW> qst, gst;
+    float2 sst = make_float2(0.f, 0.f);
+    auto fetch = [&](int p0) __attribute__((always_inline)) {
+        qst.fetch(qseq, a.q.sw, p0, T, dlim);
+        gst.fetch(gseq, a.d_o.sw, p0, T, dlim);
+        if (threadIdx.x < KB) {
+            const int64_t at = tok0 + min(p0 + (int)threadIdx.x, T - 1);
+            sst = make_float2(a.lse[at] * kLog2e, a.delta[at]);
+        }
+    };
+    auto commit = [&](int buf) __attribute__((always_inline)) {
+        qst.commit(lds_q[buf]);
+        gst.commit(lds_g[buf]);
+        if (threadIdx.x < KB) lds_stat[buf][threadIdx.x] = sst;
+    };
+    fetch(qa);
+
+    const int w0 = tl.t0 + wave * 16;
+    const bool on = w0 < T;
+    const int wa = axis_inv_lo(min(w0, T - 1), k, causal), wb = axis_inv_hi(min(w0 + 16, T) - 1, T, k, causal);
+    s16x8 kreg[G::DS], vreg[G::DS];
+    f32x4 dk[G::DT], dv[G::DT];
+    const int kt = min(w0 + n, T - 1);  // this lane's key
+    load_row<G::DS, NARROW>(kreg, bseq(a.k, tl) + kt * a.k.sw, g, dlim);
+    load_row<G::DS, NARROW>(vreg, bseq(a.v, tl) + kt * a.v.sw, g, dlim);
+#pragma unroll
+    for (int t = 0; t < G::DT; t++) {
+        dk[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        dv[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    commit(0);
+    __syncthreads();
+
+    for (int p0 = qa, buf = 0; p0 < qb; p0 += KB, buf ^= 1) {
+        const bool more = p0 + KB < qb;
+        if (more) fetch(p0 + KB);
+        const short *lq = lds_q[buf], *lg = lds_g[buf];
+        const float2 *stat = lds_stat[buf];
+#pragma unroll
+        for (int st = 0; st < KB / 32; st++) {
+            const int qq = p0 + st * 32;
+            if (!on || qq >= wb || qq + 32 <= wa) continue;
+            f32x4 c[2], cp[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int row = (st * 32 + h * 16 + n) * G::PITCH + g * 8;
+                c[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+                cp[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ds = 0; ds < G::DS; ds++) {
+                    const s16x8 qr = *reinterpret_cast<const s16x8 *>(lq + row + ds * 32);
+                    const s16x8 gr = *reinterpret_cast<const s16x8 *>(lg + row + ds * 32);
+                    c[h] = mfma16<BF>(qr, kreg[ds], c[h]);
+                    cp[h] = mfma16<BF>(gr, vreg[ds], cp[h]);
+                }
+            }
+            float2 sv[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) sv[e] = stat[st * 32 + (e >> 2) * 16 + g * 4 + (e & 3)];
+            // the keys that all 32 queries of the step see
+            const int in_lo = band_lo(min(qq + 31, T - 1), T, k, causal), in_hi = band_hi(qq, T, k, causal);
+            s16x8 ph, pl, sh, sl;
+            float x[8], y[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = c[e >> 2][e & 3] * sc2 - sv[e].x;
+            if (w0 < in_lo || w0 + 16 > in_hi || qq + 32 > T) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    // (causal: the key is one of the query and the k - 1 positions before it)
+                    const int q = qq + (e >> 2) * 16 + g * 4 + (e & 3), key = w0 + n;
+                    const unsigned at = causal ? q - key : key - win_start(q, T, k);
+                    x[e] = at < (unsigned)k && q < T ? x[e] : -INFINITY;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                x[e] = __builtin_amdgcn_exp2f(x[e]);
+                y[e] = x[e] * (cp[e >> 2][e & 3] - sv[e].y);
+            }
+            split16<BF>(x, ph, pl);
+            split16<BF>(y, sh, sl);
+            const short *qp[2], *gp[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int row = (st * 32 + h * 16 + g * 4 + (n >> 2)) * G::PITCH + (n & 3) * (D / 4);
+                qp[h] = lq + row;
+                gp[h] = lg + row;
+            }
+#pragma unroll
+            for (int t = 0; t < G::DT; t++) {
+                const s16x8 gt = cat(lds_read_tr(gp[0] + t * 4), lds_read_tr(gp[1] + t * 4));
+                const s16x8 qt = cat(lds_read_tr(qp[0] + t * 4), lds_read_tr(qp[1] + t * 4));
+                dv[t] = mfma16<BF>(gt, ph, dv[t]);
+                dk[t] = mfma16<BF>(qt, sh, dk[t]);
+                dv[t] = mfma16<BF>(gt, pl, dv[t]);
+                dk[t] = mfma16<BF>(qt, sl, dk[t]);
+            }
+        }
+        if (more) commit(buf ^ 1);
+        __syncthreads();
+    }
+    if (!on) return;
+    const bool live = w0 + n < T;
+    const int64_t at = a.grad_at(tl.bb, tl.nn, 0, kt);
+    store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dk) + at, g, dk, s.scale, live, dlim);
+    store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dv) + at, g, dv, 1.f, live, dlim);
+}
+
+// ------------------------------------------------------------------ dispatch
+// Two groups of 16 queries per wave (forward and dQ pass) where the walk is long, a key row is 256
+// bytes, and tiles of that size still give every CU its two workgroups: the LDS reads of a step then feed
+// twice the matrix instructions.  One group / two, us, causal: head_dim 128 B2 N8 T4096 k400 forward
+// 36.5 / 33.4, dQ 43.5 / 38.2; at k = 128 (B1 N16 T8192) level (43.1 / 44.1, 50.9 / 49.7); head_dim 64
+// B2 N16 T4096 k256 25.7 / 33.5 and 30.9 / 36.9: there more waves count for more.  The dK/dV
+// pass with two groups of keys: 108 / 151 at head_dim 64.
+bool two_groups(const Shape &s) {
+    return s.D == 128 && s.kw >= 256 && (int64_t)s.B * s.N * ((s.W + 127) / 128) >= 512;
+}
+int band_grid(int64_t ntiles) { return (int)((ntiles + 7) / 8 * 8); }
+
+template <bool BF, int D, int NQ, bool NARROW>
+int fwd_go(const FwdArgs &a, hipStream_t st) {
+    const int tiles_t = (a.s.W + 64 * NQ - 1) / (64 * NQ);
+    const int64_t nt = (int64_t)a.s.B * a.s.N * tiles_t;
+    {
+        ProfScope prof(ENATTEN_KERNEL_FWD, "fwd_band_mfma", st);
+        hipLaunchKernelGGL((fwd_band_mfma<BF, D, NQ, NARROW>), dim3(band_grid(nt)), dim3(256), 0, st, a, tiles_t,
+                           (int)nt);
+    }
+    return check_launch("fwd_band_mfma");
+}
+template <bool BF, int D, int NQ, bool NARROW>
+int bwd_go(const BwdArgs &a, hipStream_t st) {
+    const int tiles_t = (a.s.W + 64 * NQ - 1) / (64 * NQ);
+    const int64_t nt = (int64_t)a.s.B * a.s.N * tiles_t;
+    {
+        ProfScope prof(ENATTEN_KERNEL_BWD_DQ, "bwd_band_dq_mfma", st);
+        hipLaunchKernelGGL((bwd_band_dq_mfma<BF, D, NQ, NARROW>), dim3(band_grid(nt)), dim3(256), 0, st, a, tiles_t,
+                           (int)nt);
+    }
+    {
+        ProfScope prof(ENATTEN_KERNEL_BWD_DKDV, "bwd_band_dkdv_mfma", st);
+        const int tk = (a.s.W + 63) / 64;
+        const int64_t nk = (int64_t)a.s.B * a.s.N * tk;
+        hipLaunchKernelGGL((bwd_band_dkdv_mfma<BF, D, NARROW>), dim3(band_grid(nk)), dim3(256), 0, st, a, tk,
+                           (int)nk);
+    }
+    return check_launch("bwd_band_mfma");
+}
+
+#define ENATTEN_BAND(FN, BF, ARGS, ST)                                                         \
+    switch ((ARGS).s.D) {                                                                      \
+        case 32: return FN<BF, 32, 1, false>(ARGS, ST);                                        \
+        case 64: return FN<BF, 64, 1, false>(ARGS, ST);                                        \
+        case 128: return two ? FN<BF, 128, 2, false>(ARGS, ST) : FN<BF, 128, 1, false>(ARGS, ST); \
+    }                                                                                          \
+    if ((ARGS).s.D < 32) return FN<BF, 32, 1, true>(ARGS, ST);                                 \
+    if ((ARGS).s.D < 64) return FN<BF, 64, 1, true>(ARGS, ST);                                 \
+    return FN<BF, 128, 1, true>(ARGS, ST);
+
+bool band_layout_ok(const View &v) {
+    return reinterpret_cast<uintptr_t>(v.ptr) % 16 == 0 && v.sb % 8 == 0 && v.sn % 8 == 0 && v.sw % 8 == 0 &&
+           v.sw < (1 << 22);
+}
+bool band_shape_ok(const Shape &s, int dtype) {
+    return (dtype == ENATTEN_BF16 || dtype == ENATTEN_F16) && s.D >= 8 && s.D <= 128 && s.D % 8 == 0 && s.H == 1 &&
+           s.kh == 1 && (int64_t)s.B * s.N * ((s.W + 63) / 64) < ((int64_t)1 << 31) - 8;
+}
+
+}  // namespace
+
+bool band_supported(const FwdArgs &a, int dtype) {
+    return band_shape_ok(a.s, dtype) && !a.rpb && band_layout_ok(a.q) && band_layout_ok(a.k) &&
+           band_layout_ok(a.v) && band_layout_ok(a.o);
+}
+bool band_supported(const BwdArgs &a, int dtype) {
+    auto al = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    return band_shape_ok(a.s, dtype) && !a.rpb && band_layout_ok(a.q) && band_layout_ok(a.k) &&
+           band_layout_ok(a.v) && band_layout_ok(a.o) && band_layout_ok(a.d_o) && al(a.dq) && al(a.dk) &&
+           al(a.dv) && a.gsb % 8 == 0 && a.gsn % 8 == 0 && a.gsw % 8 == 0;
+}
+int launch_fwd_band(const FwdArgs &a, int dtype, hipStream_t st) {
+    const bool two = two_groups(a.s);
+    if (dtype == ENATTEN_BF16) {
+        ENATTEN_BAND(fwd_go, true, a, st)
+    } else {
+        ENATTEN_BAND(fwd_go, false, a, st)
+    }
+}
+int launch_bwd_band(const BwdArgs &a, int dtype, hipStream_t st) {
+    const bool two = two_groups(a.s);
+    if (dtype == ENATTEN_BF16) {
+        ENATTEN_BAND(bwd_go, true, a, st)
+    } else {
+        ENATTEN_BAND(bwd_go, false, a, st)
+    }
+}
+
+}  // namespace enatten

@@ -164,6 +164,12 @@ int launch_fwd1d_mfma(const FwdArgs &a, int dtype, hipStream_t st);
 int launch_bwd1d_mfma(const BwdArgs &a, int dtype, int path, hipStream_t st);
 int launch_fwd1d_mfma_narrow(const FwdArgs &a, int dtype, hipStream_t st);
 int launch_bwd1d_mfma_narrow(const BwdArgs &a, int dtype, int path, hipStream_t st);
+// matrix-core kernels for 1D windows of any length, centred or causal (a.s: H = 1, kh = 1; a.s.cw):
+// bf16 / f16, D a multiple of 8 up to 128
+bool band_supported(const FwdArgs &a, int dtype);
+bool band_supported(const BwdArgs &a, int dtype);
+int launch_fwd_band(const FwdArgs &a, int dtype, hipStream_t st);
+int launch_bwd_band(const BwdArgs &a, int dtype, hipStream_t st);
 // fused backward (dQ, dK, dV of every tile from one staging), where built
 bool fused_bwd_supported(const BwdArgs &a);
 int launch_bwd_fused(const BwdArgs &a, bool bf16, const TileSet &ts, int64_t ntiles,

@@ -39,7 +39,7 @@ int dtype_code(const Tensor &t) {
 // bad shapes, dtypes and kernel sizes, RuntimeError for tensors that are not on
 // the GPU.
 void validate(const char *what, const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks,
-              int64_t ndim) {
+              int64_t ndim, bool check_device = true) {
     TORCH_CHECK_VALUE(q.dim() == ndim, what, ": expected ",
                       ndim == 5 ? "[B, heads, H, W, head_dim]" : "[B, heads, T, head_dim]",
                       " tensors, got ", q.dim(), "-D q");
@@ -61,7 +61,7 @@ void validate(const char *what, const Tensor &q, const Tensor &k, const Tensor &
                       " exceeds the supported maximum of 1024");
     // meta tensors (shape inference under tracing) pass: every operator returns outputs of
     // the right shape for them without touching the library
-    TORCH_CHECK(q.is_cuda() || q.is_meta(), what,
+    TORCH_CHECK(!check_device || q.is_cuda() || q.is_meta(), what,
                 ": tensors must be on the GPU; this build has no CPU path");
 }
 
@@ -292,6 +292,132 @@ Tensor natten2d_dilated_plain(const Tensor &q, const Tensor &k, const Tensor &v,
     return std::get<0>(dilated_fwd(q, k, v, ks, scale, dil));
 }
 
+// Rectangular and causal windows and the relative position bias (enatten2d_fwd_window): the
+// rules of the Python host side, 2D ([B, heads, H, W, d], rpb [heads, 2 kh - 1, 2 kw - 1]) and 1D
+// ([B, heads, T, d] as an image of one row, rpb [heads, 2 k - 1]).
+struct Window {
+    int64_t kh, kw;
+    bool ch, cw;
+    double scale;
+};
+void validate_window(const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &rpb,
+                     const Window &w, bool two_d) {
+    const char *what = two_d ? "natten2d" : "natten1d";
+    validate(what, q, k, v, 1, two_d ? 5 : 4, false);
+    auto axis = [&](const char *name, int64_t L, int64_t ks, bool causal) {
+        TORCH_CHECK_VALUE(ks >= 1 && (causal || ks % 2 == 1), what, ": kernel_size along ", name,
+                          " must be >= 1, and odd unless that axis is causal, got ", ks);
+        TORCH_CHECK_VALUE(L >= ks, what, ": input has ", L, " ", name, ", fewer than kernel_size ", ks);
+    };
+    if (two_d) axis("rows", q.size(2), w.kh, w.ch);
+    axis(two_d ? "columns" : "positions", q.size(-2), w.kw, w.cw);
+    if (rpb.has_value()) {
+        const Tensor &r = *rpb;
+        const bool shape_ok = two_d ? r.dim() == 3 && r.size(0) == q.size(1) && r.size(1) == 2 * w.kh - 1 &&
+                                          r.size(2) == 2 * w.kw - 1
+                                    : r.dim() == 2 && r.size(0) == q.size(1) && r.size(1) == 2 * w.kw - 1;
+        TORCH_CHECK_VALUE(shape_ok, what, ": rpb must have shape [heads, 2*kernel_size-1 along each axis], got ", r.sizes());
+        TORCH_CHECK_VALUE(r.scalar_type() == q.scalar_type() && r.device() == q.device(), what,
+                          ": rpb must have the dtype and device of q");
+        TORCH_CHECK_VALUE(!w.ch && !w.cw, what, ": a relative position bias goes with centred axes only");
+    }
+    TORCH_CHECK(q.is_cuda(), what, ": tensors must be on the GPU; this build has no CPU path");
+}
+// (batch, head, row, column) extents and strides of a tensor; a sequence is an image of one row
+struct Image {
+    int B, N, H, W, D;
+    explicit Image(const Tensor &t)
+        : B(t.size(0)), N(t.size(1)), H(t.dim() == 5 ? t.size(2) : 1), W(t.size(-2)), D(t.size(-1)) {}
+};
+struct Strides {
+    int64_t s[4];
+    explicit Strides(const Tensor &t)
+        : s{t.stride(0), t.stride(1), t.dim() == 5 ? t.stride(2) : 0, t.stride(-2)} {}
+    operator const int64_t *() const { return s; }
+};
+std::tuple<Tensor, Tensor> window_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_,
+                                      const c10::optional<Tensor> &rpb_, const Window &w) {
+    const c10::DeviceGuard guard(q_.device());
+    const Tensor q = kernel_layout(q_), k = kernel_layout(k_), v = kernel_layout(v_);
+    const Tensor rpb = rpb_.has_value() ? rpb_->contiguous() : Tensor();
+    const Image im(q);
+    Tensor o = kernel_layout(at::empty_like(q));
+    Tensor lse = at::empty({im.B, im.N, im.H, im.W}, q.options().dtype(at::kFloat));
+    check_rc(enatten2d_fwd_window(q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                  rpb.defined() ? rpb.data_ptr() : nullptr, o.data_ptr(), lse.data_ptr<float>(),
+                                  im.B, im.N, im.H, im.W, im.D, (int)w.kh, (int)w.kw, w.ch, w.cw, dtype_code(q),
+                                  Strides(q), Strides(k), Strides(v), Strides(o), (float)w.scale,
+                                  c10::hip::getCurrentHIPStream().stream()));
+    return {o, lse};
+}
+struct WindowFn : public torch::autograd::Function<WindowFn> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v,
+                          const c10::optional<Tensor> &rpb, int64_t kh, int64_t kw, bool ch, bool cw,
+                          double scale) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Window w{kh, kw, ch, cw, scale};
+        Tensor o, lse;
+        std::tie(o, lse) = window_fwd(q, k, v, rpb, w);
+        ctx->save_for_backward({q, k, v, o, lse, rpb.has_value() ? *rpb : Tensor()});
+        ctx->saved_data["kh"] = kh;
+        ctx->saved_data["kw"] = kw;
+        ctx->saved_data["causal"] = (int64_t)ch | ((int64_t)cw << 1);
+        ctx->saved_data["scale"] = scale;
+        return o;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const int64_t causal = ctx->saved_data["causal"].toInt();
+        const Window w{ctx->saved_data["kh"].toInt(), ctx->saved_data["kw"].toInt(), (causal & 1) != 0,
+                       (causal & 2) != 0, ctx->saved_data["scale"].toDouble()};
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::DeviceGuard guard(s[0].device());
+        check_bwd_extras("natten", s[0], s[3], grads[0]);
+        const Tensor q = kernel_layout(s[0]), k = kernel_layout(s[1]), v = kernel_layout(s[2]);
+        const Tensor &o = s[3], &lse = s[4], d_o = kernel_layout(grads[0]);
+        const Tensor rpb = s[5].defined() ? s[5].contiguous() : Tensor();
+        const Image im(q);
+        Tensor dq = at::empty(q.sizes(), q.options());
+        Tensor dk = at::empty_like(dq), dv = at::empty_like(dq);
+        Tensor d_rpb = rpb.defined() ? at::empty(rpb.sizes(), q.options().dtype(at::kFloat)) : Tensor();
+        Tensor ws = at::empty({(int64_t)enatten2d_bwd_window_workspace_bytes(im.B, im.N, im.H, im.W, (int)w.kh,
+                                                                             (int)w.kw, rpb.defined())},
+                              q.options().dtype(at::kByte));
+        check_rc(enatten2d_bwd_window(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), rpb.defined() ? rpb.data_ptr() : nullptr, o.data_ptr(),
+            d_o.data_ptr(), lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+            rpb.defined() ? d_rpb.data_ptr<float>() : nullptr, ws.data_ptr(), im.B, im.N, im.H, im.W, im.D,
+            (int)w.kh, (int)w.kw, w.ch, w.cw, dtype_code(q), Strides(q), Strides(k), Strides(v), Strides(o),
+            Strides(d_o), (float)w.scale, c10::hip::getCurrentHIPStream().stream()));
+        if (rpb.defined() && q.scalar_type() != at::kFloat) d_rpb = d_rpb.to(q.scalar_type());
+        return {dq, dk, dv, d_rpb, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+Tensor natten2d_window_autograd(const Tensor &q, const Tensor &k, const Tensor &v,
+                                const c10::optional<Tensor> &rpb, int64_t kh, int64_t kw, bool ch, bool cw,
+                                double scale) {
+    validate_window(q, k, v, rpb, Window{kh, kw, ch, cw, scale}, true);
+    return WindowFn::apply(q, k, v, rpb, kh, kw, ch, cw, scale);
+}
+Tensor natten2d_window_plain(const Tensor &q, const Tensor &k, const Tensor &v,
+                             const c10::optional<Tensor> &rpb, int64_t kh, int64_t kw, bool ch, bool cw,
+                             double scale) {
+    const Window w{kh, kw, ch, cw, scale};
+    validate_window(q, k, v, rpb, w, true);
+    return std::get<0>(window_fwd(q, k, v, rpb, w));
+}
+Tensor natten1d_window_autograd(const Tensor &q, const Tensor &k, const Tensor &v,
+                                const c10::optional<Tensor> &rpb, int64_t ks, bool causal, double scale) {
+    validate_window(q, k, v, rpb, Window{1, ks, false, causal, scale}, false);
+    return WindowFn::apply(q, k, v, rpb, (int64_t)1, ks, false, causal, scale);
+}
+Tensor natten1d_window_plain(const Tensor &q, const Tensor &k, const Tensor &v,
+                             const c10::optional<Tensor> &rpb, int64_t ks, bool causal, double scale) {
+    const Window w{1, ks, false, causal, scale};
+    validate_window(q, k, v, rpb, w, false);
+    return std::get<0>(window_fwd(q, k, v, rpb, w));
+}
+
 Tensor natten2d_autograd(const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks,
                          double scale) {
     return NattenFn<true>::apply(q, k, v, ks, scale);
@@ -318,6 +444,10 @@ TORCH_LIBRARY(enatten, m) {
           "int kernel_size, float scale) -> (Tensor, Tensor, Tensor)");
     m.def("natten2d(Tensor q, Tensor k, Tensor v, int kernel_size=7, float scale=1.0) -> Tensor");
     m.def("natten2d_dilated(Tensor q, Tensor k, Tensor v, int kernel_size, float scale, int dilation) -> Tensor");
+    m.def("natten2d_window(Tensor q, Tensor k, Tensor v, Tensor? rpb, int kh, int kw, bool causal_h, "
+          "bool causal_w, float scale) -> Tensor");
+    m.def("natten1d_window(Tensor q, Tensor k, Tensor v, Tensor? rpb, int kernel_size, bool causal, "
+          "float scale) -> Tensor");
     m.def("natten1d(Tensor q, Tensor k, Tensor v, int kernel_size=7, float scale=1.0) -> Tensor");
 }
 
@@ -328,11 +458,15 @@ TORCH_LIBRARY_IMPL(enatten, CompositeExplicitAutograd, m) {
     m.impl("na1d_bwd", &na1d_bwd);
     m.impl("natten2d", &natten2d_plain);
     m.impl("natten2d_dilated", &natten2d_dilated_plain);
+    m.impl("natten2d_window", &natten2d_window_plain);
+    m.impl("natten1d_window", &natten1d_window_plain);
     m.impl("natten1d", &natten1d_plain);
 }
 
 TORCH_LIBRARY_IMPL(enatten, Autograd, m) {
     m.impl("natten2d", &natten2d_autograd);
     m.impl("natten2d_dilated", &natten2d_dilated_autograd);
+    m.impl("natten2d_window", &natten2d_window_autograd);
+    m.impl("natten1d_window", &natten1d_window_autograd);
     m.impl("natten1d", &natten1d_autograd);
 }

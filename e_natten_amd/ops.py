@@ -385,8 +385,9 @@ class Natten2dWindow(torch.autograd.Function):
     ``kernel = (rows, columns)``, ``causal = (rows, columns)``.  On a causal axis a query
     attends the last k positions up to and including its own.  ``rpb`` is None or a
     relative position bias ``[heads, 2*rows-1, 2*columns-1]`` that is added to the scaled
-    logits (entry key - query + kernel - 1 per axis) and gets a gradient.  Served by the
-    general kernels through ``enatten2d_fwd_window`` / ``enatten2d_bwd_window``."""
+    logits (entry key - query + kernel - 1 per axis) and gets a gradient.  Served through
+    ``enatten2d_fwd_window`` / ``enatten2d_bwd_window``; ``natten2d`` and ``natten1d`` reach the
+    same calls through the native binding where that is built."""
 
     @staticmethod
     def forward(ctx, Q, K, V, rpb, kernel, causal, scale):
@@ -407,7 +408,11 @@ class Natten2dWindow(torch.autograd.Function):
 def _window_call(q, k, v, kernel, causal, scale, dilation, rpb=None):
     """Natten2dWindow on the dilation^2 strided sub-grids (see Natten2dDilated)."""
     if dilation == 1:
-        return Natten2dWindow.apply(q, k, v, rpb, kernel, causal, float(scale))
+        if not NATIVE_BINDING:
+            return Natten2dWindow.apply(q, k, v, rpb, kernel, causal, float(scale))
+        if rpb is not None and not isinstance(rpb, torch.Tensor):
+            raise TypeError("rpb must be a tensor")
+        return torch.ops.enatten.natten2d_window(q, k, v, rpb, *kernel, *causal, float(scale))
     if not isinstance(dilation, int) or isinstance(dilation, bool) or dilation < 1:
         raise ValueError("dilation must be a positive int")
     _validate_window(q, k, v, kernel, causal)
@@ -517,11 +522,14 @@ def natten1d(q, k, v, kernel_size=7, scale=1.0, dilation=1, is_causal=False, rpb
     attends keys max(t - kernel_size + 1, 0) .. t; ``rpb`` is a relative position bias
     ``[heads, 2*kernel_size-1]``."""
     if is_causal or rpb is not None:
-        _validate(q, k, v, 1, 4)
-        if not isinstance(kernel_size, int) or isinstance(kernel_size, bool):
+        if type(kernel_size) is not int:
             raise TypeError("kernel_size must be an int")
         if rpb is not None and (not isinstance(rpb, torch.Tensor) or rpb.dim() != 2):
             raise ValueError("rpb must be a [heads, 2*kernel_size-1] tensor")
+        if NATIVE_BINDING and dilation == 1:  # (checks everything else itself)
+            return torch.ops.enatten.natten1d_window(q, k, v, rpb, kernel_size, bool(is_causal),
+                                                     float(scale))
+        _validate(q, k, v, 1, 4)
         o = _window_call(q.unsqueeze(2), k.unsqueeze(2), v.unsqueeze(2), (1, kernel_size),
                          (False, bool(is_causal)), scale, dilation,
                          None if rpb is None else rpb.unsqueeze(1))

@@ -1,0 +1,52 @@
+"""1D windows of any length on the matrix cores, causal and centred, against the dense-mask oracle."""
+import pytest
+import torch
+
+from _util import BF16_REL, O, ensure_built, make_inputs
+
+pytestmark = pytest.mark.gpu
+BF16, F16 = torch.bfloat16, torch.float16
+
+
+@pytest.mark.parametrize("shape,ks,causal,dtype,layout", [
+    ((1, 2, 65, 32), 2, True, BF16, "plain"),      # smallest window with a gradient; one position past a tile
+    ((2, 1, 64, 64), 64, True, F16, "plain"),      # plain causal attention of one tile
+    ((1, 3, 200, 128), 33, True, BF16, "proj"),    # band edges inside the steps of 32 keys
+    ((1, 2, 300, 128), 300, True, F16, "plain"),   # window = sequence
+    ((2, 2, 131, 40), 16, True, BF16, "proj"),     # head_dim below a built one
+    ((1, 2, 17, 8), 5, True, F16, "plain"),        # shorter than one step of keys
+    ((4, 128, 130, 32), 70, True, BF16, "plain"),  # two groups of queries per wave, the second cut
+    ((4, 128, 200, 128), 100, True, F16, "proj"),
+    ((1, 2, 257, 64), 51, False, BF16, "proj"),    # centred: clamped windows at both ends
+    ((2, 1, 129, 128), 129, False, F16, "plain"),  # window = sequence: plain attention
+    ((8, 64, 160, 64), 97, False, BF16, "plain"),  # two groups per wave
+])
+def test_band_windows(shape, ks, causal, dtype, layout):
+    ensure_built()
+    from e_natten_amd import natten1d
+    print("case band", shape, dtype, "k=%d" % ks, "causal" if causal else "centred", layout, flush=True)
+    q, k, v, g = make_inputs(shape, dtype, seed=31)
+    scale = shape[-1] ** -0.5
+    if layout == "proj":
+        qkv = torch.stack([t.permute(0, 2, 1, 3) for t in (q, k, v)], dim=2).cuda()
+        qg, kg, vg = (t.permute(0, 2, 1, 3).requires_grad_(True) for t in qkv.unbind(2))
+    else:
+        qg, kg, vg = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    o = natten1d(qg, kg, vg, ks, scale, 1, causal)
+    got = (o, *torch.autograd.grad(o, (qg, kg, vg), g.cuda()))
+    # (a sample of the heads: every head is the same computation on other data)
+    heads = slice(0, None, max(1, shape[1] // 4))
+    qr, kr, vr = (t[-1:, heads].double().requires_grad_(True) for t in (q, k, v))
+    o_ref = O.natten2d_window_dense_mask(qr.unsqueeze(2), kr.unsqueeze(2), vr.unsqueeze(2), (1, ks),
+                                         (False, causal), scale).squeeze(2)
+    ref = (o_ref.detach(), *torch.autograd.grad(o_ref, (qr, kr, vr), g[-1:, heads].double()))
+    for name, x, r in zip(("O", "dQ", "dK", "dV"), got, ref):
+        x = x.detach()[-1:, heads].cpu()
+        err = O.rel_err(x, r)
+        # P and dS are carried to 16 bits or more: what is left is the rounding of the results
+        # (2^-9 of an element for bfloat16, 2^-12 for float16) and of O in delta
+        norm = ((x.double() - r).norm() / r.norm()).item()
+        print("   ", name, "max-abs / max %.2e" % err, "2-norm %.2e" % norm, flush=True)
+        assert err <= BF16_REL, (name, err)
+        assert norm <= (4e-3 if dtype == BF16 else 5e-4), (name, norm)
+    assert torch.equal(o, natten1d(qg, kg, vg, ks, scale, 1, causal))
