@@ -539,6 +539,8 @@ int enatten2d_fwd_window(const void *q, const void *k, const void *v, const void
     a.rpb = rpb;
     if (dtype == ENATTEN_F64) return launch_fwd_f64(a, static_cast<hipStream_t>(stream));
     if (use_band(a, dtype)) return launch_fwd_band(a, dtype, static_cast<hipStream_t>(stream));
+    if (rpb && kernel_h == kernel_w && use_mfma(D, kernel_h, dtype))
+        return launch_fwd_mfma_bias(a, dtype, static_cast<hipStream_t>(stream));
     return launch_fwd_simt(a, dtype, static_cast<hipStream_t>(stream));
 }
 
@@ -601,6 +603,8 @@ int enatten2d_bwd_window(const void *q, const void *k, const void *v, const void
     a.ds_pairs = rpb ? a.delta + (size_t)4 * B * heads * H * W : nullptr;
     if (dtype == ENATTEN_F64) return bwd_f64(fn, a, ws_floats, static_cast<hipStream_t>(stream));
     if (use_band(a, dtype)) return launch_bwd_band(a, dtype, static_cast<hipStream_t>(stream));
+    if (rpb && kernel_h == kernel_w && use_mfma(D, kernel_h, dtype))
+        return launch_bwd_mfma_bias(a, dtype, static_cast<hipStream_t>(stream));
     return launch_bwd_simt(a, dtype, static_cast<hipStream_t>(stream));
 }
 

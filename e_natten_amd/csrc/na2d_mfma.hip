@@ -7,6 +7,7 @@ namespace enatten {
 namespace {
 constexpr bool kNarrow = false;
 constexpr bool kSub = false;
+constexpr bool kBias = false;
 }
 }  // namespace enatten
 

@@ -1,0 +1,21 @@
+// The kernels of na2d_mfma_kernels.h with a relative position bias, any head dim that is a
+// multiple of 8 up to 128 (channels a tensor does not have as in na2d_mfma_narrow.hip), square
+// centred windows.
+#include "na2d_common.h"
+
+namespace enatten {
+namespace {
+constexpr bool kNarrow = true;
+constexpr bool kSub = false;
+constexpr bool kBias = true;
+}
+}  // namespace enatten
+
+#include "na2d_mfma_kernels.h"
+
+namespace enatten {
+
+int launch_fwd_mfma_bias(const FwdArgs &a, int dtype, hipStream_t st) { return fwd_dispatch(a, dtype, st); }
+int launch_bwd_mfma_bias(const BwdArgs &a, int dtype, hipStream_t st) { return bwd_dispatch(a, dtype, 0, st); }
+
+}  // namespace enatten

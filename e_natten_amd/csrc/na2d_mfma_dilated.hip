@@ -12,6 +12,7 @@ namespace enatten {
 namespace {
 constexpr bool kNarrow = true;
 constexpr bool kSub = true;
+constexpr bool kBias = false;
 }
 }  // namespace enatten
 

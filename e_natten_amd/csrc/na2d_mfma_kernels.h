@@ -129,6 +129,194 @@ __device__ __forceinline__ LaneQ lane_at(const ARGS &a, const TL &tl, int wave, 
     return q;
 }
 
+// ------------------------------------------------------------------ operands of the second products
+// Eight probabilities (or dS) of a lane as an operand: rounded to 16 bits, or, with a bias, as the
+// sum of two 16-bit terms (the value rounded, and what that left).  Calls with a bias used to run
+// with float32 probabilities on the general kernels; two terms keep what they had (bf16: 16 bits
+// of every probability, against the 8 bits of the results).
+struct TwoTerms {
+    s16x8 hi, lo;
+};
+using Op8 = std::conditional_t<kBias, TwoTerms, s16x8>;
+template <bool BF, typename OP>
+__device__ __forceinline__ void put(OP &o, int e, float x) {
+    if constexpr (std::is_same_v<OP, TwoTerms>) {
+        o.hi[e] = cvt16<BF>(x);
+        o.lo[e] = cvt16<BF>(x - cvt32<BF>(o.hi[e]));
+    } else {
+        o[e] = cvt16<BF>(x);
+    }
+}
+template <bool BF, typename OP>
+__device__ __forceinline__ float get(const OP &o, int e) {
+    if constexpr (std::is_same_v<OP, TwoTerms>) return cvt32<BF>(o.hi[e]) + cvt32<BF>(o.lo[e]);
+    else return cvt32<BF>(o[e]);
+}
+template <bool BF, typename OP>
+__device__ __forceinline__ f32x4 mfma_op(s16x8 a, const OP &b, f32x4 c) {
+    if constexpr (std::is_same_v<OP, TwoTerms>) return mfma16<BF>(a, b.lo, mfma16<BF>(a, b.hi, c));
+    else return mfma16<BF>(a, b, c);
+}
+
+// ------------------------------------------------------------------ relative position bias
+// The head's [2k-1, 2k-1] table in LDS, times log2(e), in float32, with a margin of 3 rows and
+// columns: entry (key - query + k - 1) per axis lies at (.. + 3), so that every (token of a 4x4
+// block's halo, pixel of the block) pair has an entry, in its window or not, and the place of a
+// token's entry is a lane constant plus (token row) * TB + (token column), which folds into the
+// LDS read's offset.
+template <int KS>
+struct Bias {
+    using G = Geo<32, KS>;  // (the numbering of the halo tokens depends on KS alone)
+    static constexpr int TB = 2 * KS + 5, SPAN = 2 * KS - 1, E = SPAN * SPAN;
+    // 16-token tiles that hold tokens at all, and the largest row that their numbers stand for
+    static constexpr int W2 = G::W1 ? G::SW - G::W1 : 1, A_TILES = G::W1 ? G::SW * G::W1 / 16 : 0;
+    static constexpr int USED = G::W1 ? A_TILES + (G::SW * W2 + 15) / 16 : (G::NK + 15) / 16;
+    static constexpr int MAXR = G::W1 ? ((USED - A_TILES) * 16 - 1) / W2 : (USED * 16 - 1) / G::SWC;
+    static constexpr int WORDS = (MAXR + KS + 3) * TB + 16;
+    // (token row) * TB + (token column) of token tile * 16 + x; 0 for tiles without tokens
+    static __device__ __forceinline__ int token(int tile, int x) {
+        if (tile >= USED) return 0;
+        int r, c;
+        G::tok_rc(tile, x, r, c);
+        return r * TB + c;
+    }
+    // lane constant of a query whose halo starts at (sr0, sc0): the entry of its token is query() + token()
+    static __device__ __forceinline__ int query(const LaneQ &q) {
+        return (q.hr0 + q.orow - q.qr + KS + 2) * TB + (q.hc0 + q.ocol - q.qc + KS + 2);
+    }
+};
+// A thread's share of the table on its way to LDS
+template <bool BF, int KS, int NT>
+struct BiasRegs {
+    using T = Bias<KS>;
+    static constexpr int NB = (T::E + NT - 1) / NT;
+    short v[NB];
+    __device__ __forceinline__ void fetch(const void *rpb, int head) {
+        const short *p = static_cast<const short *>(rpb) + (int64_t)head * T::E;
+#pragma unroll
+        for (int i = 0; i < NB; i++) v[i] = p[min((int)threadIdx.x + i * NT, T::E - 1)];
+    }
+    __device__ __forceinline__ void commit(float *lds) const {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const int e = min((int)threadIdx.x + i * NT, T::E - 1);  // (the same value twice at the end)
+            lds[(e / T::SPAN + 3) * T::TB + e % T::SPAN + 3] = cvt32<BF>(v[i]) * kLog2e;
+        }
+    }
+};
+// Gradient of the bias.  A tile's dS is turned through LDS, wave by wave, one row of the block's four
+// rows of queries at a time: the four queries' dS each in a plane of their own that is laid out
+// like the wave's halo, with a margin of zeros.  A lane then owns displacements (t, u) = (token row -
+// query row, token column - query column) and sums them over the planes with constant offsets.  The waves' sums
+// of a tile are added in a fixed order and left in the workspace, one row of E floats per tile;
+// rpb_tile_reduce sums the rows.  No atomics.  (Adding every dS to a table with ds_add_f32, in an order that
+// was fixed too, took 76 cycles an instruction: dQ pass at B8 N8 112x112 d32 k7 309 us.)
+template <int KS>
+struct BiasGrad {
+    using T = Bias<KS>;
+    using G = typename T::G;
+    static constexpr int P = (G::SW + 7 + 3) / 4 * 4;          // columns of a plane: c + 4, 16-byte aligned
+    static constexpr int PLANE = (G::SW + 6) * P + 4;          // rows r + 3
+    static constexpr int SIDE = G::SW + 3;                     // displacements per axis: -3 .. SW - 1
+    static constexpr int SUMS = SIDE * SIDE, PASSES = (SUMS + 63) / 64;
+    static constexpr int WORDS = 4 * PLANE + (SUMS + 3) / 4 * 4;  // per wave: planes, sums
+    template <int NT>
+    static __device__ __forceinline__ void clear(float *lds) {
+        for (int i = threadIdx.x; i < NT / 64 * WORDS; i += NT) lds[i] = 0.f;
+    }
+    // ds[tile][i]: this lane's accumulator layout (token tile * 16 + 4 g + i, query n), zero where
+    // the pair is not in the window or the query does not exist
+    static __device__ __forceinline__ void sum(float *wave_lds, const f32x4 (&ds)[T::USED], int n, int g) {
+        const int l = n + 16 * g;
+        float *plane = wave_lds + (n & 3) * PLANE + 3 * P + 4;
+        int at[PASSES];
+        float acc[PASSES];
+#pragma unroll
+        for (int j = 0; j < PASSES; j++) {
+            const int pos = min(j * 64 + l, SUMS - 1);
+            at[j] = pos / SIDE * P + pos % SIDE + 1;
+            acc[j] = 0.f;
+        }
+#pragma unroll
+        for (int qr = 0; qr < 4; qr++) {
+            if ((n >> 2) == qr) {
+#pragma unroll
+                for (int t = 0; t < T::USED; t++) {
+                    int r, c;
+                    G::tok_rc(t, g * 4, r, c);
+                    if constexpr (G::SW == 6) {
+#pragma unroll
+                        for (int i = 0; i < 4; i++)
+                            if (G::tok_rc(t, g * 4 + i, r, c)) plane[r * P + c] = ds[t][i];
+                    } else if constexpr (T::W2 == 2) {
+                        typedef float f32x2 __attribute__((ext_vector_type(2)));
+                        if (t < T::A_TILES) {
+                            *reinterpret_cast<f32x4 *>(plane + r * P + c) = ds[t];
+                        } else if (r < G::SW) {  // two tokens of row r, two of row r + 1
+                            *reinterpret_cast<f32x2 *>(plane + r * P + c) = f32x2{ds[t][0], ds[t][1]};
+                            *reinterpret_cast<f32x2 *>(plane + (r + 1) * P + c) = f32x2{ds[t][2], ds[t][3]};
+                        }
+                    } else if (r < G::SW) {
+                        *reinterpret_cast<f32x4 *>(plane + r * P + c) = ds[t];
+                    }
+                }
+            }
+            wave_fence();
+#pragma unroll
+            for (int j = 0; j < PASSES; j++)
+#pragma unroll
+                for (int qc = 0; qc < 4; qc++) acc[j] += wave_lds[at[j] + qc * PLANE + qr * P + qc];
+            wave_fence();
+        }
+#pragma unroll
+        for (int j = 0; j < PASSES; j++)
+            if (j * 64 + l < SUMS) wave_lds[4 * PLANE + j * 64 + l] = acc[j];
+    }
+    // (LDS operations of one wave complete in program order: only the compiler has to be told that lanes read
+    // what other lanes wrote)
+    static __device__ __forceinline__ void wave_fence() {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    // the waves' sums to a tile's row of the workspace
+    template <int NW>
+    static __device__ __forceinline__ void flush(const float *lds, float *row, const Tile &tl, const Shape &s) {
+        for (int e = threadIdx.x; e < T::E; e += 64 * NW) {
+            const int dy = e / T::SPAN - (KS - 1), dx = e % T::SPAN - (KS - 1);
+            float x = 0.f;
+#pragma unroll
+            for (int w = 0; w < NW; w++) {
+                const int wr0 = tl.r0 + (w >> 1) * 4, wc0 = tl.c0 + (w & 1) * 4;
+                const int t = dy + wr0 - win_start(min(wr0, s.H - 1), s.H, KS) + 3;
+                const int u = dx + wc0 - win_start(min(wc0, s.W - 1), s.W, KS) + 3;
+                const bool in = wr0 < s.H && wc0 < s.W && (unsigned)t < (unsigned)SIDE && (unsigned)u < (unsigned)SIDE;
+                const float v = lds[w * WORDS + 4 * PLANE + (in ? t * SIDE + u : 0)];
+                x += in ? v : 0.f;
+            }
+            row[e] = x;
+        }
+    }
+};
+// d_rpb[head][entry] = the sum over batch entries and tiles of the rows that the dQ pass left, in a
+// fixed order: a workgroup takes 16 entries of a head, 64 threads a strided share of the rows each.
+template <bool BIAS>
+__global__ __launch_bounds__(1024) void rpb_tile_reduce(const float *rows, float *d_rpb, int B, int N, int tiles,
+                                                        int E) {
+    __shared__ float part[1024];
+    const int n = blockIdx.x, e = blockIdx.y * 16 + threadIdx.x % 16;
+    float acc = 0.f;
+    if (e < E)
+        for (int r = threadIdx.x / 16; r < B * tiles; r += 64)
+            acc += rows[((int64_t)(r / tiles * N + n) * tiles + r % tiles) * E + e];
+    part[threadIdx.x] = acc;
+    __syncthreads();
+    for (int w = 512; w >= 16; w >>= 1) {
+        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x < 16 && e < E) d_rpb[(int64_t)n * E + e] = part[threadIdx.x];
+}
+
 // ------------------------------------------------------------------ forward
 // ROLL: walk down the columns of an image and keep the halo rows that consecutive
 // tiles share in LDS (see make_runs); otherwise a strided walk over row-major tiles
@@ -144,6 +332,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_k[G::ROWS * G::PITCH];
     __shared__ __attribute__((aligned(16))) short lds_v[G::ROWS * G::PITCH];
+    __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
 
     const Shape &s = a.s;
     const int dlim = kNarrow ? s.D : D;  // head dim of the tensors: D, or less in the build for narrow dims
@@ -160,6 +349,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void
     const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim);
     HaloRegs<D, KS, NW> kst, vst;
     s16x8 qnext[G::DS];
+    BiasRegs<BF, KS, G::NT> bst;
     // rows [y0, y0 + nr) of the halo are what LDS does not hold yet
     auto prefetch = [&](const ATile &tl, const LaneQ &lq, int y0, int nr) __attribute__((always_inline)) {
         if constexpr (ROLL) {
@@ -170,6 +360,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void
             halo_fetch<D, KS>(vst, plan, image_at(a, a.v, tl), row_step(a, a.v), col_step(a, a.v), lq.hr0, lq.hc0, s.H, s.W);
         }
         load_row_chunks(qnext, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
+        if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
     };
 
     auto pick = [&](int t) __attribute__((always_inline)) {
@@ -192,6 +383,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void
             halo_commit<D, KS>(lds_k, plan, kst);
             halo_commit<D, KS>(lds_v, plan, vst);
         }
+        if constexpr (kBias) bst.commit(lds_bias);
 #pragma unroll
         for (int ds = 0; ds < G::DS; ds++) qreg[ds] = qnext[ds];
     };
@@ -225,6 +417,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void
 
         if (FULL || lq.wave_on) {
             // logits^T [halo token][query], masked, in units of log2
+            const int bq = kBias ? Bias<KS>::query(lq) : 0;
             f32x4 acc[G::MT];
             float mx = -INFINITY;
 #pragma unroll
@@ -237,21 +430,23 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, lq.dr, lq.dc);
-                    c[i] = ok ? c[i] * sc2 : -INFINITY;
+                    float x = c[i] * sc2;
+                    if constexpr (kBias) x += lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)];
+                    c[i] = ok ? x : -INFINITY;
                     mx = fmaxf(mx, c[i]);
                 }
                 acc[mt] = c;
             }
             mx = col_max(mx);
             float sum = 0.f;
-            s16x8 pb[G::KSTEPS];
+            Op8 pb[G::KSTEPS];
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const float p = __builtin_amdgcn_exp2f(acc[mt][i] - mx);
                     sum += p;
-                    pb[mt >> 1][(mt & 1) * 4 + i] = cvt16<BF>(p);
+                    put<BF>(pb[mt >> 1], (mt & 1) * 4 + i, p);
                 }
             }
             sum = col_sum(sum);
@@ -268,8 +463,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void
                     vp[h] = G::t_row(lds_v, trow(ks * 2 + h, g * 4 + (n >> 2)), n);
 #pragma unroll
                 for (int mt = 0; mt < G::DT; mt++)
-                    o[mt] = mfma16<BF>(
-                        cat(lds_read_tr(G::t_at(vp[0], mt)), lds_read_tr(G::t_at(vp[1], mt))), pb[ks],
+                    o[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(vp[0], mt)), lds_read_tr(G::t_at(vp[1], mt))), pb[ks],
                         o[mt]);
             }
 
@@ -318,6 +512,7 @@ template <bool BF, int D, int KS, int NW = 4, bool FULL = false>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS> : 1)) void fwd2_mfma(FArgs a, int tiles_r, int tiles_c, int ntiles) {
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_x[G::ROWS * G::PITCH];
+    __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
     const Shape &s = a.s;
     const int dlim = kNarrow ? s.D : D;  // head dim of the tensors: D, or less in the build for narrow dims
     Sched sc = make_sched(ntiles, blockIdx.x, gridDim.x);
@@ -330,11 +525,13 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim);
     HaloRegs<D, KS, NW> st;
     s16x8 qnext[G::DS];
+    BiasRegs<BF, KS, G::NT> bst;
     auto fetch_rows = [&](const View &vw, const ATile &tl, const LaneQ &lq) __attribute__((always_inline)) {
         halo_fetch<D, KS>(st, plan, image_at(a, vw, tl), row_step(a, vw), col_step(a, vw), lq.hr0, lq.hc0, s.H, s.W);
     };
     auto fetch_q = [&](const ATile &tl, const LaneQ &lq) __attribute__((always_inline)) {
         load_row_chunks(qnext, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
+        if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
     };
     ATile cur = in_sub(tile_of(sc.t, tiles_r, tiles_c, s.N, G::TH), a);
     LaneQ lq = lane_at<KS>(a, cur, wave, n);
@@ -345,6 +542,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     // see fwd_mfma)
     auto commit_k = [&]() __attribute__((always_inline)) {
         halo_commit<D, KS>(lds_x, plan, st);
+        if constexpr (kBias) bst.commit(lds_bias);
 #pragma unroll
         for (int ds = 0; ds < G::DS; ds++) qreg[ds] = qnext[ds];
     };
@@ -354,9 +552,10 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
         __syncthreads();
         fetch_rows(a.v, cur, lq);
         auto trow = [&](int tile, int x) __attribute__((always_inline)) { return G::token_row(tile, x, lq.orow, lq.ocol); };
-        s16x8 pb[G::KSTEPS];
+        Op8 pb[G::KSTEPS];
         float mx = -INFINITY, sum = 0.f;
         if (FULL || lq.wave_on) {
+            const int bq = kBias ? Bias<KS>::query(lq) : 0;
             f32x4 acc[G::MT];
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
@@ -368,7 +567,9 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, lq.dr, lq.dc);
-                    c[i] = ok ? c[i] * sc2 : -INFINITY;
+                    float x = c[i] * sc2;
+                    if constexpr (kBias) x += lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)];
+                    c[i] = ok ? x : -INFINITY;
                     mx = fmaxf(mx, c[i]);
                 }
                 acc[mt] = c;
@@ -380,7 +581,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                 for (int i = 0; i < 4; i++) {
                     const float p = __builtin_amdgcn_exp2f(acc[mt][i] - mx);
                     sum += p;
-                    pb[mt >> 1][(mt & 1) * 4 + i] = cvt16<BF>(p);
+                    put<BF>(pb[mt >> 1], (mt & 1) * 4 + i, p);
                 }
             sum = col_sum(sum);
         }
@@ -412,8 +613,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                     vp[h] = G::t_row(lds_x, trow(ks * 2 + h, g * 4 + (n >> 2)), n);
 #pragma unroll
                 for (int mt = 0; mt < G::DT; mt++)
-                    o[mt] = mfma16<BF>(
-                        cat(lds_read_tr(G::t_at(vp[0], mt)), lds_read_tr(G::t_at(vp[1], mt))), pb[ks],
+                    o[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(vp[0], mt)), lds_read_tr(G::t_at(vp[1], mt))), pb[ks],
                         o[mt]);
             }
             store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(const_cast<short *>(image_at(a, a.o, cur)) + lq.qr * row_step(a, a.o) + lq.qc * col_step(a, a.o),
@@ -443,10 +643,10 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
 // the fused backward).
 // head_dim 32 with kernel_size 7 and 9: the dQ pass fits the 168 registers of three waves
 // per SIMD (LDS admits three workgroups per CU and more); B8 N2 112x112 k = 7: 27.8 -> 24.4
-// us, B4 N4 128x128 k = 9: 37.1 -> 35.0.  The forward is as fast or faster compiled for two
+// us, B4 N4 128x128 k = 9: 37.1 -> 35.0 (with a bias it spills 55 there).  The forward is as fast or faster compiled for two
 // (it then takes about 150 registers and runs three per SIMD anyway).
 template <int D, int KS, int NW>
-constexpr int kDqWaves = D == 32 && (KS == 7 || KS == 9) && NW == 4 ? 3 : Geo<D, KS, NW>::WAVES;
+constexpr int kDqWaves = D == 32 && (KS == 7 || KS == 9) && NW == 4 && !kBias ? 3 : Geo<D, KS, NW>::WAVES;
 // FULL: as in fwd_mfma (no wave switched off, no store predicated, the staged rows go to LDS at
 // the end of a tile's pass through the loop).
 template <bool BF, int D, int KS, bool FRAME, bool ROLL, int NW = 4, bool FULL = false>
@@ -456,6 +656,8 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_k[G::ROWS * G::PITCH];
     __shared__ __attribute__((aligned(16))) short lds_v[G::ROWS * G::PITCH];
+    __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
+    __shared__ __attribute__((aligned(16))) float lds_dbias[kBias ? NW * BiasGrad<KS>::WORDS : 1];
 
     const Shape &s = a.s;
     const int dlim = kNarrow ? s.D : D;  // head dim of the tensors: D, or less in the build for narrow dims
@@ -478,6 +680,8 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
     HaloRegs<D, KS, NW> kst, vst;
     s16x8 qnext[G::DS], gnext[G::DS];
     float lse_next = 0.f;
+    BiasRegs<BF, KS, G::NT> bst;
+    if constexpr (kBias) BiasGrad<KS>::template clear<G::NT>(lds_dbias);
     // rows [y0, y0 + nr) of the halo are what LDS does not hold yet
     auto prefetch = [&](const ATile &tl, const LaneQ &lq, int y0, int nr) __attribute__((always_inline)) {
         if constexpr (ROLL) {
@@ -490,6 +694,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
         load_row_chunks(qnext, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
         load_row_chunks(gnext, image_at(a, a.d_o, tl) + lq.qr * row_step(a, a.d_o) + lq.qc * col_step(a, a.d_o), g, dlim);
         lse_next = a.lse[lq.tok];
+        if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
     };
 
     ATile cur = pick(sc.t);
@@ -513,6 +718,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             greg[ds] = gnext[ds];
         }
         lse2 = lse_next * kLog2e;
+        if constexpr (kBias) bst.commit(lds_bias);
     };
     if constexpr (FULL) commit();
     for (;;) {
@@ -548,9 +754,10 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             // the largest halos it is not kept but formed a second time once delta
             // is known (measured faster there: the matrix cores are idle, the
             // registers are not).
+            const int bq = kBias ? Bias<KS>::query(lq) : 0;
             constexpr bool kKeepDp = !(G::WAVES == 1 && G::MT >= 16);
             f32x4 dp[kKeepDp ? G::MT : 1];
-            s16x8 dsb[G::KSTEPS];
+            Op8 dsb[G::KSTEPS];
             float dpart = 0.f;
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
@@ -565,13 +772,16 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, lq.dr, lq.dc);
-                    cs[i] = __builtin_amdgcn_exp2f(ok ? cs[i] * sc2 - lse2 : -INFINITY);
+                    float x = cs[i] * sc2 - lse2;
+                    if constexpr (kBias) x += lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)];
+                    cs[i] = __builtin_amdgcn_exp2f(ok ? x : -INFINITY);
                     dpart = fmaf(cs[i], cp[i], dpart);
-                    dsb[mt >> 1][(mt & 1) * 4 + i] = cvt16<BF>(cs[i]);
+                    put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, cs[i]);
                 }
                 if constexpr (kKeepDp) dp[mt] = cp;
             }
             const float delta = col_sum(dpart);
+            f32x4 ds_all[kBias ? Bias<KS>::USED : 1];
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
                 f32x4 cp;
@@ -586,11 +796,15 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                 }
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float p = cvt32<BF>(dsb[mt >> 1][(mt & 1) * 4 + i]);
-                    dsb[mt >> 1][(mt & 1) * 4 + i] = cvt16<BF>(p * (cp[i] - delta));
+                    const float p = get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i);
+                    const float ds = p * (cp[i] - delta);
+                    put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
+                    if constexpr (kBias)
+                        if (mt < Bias<KS>::USED) ds_all[mt][i] = lq.live ? ds : 0.f;
                 }
             }
 
+            if constexpr (kBias) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
             f32x4 dq[G::DT];
 #pragma unroll
             for (int mt = 0; mt < G::DT; mt++) dq[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -602,13 +816,16 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                     kp[h] = G::t_row(lds_k, trow(ks * 2 + h, g * 4 + (n >> 2)), n);
 #pragma unroll
                 for (int mt = 0; mt < G::DT; mt++)
-                    dq[mt] = mfma16<BF>(
-                        cat(lds_read_tr(G::t_at(kp[0], mt)), lds_read_tr(G::t_at(kp[1], mt))), dsb[ks],
+                    dq[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(kp[0], mt)), lds_read_tr(G::t_at(kp[1], mt))), dsb[ks],
                         dq[mt]);
             }
 
             store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale, lq.live, dlim);
             if (FULL || (lq.live && g == 0)) a.delta[lq.tok] = delta;
+        }
+        if constexpr (kBias) {
+            __syncthreads();
+            BiasGrad<KS>::template flush<NW>(lds_dbias, a.ds_pairs + (int64_t)sc.t * Bias<KS>::E, cur, s);
         }
 
         if (!more) {
@@ -647,6 +864,8 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv) *reinterpret_cast<int *>(a.zinv) = 0;
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_x[G::ROWS * G::PITCH];
+    __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
+    __shared__ __attribute__((aligned(16))) float lds_dbias[kBias ? NW * BiasGrad<KS>::WORDS : 1];
     const Shape &s = a.s;
     const int dlim = kNarrow ? s.D : D;  // head dim of the tensors: D, or less in the build for narrow dims
     Sched sc = make_sched(ntiles, blockIdx.x, gridDim.x);
@@ -662,6 +881,8 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     // phase ahead of phase 2: one spare set of row registers instead of two.
     s16x8 qreg[G::DS], gnext[G::DS];
     float lse_cur = 0.f;
+    BiasRegs<BF, KS, G::NT> bst;
+    if constexpr (kBias) BiasGrad<KS>::template clear<G::NT>(lds_dbias);
     // The last TAIL chunks of a halo are loaded when the arithmetic of the phase is over
     // (fetch_tail): where the registers do not hold a whole halo beside it.
     constexpr int TAIL = kDq2Tail<D, KS, NW>, HEAD = G::NL - TAIL;
@@ -678,6 +899,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     auto fetch_q = [&](const ATile &tl, const LaneQ &lq) __attribute__((always_inline)) {
         load_row_chunks(qreg, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
         lse_cur = a.lse[lq.tok];
+        if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
     };
 
     ATile cur = in_sub(tile_of(sc.t, ts.tiles_r, ts.tiles_c, s.N, G::TH), a);
@@ -716,6 +938,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
         fetch_tail(a.k, cur, lq);
         __syncthreads();                      // every wave has read V
         halo_commit<D, KS>(lds_x, plan, st);  // K
+        if constexpr (kBias) bst.commit(lds_bias);
         __syncthreads();
 
         const int tn = sched_peek(sc);
@@ -732,7 +955,8 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
         }
         const float lse2 = lse_cur * kLog2e;
         if (FULL || lq.wave_on) {
-            s16x8 dsb[G::KSTEPS];
+            const int bq = kBias ? Bias<KS>::query(lq) : 0;
+            Op8 dsb[G::KSTEPS];
             float dpart = 0.f;
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
@@ -744,19 +968,26 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, lq.dr, lq.dc);
-                    const float p = __builtin_amdgcn_exp2f(ok ? cs[i] * sc2 - lse2 : -INFINITY);
+                    float x = cs[i] * sc2 - lse2;
+                    if constexpr (kBias) x += lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)];
+                    const float p = __builtin_amdgcn_exp2f(ok ? x : -INFINITY);
                     dpart = fmaf(p, dp[mt][i], dpart);
-                    dsb[mt >> 1][(mt & 1) * 4 + i] = cvt16<BF>(p);
+                    put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, p);
                 }
             }
             const float delta = col_sum(dpart);
+            f32x4 ds_all[kBias ? Bias<KS>::USED : 1];
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float p = cvt32<BF>(dsb[mt >> 1][(mt & 1) * 4 + i]);
-                    dsb[mt >> 1][(mt & 1) * 4 + i] = cvt16<BF>(p * (dp[mt][i] - delta));
+                    const float p = get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i);
+                    const float ds = p * (dp[mt][i] - delta);
+                    put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
+                    if constexpr (kBias)
+                        if (mt < Bias<KS>::USED) ds_all[mt][i] = lq.live ? ds : 0.f;
                 }
+            if constexpr (kBias) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
             f32x4 dq[G::DT];
 #pragma unroll
             for (int mt = 0; mt < G::DT; mt++) dq[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -768,12 +999,15 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                     kp[h] = G::t_row(lds_x, trow(ks * 2 + h, g * 4 + (n >> 2)), n);
 #pragma unroll
                 for (int mt = 0; mt < G::DT; mt++)
-                    dq[mt] = mfma16<BF>(
-                        cat(lds_read_tr(G::t_at(kp[0], mt)), lds_read_tr(G::t_at(kp[1], mt))), dsb[ks],
+                    dq[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(kp[0], mt)), lds_read_tr(G::t_at(kp[1], mt))), dsb[ks],
                         dq[mt]);
             }
             store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale, lq.live, dlim);
             if (FULL || (lq.live && g == 0)) a.delta[lq.tok] = delta;
+        }
+        if constexpr (kBias) {
+            __syncthreads();
+            BiasGrad<KS>::template flush<NW>(lds_dbias, a.ds_pairs + (int64_t)sc.t * Bias<KS>::E, cur, s);
         }
         if (more) fetch_tail(a.v, nxt, lqn);
         if (!more) {
@@ -830,7 +1064,7 @@ __device__ __forceinline__ bool next_block(KeyBlock &b) {
 template <bool BF, int D, int KS, bool ROLL, int SP, int PART>
 __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, int ntiles, Runs rp,
                                            int block, int nblocks, short *lds_q, short *lds_g,
-                                           float2 *lds_stat, f32x4 *lds_red) {
+                                           float2 *lds_stat, f32x4 *lds_red, float *lds_bias) {
     using G = Geo<D, KS, 4, SP>;
     const Shape &s = a.s;
     const int dlim = kNarrow ? s.D : D;  // head dim of the tensors: D, or less in the build for narrow dims
@@ -861,6 +1095,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
     const HaloPlan<D, KS, 4, SP> plan = make_plan<D, KS, 4, SP>(dlim);
     HaloRegs<D, KS, 4, SP> qst, gst;
     float2 sst[G::NST];
+    BiasRegs<BF, KS, G::NT> bst;
     // ROLL: rows [y0, y0 + nr) of the block are what LDS does not hold yet
     auto prefetch = [&](const ATile &tl, int y0, int nr) __attribute__((always_inline)) {
         const int64_t img_tok = image_token(a, tl);
@@ -881,6 +1116,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
                 sst[i] = make_float2(a.lse[qt] * kLog2e, a.delta[qt]);
             }
         }
+        if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
     };
     auto commit = [&](int y0, int nr) __attribute__((always_inline)) {
         if constexpr (ROLL) {
@@ -906,7 +1142,10 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
                 if (id < G::ZROW) lds_stat[id] = sst[i];
             }
         }
+        if constexpr (kBias) bst.commit(lds_bias);
     };
+    // (entry of this lane's key and a token of its halo: bk - token, see Bias)
+    const int bk = kBias ? ((n >> 2) + KS / 2 + KS + 2) * Bias<KS>::TB + (n & 3) + KS / 2 + KS + 2 : 0;
     // B operands of a tile: this lane's key, channels ds*32 + g*8 ..  Loaded when
     // the previous tile's math is over (they would not fit beside it) and complete
     // before the barrier below, i.e. before any newer load is in flight.
@@ -949,7 +1188,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
         }
 #pragma unroll
         for (int ks = K0; ks < K1; ks++) {
-            s16x8 pb, dsb;
+            Op8 pb, dsb;
 #pragma unroll
             for (int m2 = 0; m2 < 2; m2++) {
                 const int mt = ks * 2 + m2;
@@ -965,9 +1204,11 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
                 for (int i = 0; i < 4; i++) {
                     const float2 st = lds_stat[row_of(mt, g * 4 + i)];  // query of accumulator row g*4+i
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, n >> 2, n & 3);
-                    const float p = __builtin_amdgcn_exp2f(ok ? cs[i] * sc2 - st.x : -INFINITY);
-                    pb[m2 * 4 + i] = cvt16<BF>(p);
-                    dsb[m2 * 4 + i] = cvt16<BF>(p * (cp[i] - st.y));
+                    float x = cs[i] * sc2 - st.x;
+                    if constexpr (kBias) x += lds_bias[ok ? bk - Bias<KS>::token(mt, g * 4 + i) : 0];
+                    const float p = __builtin_amdgcn_exp2f(ok ? x : -INFINITY);
+                    put<BF>(pb, m2 * 4 + i, p);
+                    put<BF>(dsb, m2 * 4 + i, p * (cp[i] - st.y));
                 }
             }
             typename G::TRow qt[2], gt[2];
@@ -979,9 +1220,9 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
             }
 #pragma unroll
             for (int mt = 0; mt < G::DT; mt++) {
-                dv[mt] = mfma16<BF>(cat(lds_read_tr(G::t_at(gt[0], mt)), lds_read_tr(G::t_at(gt[1], mt))),
+                dv[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(gt[0], mt)), lds_read_tr(G::t_at(gt[1], mt))),
                                     pb, dv[mt]);
-                dk[mt] = mfma16<BF>(cat(lds_read_tr(G::t_at(qt[0], mt)), lds_read_tr(G::t_at(qt[1], mt))),
+                dk[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(qt[0], mt)), lds_read_tr(G::t_at(qt[1], mt))),
                                     dsb, dk[mt]);
             }
         }
@@ -1033,7 +1274,8 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
 template <bool BF, int D, int KS, int SP, int KSG, bool RED_OVER>
 __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, int ntiles,
                                            int block, int nblocks, short *lds_q, short *lds_g,
-                                           float4 *lds_stat, f32x4 *lds_red, int *tile_ctr, int *lds_tile) {
+                                           float4 *lds_stat, f32x4 *lds_red, int *tile_ctr, int *lds_tile,
+                                           float *lds_bias) {
     using G = Geo<D, KSG, 4, SP>;
     const Shape &s = a.s;
     const int dlim = kNarrow ? s.D : D;  // head dim of the tensors: D, or less in the build for narrow dims
@@ -1066,6 +1308,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
     const HaloPlan<D, KSG, 4, SP> plan = make_plan<D, KSG, 4, SP>(dlim);
     HaloRegs<D, KSG, 4, SP> qst, gst;
     float2 sst[G::NST];
+    BiasRegs<BF, KS, G::NT> bst;
     // the wave's 4x4 keys of a tile: this lane's key pixel (clamped into the image)
     auto key_of = [&](const ATile &tl, int &kr, int &kc) __attribute__((always_inline)) {
         kr = min(tl.r0 + (wave >> 1) * 4 + (n >> 2), s.H - 1);
@@ -1082,6 +1325,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
             const int64_t qt = img_tok + (int64_t)r * s.W + c;
             sst[i] = make_float2(a.lse[qt] * kLog2e, a.delta[qt]);
         }
+        if constexpr (kBias) bst.fetch(a.rpb, b.tl.nn);
     };
     // B operands of the tile: this lane's key, channels ds*32 + g*8 ..
     s16x8 kreg[G::DS], vreg[G::DS];
@@ -1128,9 +1372,12 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
             // differences; the padding row's window is nowhere
             const int r = min(cur.br + id / G::HC, cur.qb - 1), c = min(cur.bc + id % G::HC, cur.cb - 1);
             const int ws = win_start(r, s.H, KS) | (win_start(c, s.W, KS) << 16);
-            if (id < G::ZROW) lds_stat[id] = make_float4(sst[i].x, sst[i].y, __int_as_float(ws), 0.f);
+            // (with a bias also the query's place in a table with TB columns, from the block's origin)
+            const int at = kBias ? (id / G::HC) * Bias<KS>::TB + id % G::HC : 0;
+            if (id < G::ZROW) lds_stat[id] = make_float4(sst[i].x, sst[i].y, __int_as_float(ws), __int_as_float(at));
             else if (id == G::ZROW) lds_stat[id] = make_float4(0.f, 0.f, __int_as_float(0x7fff7fff), 0.f);
         }
+        if constexpr (kBias) bst.commit(lds_bias);
         if (cur.first) {
 #pragma unroll
             for (int mt = 0; mt < G::DT; mt++) {
@@ -1153,6 +1400,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
         const bool wave_on = wr0 < s.H && wc0 < s.W;
         int kr, kc;
         key_of(cur.tl, kr, kc);
+        const int bk = kBias ? (kr - cur.br + KS + 2) * Bias<KS>::TB + (kc - cur.bc + KS + 2) : 0;
         if (wave_on) {
             // this wave's queries inside the staged block: those that attend to any
             // of its 4x4 keys, numbered row-major over their rectangle
@@ -1171,7 +1419,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
                 return qi < nq ? row : (int)G::ZROW;
             };
             for (int q0 = part * 32; q0 < nq; q0 += 32 * SP) {
-                s16x8 pb, dsb;
+                Op8 pb, dsb;
 #pragma unroll
                 for (int m2 = 0; m2 < 2; m2++) {
                     const int row = row_of(q0 + m2 * 16 + n);
@@ -1189,10 +1437,11 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
                         const int ws = __float_as_int(st.z);
                         const bool ok = ((unsigned)(kr - (ws & 0xffff)) < (unsigned)KS) &
                                         ((unsigned)(kc - (ws >> 16)) < (unsigned)KS);
-                        const float p =
-                            __builtin_amdgcn_exp2f(ok ? cs[i] * sc2 - st.x : -INFINITY);
-                        pb[m2 * 4 + i] = cvt16<BF>(p);
-                        dsb[m2 * 4 + i] = cvt16<BF>(p * (cp[i] - st.y));
+                        float x = cs[i] * sc2 - st.x;
+                        if constexpr (kBias) x += lds_bias[ok ? bk - __float_as_int(st.w) : 0];
+                        const float p = __builtin_amdgcn_exp2f(ok ? x : -INFINITY);
+                        put<BF>(pb, m2 * 4 + i, p);
+                        put<BF>(dsb, m2 * 4 + i, p * (cp[i] - st.y));
                     }
                 }
                 typename G::TRow qt[2], gt[2];
@@ -1204,10 +1453,8 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
                 }
 #pragma unroll
                 for (int mt = 0; mt < G::DT; mt++) {
-                    dv[mt] = mfma16<BF>(
-                        cat(lds_read_tr(G::t_at(gt[0], mt)), lds_read_tr(G::t_at(gt[1], mt))), pb, dv[mt]);
-                    dk[mt] = mfma16<BF>(
-                        cat(lds_read_tr(G::t_at(qt[0], mt)), lds_read_tr(G::t_at(qt[1], mt))), dsb, dk[mt]);
+                    dv[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(gt[0], mt)), lds_read_tr(G::t_at(gt[1], mt))), pb, dv[mt]);
+                    dk[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(qt[0], mt)), lds_read_tr(G::t_at(qt[1], mt))), dsb, dk[mt]);
                 }
             }
         }
@@ -1303,6 +1550,7 @@ __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) v
     // when their walk is over; the counter lies where the general kernels keep 1 / Z per query,
     // and the dQ pass, which runs before this one on the stream, has cleared it.
     __shared__ int lds_tile[2];
+    __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
     int *tile_ctr = dyn ? reinterpret_cast<int *>(a.zinv) : nullptr;
     if constexpr (!FRAME_ONLY) {
         if ((int)blockIdx.x < inner_blocks) {
@@ -1312,10 +1560,10 @@ __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) v
             f32x4 *lds_red = reinterpret_cast<f32x4 *>(lds_raw + 2 * I_ROWS + I_STAT);
             if (SP == 1 || threadIdx.x < 256)
                 dkdv_inner<BF, D, KS, ROLL, SP, 0>(a, ts, n_inner, rp, blockIdx.x, inner_blocks, lds_q,
-                                                   lds_g, lds_stat, lds_red);
+                                                   lds_g, lds_stat, lds_red, lds_bias);
             else  // the same number of barriers as the first part
                 dkdv_inner<BF, D, KS, ROLL, SP, SP - 1>(a, ts, n_inner, rp, blockIdx.x, inner_blocks,
-                                                        lds_q, lds_g, lds_stat, lds_red);
+                                                        lds_q, lds_g, lds_stat, lds_red, lds_bias);
             if (!dyn) return;
             __syncthreads();
         }
@@ -1327,7 +1575,7 @@ __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) v
         f32x4 *lds_red = reinterpret_cast<f32x4 *>(RED_OVER ? lds_raw : lds_raw + 2 * F_ROWS + F_STAT);
         dkdv_frame<BF, D, KS, SP, kFrameKS<D, KS, SP>, RED_OVER>(
             a, ts, n_frame, dyn ? blockIdx.x : blockIdx.x - inner_blocks,
-            dyn ? gridDim.x : gridDim.x - inner_blocks, lds_q, lds_g, lds_stat, lds_red, tile_ctr, lds_tile);
+            dyn ? gridDim.x : gridDim.x - inner_blocks, lds_q, lds_g, lds_stat, lds_red, tile_ctr, lds_tile, lds_bias);
     }
 }
 
@@ -1356,9 +1604,10 @@ bool roll_pays(int64_t ntiles, int grid) {
 template <int D, int KS>
 constexpr bool kTallBuilt =
     D == 64 && KS >= 7 &&
-    (size_t)2 * Geo<D, KS, 8>::ROWS * Geo<D, KS, 8>::PITCH * sizeof(short) <= 160 * 1024;
+    (size_t)2 * Geo<D, KS, 8>::ROWS * Geo<D, KS, 8>::PITCH * sizeof(short) +
+            (kBias ? Bias<KS>::WORDS * sizeof(float) : 0) <= 160 * 1024;
 template <int D, int KS>
-constexpr bool kTallDqBuilt = kTallBuilt<D, KS> && KS <= 9;
+constexpr bool kTallDqBuilt = kTallBuilt<D, KS> && KS <= (kBias ? 7 : 9);  // (a bias's planes take LDS too)
 
 // The dQ pass with one halo in LDS at a time (bwd_dq2_mfma): where two halos leave LDS for
 // one workgroup per CU, one halo fits twice, and the 16x8 tiles are not used.  head_dim 64
@@ -1389,9 +1638,9 @@ constexpr bool kFwd2TallBuilt = D == 128 && kOneHaloWgs<D, KS> == 1 && kOneHaloF
                                 (size_t)Geo<D, KS, 8>::ROWS * Geo<D, KS, 8>::PITCH * 2 + 1024 <= 160 * 1024;
 // At head_dim 64 (kernel_size 11 and 13, where one halo of an 8x8 tile fits LDS twice) the one-halo dQ
 // pass takes the 16x8 tiles too: one workgroup of eight waves instead of two of four, a quarter less halo
-// per pixel.  B2 N8 128x128 k13 81.5 -> 76.2 us, B4 N8 256x256 626 -> 606, B4 N4 128x128 k11 77.1 -> 76.3.
+// per pixel.  (With a bias, whose planes take LDS too, only at k11.)  B2 N8 128x128 k13 81.5 -> 76.2 us, B4 N8 256x256 626 -> 606, B4 N4 128x128 k11 77.1 -> 76.3.
 template <int D, int KS>
-constexpr bool kDq2TallBuilt = kFwd2TallBuilt<D, KS> || (D == 64 && KS >= 11);
+constexpr bool kDq2TallBuilt = (kFwd2TallBuilt<D, KS> && !kBias) || (D == 64 && KS >= 11 && !(kBias && KS == 13));
 template <int D, int KS>
 constexpr bool kFwd2Built = D == 128 && Geo<D, KS>::WAVES == 1 && kOneHaloFits<D, KS>;
 // Built at all: two halos fit, or the one-halo kernels serve the forward and the dQ pass and
@@ -1516,7 +1765,7 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
         // The fused backward wherever it is built (fused_bwd_supported): 5-25% faster than the
         // two passes at every size measured, from B64 N16 8x8 (45.7 against 47.3 us) and B4 N4
         // 32x32 (14.8 against 24.1) to B16 N8 128x128 (938 against 1174).
-        if (!kSub && !split_forced(path) && fused_bwd_supported(a)) {
+        if (!kSub && !kBias && !split_forced(path) && fused_bwd_supported(a)) {
             const int rc = launch_bwd_fused(a, BF, ts, nb, st);
             return rc ? rc : check_launch("enatten2d_bwd");
         }
@@ -1533,13 +1782,14 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
         // 56x56 52.7 vs 49.0.  So it is the default only where at most one tile in eight is an
         // inner tile (level with the two passes there, one launch less);
         // ENATTEN_PATH_MFMA_FUSED forces it wherever it is built.
-        if (!kSub && !split_forced(path) && onepass_bwd_supported(a) &&
+        if (!kSub && !kBias && !split_forced(path) && onepass_bwd_supported(a) &&
             (path == ENATTEN_PATH_MFMA_FUSED || 8 * n_inner <= nb)) {
             const int rc = launch_bwd_onepass(a, BF, ts, nb, st);
             return rc ? rc : check_launch("enatten2d_bwd");
         }
 
         bool dq_done = false;
+        int dq_tiles = tiles_r * tiles_c;  // per image, of the dQ pass
         if constexpr (kDq2TallBuilt<D, KS>) {
             using G8 = Geo<D, KS, 8>;
             TileSet tall = ts;  // only the tile counts are used by this pass
@@ -1555,6 +1805,7 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                     hipLaunchKernelGGL((bwd_dq2_mfma<BF, D, KS, 8>), dim3(grid), dim3(G8::NT), 0, st, a, tall,
                                        (int)nb8);
                 dq_done = true;
+                dq_tiles = tall.tiles_r * tiles_c;
             }
         }
         if constexpr (kDq2Built<D, KS>) {
@@ -1583,9 +1834,10 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                     hipLaunchKernelGGL((bwd_dq_mfma<BF, D, KS, false, false, 8>), dim3(grid), dim3(G8::NT),
                                        0, st, a, tall, (int)nb8, Runs{0, 0});
                 dq_done = true;
+                dq_tiles = tall.tiles_r * tiles_c;
             }
         }
-        if constexpr (fits<D, KS>()) if (!dq_done) {
+        if constexpr (fits<D, KS>() && !kDq2Built<D, KS>) if (!dq_done) {
             const int grid = persistent_grid<bwd_dq_mfma<BF, D, KS, false, false>>(nb);
             ProfScope prof(ENATTEN_KERNEL_BWD_DQ, "bwd_dq_mfma", st);
             const bool full = !kNarrow && a.s.H % G::TH == 0 && a.s.W % G::TW == 0;
@@ -1684,6 +1936,9 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                 hipLaunchKernelGGL((bwd_dkdv_mfma<BF, D, KS, false, SP>), dim3(grid), dim3(NT), 0, st,
                                    a, ts, (int)n_inner, (int)n_frame, inner_blocks, Runs{0, 0}, dyn);
         }
+        if constexpr (kBias)
+            hipLaunchKernelGGL((rpb_tile_reduce<kBias>), dim3(a.s.N, (Bias<KS>::E + 15) / 16), dim3(1024), 0, st,
+                               a.ds_pairs, a.d_rpb, a.s.B, a.s.N, dq_tiles, Bias<KS>::E);
         return check_launch("enatten2d_bwd");
     } else {
         set_error("no matrix-core kernel for head_dim %d, kernel_size %d", D, KS);

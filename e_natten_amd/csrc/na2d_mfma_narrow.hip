@@ -9,6 +9,7 @@ namespace enatten {
 namespace {
 constexpr bool kNarrow = true;
 constexpr bool kSub = false;
+constexpr bool kBias = false;
 }
 }  // namespace enatten
 

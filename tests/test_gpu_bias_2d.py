@@ -1,0 +1,57 @@
+"""Relative position bias on the matrix-core kernels, against the dense-mask oracle."""
+import pytest
+import torch
+
+from _util import BF16_REL, O, ensure_built, make_inputs
+
+pytestmark = pytest.mark.gpu
+BF16, F16 = torch.bfloat16, torch.float16
+
+
+@pytest.mark.parametrize("shape,ks,dtype,layout", [
+    ((2, 3, 14, 14, 32), 7, BF16, "proj"),      # border tiles only
+    ((1, 2, 41, 35, 32), 5, F16, "plain"),      # inner tiles, ragged sides
+    ((1, 2, 33, 30, 32), 3, BF16, "plain"),     # 6 tokens to a row: lane groups take turns
+    ((2, 2, 40, 48, 64), 9, BF16, "proj"),      # tokens in two blocks, four to a row in the second
+    ((8, 16, 32, 40, 64), 7, F16, "plain"),     # 16x8 tiles
+    ((1, 2, 30, 41, 48), 7, BF16, "proj"),      # head_dim below a built one
+    ((1, 2, 40, 31, 64), 13, BF16, "plain"),    # 16 tokens to a row, two waves per block of keys
+    ((4, 20, 32, 40, 64), 11, F16, "plain"),    # one halo in LDS at a time, 16x8 tiles
+    ((1, 2, 24, 32, 128), 5, BF16, "plain"),
+    ((1, 1, 26, 29, 128), 9, F16, "proj"),      # one halo in LDS at a time
+    ((1, 1, 22, 13, 128), 13, BF16, "plain"),   # frame body only; window = image on one axis
+    ((1, 2, 5, 5, 16), 5, F16, "plain"),        # window = image
+])
+def test_bias(shape, ks, dtype, layout):
+    ensure_built()
+    from e_natten_amd import natten2d
+    print("case bias", shape, dtype, "k=%d" % ks, layout, flush=True)
+    q, k, v, g = make_inputs(shape, dtype, seed=37)
+    scale = shape[-1] ** -0.5
+    gen = torch.Generator().manual_seed(5)
+    rpb = torch.randn(shape[1], 2 * ks - 1, 2 * ks - 1, generator=gen).to(dtype)
+    if layout == "proj":
+        qkv = torch.stack([t.permute(0, 2, 3, 1, 4) for t in (q, k, v)], dim=3).cuda()
+        qg, kg, vg = (t.permute(0, 3, 1, 2, 4).requires_grad_(True) for t in qkv.unbind(3))
+    else:
+        qg, kg, vg = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    bg = rpb.cuda().requires_grad_(True)
+    o = natten2d(qg, kg, vg, ks, scale, rpb=bg)
+    got = (o, *torch.autograd.grad(o, (qg, kg, vg, bg), g.cuda()))
+    # (the last heads only where there are many: a head is the same computation on other data; its
+    # bias gradient sums over the whole batch)
+    heads = slice(max(0, shape[1] - 3), None)
+    qr, kr, vr, br = (t[:, heads].double().requires_grad_(True) for t in (q, k, v, rpb.unsqueeze(0)))
+    o_ref = O.natten2d_window_dense_mask(qr, kr, vr, (ks, ks), scale=scale, rpb=br[0])
+    ref = (o_ref.detach(), *torch.autograd.grad(o_ref, (qr, kr, vr, br), g[:, heads].double()))
+    for name, x, r in zip(("O", "dQ", "dK", "dV", "dRPB"), got, ref):
+        x = x.detach()
+        x = (x[:, heads] if name != "dRPB" else x[heads].unsqueeze(0)).cpu()
+        err, norm = O.rel_err(x, r), ((x.double() - r).norm() / r.norm()).item()
+        print("   ", name, "max-abs / max %.2e" % err, "2-norm %.2e" % norm, flush=True)
+        assert err <= BF16_REL, (name, err)
+        # P and dS are carried to 16 bits or more: what is left is the rounding of the results (2^-9
+        # of an element for bfloat16, 2^-12 for float16)
+        assert norm <= (4e-3 if dtype == BF16 else 5e-4), (name, norm)
+    again = torch.autograd.grad(natten2d(qg, kg, vg, ks, scale, rpb=bg), (qg, kg, vg, bg), g.cuda())
+    assert all(torch.equal(a, b) for a, b in zip(again, got[1:])), "not bit-reproducible"
