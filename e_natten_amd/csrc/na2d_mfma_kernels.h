@@ -327,8 +327,12 @@ __global__ __launch_bounds__(1024) void rpb_tile_reduce(const float *rows, float
 // not wait for the stores as well.  With a branch around the stores, even a uniform one with
 // an explicit wait on its other side, it falls back to waiting for everything outstanding
 // (B4 N4 128x128 d128 k5: 58.8 -> 56.7 us, 256x256: 198.2 -> 189.3, d64 k5: 60.4 -> 58.5).
+// With a bias the head_dim 32 forward takes 169 to 175 registers (k = 7 and 9), one more than three
+// waves per SIMD have: budgeted for three, B8 N8 112x112 k7 114.8 -> 97.8 us.
+template <int D, int KS, int NW>
+constexpr int kFwdWaves = kBias && D == 32 && KS <= 9 ? 3 : Geo<D, KS, NW>::WAVES;
 template <bool BF, int D, int KS, bool ROLL, int NW = 4, bool FULL = false>
-__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (Geo<D, KS, NW>::WAVES)) void fwd_mfma(FArgs a, int tiles_r, int tiles_c, int ntiles, Runs rp) {
+__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void fwd_mfma(FArgs a, int tiles_r, int tiles_c, int ntiles, Runs rp) {
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_k[G::ROWS * G::PITCH];
     __shared__ __attribute__((aligned(16))) short lds_v[G::ROWS * G::PITCH];
@@ -1511,7 +1515,8 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
 // Waves per SIMD that the dK/dV pass budgets its registers for: three where LDS admits
 // three workgroups per CU (head_dim <= 64 with small halos; it fits 168 registers there,
 // measured 35 -> 32 us at B8 N2 112x112 d32 k7 and 67 -> 60 us at B4 N4 128x128 d32 k9;
-// the forward and the dQ pass spill under that budget and get slower).
+// the forward and the dQ pass spill under that budget and get slower; with a bias so does this
+// one at head_dim 64: B8 N8 64x64 k5 60 us with two waves, 84 with three).
 // Size of the frame body's blocks as a kernel size (see dkdv_frame): larger than KS where the
 // pass has one workgroup per CU anyway (two parts per block) and LDS has the room.
 // Where not even one workgroup's Q and dO halos fit LDS (head_dim 128 with kernel_size 11 and
@@ -1524,7 +1529,7 @@ constexpr int kFrameKS = kDkdvFrameOnly<D, KS> ? 5 : SP == 2 && KS >= 9 ? 9 + KS
 template <int D, int KS, int SP>
 constexpr int kDkdvWaves =
     kDkdvFrameOnly<D, KS> ? 2 :
-    SP == 1 && D <= 64 && 3 * (Geo<D, KS>::LDS_BYTES + 2048) <= 160 * 1024 ? 3 : Geo<D, KS, 4, SP>::WAVES;
+    SP == 1 && D <= (kBias ? 32 : 64) && 3 * (Geo<D, KS>::LDS_BYTES + 2048) <= 160 * 1024 ? 3 : Geo<D, KS, 4, SP>::WAVES;
 template <bool BF, int D, int KS, bool ROLL, int SP = 1>
 __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) void bwd_dkdv_mfma(
     BArgs a, TileSet ts, int n_inner, int n_frame, int inner_blocks, Runs rp, int dyn) {
