@@ -13,8 +13,10 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/library.h>
 
+#include <algorithm>
 #include <tuple>
 
 #include "enatten.h"
@@ -228,16 +230,33 @@ struct NattenFn : public torch::autograd::Function<NattenFn<TWO_D>> {
     }
 };
 
-// Dilated neighborhoods: the contract of enatten2d_fwd_dilated, with an autograd node of its own.
-// The output is contiguous.
-void validate_dilation(const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks, int64_t dil) {
-    validate("enatten::natten2d_dilated", q, k, v, ks, 5);
-    TORCH_CHECK_VALUE(dil >= 1, "enatten::natten2d_dilated: dilation must be >= 1, got ", dil);
-    TORCH_CHECK(q.is_cuda(), "enatten::natten2d_dilated: tensors must be on the GPU; this build has no CPU path");
+// Gradients that carry no graph of their own.  Where the upstream gradient requires one
+// (create_graph), they are handed on through a node that raises when it is differentiated, as a
+// Python function marked once_differentiable does, instead of counting as constants.
+variable_list once_differentiable(variable_list out, const variable_list &grads) {
+    bool wanted = false;
+    for (const Tensor &g : grads) wanted = wanted || (g.defined() && g.requires_grad());
+    if (!wanted || !at::GradMode::is_enabled()) return out;
+    for (Tensor &t : out)
+        if (t.defined()) t = t.detach().set_requires_grad(true);
+    return torch::autograd::DelayedError("the gradients of this operator cannot be differentiated again",
+                                         (int64_t)out.size())(std::move(out));
 }
-std::tuple<Tensor, Tensor> dilated_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, int64_t ks,
-                                       double scale, int64_t dil) {
-    validate_dilation(q_, k_, v_, ks, dil);
+
+// Dilated neighborhoods: the contract of enatten2d_fwd_dilated.  The output is contiguous.
+void validate_dilation(const char *what, const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks,
+                       int64_t dil) {
+    validate(what, q, k, v, ks, 5);
+    TORCH_CHECK_VALUE(dil >= 1, what, ": dilation must be >= 1, got ", dil);
+    TORCH_CHECK_VALUE(std::min(q.size(2), q.size(3)) / dil >= ks, what, ": input of extent ",
+                      q.sizes().slice(2, 2), " is smaller than kernel_size * dilation = ", ks, " * ", dil);
+}
+std::tuple<Tensor, Tensor> na2d_dilated_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_,
+                                            int64_t ks, double scale, int64_t dil) {
+    validate_dilation("enatten::na2d_dilated_fwd", q_, k_, v_, ks, dil);
+    if (q_.is_meta())
+        return {at::empty(q_.sizes(), q_.options()),
+                at::empty(q_.sizes().slice(0, 4), q_.options().dtype(at::kFloat))};
     const c10::DeviceGuard guard(q_.device());
     const Tensor q = kernel_layout(q_), k = kernel_layout(k_), v = kernel_layout(v_);
     const int B = q.size(0), N = q.size(1), H = q.size(2), W = q.size(3), D = q.size(4);
@@ -245,16 +264,50 @@ std::tuple<Tensor, Tensor> dilated_fwd(const Tensor &q_, const Tensor &k_, const
     Tensor lse = at::empty({B, N, H, W}, q.options().dtype(at::kFloat));
     check_rc(enatten2d_fwd_dilated(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                                    lse.data_ptr<float>(), B, N, H, W, D, (int)ks, (int)dil, dtype_code(q),
-                                   q.strides().data(), k.strides().data(), v.strides().data(), nullptr,
-                                   (float)scale, c10::hip::getCurrentHIPStream().stream()));
+                                   q.strides().data(), k.strides().data(), v.strides().data(),
+                                   o.strides().data(), (float)scale,
+                                   c10::hip::getCurrentHIPStream().stream()));
     return {o, lse};
+}
+std::tuple<Tensor, Tensor, Tensor> na2d_dilated_bwd(const Tensor &q_, const Tensor &k_, const Tensor &v_,
+                                                    const Tensor &o_, const Tensor &lse_,
+                                                    const Tensor &d_o_, int64_t ks, double scale,
+                                                    int64_t dil) {
+    validate_dilation("enatten::na2d_dilated_bwd", q_, k_, v_, ks, dil);
+    check_bwd_extras("enatten::na2d_dilated_bwd", q_, o_, d_o_);
+    if (q_.is_meta()) {
+        const Tensor g = at::empty(q_.sizes(), q_.options());
+        return {g, at::empty_like(g), at::empty_like(g)};
+    }
+    const c10::DeviceGuard guard(q_.device());
+    const Tensor q = kernel_layout(q_), k = kernel_layout(k_), v = kernel_layout(v_);
+    const Tensor o = kernel_layout(o_), d_o = kernel_layout(d_o_), lse = lse_.contiguous();
+    const int B = q.size(0), N = q.size(1), H = q.size(2), W = q.size(3), D = q.size(4);
+    Tensor dq = at::empty(q.sizes(), q.options());
+    Tensor dk = at::empty_like(dq), dv = at::empty_like(dq);
+    Tensor ws = at::empty({(int64_t)enatten2d_bwd_dilated_workspace_bytes(B, N, H, W, dtype_code(q))},
+                          q.options().dtype(at::kByte));
+    check_rc(enatten2d_bwd_dilated(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr<float>(),
+        dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), B, N, H, W, D, (int)ks, (int)dil,
+        dtype_code(q), q.strides().data(), k.strides().data(), v.strides().data(), o.strides().data(),
+        d_o.strides().data(), (float)scale, c10::hip::getCurrentHIPStream().stream()));
+    return {dq, dk, dv};
+}
+// (through the dispatcher, as call_fwd and call_bwd)
+std::tuple<Tensor, Tensor> call_dilated_fwd(const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks,
+                                            double scale, int64_t dil) {
+    static const auto op = c10::Dispatcher::singleton()
+                               .findSchemaOrThrow("enatten::na2d_dilated_fwd", "")
+                               .typed<decltype(na2d_dilated_fwd)>();
+    return op.call(q, k, v, ks, scale, dil);
 }
 struct DilatedFn : public torch::autograd::Function<DilatedFn> {
     static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v,
                           int64_t ks, double scale, int64_t dil) {
         at::AutoDispatchBelowADInplaceOrView below;
         Tensor o, lse;
-        std::tie(o, lse) = dilated_fwd(q, k, v, ks, scale, dil);
+        std::tie(o, lse) = call_dilated_fwd(q, k, v, ks, scale, dil);
         ctx->save_for_backward({q, k, v, o, lse});
         ctx->saved_data["kernel_size"] = ks;
         ctx->saved_data["scale"] = scale;
@@ -265,22 +318,15 @@ struct DilatedFn : public torch::autograd::Function<DilatedFn> {
         const variable_list s = ctx->get_saved_variables();
         const int64_t ks = ctx->saved_data["kernel_size"].toInt(), dil = ctx->saved_data["dilation"].toInt();
         const double scale = ctx->saved_data["scale"].toDouble();
-        at::AutoDispatchBelowADInplaceOrView below;
-        const c10::DeviceGuard guard(s[0].device());
-        check_bwd_extras("enatten::natten2d_dilated", s[0], s[3], grads[0]);
-        const Tensor q = kernel_layout(s[0]), k = kernel_layout(s[1]), v = kernel_layout(s[2]);
-        const Tensor &o = s[3], &lse = s[4], d_o = kernel_layout(grads[0]);
-        const int B = q.size(0), N = q.size(1), H = q.size(2), W = q.size(3), D = q.size(4);
-        Tensor dq = at::empty(q.sizes(), q.options());
-        Tensor dk = at::empty_like(dq), dv = at::empty_like(dq);
-        Tensor ws = at::empty({(int64_t)enatten2d_bwd_dilated_workspace_bytes(B, N, H, W, dtype_code(q))},
-                              q.options().dtype(at::kByte));
-        check_rc(enatten2d_bwd_dilated(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr<float>(),
-            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), B, N, H, W, D, (int)ks, (int)dil,
-            dtype_code(q), q.strides().data(), k.strides().data(), v.strides().data(), o.strides().data(),
-            d_o.strides().data(), (float)scale, c10::hip::getCurrentHIPStream().stream()));
-        return {dq, dk, dv, Tensor(), Tensor(), Tensor()};
+        static const auto op = c10::Dispatcher::singleton()
+                                   .findSchemaOrThrow("enatten::na2d_dilated_bwd", "")
+                                   .typed<decltype(na2d_dilated_bwd)>();
+        Tensor dq, dk, dv;
+        {
+            at::AutoDispatchBelowADInplaceOrView below;
+            std::tie(dq, dk, dv) = op.call(s[0], s[1], s[2], s[3], s[4], grads[0], ks, scale, dil);
+        }
+        return once_differentiable({dq, dk, dv, Tensor(), Tensor(), Tensor()}, grads);
     }
 };
 Tensor natten2d_dilated_autograd(const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks,
@@ -289,7 +335,7 @@ Tensor natten2d_dilated_autograd(const Tensor &q, const Tensor &k, const Tensor 
 }
 Tensor natten2d_dilated_plain(const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks,
                               double scale, int64_t dil) {
-    return std::get<0>(dilated_fwd(q, k, v, ks, scale, dil));
+    return std::get<0>(call_dilated_fwd(q, k, v, ks, scale, dil));
 }
 
 // Rectangular and causal windows and the relative position bias (enatten2d_fwd_window): the
@@ -321,7 +367,8 @@ void validate_window(const Tensor &q, const Tensor &k, const Tensor &v, const c1
                           ": rpb must have the dtype and device of q");
         TORCH_CHECK_VALUE(!w.ch && !w.cw, what, ": a relative position bias goes with centred axes only");
     }
-    TORCH_CHECK(q.is_cuda(), what, ": tensors must be on the GPU; this build has no CPU path");
+    TORCH_CHECK(q.is_cuda() || q.is_meta(), what,
+                ": tensors must be on the GPU; this build has no CPU path");
 }
 // (batch, head, row, column) extents and strides of a tensor; a sequence is an image of one row
 struct Image {
@@ -335,29 +382,73 @@ struct Strides {
         : s{t.stride(0), t.stride(1), t.dim() == 5 ? t.stride(2) : 0, t.stride(-2)} {}
     operator const int64_t *() const { return s; }
 };
-std::tuple<Tensor, Tensor> window_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_,
-                                      const c10::optional<Tensor> &rpb_, const Window &w) {
+// One pair of operators for both: [B, heads, H, W, d] or [B, heads, T, d] with kh = 1, ch = false.
+std::tuple<Tensor, Tensor> na_window_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_,
+                                         const c10::optional<Tensor> &rpb_, int64_t kh, int64_t kw, bool ch,
+                                         bool cw, double scale) {
+    const bool two_d = q_.dim() == 5;
+    validate_window(q_, k_, v_, rpb_, Window{kh, kw, ch, cw, scale}, two_d);
+    const Image im(q_);
+    const auto lse_of = [&] { return at::empty({im.B, im.N, im.H, im.W}, q_.options().dtype(at::kFloat)); };
+    if (q_.is_meta()) return {kernel_layout(at::empty_like(kernel_layout(q_))), lse_of()};
     const c10::DeviceGuard guard(q_.device());
     const Tensor q = kernel_layout(q_), k = kernel_layout(k_), v = kernel_layout(v_);
     const Tensor rpb = rpb_.has_value() ? rpb_->contiguous() : Tensor();
-    const Image im(q);
-    Tensor o = kernel_layout(at::empty_like(q));
-    Tensor lse = at::empty({im.B, im.N, im.H, im.W}, q.options().dtype(at::kFloat));
+    Tensor o = kernel_layout(at::empty_like(q)), lse = lse_of();
     check_rc(enatten2d_fwd_window(q.data_ptr(), k.data_ptr(), v.data_ptr(),
                                   rpb.defined() ? rpb.data_ptr() : nullptr, o.data_ptr(), lse.data_ptr<float>(),
-                                  im.B, im.N, im.H, im.W, im.D, (int)w.kh, (int)w.kw, w.ch, w.cw, dtype_code(q),
-                                  Strides(q), Strides(k), Strides(v), Strides(o), (float)w.scale,
+                                  im.B, im.N, im.H, im.W, im.D, (int)kh, (int)kw, ch, cw, dtype_code(q),
+                                  Strides(q), Strides(k), Strides(v), Strides(o), (float)scale,
                                   c10::hip::getCurrentHIPStream().stream()));
     return {o, lse};
+}
+// (dQ, dK, dV, dRPB); without a bias the last one is empty
+std::tuple<Tensor, Tensor, Tensor, Tensor> na_window_bwd(const Tensor &q_, const Tensor &k_, const Tensor &v_,
+                                                         const c10::optional<Tensor> &rpb_, const Tensor &o_,
+                                                         const Tensor &lse_, const Tensor &d_o_, int64_t kh,
+                                                         int64_t kw, bool ch, bool cw, double scale) {
+    validate_window(q_, k_, v_, rpb_, Window{kh, kw, ch, cw, scale}, q_.dim() == 5);
+    check_bwd_extras("enatten::na_window_bwd", q_, o_, d_o_);
+    const bool bias = rpb_.has_value();
+    Tensor dq, dk, dv, d_rpb;
+    const c10::DeviceGuard guard(q_.device());
+    dq = at::empty(q_.sizes(), q_.options());
+    dk = at::empty_like(dq), dv = at::empty_like(dq);
+    d_rpb = at::empty(bias ? rpb_->sizes() : at::IntArrayRef({0}), q_.options().dtype(at::kFloat));
+    if (!q_.is_meta()) {
+        const Tensor q = kernel_layout(q_), k = kernel_layout(k_), v = kernel_layout(v_);
+        const Tensor o = kernel_layout(o_), d_o = kernel_layout(d_o_), lse = lse_.contiguous();
+        const Tensor rpb = bias ? rpb_->contiguous() : Tensor();
+        const Image im(q);
+        Tensor ws = at::empty({(int64_t)enatten2d_bwd_window_workspace_bytes(im.B, im.N, im.H, im.W, (int)kh,
+                                                                             (int)kw, bias)},
+                              q.options().dtype(at::kByte));
+        check_rc(enatten2d_bwd_window(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), bias ? rpb.data_ptr() : nullptr, o.data_ptr(),
+            d_o.data_ptr(), lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+            bias ? d_rpb.data_ptr<float>() : nullptr, ws.data_ptr(), im.B, im.N, im.H, im.W, im.D, (int)kh,
+            (int)kw, ch, cw, dtype_code(q), Strides(q), Strides(k), Strides(v), Strides(o), Strides(d_o),
+            (float)scale, c10::hip::getCurrentHIPStream().stream()));
+    }
+    if (bias && q_.scalar_type() != at::kFloat) d_rpb = d_rpb.to(q_.scalar_type());
+    return {dq, dk, dv, d_rpb};
+}
+// (through the dispatcher, as call_fwd and call_bwd)
+std::tuple<Tensor, Tensor> call_window_fwd(const Tensor &q, const Tensor &k, const Tensor &v,
+                                           const c10::optional<Tensor> &rpb, int64_t kh, int64_t kw, bool ch,
+                                           bool cw, double scale) {
+    static const auto op = c10::Dispatcher::singleton()
+                               .findSchemaOrThrow("enatten::na_window_fwd", "")
+                               .typed<decltype(na_window_fwd)>();
+    return op.call(q, k, v, rpb, kh, kw, ch, cw, scale);
 }
 struct WindowFn : public torch::autograd::Function<WindowFn> {
     static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v,
                           const c10::optional<Tensor> &rpb, int64_t kh, int64_t kw, bool ch, bool cw,
                           double scale) {
         at::AutoDispatchBelowADInplaceOrView below;
-        const Window w{kh, kw, ch, cw, scale};
         Tensor o, lse;
-        std::tie(o, lse) = window_fwd(q, k, v, rpb, w);
+        std::tie(o, lse) = call_window_fwd(q, k, v, rpb, kh, kw, ch, cw, scale);
         ctx->save_for_backward({q, k, v, o, lse, rpb.has_value() ? *rpb : Tensor()});
         ctx->saved_data["kh"] = kh;
         ctx->saved_data["kw"] = kw;
@@ -368,29 +459,20 @@ struct WindowFn : public torch::autograd::Function<WindowFn> {
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const variable_list s = ctx->get_saved_variables();
         const int64_t causal = ctx->saved_data["causal"].toInt();
-        const Window w{ctx->saved_data["kh"].toInt(), ctx->saved_data["kw"].toInt(), (causal & 1) != 0,
-                       (causal & 2) != 0, ctx->saved_data["scale"].toDouble()};
-        at::AutoDispatchBelowADInplaceOrView below;
-        const c10::DeviceGuard guard(s[0].device());
-        check_bwd_extras("natten", s[0], s[3], grads[0]);
-        const Tensor q = kernel_layout(s[0]), k = kernel_layout(s[1]), v = kernel_layout(s[2]);
-        const Tensor &o = s[3], &lse = s[4], d_o = kernel_layout(grads[0]);
-        const Tensor rpb = s[5].defined() ? s[5].contiguous() : Tensor();
-        const Image im(q);
-        Tensor dq = at::empty(q.sizes(), q.options());
-        Tensor dk = at::empty_like(dq), dv = at::empty_like(dq);
-        Tensor d_rpb = rpb.defined() ? at::empty(rpb.sizes(), q.options().dtype(at::kFloat)) : Tensor();
-        Tensor ws = at::empty({(int64_t)enatten2d_bwd_window_workspace_bytes(im.B, im.N, im.H, im.W, (int)w.kh,
-                                                                             (int)w.kw, rpb.defined())},
-                              q.options().dtype(at::kByte));
-        check_rc(enatten2d_bwd_window(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), rpb.defined() ? rpb.data_ptr() : nullptr, o.data_ptr(),
-            d_o.data_ptr(), lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-            rpb.defined() ? d_rpb.data_ptr<float>() : nullptr, ws.data_ptr(), im.B, im.N, im.H, im.W, im.D,
-            (int)w.kh, (int)w.kw, w.ch, w.cw, dtype_code(q), Strides(q), Strides(k), Strides(v), Strides(o),
-            Strides(d_o), (float)w.scale, c10::hip::getCurrentHIPStream().stream()));
-        if (rpb.defined() && q.scalar_type() != at::kFloat) d_rpb = d_rpb.to(q.scalar_type());
-        return {dq, dk, dv, d_rpb, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        const c10::optional<Tensor> rpb = s[5].defined() ? c10::optional<Tensor>(s[5]) : c10::nullopt;
+        static const auto op = c10::Dispatcher::singleton()
+                                   .findSchemaOrThrow("enatten::na_window_bwd", "")
+                                   .typed<decltype(na_window_bwd)>();
+        Tensor dq, dk, dv, d_rpb;
+        {
+            at::AutoDispatchBelowADInplaceOrView below;
+            std::tie(dq, dk, dv, d_rpb) =
+                op.call(s[0], s[1], s[2], rpb, s[3], s[4], grads[0], ctx->saved_data["kh"].toInt(),
+                        ctx->saved_data["kw"].toInt(), (causal & 1) != 0, (causal & 2) != 0,
+                        ctx->saved_data["scale"].toDouble());
+        }
+        return once_differentiable({dq, dk, dv, rpb.has_value() ? d_rpb : Tensor(), Tensor(), Tensor(),
+                                    Tensor(), Tensor(), Tensor()}, grads);
     }
 };
 Tensor natten2d_window_autograd(const Tensor &q, const Tensor &k, const Tensor &v,
@@ -402,9 +484,8 @@ Tensor natten2d_window_autograd(const Tensor &q, const Tensor &k, const Tensor &
 Tensor natten2d_window_plain(const Tensor &q, const Tensor &k, const Tensor &v,
                              const c10::optional<Tensor> &rpb, int64_t kh, int64_t kw, bool ch, bool cw,
                              double scale) {
-    const Window w{kh, kw, ch, cw, scale};
-    validate_window(q, k, v, rpb, w, true);
-    return std::get<0>(window_fwd(q, k, v, rpb, w));
+    validate_window(q, k, v, rpb, Window{kh, kw, ch, cw, scale}, true);
+    return std::get<0>(call_window_fwd(q, k, v, rpb, kh, kw, ch, cw, scale));
 }
 Tensor natten1d_window_autograd(const Tensor &q, const Tensor &k, const Tensor &v,
                                 const c10::optional<Tensor> &rpb, int64_t ks, bool causal, double scale) {
@@ -413,9 +494,8 @@ Tensor natten1d_window_autograd(const Tensor &q, const Tensor &k, const Tensor &
 }
 Tensor natten1d_window_plain(const Tensor &q, const Tensor &k, const Tensor &v,
                              const c10::optional<Tensor> &rpb, int64_t ks, bool causal, double scale) {
-    const Window w{1, ks, false, causal, scale};
-    validate_window(q, k, v, rpb, w, false);
-    return std::get<0>(window_fwd(q, k, v, rpb, w));
+    validate_window(q, k, v, rpb, Window{1, ks, false, causal, scale}, false);
+    return std::get<0>(call_window_fwd(q, k, v, rpb, 1, ks, false, causal, scale));
 }
 
 Tensor natten2d_autograd(const Tensor &q, const Tensor &k, const Tensor &v, int64_t ks,
@@ -442,6 +522,14 @@ TORCH_LIBRARY(enatten, m) {
     m.def("na1d_fwd(Tensor q, Tensor k, Tensor v, int kernel_size, float scale) -> (Tensor, Tensor)");
     m.def("na1d_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor d_o, "
           "int kernel_size, float scale) -> (Tensor, Tensor, Tensor)");
+    m.def("na2d_dilated_fwd(Tensor q, Tensor k, Tensor v, int kernel_size, float scale, int dilation) "
+          "-> (Tensor, Tensor)");
+    m.def("na2d_dilated_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor d_o, "
+          "int kernel_size, float scale, int dilation) -> (Tensor, Tensor, Tensor)");
+    m.def("na_window_fwd(Tensor q, Tensor k, Tensor v, Tensor? rpb, int kh, int kw, bool causal_h, "
+          "bool causal_w, float scale) -> (Tensor, Tensor)");
+    m.def("na_window_bwd(Tensor q, Tensor k, Tensor v, Tensor? rpb, Tensor o, Tensor lse, Tensor d_o, "
+          "int kh, int kw, bool causal_h, bool causal_w, float scale) -> (Tensor, Tensor, Tensor, Tensor)");
     m.def("natten2d(Tensor q, Tensor k, Tensor v, int kernel_size=7, float scale=1.0) -> Tensor");
     m.def("natten2d_dilated(Tensor q, Tensor k, Tensor v, int kernel_size, float scale, int dilation) -> Tensor");
     m.def("natten2d_window(Tensor q, Tensor k, Tensor v, Tensor? rpb, int kh, int kw, bool causal_h, "
@@ -456,6 +544,10 @@ TORCH_LIBRARY_IMPL(enatten, CompositeExplicitAutograd, m) {
     m.impl("na2d_bwd", &na2d_bwd);
     m.impl("na1d_fwd", &na1d_fwd);
     m.impl("na1d_bwd", &na1d_bwd);
+    m.impl("na2d_dilated_fwd", &na2d_dilated_fwd);
+    m.impl("na2d_dilated_bwd", &na2d_dilated_bwd);
+    m.impl("na_window_fwd", &na_window_fwd);
+    m.impl("na_window_bwd", &na_window_bwd);
     m.impl("natten2d", &natten2d_plain);
     m.impl("natten2d_dilated", &natten2d_dilated_plain);
     m.impl("natten2d_window", &natten2d_window_plain);

@@ -72,6 +72,16 @@ def _require_gpu(t: torch.Tensor, what: str) -> None:
         raise RuntimeError("%s: tensors must be on the GPU; this build has no CPU path" % what)
 
 
+def _window_operands(q, k, v) -> None:
+    """What the native dilated and window operators leave to this side: they take meta tensors for
+    tracing only (fake tensors name the GPU as their device)."""
+    for name, t in (("q", q), ("k", k), ("v", v)):
+        if not isinstance(t, torch.Tensor):
+            raise TypeError("%s must be a tensor" % name)
+    if q.device.type == "meta":
+        raise RuntimeError("natten: dilated, rectangular, causal and biased windows need tensors on the GPU")
+
+
 def _stream_of(t: torch.Tensor) -> int:
     """Raw HIP stream that torch orders work on for the tensor's device.  Called
     with that device current (the callers hold ``torch.cuda.device(t.device)``,
@@ -412,6 +422,7 @@ def _window_call(q, k, v, kernel, causal, scale, dilation, rpb=None):
             return Natten2dWindow.apply(q, k, v, rpb, kernel, causal, float(scale))
         if rpb is not None and not isinstance(rpb, torch.Tensor):
             raise TypeError("rpb must be a tensor")
+        _window_operands(q, k, v)
         return torch.ops.enatten.natten2d_window(q, k, v, rpb, *kernel, *causal, float(scale))
     if not isinstance(dilation, int) or isinstance(dilation, bool) or dilation < 1:
         raise ValueError("dilation must be a positive int")
@@ -455,6 +466,7 @@ def natten2d(q, k, v, kernel_size=7, scale=1.0, dilation=1, is_causal=False, rpb
                              % (q.shape[2], q.shape[3], kernel_size * dilation))
         if not NATIVE_BINDING:
             return Natten2dDilated.apply(q, k, v, kernel_size, float(scale), dilation)
+        _window_operands(q, k, v)
         return torch.ops.enatten.natten2d_dilated(q, k, v, kernel_size, float(scale), dilation)
     if not NATIVE_BINDING:
         return Natten2d.apply(q, k, v, kernel_size, scale)
@@ -527,6 +539,7 @@ def natten1d(q, k, v, kernel_size=7, scale=1.0, dilation=1, is_causal=False, rpb
         if rpb is not None and (not isinstance(rpb, torch.Tensor) or rpb.dim() != 2):
             raise ValueError("rpb must be a [heads, 2*kernel_size-1] tensor")
         if NATIVE_BINDING and dilation == 1:  # (checks everything else itself)
+            _window_operands(q, k, v)
             return torch.ops.enatten.natten1d_window(q, k, v, rpb, kernel_size, bool(is_causal),
                                                      float(scale))
         _validate(q, k, v, 1, 4)

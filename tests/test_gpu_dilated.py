@@ -39,3 +39,26 @@ def test_dilated_sub_grids_in_one_launch(shape, ks, dil, dtype, layout):
     got = torch.autograd.grad(o, (qg, kg, vg), gg)
     assert o.is_contiguous() and all(t.is_contiguous() for t in got)
     assert_close(tuple(t.detach().cpu() for t in (o, *got)), (o_ref.detach(), *ref), dtype, "dilated")
+
+
+def test_every_kind_of_window_traced_by_torch_compile():
+    # as one graph: the operators carry meta kernels; the compiled function runs the same kernels
+    ensure_built()
+    from e_natten_amd import natten1d, natten2d, ops
+    if not ops.NATIVE_BINDING:
+        pytest.skip("native torch binding not built")
+
+    def f(q, k, v, rpb, s):
+        a = natten2d(q * 1.0, k, v, 5, 0.2, 2) + natten2d(q, k, v, 5, 0.2, rpb=rpb)
+        a = a + natten2d(q, k, v, (3, 5), 0.2)
+        return (a.float() ** 2).sum() + natten1d(s, s, s, 6, 0.2, is_causal=True).float().sum()
+
+    q, k, v, _ = make_inputs((2, 2, 24, 20, 32), BF16, seed=5)
+    x = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    x.append(torch.randn(2, 9, 9, device="cuda", dtype=BF16, requires_grad=True))
+    x.append(torch.randn(2, 2, 200, 32, device="cuda", dtype=F16, requires_grad=True))
+    want = f(*x)
+    got = torch.compile(f, backend="aot_eager", fullgraph=True)(*x)
+    assert torch.equal(got.detach(), want.detach())
+    for a, b in zip(torch.autograd.grad(got, x), torch.autograd.grad(want, x)):
+        assert torch.equal(a, b)

@@ -209,6 +209,53 @@ def test_meta_tensors_give_shapes_without_a_gpu():
         natten2d(q, q, q, 4)
 
 
+def _window_calls(device):
+    """(call, inputs) for every kind of window beyond the plain one."""
+    ops = torch.ops.enatten
+    new = lambda *shape: torch.empty(shape, device=device, dtype=torch.bfloat16, requires_grad=True)
+    x, s, b, b1 = [new(2, 3, 16, 12, 32) for _ in range(3)], [new(2, 3, 40, 32) for _ in range(3)], new(3, 9, 9), new(3, 9)
+    return [(lambda: ops.natten2d_dilated(*x, 5, 0.5, 2), x),
+            (lambda: ops.natten2d_window(*x, None, 4, 5, True, False, 1.0), x),
+            (lambda: ops.natten2d_window(*x, None, 3, 5, False, False, 1.0), x),
+            (lambda: ops.natten2d_window(*x, b, 5, 5, False, False, 1.0), [*x, b]),
+            (lambda: ops.natten1d_window(*s, None, 6, True, 1.0), s),
+            (lambda: ops.natten1d_window(*s, b1, 5, False, 1.0), [*s, b1])]
+
+
+def test_every_kind_of_window_can_be_traced():
+    # what a tracer does: fake tensors that name the GPU as their device (forward; the engine wants
+    # a device for their backward) and shape inference of forward and backward on meta tensors
+    from torch._subclasses import FakeTensorMode
+    from e_natten_amd import ops
+    if not ops.NATIVE_BINDING:
+        pytest.skip("native torch binding not built")
+    with FakeTensorMode():
+        for call, inputs in _window_calls("cuda"):
+            o = call()
+            assert o.shape == inputs[0].shape and o.dtype == inputs[0].dtype and o.device.type == "cuda"
+    for call, inputs in _window_calls("meta"):
+        o = call()
+        upstream = torch.empty_like(o).requires_grad_(True)
+        for x, g in zip(inputs, torch.autograd.grad(o, inputs, upstream, create_graph=True)):
+            assert g.shape == x.shape and g.dtype == x.dtype
+            # no second derivative: asking for one is an error, not a zero
+            with pytest.raises(RuntimeError, match="cannot be differentiated again"):
+                g.backward(torch.empty_like(g))
+
+
+def test_window_calls_refuse_meta_tensors_and_other_types():
+    from e_natten_amd import natten1d, natten2d
+    q = torch.empty(1, 2, 16, 12, 32, device="meta")
+    for f in (lambda: natten2d(q, q, q, 3, 1.0, 2), lambda: natten2d(q, q, q, (3, 5)),
+              lambda: natten1d(q[0], q[0], q[0], 4, is_causal=True)):
+        with pytest.raises(RuntimeError, match="on the GPU"):
+            f()
+    for f in (lambda: natten2d(q, None, q, 3, 1.0, 2), lambda: natten2d(q, None, q, (3, 5)),
+              lambda: natten1d(q[0], None, q[0], 4, is_causal=True)):
+        with pytest.raises(TypeError, match="must be a tensor"):
+            f()
+
+
 def test_window_entry_points_validate(lib):
     from e_natten_amd import _lib, natten1d, natten2d
     f = lambda kh, kw, ch=0, cw=0, H=8, W=8, q=1, rpb=None: lib.enatten2d_fwd_window(
