@@ -570,9 +570,11 @@ bool band_layout_ok(const View &v) {
     return reinterpret_cast<uintptr_t>(v.ptr) % 16 == 0 && v.sb % 8 == 0 && v.sn % 8 == 0 && v.sw % 8 == 0 &&
            v.sw < (1 << 22);
 }
+// (not windows of one key, whose probability is 1: dP - delta must cancel to an exact zero, which
+// takes the two sums in one order, as in the general kernels)
 bool band_shape_ok(const Shape &s, int dtype) {
-    return (dtype == ENATTEN_BF16 || dtype == ENATTEN_F16) && s.D >= 8 && s.D <= 128 && s.D % 8 == 0 && s.H == 1 &&
-           s.kh == 1 && (int64_t)s.B * s.N * ((s.W + 63) / 64) < ((int64_t)1 << 31) - 8;
+    return s.kw > 1 && (dtype == ENATTEN_BF16 || dtype == ENATTEN_F16) && s.D >= 8 && s.D <= 128 && s.D % 8 == 0 &&
+           s.H == 1 && s.kh == 1 && (int64_t)s.B * s.N * ((s.W + 63) / 64) < ((int64_t)1 << 31) - 8;
 }
 
 }  // namespace
