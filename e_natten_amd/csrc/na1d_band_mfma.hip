@@ -120,6 +120,39 @@ __device__ __forceinline__ void load_row(s16x8 (&reg)[DS], const short *row, int
     }
 }
 
+// ---- results that are not finite
+// A matrix instruction multiplies every staged row by every weight, and zero times an infinity or
+// a NaN is NaN: such a value in a position that a query does not see (the future of a causal
+// sequence) would reach the query's result through its zero probability, and a dS beyond float16
+// would as infinity minus infinity.  So each wave looks at its results before it stores them (one
+// instruction per value, once a tile) and computes the tokens with a value that is not finite
+// again, one after the other, from the rows in their windows alone, in float32.  A lane then holds
+// channels lane and lane + 64.
+struct Chan2 {
+    float a, b;
+};
+template <bool BF>
+__device__ __forceinline__ Chan2 chan_load(const short *row, int dlim) {
+    const int c = threadIdx.x & 63;
+    Chan2 r{0.f, 0.f};
+    if (c < dlim) r.a = cvt32<BF>(row[c]);
+    if (c + 64 < dlim) r.b = cvt32<BF>(row[c + 64]);
+    return r;
+}
+template <bool BF>
+__device__ __forceinline__ void chan_store(short *row, int dlim, const Chan2 &x, float mul) {
+    const int c = threadIdx.x & 63;
+    if (c < dlim) row[c] = cvt16<BF>(x.a * mul);
+    if (c + 64 < dlim) row[c + 64] = cvt16<BF>(x.b * mul);
+}
+__device__ __forceinline__ float chan_dot(const Chan2 &x, const Chan2 &y) {
+    return wave_sum(x.a * y.a + x.b * y.b);
+}
+__device__ __forceinline__ void chan_add(Chan2 &acc, float w, const Chan2 &x) {
+    acc.a += w * x.a;
+    acc.b += w * x.b;
+}
+
 // ------------------------------------------------------------------ forward
 template <bool BF, int D, int NQ, bool NARROW>
 __global__ __launch_bounds__(256, 2) void fwd_band_mfma(FwdArgs a, int tiles_t, int ntiles) {
@@ -245,9 +278,31 @@ __global__ __launch_bounds__(256, 2) void fwd_band_mfma(FwdArgs a, int tiles_t, 
         const int q0 = w0 + u * 16 + n, qt = min(q0, T - 1);
         const bool live = q0 < T;
         const float total = col_sum(sum[u]);
-        store_token<BF, D, (D >= 64 && !NARROW)>(oseq + qt * a.o.sw, g, o[u], 1.f / total, live, dlim);
-        if (a.lse && live && g == 0)
+        unsigned bad = bad_columns(o[u], total);
+        const bool here = live && !(bad >> n & 1);
+        store_token<BF, D, (D >= 64 && !NARROW)>(oseq + qt * a.o.sw, g, o[u], 1.f / total, here, dlim);
+        if (a.lse && here && g == 0)
             a.lse[((int64_t)tl.bb * s.N + tl.nn) * T + qt] = (m[u] + __builtin_amdgcn_logf(total)) * kLn2;
+        for (; bad; bad &= bad - 1) {
+            const int t = w0 + u * 16 + __builtin_ctz(bad);
+            if (t >= T) break;
+            const Chan2 q = chan_load<BF>(qseq + t * a.q.sw, dlim);
+            Chan2 acc{0.f, 0.f};
+            float mx = -1e30f, z = 0.f;
+            for (int key = band_lo(t, T, k, causal); key < band_hi(t, T, k, causal); key++) {
+                const float x = chan_dot(q, chan_load<BF>(kseq + key * a.k.sw, dlim)) * sc2;
+                const float mn = fmaxf(mx, x), corr = __builtin_amdgcn_exp2f(mx - mn);
+                const float p = __builtin_amdgcn_exp2f(x - mn);
+                mx = mn;
+                z = z * corr + p;
+                acc.a *= corr;
+                acc.b *= corr;
+                chan_add(acc, p, chan_load<BF>(vseq + key * a.v.sw, dlim));
+            }
+            chan_store<BF>(oseq + t * a.o.sw, dlim, acc, 1.f / z);
+            if (a.lse && l == 0)
+                a.lse[((int64_t)tl.bb * s.N + tl.nn) * T + t] = (mx + __builtin_amdgcn_logf(z)) * kLn2;
+        }
     }
 }
 
@@ -380,8 +435,23 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
 #pragma unroll
     for (int u = 0; u < NQ; u++) {
         const int q0 = w0 + u * 16 + n, qt = min(q0, T - 1);
+        unsigned bad = bad_columns(dq[u]);
         store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dq) + a.grad_at(tl.bb, tl.nn, 0, qt), g,
-                                                 dq[u], s.scale, q0 < T, dlim);
+                                                 dq[u], s.scale, q0 < T && !(bad >> n & 1), dlim);
+        for (; bad; bad &= bad - 1) {
+            const int col = __builtin_ctz(bad), t = w0 + u * 16 + col;
+            if (t >= T) break;
+            const Chan2 q = chan_load<BF>(bseq(a.q, tl) + t * a.q.sw, dlim);
+            const Chan2 go = chan_load<BF>(bseq(a.d_o, tl) + t * a.d_o.sw, dlim);
+            const float lse_t = __shfl(lse2[u], col, 64), delta_t = __shfl(delta[u], col, 64);
+            Chan2 acc{0.f, 0.f};
+            for (int key = band_lo(t, T, k, causal); key < band_hi(t, T, k, causal); key++) {
+                const Chan2 kr = chan_load<BF>(kseq + key * a.k.sw, dlim);
+                const float p = __builtin_amdgcn_exp2f(chan_dot(q, kr) * sc2 - lse_t);
+                chan_add(acc, p * (chan_dot(go, chan_load<BF>(vseq + key * a.v.sw, dlim)) - delta_t), kr);
+            }
+            chan_store<BF>(static_cast<short *>(a.dq) + a.grad_at(tl.bb, tl.nn, 0, t), dlim, acc, s.scale);
+        }
     }
 }
 
@@ -508,10 +578,28 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
         __syncthreads();
     }
     if (!on) return;
-    const bool live = w0 + n < T;
+    unsigned bad = bad_columns(dk) | bad_columns(dv);
+    const bool live = w0 + n < T && !(bad >> n & 1);
     const int64_t at = a.grad_at(tl.bb, tl.nn, 0, kt);
     store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dk) + at, g, dk, s.scale, live, dlim);
     store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dv) + at, g, dv, 1.f, live, dlim);
+    for (; bad; bad &= bad - 1) {
+        const int key = w0 + __builtin_ctz(bad);
+        if (key >= T) break;
+        const Chan2 kr = chan_load<BF>(bseq(a.k, tl) + key * a.k.sw, dlim);
+        const Chan2 vr = chan_load<BF>(bseq(a.v, tl) + key * a.v.sw, dlim);
+        Chan2 ak{0.f, 0.f}, av{0.f, 0.f};
+        for (int q = axis_inv_lo(key, k, causal); q < axis_inv_hi(key, T, k, causal); q++) {
+            if ((unsigned)(key - band_lo(q, T, k, causal)) >= (unsigned)k) continue;
+            const Chan2 qr = chan_load<BF>(qseq + q * a.q.sw, dlim), gr = chan_load<BF>(gseq + q * a.d_o.sw, dlim);
+            const float p = __builtin_amdgcn_exp2f(chan_dot(qr, kr) * sc2 - a.lse[tok0 + q] * kLog2e);
+            chan_add(av, p, gr);
+            chan_add(ak, p * (chan_dot(gr, vr) - a.delta[tok0 + q]), qr);
+        }
+        const int64_t to = a.grad_at(tl.bb, tl.nn, 0, key);
+        chan_store<BF>(static_cast<short *>(a.dk) + to, dlim, ak, s.scale);
+        chan_store<BF>(static_cast<short *>(a.dv) + to, dlim, av, 1.f);
+    }
 }
 
 // ------------------------------------------------------------------ dispatch

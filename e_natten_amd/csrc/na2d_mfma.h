@@ -66,6 +66,25 @@ __device__ __forceinline__ float col_sum(float x) {
     return x + __shfl_xor(x, 32, 64);
 }
 
+// bit n: column n of the accumulators (lanes n, n + 16, n + 32, n + 48) has a value that is not
+// finite
+template <int DT>
+__device__ __forceinline__ unsigned bad_columns(const f32x4 (&acc)[DT], float also = 0.f) {
+    float z = also * 0.f;
+#pragma unroll
+    for (int t = 0; t < DT; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) z = fmaf(acc[t][i], 0.f, z);
+    const unsigned long long m = __ballot(!(z == 0.f));
+    return (unsigned)(m | m >> 16 | m >> 32 | m >> 48) & 0xffffu;
+}
+// sum over the wave
+__device__ __forceinline__ float wave_sum(float x) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) x += __shfl_xor(x, o, 64);
+    return x;
+}
+
 // dO . O over the 8 channels of one 16-byte chunk: four two-element dot products that
 // accumulate in float32 (v_dot2c_f32_bf16 / v_dot2c_f32_f16), one instruction per dword where
 // taking the halves apart and multiplying them took six.

@@ -50,3 +50,57 @@ def test_band_windows(shape, ks, causal, dtype, layout):
         assert err <= BF16_REL, (name, err)
         assert norm <= (4e-3 if dtype == BF16 else 5e-4), (name, norm)
     assert torch.equal(o, natten1d(qg, kg, vg, ks, scale, 1, causal))
+
+
+@pytest.mark.parametrize("ks,causal,d,dtype", [(33, True, 64, BF16), (51, False, 128, F16), (70, True, 40, F16)])
+def test_values_that_are_not_finite_stay_in_their_windows(ks, causal, d, dtype):
+    # a NaN in v at one position: only queries that see it, and the keys that such queries see, may
+    # be touched (in a causal sequence nothing before it), though rows outside a window are staged
+    ensure_built()
+    from e_natten_amd import natten1d
+    print("case not finite", ks, causal, d, dtype, flush=True)
+    T, pos, scale = 260, 140, d ** -0.5
+    q, k, v, g = make_inputs((1, 2, T, d), dtype, seed=41)
+    qr, kr, vr = (t.double().requires_grad_(True) for t in (q, k, v))
+    o_ref = O.natten2d_window_dense_mask(qr.unsqueeze(2), kr.unsqueeze(2), vr.unsqueeze(2), (1, ks),
+                                         (False, causal), scale).squeeze(2)
+    ref = (o_ref.detach(), *torch.autograd.grad(o_ref, (qr, kr, vr), g.double()))
+    vbad = v.clone()
+    vbad[:, :, pos] = float("nan")
+    qg, kg, vg = (t.cuda().requires_grad_(True) for t in (q, k, vbad))
+    o = natten1d(qg, kg, vg, ks, scale, 1, causal)
+    got = [t.detach().cpu() for t in (o, *torch.autograd.grad(o, (qg, kg, vg), g.cuda()))]
+    start = lambda t: max(0, t - ks + 1) if causal else min(max(t - ks // 2, 0), T - ks)
+    windows = [range(start(t), t + 1 if causal else start(t) + ks) for t in range(T)]
+    sees = torch.tensor([pos in w for w in windows])
+    reached = torch.zeros(T, dtype=torch.bool)
+    for w in (w for w in windows if pos in w):
+        reached[w.start:w.stop] = True
+    assert got[0][:, :, sees].isnan().all() and got[1][:, :, sees].isnan().all()
+    assert got[2][:, :, reached].isnan().all()
+    for name, x, r, touched in zip(("O", "dQ", "dK", "dV"), got, ref,
+                                   (sees, sees, reached, torch.zeros(T, dtype=torch.bool))):
+        x, r = x[:, :, ~touched].double(), r[:, :, ~touched]
+        norm = ((x - r).norm() / r.norm()).item()
+        print("   ", name, "2-norm %.2e" % norm, flush=True)
+        assert norm <= (4e-3 if dtype == BF16 else 5e-4), (name, norm)  # (as in test_band_windows)
+
+
+def test_gradients_of_logits_beyond_float16():
+    # dS of some 1e5, whose 16-bit terms would be an infinity and its negative, under a small
+    # softmax scale: the gradients of q and k themselves are in range
+    ensure_built()
+    from e_natten_amd import natten1d
+    q, k, v, g = make_inputs((1, 2, 130, 64), F16, seed=43)
+    v, g, scale = v * 200, g * 200, 2.0 ** -10
+    qr, kr, vr = (t.double().requires_grad_(True) for t in (q, k, v))
+    o_ref = O.natten2d_window_dense_mask(qr.unsqueeze(2), kr.unsqueeze(2), vr.unsqueeze(2), (1, 3),
+                                         (False, True), scale).squeeze(2)
+    ref = torch.autograd.grad(o_ref, (qr, kr, vr), g.double())
+    qg, kg, vg = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    got = torch.autograd.grad(natten1d(qg, kg, vg, 3, scale, 1, True), (qg, kg, vg), g.cuda())
+    for name, x, r in zip(("dQ", "dK", "dV"), got, ref):
+        norm = ((x.cpu().double() - r).norm() / r.norm()).item()
+        print("   ", name, "2-norm %.2e" % norm, flush=True)
+        # dP - delta loses what O was rounded to: 2^-12 of dO . O, three such errors in a sum of three
+        assert norm <= 2e-3, (name, norm)
