@@ -157,6 +157,11 @@ bool sub_layout_ok(const FwdArgsSub &a);
 bool sub_layout_ok(const BwdArgsSub &a);
 int launch_fwd_mfma_sub(const FwdArgsSub &a, int dtype, hipStream_t st);
 int launch_bwd_mfma_sub(const BwdArgsSub &a, int dtype, hipStream_t st);
+// ... and where a sub-grid fits one workgroup's LDS, the kernels that take it whole
+bool small_fwd_supported(const FwdArgsSub &a);
+bool small_bwd_supported(const BwdArgsSub &a);
+int launch_fwd_small(const FwdArgsSub &a, int dtype, hipStream_t st);
+int launch_bwd_small(const BwdArgsSub &a, int dtype, hipStream_t st);
 // the same kernels with a relative position bias (a.rpb, a.d_rpb; a.ds_pairs takes one row of
 // (2k-1)^2 floats per tile): square centred windows that mfma_supported takes
 int launch_fwd_mfma_bias(const FwdArgs &a, int dtype, hipStream_t st);

@@ -5,7 +5,8 @@
 // per sub-grid left most CUs without a tile, and dilation^2 launches of each kernel and as many
 // calls through Python bounded the call.  One launch for all of one size: B8 N4 56x56 d32 k7
 // dilation 4, views of a projection, forward and backward 1060 -> 70 us (16 launches each of 5 +
-// 14 us of kernels and 1100 us of host time before; three kernels of 16 + 26 + 32 us now).
+// 14 us of kernels and 1100 us of host time before; three kernels of 14 + 25 + 31 us).  Sub-grids
+// that fit one workgroup's LDS go to na2d_mfma_small.hip.
 #include "na2d_common.h"
 
 namespace enatten {
@@ -34,9 +35,11 @@ bool sub_layout_ok(const BwdArgsSub &a) {
 }
 
 int launch_fwd_mfma_sub(const FwdArgsSub &a, int dtype, hipStream_t st) {
+    if (small_fwd_supported(a)) return launch_fwd_small(a, dtype, st);
     return fwd_dispatch(a, dtype, st);
 }
 int launch_bwd_mfma_sub(const BwdArgsSub &a, int dtype, hipStream_t st) {
+    if (small_bwd_supported(a)) return launch_bwd_small(a, dtype, st);
     return bwd_dispatch(a, dtype, 0, st);
 }
 

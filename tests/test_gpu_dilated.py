@@ -14,6 +14,13 @@ BF16, F16 = torch.bfloat16, torch.float16
     ((2, 2, 38, 54, 48), 7, 2, F16, "proj"),     # head_dim below a built one, inner tiles
     ((1, 1, 67, 70, 64), 13, 5, BF16, "plain"),  # largest window: two waves per block of keys
     ((1, 2, 44, 45, 128), 11, 4, F16, "proj"),   # one halo in LDS at a time, border tiles only
+    ((2, 2, 26, 32, 64), 13, 2, F16, "proj"),    # whole sub-grids of 208 pixels, the window as large
+    ((1, 3, 21, 40, 56), 5, 3, F16, "plain"),    # whole ones of two sizes, head_dim below a built one
+    ((2, 1, 40, 48, 16), 3, 7, BF16, "plain"),   # ... of four sizes, 30 to 42 pixels
+    ((1, 2, 28, 30, 32), 7, 2, BF16, "plain"),   # 210 pixels: two beyond the middle size
+    ((3, 22, 32, 32, 64), 5, 2, F16, "proj"),    # 256 pixels: the largest, whole in the backward only
+    ((9, 8, 16, 24, 32), 7, 2, BF16, "proj"),    # 96 pixels: all of the smallest size
+    ((1, 2, 34, 32, 32), 9, 2, BF16, "plain"),   # 272 pixels: one row more than a workgroup takes
     ((1, 2, 24, 26, 64), 3, 8, BF16, "odd"),     # upstream gradient the 16-byte loads cannot take:
                                                  # the backward runs sub-grid by sub-grid
 ])
@@ -39,6 +46,42 @@ def test_dilated_sub_grids_in_one_launch(shape, ks, dil, dtype, layout):
     got = torch.autograd.grad(o, (qg, kg, vg), gg)
     assert o.is_contiguous() and all(t.is_contiguous() for t in got)
     assert_close(tuple(t.detach().cpu() for t in (o, *got)), (o_ref.detach(), *ref), dtype, "dilated")
+
+
+def test_values_that_are_not_finite_stay_in_their_windows():
+    # sub-grids that a workgroup takes whole: a NaN in v reaches the queries that see it, and the
+    # keys that those see, alone
+    ensure_built()
+    from e_natten_amd import natten2d
+    ks, dil, side, at = 5, 2, 28, (9, 14)
+    q, k, v, g = make_inputs((1, 66, side, side, 32), BF16, seed=29)  # (more images than CUs)
+    clean = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    v[:, :, at[0], at[1]] = float("nan")
+    dirty = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    res = []
+    for x in (clean, dirty):
+        o = natten2d(*x, ks, 0.2, dil)
+        res.append([t.detach().float().cpu() for t in (o, *torch.autograd.grad(o, x, g.cuda()))])
+    # along an axis: the window of each position of the residue class, as positions of the axis
+    def windows(c):
+        n = side // dil
+        start = lambda i: min(max(i - ks // 2, 0), n - ks)
+        return {i * dil + c % dil: [j * dil + c % dil for j in range(start(i), start(i) + ks)] for i in range(n)}
+    rows, cols = windows(at[0]), windows(at[1])
+    sees, reached = torch.zeros(side, side, dtype=torch.bool), torch.zeros(side, side, dtype=torch.bool)
+    for y in (y for y in rows if at[0] in rows[y]):
+        for x in (x for x in cols if at[1] in cols[x]):
+            sees[y, x] = True
+            for ky in rows[y]:
+                reached[ky, cols[x]] = True
+    for name, c, d, touched in zip(("O", "dQ", "dK", "dV"), *res,
+                                   (sees, sees, reached, torch.zeros_like(sees))):
+        assert d[:, :, touched].isnan().all(), name
+        # (bfloat16 results of the same sums in another order, P and dS rounded to it on one side)
+        c, d = c[:, :, ~touched], d[:, :, ~touched]
+        norm = ((c - d).norm() / c.norm()).item()
+        print("   ", name, "2-norm %.2e" % norm, flush=True)
+        assert norm <= 6e-3, (name, norm)
 
 
 def test_every_kind_of_window_traced_by_torch_compile():
