@@ -130,18 +130,35 @@ int bwd_f64(const char *fn, const BwdArgs &a, size_t ws_floats, hipStream_t st) 
     return launch_bwd_f64(a, st);
 }
 
+// an undilated call as a dilated one with a single sub-grid
+template <typename SUB, typename ARGS>
+SUB whole(const ARGS &a) {
+    SUB w;
+    static_cast<ARGS &>(w) = a;
+    w.sub_r = w.sub_c = w.dil = 1;
+    return w;
+}
 // a square, centred, undilated window: the kernel family that serves the call
 int run_fwd(const FwdArgs &a, int dtype, hipStream_t st) {
     const int D = a.s.D, ks = a.s.kh;
     if (dtype == ENATTEN_F64) return launch_fwd_f64(a, st);
-    if (use_mfma(D, ks, dtype)) return launch_fwd_mfma(a, dtype, st);
+    if (use_mfma(D, ks, dtype)) {
+        const FwdArgsSub w = whole<FwdArgsSub>(a);
+        if (g_path.load() == 0 && small_fwd_supported(w) && sub_layout_ok(w)) return launch_fwd_small(w, dtype, st);
+        return launch_fwd_mfma(a, dtype, st);
+    }
     if (use_mfma_f32(D, ks, dtype)) return launch_fwd_mfma_f32(a, st);
     return launch_fwd_simt(a, dtype, st);
 }
 int run_bwd(const char *fn, const BwdArgs &a, int dtype, size_t ws_floats, hipStream_t st) {
     const int D = a.s.D, ks = a.s.kh;
     if (dtype == ENATTEN_F64) return bwd_f64(fn, a, ws_floats, st);
-    if (use_mfma(D, ks, dtype)) return launch_bwd_mfma(a, dtype, g_path.load(), st);
+    if (use_mfma(D, ks, dtype)) {
+        const int path = g_path.load();
+        const BwdArgsSub w = whole<BwdArgsSub>(a);
+        if (path == 0 && small_bwd_supported(w) && sub_layout_ok(w)) return launch_bwd_small(w, dtype, st);
+        return launch_bwd_mfma(a, dtype, path, st);
+    }
     // the float32 matrix-core backward where the workspace at hand holds its P and dS (it
     // writes contiguous gradients only)
     if (use_mfma_f32(D, ks, dtype) && a.grads_contiguous() &&

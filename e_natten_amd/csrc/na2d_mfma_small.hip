@@ -1,5 +1,5 @@
-// Sub-grids of at most 256 pixels (a dilated call's, such as 14x14 for 56x56 at dilation
-// 4): one workgroup per image, everything it needs in LDS at once.  bf16 / fp16, head dims that are
+// Images of at most 256 pixels, above all the sub-grids of a dilated call (14x14 for 56x56 at
+// dilation 4): one workgroup per image, everything it needs in LDS at once.  bf16 / fp16, head dims that are
 // multiples of 8 up to 64, any window.
 //
 // The tiled kernels of na2d_mfma_kernels.h cut such an image into four tiles that all touch the
@@ -428,9 +428,19 @@ int bwd_size(const BwdArgsSub &a, hipStream_t st) {
 // two whose dK/dV pass walks the border: always (4 images 14x14 d64 20.5 / 17.5, 32 images d32
 // 18.8 / 13.2, 512 images 55.9 / 20.1, 3200 images 8x8 68 / 31, 8192 images 16x16 652 / 415).
 // With one size (208 tokens, eight waves) for all, 3200 images 8x8 took 18.6 + 39.4 instead of
-// 15.9 + 31.3.
-bool small_fwd_supported(const FwdArgsSub &a) { return size_ok(a.s, images_of(a), 208) && images_of(a) > 256; }
-bool small_bwd_supported(const BwdArgsSub &a) { return size_ok(a.s, images_of(a), 256); }
+// 15.9 + 31.3.  Not where a few workgroups hold the largest size with one to a CU (d64 k13 16x16: 4
+// images 25.5 / 27.7, 32 images 25.2 / 24.7).
+// Undilated images: for k >= 7 and from 128 images on (14x14 d32 k7: 128 images 16.4 / 13.3, 1024
+// images 99.7 / 38.4; 14x18 d48 k9: 32 images 23.5 / 24.8, 128 images 36.9 / 25.0; 9x10 d64 k9, 1024
+// images 103 / 30); at k = 3 and 5 the other passes have little border to walk (14x14 d64 k3, 128
+// images 10.8 / 14.5).  Their forward from the second tile on (8x8 d32, 1024 images 7.1 / 7.5).
+bool small_fwd_supported(const FwdArgsSub &a) {
+    return size_ok(a.s, images_of(a), 208) && images_of(a) > 256 && (a.dil > 1 || (a.s.kh >= 7 && a.s.H * a.s.W > 64));
+}
+bool small_bwd_supported(const BwdArgsSub &a) {
+    const int64_t ni = images_of(a);
+    return size_ok(a.s, ni, a.s.D > 32 && ni < 64 ? 208 : 256) && (a.dil > 1 || (a.s.kh >= 7 && ni >= 128));
+}
 int launch_fwd_small(const FwdArgsSub &a, int dtype, hipStream_t st) {
     if (dtype == ENATTEN_BF16) return a.s.D <= 32 ? fwd_size<true, 32>(a, st) : fwd_size<true, 64>(a, st);
     return a.s.D <= 32 ? fwd_size<false, 32>(a, st) : fwd_size<false, 64>(a, st);
