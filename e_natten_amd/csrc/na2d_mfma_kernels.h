@@ -72,6 +72,15 @@ struct SubTile : Tile {
 };
 using ATile = std::conditional_t<kSub, SubTile, Tile>;
 
+// two tiles in one column of one image, the sub-grid included: a walk that hops from segment to
+// segment may meet the same place of another sub-grid next
+template <typename TL>
+__device__ __forceinline__ bool same_column(const TL &x, const TL &y) {
+    bool same = x.bb == y.bb && x.nn == y.nn && x.c0 == y.c0;
+    if constexpr (kSub) same = same && x.ri == y.ri && x.rj == y.rj;
+    return same;
+}
+
 // Images (one batch entry, head and sub-grid each) of a launch
 template <typename ARGS>
 int64_t images_of(const ARGS &a) {
@@ -404,7 +413,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
             nxt = pick(tn);
             lqn = lane_at<KS>(a, nxt, wave, n);
             // the tile below in the same image keeps the rows the two halos share
-            const bool below = ROLL && nxt.bb == cur.bb && nxt.nn == cur.nn && nxt.c0 == cur.c0 &&
+            const bool below = ROLL && same_column(nxt, cur) &&
                                nxt.r0 > cur.r0 && lqn.hr0 < lq.hr0 + G::HR;
             y0 = below ? lq.hr0 + G::HR : lqn.hr0;
             nr = below ? lqn.hr0 - lq.hr0 : G::HR;
@@ -737,7 +746,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             nxt = pick(tn);
             lqn = lane_at<KS>(a, nxt, wave, n);
             // the tile below in the same image keeps the rows the two halos share
-            const bool below = ROLL && nxt.bb == cur.bb && nxt.nn == cur.nn && nxt.c0 == cur.c0 &&
+            const bool below = ROLL && same_column(nxt, cur) &&
                                nxt.r0 > cur.r0 && lqn.hr0 < lq.hr0 + G::HR;
             y0 = below ? lq.hr0 + G::HR : lqn.hr0;
             nr = below ? lqn.hr0 - lq.hr0 : G::HR;
@@ -1177,7 +1186,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
         if (more) {
             nxt = pick(tn);
             // the tile below in the same image keeps the rows the two blocks share
-            const bool below = ROLL && nxt.bb == cur.bb && nxt.nn == cur.nn && nxt.c0 == cur.c0 &&
+            const bool below = ROLL && same_column(nxt, cur) &&
                                nxt.r0 > cur.r0 && nxt.r0 - cur.r0 < G::HR;
             y0 = below ? cur.r0 - KS / 2 + G::HR : nxt.r0 - KS / 2;
             nr = below ? nxt.r0 - cur.r0 : G::HR;

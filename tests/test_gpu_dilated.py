@@ -50,6 +50,27 @@ def test_dilated_sub_grids_in_one_launch(shape, ks, dil, dtype, layout):
     assert_close(tuple(t.detach().cpu() for t in (o, *got)), (o_ref.detach(), *ref), dtype, "dilated")
 
 
+def test_column_walk_keeps_rows_of_its_own_sub_grid_only():
+    # 4032 tiles over 512 workgroups in segments of a third of a column: the tile after a segment lies
+    # one row of tiles lower in the next sub-grid of the same batch entry and head
+    ensure_built()
+    from e_natten_amd import natten2d
+    shape, ks, dil = (8, 7, 96, 48, 128), 5, 2
+    q, k, v, g = make_inputs(shape, BF16, seed=47)
+    print("case column walk", shape, "k=%d dilation=%d" % (ks, dil), flush=True)
+    scale = shape[-1] ** -0.5
+    x = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    o = natten2d(*x, ks, scale, dil)
+    got = [t.detach().cpu() for t in (o, *torch.autograd.grad(o, x, g.cuda()))]
+    for i in range(dil):
+        for j in range(dil):
+            sub = (slice(0, 1), slice(None), slice(i, None, dil), slice(j, None, dil))
+            ref_x = [t[sub].double().requires_grad_(True) for t in (q, k, v)]
+            o_ref = O.natten2d_dense_mask(*ref_x, ks, scale)
+            ref = (o_ref.detach(), *torch.autograd.grad(o_ref, ref_x, g[sub].double()))
+            assert_close([t[sub] for t in got], ref, BF16, "sub-grid %d %d" % (i, j))
+
+
 def test_values_that_are_not_finite_stay_in_their_windows():
     # sub-grids that a workgroup takes whole: a NaN in v reaches the queries that see it, and the
     # keys that those see, alone
