@@ -8,7 +8,8 @@
 // a time: as queries against the run of tokens that their windows' rows span (forward, dQ), or as
 // keys against the run of queries that see them (dK, dV), 32 tokens to a step, the window being a
 // mask from a table of the tokens' places.  The backward is one kernel: five tensors read, three
-// written, its jobs (16 queries' dQ, 16 keys' dK and dV) dealt to the waves in turn.
+// written, its jobs (16 queries' dQ, and behind a barrier 16 keys' dK and dV) dealt to the waves in
+// turn, from both ends.
 // A result that is not finite is computed again from its window alone, as in na1d_band_mfma.hip.
 // Bound by the latency of the staging loads and the vector work on the logits (half of a step's
 // pairs are inside a window at 14x14, k = 7).  B8 N4 56x56 d32 k7 dilation 4, forward and backward
@@ -133,6 +134,18 @@ __device__ __forceinline__ void second_product(f32x4 (&acc)[D / 16], const short
 #pragma unroll
     for (int t = 0; t < D / 16; t++)
         acc[t] = mfma16<BF>(cat(lds_read_tr(p + t * 4), lds_read_tr(p + 16 * kPitch<D> + t * 4)), w, acc[t]);
+}
+// ... and acc2 += X^T w2 with the same rows
+template <bool BF, int D>
+__device__ __forceinline__ void second_product(f32x4 (&acc)[D / 16], const short *lds, int t0, int n, int g, s16x8 w,
+                                               f32x4 (&acc2)[D / 16], s16x8 w2) {
+    const short *p = lds + (t0 + g * 4 + (n >> 2)) * kPitch<D> + (n & 3) * (D / 4);
+#pragma unroll
+    for (int t = 0; t < D / 16; t++) {
+        const s16x8 x = cat(lds_read_tr(p + t * 4), lds_read_tr(p + 16 * kPitch<D> + t * 4));
+        acc[t] = mfma16<BF>(x, w, acc[t]);
+        acc2[t] = mfma16<BF>(x, w2, acc2[t]);
+    }
 }
 // element e of a lane's eight: row t0 + (e >> 2) * 16 + g * 4 + (e & 3)
 __device__ __forceinline__ void lane_places(int (&x)[8], const int *table, int t0, int g) {
@@ -272,111 +285,134 @@ __global__ __launch_bounds__(G::NT, G::WPS) void bwd_small_mfma(BwdArgsSub a, in
     }
     __syncthreads();
     const int blocks = (P + 15) / 16;
-    for (int job = wave; job < 2 * blocks; job += G::NW) {
-        const bool keys = job >= blocks;
-        const int t0 = (keys ? job - blocks : job) * 16;
+    auto grad_pix = [&](int t) __attribute__((always_inline)) {
+        return a.grad_at(im.bb, im.nn, im.ri + t / s.W * a.dil, im.rj + t % s.W * a.dil);
+    };
+    // dQ.  delta = dO . O is what O was rounded to away from the sum of P dP, an error that all keys
+    // of a window share and that keys or values with a common component multiply.  So the residual
+    // E = sum p (dP - delta) is summed beside the products, dQ = A - E / Z sum p k, and the dK/dV jobs
+    // find delta + E / Z (14x14 d64 k9 bf16, k and v of mean 2: dQ off by 4.4e-2 in 2-norm without, 4.1e-3 with).
+    for (int t0 = wave * 16; t0 < P; t0 += G::NW * 16) {
         const int own = min(t0 + n, P - 1);
-        auto grad_pix = [&](int t) __attribute__((always_inline)) {
-            return a.grad_at(im.bb, im.nn, im.ri + t / s.W * a.dil, im.rj + t % s.W * a.dil);
-        };
-        const int64_t at = grad_pix(own);
-        const bool live = t0 + n < P;
+        s16x8 qreg[G::DS], greg[G::DS];
+        lds_row(qreg, lds_q + own * G::PITCH, g);
+        lds_row(greg, lds_g + own * G::PITCH, g);
+        const int win = lds_win[own];
+        const float lse2 = lds_lse[own], delta = lds_delta[own];
         int lo, hi;
-        if (!keys) {
-            s16x8 qreg[G::DS], greg[G::DS];
-            lds_row(qreg, lds_q + own * G::PITCH, g);
-            lds_row(greg, lds_g + own * G::PITCH, g);
-            const int win = lds_win[own];
-            const float lse2 = lds_lse[own], delta = lds_delta[own];
-            key_run(t0, P, s, lo, hi);
-            f32x4 dq[G::DT];
+        key_run(t0, P, s, lo, hi);
+        f32x4 dq[G::DT], pk[G::DT];
+        float zsum = 0.f, esum = 0.f;
 #pragma unroll
-            for (int t = 0; t < G::DT; t++) dq[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-            for (int kk = lo & ~15; kk < hi; kk += 32) {
-                f32x4 c[2], cp[2];
-                first_product<BF, D>(c, lds_k, kk, n, g, qreg);
-                first_product<BF, D>(cp, lds_v, kk, n, g, greg);
-                int pos[8];
-                lane_places(pos, lds_pos, kk, g);
-                s16x8 ds;
+        for (int t = 0; t < G::DT; t++) {
+            dq[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            pk[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        for (int kk = lo & ~15; kk < hi; kk += 32) {
+            f32x4 c[2], cp[2];
+            first_product<BF, D>(c, lds_k, kk, n, g, qreg);
+            first_product<BF, D>(cp, lds_v, kk, n, g, greg);
+            int pos[8];
+            lane_places(pos, lds_pos, kk, g);
+            s16x8 ph, ds;
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const float x = c[e >> 2][e & 3] * sc2 - lse2;
-                    const float p = __builtin_amdgcn_exp2f(inside(pos[e], win, ks) ? x : -INFINITY);
-                    ds[e] = cvt16<BF>(p * (cp[e >> 2][e & 3] - delta));
-                }
-                second_product<BF, D>(dq, lds_k, kk, n, g, ds);
+            for (int e = 0; e < 8; e++) {
+                const float x = c[e >> 2][e & 3] * sc2 - lse2;
+                const float p = __builtin_amdgcn_exp2f(inside(pos[e], win, ks) ? x : -INFINITY);
+                const float y = p * (cp[e >> 2][e & 3] - delta);
+                zsum += p;
+                esum += y;
+                ph[e] = cvt16<BF>(p);
+                ds[e] = cvt16<BF>(y);
             }
-            unsigned bad = bad_columns(dq);
-            store_token<BF, D>(static_cast<short *>(a.dq) + at, g, dq, s.scale, live && !(bad >> n & 1), s.D);
-            for (; bad; bad &= bad - 1) {
-                const int t = t0 + __builtin_ctz(bad);
-                if (t >= P) break;
-                const float q = chan<BF>(lds_q + t * G::PITCH, l, D), go = chan<BF>(lds_g + t * G::PITCH, l, D);
-                float acc = 0.f;
-                for (int j = 0; j < ks * ks; j++) {
-                    const int w = lds_win[t], key = ((w & 0xffff) + j / ks) * s.W + (w >> 16) + j % ks;
-                    const float kr = chan<BF>(lds_k + key * G::PITCH, l, D);
-                    const float p = __builtin_amdgcn_exp2f(wave_sum(q * kr) * sc2 - lds_lse[t]);
-                    acc += p * (wave_sum(go * chan<BF>(lds_v + key * G::PITCH, l, D)) - lds_delta[t]) * kr;
-                }
-                if (l < s.D) static_cast<short *>(a.dq)[grad_pix(t) + l] = cvt16<BF>(acc * s.scale);
-            }
-        } else {
-            s16x8 kreg[G::DS], vreg[G::DS];
-            lds_row(kreg, lds_k + own * G::PITCH, g);
-            lds_row(vreg, lds_v + own * G::PITCH, g);
-            const int pos = lds_pos[own];
-            query_run(t0, P, s, lo, hi);
-            f32x4 dk[G::DT], dv[G::DT];
+            second_product<BF, D>(dq, lds_k, kk, n, g, ds, pk, ph);
+        }
+        const float shift = col_sum(esum) / col_sum(zsum);
 #pragma unroll
-            for (int t = 0; t < G::DT; t++) {
-                dk[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                dv[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < G::DT; t++) dq[t] -= shift * pk[t];
+        unsigned bad = bad_columns(dq);
+        const bool here = t0 + n < P && !(bad >> n & 1);
+        store_token<BF, D>(static_cast<short *>(a.dq) + grad_pix(own), g, dq, s.scale, here, s.D);
+        // (only the jobs behind the barrier read another block's)
+        if (here && g == 0) lds_delta[own] = delta + shift;
+        for (; bad; bad &= bad - 1) {
+            const int t = t0 + __builtin_ctz(bad);
+            if (t >= P) break;
+            const float q = chan<BF>(lds_q + t * G::PITCH, l, D), go = chan<BF>(lds_g + t * G::PITCH, l, D);
+            float acc = 0.f, accp = 0.f, z = 0.f, res = 0.f;
+            const int w = lds_win[t];
+            for (int j = 0; j < ks * ks; j++) {
+                const int key = ((w & 0xffff) + j / ks) * s.W + (w >> 16) + j % ks;
+                const float kr = chan<BF>(lds_k + key * G::PITCH, l, D);
+                const float p = __builtin_amdgcn_exp2f(wave_sum(q * kr) * sc2 - lds_lse[t]);
+                const float y = p * (wave_sum(go * chan<BF>(lds_v + key * G::PITCH, l, D)) - lds_delta[t]);
+                z += p;
+                res += y;
+                acc += y * kr;
+                accp += p * kr;
             }
-            for (int qq = lo & ~15; qq < hi; qq += 32) {
-                f32x4 c[2], cp[2];
-                first_product<BF, D>(c, lds_q, qq, n, g, kreg);
-                first_product<BF, D>(cp, lds_g, qq, n, g, vreg);
-                int win[8];
-                lane_places(win, lds_win, qq, g);
-                s16x8 ph, ds;
+            if (l < s.D) static_cast<short *>(a.dq)[grad_pix(t) + l] = cvt16<BF>((acc - res / z * accp) * s.scale);
+            if (l == 0) lds_delta[t] += res / z;
+        }
+    }
+    __syncthreads();
+    for (int t0 = (G::NW - 1 - wave) * 16; t0 < P; t0 += G::NW * 16) {
+        const int own = min(t0 + n, P - 1);
+        const int64_t at = grad_pix(own);
+        s16x8 kreg[G::DS], vreg[G::DS];
+        lds_row(kreg, lds_k + own * G::PITCH, g);
+        lds_row(vreg, lds_v + own * G::PITCH, g);
+        const int pos = lds_pos[own];
+        int lo, hi;
+        query_run(t0, P, s, lo, hi);
+        f32x4 dk[G::DT], dv[G::DT];
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const f32x4 lse2 = *reinterpret_cast<const f32x4 *>(lds_lse + qq + h * 16 + g * 4);
-                    const f32x4 delta = *reinterpret_cast<const f32x4 *>(lds_delta + qq + h * 16 + g * 4);
+        for (int t = 0; t < G::DT; t++) {
+            dk[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            dv[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        for (int qq = lo & ~15; qq < hi; qq += 32) {
+            f32x4 c[2], cp[2];
+            first_product<BF, D>(c, lds_q, qq, n, g, kreg);
+            first_product<BF, D>(cp, lds_g, qq, n, g, vreg);
+            int win[8];
+            lane_places(win, lds_win, qq, g);
+            s16x8 ph, ds;
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float x = c[h][i] * sc2 - lse2[i];
-                        const float p = __builtin_amdgcn_exp2f(inside(pos, win[h * 4 + i], ks) ? x : -INFINITY);
-                        ph[h * 4 + i] = cvt16<BF>(p);
-                        ds[h * 4 + i] = cvt16<BF>(p * (cp[h][i] - delta[i]));
-                    }
+            for (int h = 0; h < 2; h++) {
+                const f32x4 lse2 = *reinterpret_cast<const f32x4 *>(lds_lse + qq + h * 16 + g * 4);
+                const f32x4 delta = *reinterpret_cast<const f32x4 *>(lds_delta + qq + h * 16 + g * 4);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float x = c[h][i] * sc2 - lse2[i];
+                    const float p = __builtin_amdgcn_exp2f(inside(pos, win[h * 4 + i], ks) ? x : -INFINITY);
+                    ph[h * 4 + i] = cvt16<BF>(p);
+                    ds[h * 4 + i] = cvt16<BF>(p * (cp[h][i] - delta[i]));
                 }
-                second_product<BF, D>(dv, lds_g, qq, n, g, ph);
-                second_product<BF, D>(dk, lds_q, qq, n, g, ds);
             }
-            unsigned bad = bad_columns(dk) | bad_columns(dv);
-            const bool here = live && !(bad >> n & 1);
-            store_token<BF, D>(static_cast<short *>(a.dk) + at, g, dk, s.scale, here, s.D);
-            store_token<BF, D>(static_cast<short *>(a.dv) + at, g, dv, 1.f, here, s.D);
-            for (; bad; bad &= bad - 1) {
-                const int t = t0 + __builtin_ctz(bad);
-                if (t >= P) break;
-                const float kr = chan<BF>(lds_k + t * G::PITCH, l, D), vr = chan<BF>(lds_v + t * G::PITCH, l, D);
-                float ak = 0.f, av = 0.f;
-                query_run(t, t + 1, s, lo, hi);
-                for (int q = lo; q < hi; q++) {
-                    if (!inside(lds_pos[t], lds_win[q], ks)) continue;
-                    const float qr = chan<BF>(lds_q + q * G::PITCH, l, D), gr = chan<BF>(lds_g + q * G::PITCH, l, D);
-                    const float p = __builtin_amdgcn_exp2f(wave_sum(qr * kr) * sc2 - lds_lse[q]);
-                    av += p * gr;
-                    ak += p * (wave_sum(gr * vr) - lds_delta[q]) * qr;
-                }
-                if (l < s.D) {
-                    static_cast<short *>(a.dk)[grad_pix(t) + l] = cvt16<BF>(ak * s.scale);
-                    static_cast<short *>(a.dv)[grad_pix(t) + l] = cvt16<BF>(av);
-                }
+            second_product<BF, D>(dv, lds_g, qq, n, g, ph);
+            second_product<BF, D>(dk, lds_q, qq, n, g, ds);
+        }
+        unsigned bad = bad_columns(dk) | bad_columns(dv);
+        const bool here = t0 + n < P && !(bad >> n & 1);
+        store_token<BF, D>(static_cast<short *>(a.dk) + at, g, dk, s.scale, here, s.D);
+        store_token<BF, D>(static_cast<short *>(a.dv) + at, g, dv, 1.f, here, s.D);
+        for (; bad; bad &= bad - 1) {
+            const int t = t0 + __builtin_ctz(bad);
+            if (t >= P) break;
+            const float kr = chan<BF>(lds_k + t * G::PITCH, l, D), vr = chan<BF>(lds_v + t * G::PITCH, l, D);
+            float ak = 0.f, av = 0.f;
+            query_run(t, t + 1, s, lo, hi);
+            for (int q = lo; q < hi; q++) {
+                if (!inside(lds_pos[t], lds_win[q], ks)) continue;
+                const float qr = chan<BF>(lds_q + q * G::PITCH, l, D), gr = chan<BF>(lds_g + q * G::PITCH, l, D);
+                const float p = __builtin_amdgcn_exp2f(wave_sum(qr * kr) * sc2 - lds_lse[q]);
+                av += p * gr;
+                ak += p * (wave_sum(gr * vr) - lds_delta[q]) * qr;
+            }
+            if (l < s.D) {
+                static_cast<short *>(a.dk)[grad_pix(t) + l] = cvt16<BF>(ak * s.scale);
+                static_cast<short *>(a.dv)[grad_pix(t) + l] = cvt16<BF>(av);
             }
         }
     }

@@ -71,6 +71,37 @@ def test_column_walk_keeps_rows_of_its_own_sub_grid_only():
             assert_close([t[sub] for t in got], ref, BF16, "sub-grid %d %d" % (i, j))
 
 
+@pytest.mark.parametrize("shape,ks,dil,dtype", [
+    ((8, 16, 14, 14, 64), 9, 1, BF16),
+    ((2, 64, 14, 14, 32), 7, 1, F16),
+    ((2, 64, 9, 10, 40), 9, 1, F16),
+    ((2, 4, 28, 28, 32), 7, 2, BF16),
+    ((1, 6, 32, 32, 64), 5, 2, F16),
+])
+def test_keys_and_values_with_a_common_component(shape, ks, dil, dtype):
+    # dP is then large against its spread over a window, and an error of delta, which the whole
+    # window shares, is multiplied by the common component of the keys
+    ensure_built()
+    from e_natten_amd import natten2d
+    q, k, v, g = make_inputs(shape, torch.float32, seed=53)
+    q, k, v, g = (t.to(dtype) for t in (q, k + 2, v + 2, g))
+    print("case common component", shape, dtype, "k=%d dilation=%d" % (ks, dil), flush=True)
+    scale = shape[-1] ** -0.5
+    x = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    o = natten2d(*x, ks, scale, dil)
+    got = [t.detach().cpu()[:1] for t in (o, *torch.autograd.grad(o, x, g.cuda()))]
+    x = [t[:1].double().requires_grad_(True) for t in (q, k, v)]
+    o_ref = O.natten2d_dilated_dense_mask(*x, ks, dil, scale)
+    ref = (o_ref.detach(), *torch.autograd.grad(o_ref, x, g[:1].double()))
+    for name, a, b in zip(("O", "dQ", "dK", "dV"), got, ref):
+        norm = ((a.double() - b).norm() / b.norm()).item()
+        print("   ", name, "2-norm %.2e" % norm, flush=True)
+        # a bfloat16 rounding is 1.7e-3 of a tensor in 2-norm (float16: an eighth); P and dS carry one
+        # each, and in dQ keys of rms sqrt(5) multiply it, of which only the spread of 1 shows in the
+        # result: sqrt(2 * 5) * 1.7e-3 = 5.4e-3, and half as much again for the results' own
+        assert norm <= (8e-3 if dtype == BF16 else 1e-3), (name, norm)
+
+
 def test_values_that_are_not_finite_stay_in_their_windows():
     # sub-grids that a workgroup takes whole: a NaN in v reaches the queries that see it, and the
     # keys that those see, alone
