@@ -5,9 +5,9 @@
 // kernel_size of 49.  Here a workgroup of four waves owns a tile of queries and walks the keys
 // that any of them sees, 64 at a time, with an online softmax: K and V rows of a block are in
 // LDS, the next block's are in flight into registers and go into a second buffer, one barrier
-// per block.  A wave owns NQ groups of 16 queries (the columns of v_mfma_f32_16x16x32); with two
-// groups every operand that comes out of LDS feeds two or four matrix instructions.  It takes the
-// keys 32 at a time, skips the steps its own queries do not reach, and masks only the steps that
+// per block.  A wave owns 16 queries (the columns of v_mfma_f32_16x16x32), or in the forward of long
+// windows two groups of 16, where every operand that comes out of LDS feeds twice the matrix
+// instructions.  It takes the keys 32 at a time, skips the steps its own queries do not reach, and masks only the steps that
 // the band's edges cut.  Operand layouts are those of na2d_mfma_kernels.h (tokens as MFMA rows,
 // the second product's other operand through the transposing LDS read).
 //
@@ -16,9 +16,14 @@
 // sums nor 16-bit operands lose anything by, and no cross-lane maximum is formed.
 //
 // Probabilities and dS enter the second products as the sum of two 16-bit terms (the value
-// rounded, and what the rounding left): the products are exact to 16 (bf16) or 22 (fp16)
-// bits of them, as close as the results' own type can show to the float32 probabilities of the
-// general kernels, which served these calls before.
+// rounded, and what the rounding left): the products are exact to 16 (bf16) or 22 (fp16) bits of them, as close as the results' own type can show to the float32
+// probabilities of the general kernels.
+//
+// The backward is renormalised as that of the general kernels: delta = dO . O carries what O was
+// rounded to, and the recomputed probabilities what the log-sum-exp was.  The dQ pass sums
+// Z = sum p and E = sum p (dP - delta) beside the products, dQ = (A - E / Z sum p k) / Z, and leaves
+// delta + E / Z and 1 / Z for the dK/dV pass.  (k and v of mean 2, bf16, d64 k128 causal: dQ off by
+// 4.7e-2 in 2-norm without, 1.7e-3 with.)
 //
 // What bounds it: at k = 128 the bytes (each key row is read by two or three workgroups of one
 // XCD, out of its L2); from k of about 512 the matrix pipe and the LDS reads that feed it.
@@ -128,6 +133,7 @@ __device__ __forceinline__ void load_row(s16x8 (&reg)[DS], const short *row, int
 // instruction per value, once a tile) and computes the tokens with a value that is not finite
 // again, one after the other, from the rows in their windows alone, in float32.  A lane then holds
 // channels lane and lane + 64.
+__device__ __forceinline__ float exp_neg(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 struct Chan2 {
     float a, b;
 };
@@ -290,27 +296,27 @@ __global__ __launch_bounds__(256, 2) void fwd_band_mfma(FwdArgs a, int tiles_t, 
             Chan2 acc{0.f, 0.f};
             float mx = -1e30f, z = 0.f;
             for (int key = band_lo(t, T, k, causal); key < band_hi(t, T, k, causal); key++) {
-                const float x = chan_dot(q, chan_load<BF>(kseq + key * a.k.sw, dlim)) * sc2;
-                const float mn = fmaxf(mx, x), corr = __builtin_amdgcn_exp2f(mx - mn);
-                const float p = __builtin_amdgcn_exp2f(x - mn);
+                const float x = chan_dot(q, chan_load<BF>(kseq + key * a.k.sw, dlim)) * s.scale;
+                const float mn = x > mx ? x : mx, corr = exp_neg(mx - mn), p = exp_neg(x - mn);
                 mx = mn;
                 z = z * corr + p;
                 acc.a *= corr;
                 acc.b *= corr;
                 chan_add(acc, p, chan_load<BF>(vseq + key * a.v.sw, dlim));
+                if (z != z) break;  // nothing finite can come of it
             }
             chan_store<BF>(oseq + t * a.o.sw, dlim, acc, 1.f / z);
             if (a.lse && l == 0)
-                a.lse[((int64_t)tl.bb * s.N + tl.nn) * T + t] = (mx + __builtin_amdgcn_logf(z)) * kLn2;
+                a.lse[((int64_t)tl.bb * s.N + tl.nn) * T + t] = mx + __builtin_amdgcn_logf(z) * kLn2;
         }
     }
 }
 
 // ------------------------------------------------------------------ dQ
 // The forward's walk with P from the saved log-sum-exp, dP^T = V dO^T, dS = P (dP - delta),
-// dQ^T += K^T dS^T.  delta = dO . O of the tile's queries is formed first and left for the
-// dK/dV pass.
-template <bool BF, int D, int NQ, bool NARROW>
+// dQ^T += K^T dS^T, and the sums that correct delta = dO . O (see the top of the file).  sum p k
+// takes P rounded to 16 bits: what it multiplies is of the size of O's rounding.
+template <bool BF, int D, bool NARROW>
 __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_t, int ntiles) {
     constexpr int KB = kRowsQ;
     using G = BGeo<D, KB>;
@@ -319,44 +325,44 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
     const Shape &s = a.s;
     const int T = s.W, k = s.kw, causal = s.cw, dlim = NARROW ? s.D : D;
     BTile tl;
-    if (!btile(blockIdx.x, gridDim.x, ntiles, tiles_t, 64 * NQ, s.N, tl)) return;
+    if (!btile(blockIdx.x, gridDim.x, ntiles, tiles_t, 64, s.N, tl)) return;
     const int wave = uni(threadIdx.x >> 6), l = threadIdx.x & 63, n = l & 15, g = l >> 4;
     const float sc2 = s.scale * kLog2e;
 
     const short *kseq = bseq(a.k, tl), *vseq = bseq(a.v, tl);
-    const int ka = band_lo(tl.t0, T, k, causal), kb = band_hi(min(tl.t0 + 64 * NQ, T) - 1, T, k, causal);
+    const int ka = band_lo(tl.t0, T, k, causal), kb = band_hi(min(tl.t0 + 64, T) - 1, T, k, causal);
     Block<D, KB, NARROW> kst, vst;
     kst.fetch(kseq, a.k.sw, ka, T, dlim);
     vst.fetch(vseq, a.v.sw, ka, T, dlim);
 
-    const int w0 = tl.t0 + wave * 16 * NQ;
+    const int w0 = tl.t0 + wave * 16;
     const bool on = w0 < T;
-    const int wa = band_lo(min(w0, T - 1), T, k, causal), wb = band_hi(min(w0 + 16 * NQ, T) - 1, T, k, causal);
+    const int wa = band_lo(min(w0, T - 1), T, k, causal), wb = band_hi(min(w0 + 16, T) - 1, T, k, causal);
     const int64_t tok0 = ((int64_t)tl.bb * s.N + tl.nn) * T;
-    s16x8 qreg[NQ][G::DS], greg[NQ][G::DS];
-    int lo[NQ], cnt[NQ], in_lo[NQ], in_hi[NQ];
-    f32x4 dq[NQ][G::DT];
-    float lse2[NQ], delta[NQ];
+    s16x8 qreg[G::DS], greg[G::DS];
+    int lo, cnt, in_lo, in_hi;
+    f32x4 dq[G::DT], pk[G::DT];
+    float lse2, delta, zsum, esum;
+    const int qt = min(w0 + n, T - 1);
+    load_row<G::DS, NARROW>(qreg, bseq(a.q, tl) + qt * a.q.sw, g, dlim);
+    load_row<G::DS, NARROW>(greg, bseq(a.d_o, tl) + qt * a.d_o.sw, g, dlim);
+    s16x8 orow[G::DS];
+    load_row<G::DS, NARROW>(orow, bseq(a.o, tl) + qt * a.o.sw, g, dlim);
+    lse2 = a.lse[tok0 + qt] * kLog2e;
+    zsum = esum = 0.f;
+    lo = band_lo(qt, T, k, causal);
+    cnt = band_hi(qt, T, k, causal) - lo;
+    in_lo = band_lo(min(w0 + 15, T - 1), T, k, causal);
+    in_hi = band_hi(min(w0, T - 1), T, k, causal);
+    float d = 0.f;
 #pragma unroll
-    for (int u = 0; u < NQ; u++) {
-        const int qt = min(w0 + u * 16 + n, T - 1);
-        load_row<G::DS, NARROW>(qreg[u], bseq(a.q, tl) + qt * a.q.sw, g, dlim);
-        load_row<G::DS, NARROW>(greg[u], bseq(a.d_o, tl) + qt * a.d_o.sw, g, dlim);
-        s16x8 orow[G::DS];
-        load_row<G::DS, NARROW>(orow, bseq(a.o, tl) + qt * a.o.sw, g, dlim);
-        lse2[u] = a.lse[tok0 + qt] * kLog2e;
-        lo[u] = band_lo(qt, T, k, causal);
-        cnt[u] = band_hi(qt, T, k, causal) - lo[u];
-        in_lo[u] = band_lo(min(w0 + u * 16 + 15, T - 1), T, k, causal);
-        in_hi[u] = band_hi(min(w0 + u * 16, T - 1), T, k, causal);
-        float d = 0.f;
+    for (int ds = 0; ds < G::DS; ds++)
+        d += dot8<BF>(__builtin_bit_cast(u32x4, greg[ds]), __builtin_bit_cast(u32x4, orow[ds]));
+    delta = col_sum(d);
 #pragma unroll
-        for (int ds = 0; ds < G::DS; ds++)
-            d += dot8<BF>(__builtin_bit_cast(u32x4, greg[u][ds]), __builtin_bit_cast(u32x4, orow[ds]));
-        delta[u] = col_sum(d);
-        if (w0 + u * 16 + n < T && g == 0) a.delta[tok0 + qt] = delta[u];
-#pragma unroll
-        for (int t = 0; t < G::DT; t++) dq[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < G::DT; t++) {
+        dq[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        pk[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     kst.commit(lds_k[0]);
     vst.commit(lds_v[0]);
@@ -373,44 +379,40 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
         for (int st = 0; st < KB / 32; st++) {
             const int kk = k0 + st * 32;
             if (!on || kk >= wb || kk + 32 <= wa) continue;
-            f32x4 c[NQ][2], cp[NQ][2];
+            f32x4 c[2], cp[2];
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 const int row = (st * 32 + h * 16 + n) * G::PITCH + g * 8;
-#pragma unroll
-                for (int u = 0; u < NQ; u++) {
-                    c[u][h] = f32x4{0.f, 0.f, 0.f, 0.f};
-                    cp[u][h] = f32x4{0.f, 0.f, 0.f, 0.f};
-                }
+                c[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+                cp[h] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int ds = 0; ds < G::DS; ds++) {
                     const s16x8 kr = *reinterpret_cast<const s16x8 *>(lk + row + ds * 32);
                     const s16x8 vr = *reinterpret_cast<const s16x8 *>(lv + row + ds * 32);
-#pragma unroll
-                    for (int u = 0; u < NQ; u++) {
-                        c[u][h] = mfma16<BF>(kr, qreg[u][ds], c[u][h]);
-                        cp[u][h] = mfma16<BF>(vr, greg[u][ds], cp[u][h]);
-                    }
+                    c[h] = mfma16<BF>(kr, qreg[ds], c[h]);
+                    cp[h] = mfma16<BF>(vr, greg[ds], cp[h]);
                 }
             }
-            s16x8 sh[NQ], sl[NQ];
+            s16x8 sh, sl, ph;
+            float x[8];
 #pragma unroll
-            for (int u = 0; u < NQ; u++) {
-                float x[8];
+            for (int e = 0; e < 8; e++) x[e] = c[e >> 2][e & 3] * sc2 - lse2;
+            if (kk < in_lo || kk + 32 > in_hi) {
 #pragma unroll
-                for (int e = 0; e < 8; e++) x[e] = c[u][e >> 2][e & 3] * sc2 - lse2[u];
-                if (kk < in_lo[u] || kk + 32 > in_hi[u]) {
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const int key = kk + (e >> 2) * 16 + g * 4 + (e & 3);
-                        x[e] = (unsigned)(key - lo[u]) < (unsigned)cnt[u] ? x[e] : -INFINITY;
-                    }
+                for (int e = 0; e < 8; e++) {
+                    const int key = kk + (e >> 2) * 16 + g * 4 + (e & 3);
+                    x[e] = (unsigned)(key - lo) < (unsigned)cnt ? x[e] : -INFINITY;
                 }
-#pragma unroll
-                for (int e = 0; e < 8; e++)
-                    x[e] = __builtin_amdgcn_exp2f(x[e]) * (cp[u][e >> 2][e & 3] - delta[u]);
-                split16<BF>(x, sh[u], sl[u]);
             }
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float p = __builtin_amdgcn_exp2f(x[e]);
+                x[e] = p * (cp[e >> 2][e & 3] - delta);
+                zsum += p;
+                esum += x[e];
+                ph[e] = cvt16<BF>(p);
+            }
+            split16<BF>(x, sh, sl);
             const short *kp[2];
 #pragma unroll
             for (int h = 0; h < 2; h++)
@@ -418,11 +420,9 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
 #pragma unroll
             for (int t = 0; t < G::DT; t++) {
                 const s16x8 kt = cat(lds_read_tr(kp[0] + t * 4), lds_read_tr(kp[1] + t * 4));
-#pragma unroll
-                for (int u = 0; u < NQ; u++) {
-                    dq[u][t] = mfma16<BF>(kt, sh[u], dq[u][t]);
-                    dq[u][t] = mfma16<BF>(kt, sl[u], dq[u][t]);
-                }
+                dq[t] = mfma16<BF>(kt, sh, dq[t]);
+                pk[t] = mfma16<BF>(kt, ph, pk[t]);
+                dq[t] = mfma16<BF>(kt, sl, dq[t]);
             }
         }
         if (more) {
@@ -432,25 +432,41 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
         __syncthreads();
     }
     if (!on) return;
+    const float zinv = 1.f / col_sum(zsum), shift = col_sum(esum) * zinv;
 #pragma unroll
-    for (int u = 0; u < NQ; u++) {
-        const int q0 = w0 + u * 16 + n, qt = min(q0, T - 1);
-        unsigned bad = bad_columns(dq[u]);
-        store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dq) + a.grad_at(tl.bb, tl.nn, 0, qt), g,
-                                                 dq[u], s.scale, q0 < T && !(bad >> n & 1), dlim);
-        for (; bad; bad &= bad - 1) {
-            const int col = __builtin_ctz(bad), t = w0 + u * 16 + col;
-            if (t >= T) break;
-            const Chan2 q = chan_load<BF>(bseq(a.q, tl) + t * a.q.sw, dlim);
-            const Chan2 go = chan_load<BF>(bseq(a.d_o, tl) + t * a.d_o.sw, dlim);
-            const float lse_t = __shfl(lse2[u], col, 64), delta_t = __shfl(delta[u], col, 64);
-            Chan2 acc{0.f, 0.f};
-            for (int key = band_lo(t, T, k, causal); key < band_hi(t, T, k, causal); key++) {
-                const Chan2 kr = chan_load<BF>(kseq + key * a.k.sw, dlim);
-                const float p = __builtin_amdgcn_exp2f(chan_dot(q, kr) * sc2 - lse_t);
-                chan_add(acc, p * (chan_dot(go, chan_load<BF>(vseq + key * a.v.sw, dlim)) - delta_t), kr);
-            }
-            chan_store<BF>(static_cast<short *>(a.dq) + a.grad_at(tl.bb, tl.nn, 0, t), dlim, acc, s.scale);
+    for (int t = 0; t < G::DT; t++) dq[t] -= shift * pk[t];
+    unsigned bad = bad_columns(dq, zinv);
+    const bool here = w0 + n < T && !(bad >> n & 1);
+    store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dq) + a.grad_at(tl.bb, tl.nn, 0, qt), g,
+                                             dq, s.scale * zinv, here, dlim);
+    if (here && g == 0) {
+        a.delta[tok0 + qt] = delta + shift;
+        a.zinv[tok0 + qt] = zinv;
+    }
+    for (; bad; bad &= bad - 1) {
+        const int col = __builtin_ctz(bad), t = w0 + col;
+        if (t >= T) break;
+        const Chan2 q = chan_load<BF>(bseq(a.q, tl) + t * a.q.sw, dlim);
+        const Chan2 go = chan_load<BF>(bseq(a.d_o, tl) + t * a.d_o.sw, dlim);
+        const float lse_t = a.lse[tok0 + t], delta_t = __shfl(delta, col, 64);
+        Chan2 acc{0.f, 0.f}, accp{0.f, 0.f};
+        float z = 0.f, res = 0.f;
+        for (int key = band_lo(t, T, k, causal); key < band_hi(t, T, k, causal); key++) {
+            const Chan2 kr = chan_load<BF>(kseq + key * a.k.sw, dlim);
+            const float p = exp_neg(chan_dot(q, kr) * s.scale - lse_t);
+            const float y = p * (chan_dot(go, chan_load<BF>(vseq + key * a.v.sw, dlim)) - delta_t);
+            z += p;
+            res += y;
+            chan_add(acc, y, kr);
+            chan_add(accp, p, kr);
+            if (z != z) break;  // nothing finite can come of it
+        }
+        const float sh_t = res / z;
+        chan_add(acc, -sh_t, accp);
+        chan_store<BF>(static_cast<short *>(a.dq) + a.grad_at(tl.bb, tl.nn, 0, t), dlim, acc, s.scale / z);
+        if (l == 0) {
+            a.delta[tok0 + t] = delta_t + sh_t;
+            a.zinv[tok0 + t] = 1.f / z;
         }
     }
 }
@@ -458,14 +474,14 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
 // ------------------------------------------------------------------ dK, dV
 // The tile is 64 keys, 16 per wave (columns), and the walk is over the queries
 // that see any of them, the inverse neighbourhood (e_natten/pytorch.py:13-23), a block at a time: Q
-// and dO rows, the log-sum-exp and delta of a block in LDS.  dV^T += dO^T P, dK^T += Q^T dS.
+// and dO rows, the log-sum-exp, delta and 1 / Z of a block in LDS.  dV^T += dO^T P, dK^T += Q^T dS.
 template <bool BF, int D, bool NARROW>
 __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tiles_t, int ntiles) {
     constexpr int KB = kRowsK<D>;
     using G = BGeo<D, KB>;
     __shared__ __attribute__((aligned(16))) short lds_q[2][KB * G::PITCH];
     __shared__ __attribute__((aligned(16))) short lds_g[2][KB * G::PITCH];
-    __shared__ __attribute__((aligned(16))) float2 lds_stat[2][KB];  // (lse * log2e, delta)
+    __shared__ __attribute__((aligned(16))) float lds_stat[2][3][KB];  // lse * log2e, delta, 1 / Z
     const Shape &s = a.s;
     const int T = s.W, k = s.kw, causal = s.cw, dlim = NARROW ? s.D : D;
     BTile tl;
@@ -477,19 +493,24 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
     const int64_t tok0 = ((int64_t)tl.bb * s.N + tl.nn) * T;
     const int qa = axis_inv_lo(tl.t0, k, causal), qb = axis_inv_hi(min(tl.t0 + 64, T) - 1, T, k, causal);
     Block<D, KB, NARROW> qst, gst;
-    float2 sst = make_float2(0.f, 0.f);
+    float sst[3] = {0.f, 0.f, 0.f};
     auto fetch = [&](int p0) __attribute__((always_inline)) {
         qst.fetch(qseq, a.q.sw, p0, T, dlim);
         gst.fetch(gseq, a.d_o.sw, p0, T, dlim);
         if (threadIdx.x < KB) {
             const int64_t at = tok0 + min(p0 + (int)threadIdx.x, T - 1);
-            sst = make_float2(a.lse[at] * kLog2e, a.delta[at]);
+            sst[0] = a.lse[at] * kLog2e;
+            sst[1] = a.delta[at];
+            sst[2] = a.zinv[at];
         }
     };
     auto commit = [&](int buf) __attribute__((always_inline)) {
         qst.commit(lds_q[buf]);
         gst.commit(lds_g[buf]);
-        if (threadIdx.x < KB) lds_stat[buf][threadIdx.x] = sst;
+        if (threadIdx.x < KB) {
+#pragma unroll
+            for (int j = 0; j < 3; j++) lds_stat[buf][j][threadIdx.x] = sst[j];
+        }
     };
     fetch(qa);
 
@@ -513,7 +534,6 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
         const bool more = p0 + KB < qb;
         if (more) fetch(p0 + KB);
         const short *lq = lds_q[buf], *lg = lds_g[buf];
-        const float2 *stat = lds_stat[buf];
 #pragma unroll
         for (int st = 0; st < KB / 32; st++) {
             const int qq = p0 + st * 32;
@@ -532,15 +552,18 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
                     cp[h] = mfma16<BF>(gr, vreg[ds], cp[h]);
                 }
             }
-            float2 sv[8];
+            f32x4 sv[3][2];
 #pragma unroll
-            for (int e = 0; e < 8; e++) sv[e] = stat[st * 32 + (e >> 2) * 16 + g * 4 + (e & 3)];
+            for (int j = 0; j < 3; j++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    sv[j][h] = *reinterpret_cast<const f32x4 *>(&lds_stat[buf][j][st * 32 + h * 16 + g * 4]);
             // the keys that all 32 queries of the step see
             const int in_lo = band_lo(min(qq + 31, T - 1), T, k, causal), in_hi = band_hi(qq, T, k, causal);
             s16x8 ph, pl, sh, sl;
             float x[8], y[8];
 #pragma unroll
-            for (int e = 0; e < 8; e++) x[e] = c[e >> 2][e & 3] * sc2 - sv[e].x;
+            for (int e = 0; e < 8; e++) x[e] = c[e >> 2][e & 3] * sc2 - sv[0][e >> 2][e & 3];
             if (w0 < in_lo || w0 + 16 > in_hi || qq + 32 > T) {
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
@@ -552,8 +575,8 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
             }
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                x[e] = __builtin_amdgcn_exp2f(x[e]);
-                y[e] = x[e] * (cp[e >> 2][e & 3] - sv[e].y);
+                x[e] = __builtin_amdgcn_exp2f(x[e]) * sv[2][e >> 2][e & 3];
+                y[e] = x[e] * (cp[e >> 2][e & 3] - sv[1][e >> 2][e & 3]);
             }
             split16<BF>(x, ph, pl);
             split16<BF>(y, sh, sl);
@@ -592,9 +615,10 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
         for (int q = axis_inv_lo(key, k, causal); q < axis_inv_hi(key, T, k, causal); q++) {
             if ((unsigned)(key - band_lo(q, T, k, causal)) >= (unsigned)k) continue;
             const Chan2 qr = chan_load<BF>(qseq + q * a.q.sw, dlim), gr = chan_load<BF>(gseq + q * a.d_o.sw, dlim);
-            const float p = __builtin_amdgcn_exp2f(chan_dot(qr, kr) * sc2 - a.lse[tok0 + q] * kLog2e);
+            const float p = exp_neg(chan_dot(qr, kr) * s.scale - a.lse[tok0 + q]) * a.zinv[tok0 + q];
             chan_add(av, p, gr);
             chan_add(ak, p * (chan_dot(gr, vr) - a.delta[tok0 + q]), qr);
+            if (p != p) break;  // nothing finite can come of it
         }
         const int64_t to = a.grad_at(tl.bb, tl.nn, 0, key);
         chan_store<BF>(static_cast<short *>(a.dk) + to, dlim, ak, s.scale);
@@ -603,12 +627,13 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
 }
 
 // ------------------------------------------------------------------ dispatch
-// Two groups of 16 queries per wave (forward and dQ pass) where the walk is long, a key row is 256
-// bytes, and tiles of that size still give every CU its two workgroups: the LDS reads of a step then feed
-// twice the matrix instructions.  One group / two, us, causal: head_dim 128 B2 N8 T4096 k400 forward
-// 36.5 / 33.4, dQ 43.5 / 38.2; at k = 128 (B1 N16 T8192) level (43.1 / 44.1, 50.9 / 49.7); head_dim 64
-// B2 N16 T4096 k256 25.7 / 33.5 and 30.9 / 36.9: there more waves count for more.  The dK/dV
-// pass with two groups of keys: 108 / 151 at head_dim 64.
+// Two groups of 16 queries per wave (forward) where the walk is long, a key row is 256 bytes, and
+// tiles of that size still give every CU its two workgroups: the LDS reads of a step then feed twice the
+// matrix instructions.  One group / two, us, causal: head_dim 128 B2 N8 T4096 k400 40.4 / 35.0, B2 N32
+// T8192 k512 351 / 294; at k = 128 (B1 N16 T8192) level (43.1 / 44.1); head_dim 64 B2 N16 T4096 k256
+// 25.7 / 33.5: there more waves count for more.  Not in the dQ pass: its third product takes the
+// registers that a second group needs (with two, B2 N32 T8192 d128 k512 spills and its backward
+// takes 1432 us instead of 1005), nor in the dK/dV pass (head_dim 64: 108 / 151).
 bool two_groups(const Shape &s) {
     return s.D == 128 && s.kw >= 256 && (int64_t)s.B * s.N * ((s.W + 127) / 128) >= 512;
 }
@@ -625,34 +650,22 @@ int fwd_go(const FwdArgs &a, hipStream_t st) {
     }
     return check_launch("fwd_band_mfma");
 }
-template <bool BF, int D, int NQ, bool NARROW>
+template <bool BF, int D, bool NARROW>
 int bwd_go(const BwdArgs &a, hipStream_t st) {
-    const int tiles_t = (a.s.W + 64 * NQ - 1) / (64 * NQ);
+    const int tiles_t = (a.s.W + 63) / 64;
     const int64_t nt = (int64_t)a.s.B * a.s.N * tiles_t;
     {
         ProfScope prof(ENATTEN_KERNEL_BWD_DQ, "bwd_band_dq_mfma", st);
-        hipLaunchKernelGGL((bwd_band_dq_mfma<BF, D, NQ, NARROW>), dim3(band_grid(nt)), dim3(256), 0, st, a, tiles_t,
+        hipLaunchKernelGGL((bwd_band_dq_mfma<BF, D, NARROW>), dim3(band_grid(nt)), dim3(256), 0, st, a, tiles_t,
                            (int)nt);
     }
     {
         ProfScope prof(ENATTEN_KERNEL_BWD_DKDV, "bwd_band_dkdv_mfma", st);
-        const int tk = (a.s.W + 63) / 64;
-        const int64_t nk = (int64_t)a.s.B * a.s.N * tk;
-        hipLaunchKernelGGL((bwd_band_dkdv_mfma<BF, D, NARROW>), dim3(band_grid(nk)), dim3(256), 0, st, a, tk,
-                           (int)nk);
+        hipLaunchKernelGGL((bwd_band_dkdv_mfma<BF, D, NARROW>), dim3(band_grid(nt)), dim3(256), 0, st, a, tiles_t,
+                           (int)nt);
     }
     return check_launch("bwd_band_mfma");
 }
-
-#define ENATTEN_BAND(FN, BF, ARGS, ST)                                                         \
-    switch ((ARGS).s.D) {                                                                      \
-        case 32: return FN<BF, 32, 1, false>(ARGS, ST);                                        \
-        case 64: return FN<BF, 64, 1, false>(ARGS, ST);                                        \
-        case 128: return two ? FN<BF, 128, 2, false>(ARGS, ST) : FN<BF, 128, 1, false>(ARGS, ST); \
-    }                                                                                          \
-    if ((ARGS).s.D < 32) return FN<BF, 32, 1, true>(ARGS, ST);                                 \
-    if ((ARGS).s.D < 64) return FN<BF, 64, 1, true>(ARGS, ST);                                 \
-    return FN<BF, 128, 1, true>(ARGS, ST);
 
 bool band_layout_ok(const View &v) {
     return reinterpret_cast<uintptr_t>(v.ptr) % 16 == 0 && v.sb % 8 == 0 && v.sn % 8 == 0 && v.sw % 8 == 0 &&
@@ -677,21 +690,30 @@ bool band_supported(const BwdArgs &a, int dtype) {
            band_layout_ok(a.v) && band_layout_ok(a.o) && band_layout_ok(a.d_o) && al(a.dq) && al(a.dk) &&
            al(a.dv) && a.gsb % 8 == 0 && a.gsn % 8 == 0 && a.gsw % 8 == 0;
 }
-int launch_fwd_band(const FwdArgs &a, int dtype, hipStream_t st) {
-    const bool two = two_groups(a.s);
-    if (dtype == ENATTEN_BF16) {
-        ENATTEN_BAND(fwd_go, true, a, st)
-    } else {
-        ENATTEN_BAND(fwd_go, false, a, st)
+template <bool BF>
+int fwd_dim(const FwdArgs &a, hipStream_t st) {
+    switch (a.s.D) {
+        case 32: return fwd_go<BF, 32, 1, false>(a, st);
+        case 64: return fwd_go<BF, 64, 1, false>(a, st);
+        case 128: return two_groups(a.s) ? fwd_go<BF, 128, 2, false>(a, st) : fwd_go<BF, 128, 1, false>(a, st);
     }
+    return a.s.D < 32   ? fwd_go<BF, 32, 1, true>(a, st)
+           : a.s.D < 64 ? fwd_go<BF, 64, 1, true>(a, st) : fwd_go<BF, 128, 1, true>(a, st);
+}
+template <bool BF>
+int bwd_dim(const BwdArgs &a, hipStream_t st) {
+    switch (a.s.D) {
+        case 32: return bwd_go<BF, 32, false>(a, st);
+        case 64: return bwd_go<BF, 64, false>(a, st);
+        case 128: return bwd_go<BF, 128, false>(a, st);
+    }
+    return a.s.D < 32 ? bwd_go<BF, 32, true>(a, st) : a.s.D < 64 ? bwd_go<BF, 64, true>(a, st) : bwd_go<BF, 128, true>(a, st);
+}
+int launch_fwd_band(const FwdArgs &a, int dtype, hipStream_t st) {
+    return dtype == ENATTEN_BF16 ? fwd_dim<true>(a, st) : fwd_dim<false>(a, st);
 }
 int launch_bwd_band(const BwdArgs &a, int dtype, hipStream_t st) {
-    const bool two = two_groups(a.s);
-    if (dtype == ENATTEN_BF16) {
-        ENATTEN_BAND(bwd_go, true, a, st)
-    } else {
-        ENATTEN_BAND(bwd_go, false, a, st)
-    }
+    return dtype == ENATTEN_BF16 ? bwd_dim<true>(a, st) : bwd_dim<false>(a, st);
 }
 
 }  // namespace enatten
