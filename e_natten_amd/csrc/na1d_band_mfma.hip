@@ -16,8 +16,10 @@
 // sums nor 16-bit operands lose anything by, and no cross-lane maximum is formed.
 //
 // Probabilities and dS enter the second products as the sum of two 16-bit terms (the value
-// rounded, and what the rounding left): the products are exact to 16 (bf16) or 22 (fp16) bits of them, as close as the results' own type can show to the float32
-// probabilities of the general kernels.
+// rounded, and what the rounding left): the products are exact to 16 (bf16) or 22 (fp16, down to
+// 2^-25 of the largest) bits of them, as close as the results' own type can show to the float32
+// probabilities of the general kernels.  float16 dS, and P in the dK/dV pass, are scaled by a power
+// of two for that (DsScale; kPScale).
 //
 // The backward is renormalised as that of the general kernels: delta = dO . O carries what O was
 // rounded to, and the recomputed probabilities what the log-sum-exp was.  The dQ pass sums
@@ -343,6 +345,7 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
     int lo, cnt, in_lo, in_hi;
     f32x4 dq[G::DT], pk[G::DT];
     float lse2, delta, zsum, esum;
+    DsScale<BF> scl;
     const int qt = min(w0 + n, T - 1);
     load_row<G::DS, NARROW>(qreg, bseq(a.q, tl) + qt * a.q.sw, g, dlim);
     load_row<G::DS, NARROW>(greg, bseq(a.d_o, tl) + qt * a.d_o.sw, g, dlim);
@@ -394,7 +397,7 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
                 }
             }
             s16x8 sh, sl, ph;
-            float x[8];
+            float x[8], mag = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; e++) x[e] = c[e >> 2][e & 3] * sc2 - lse2;
             if (kk < in_lo || kk + 32 > in_hi) {
@@ -411,6 +414,13 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
                 zsum += p;
                 esum += x[e];
                 ph[e] = cvt16<BF>(p);
+                if (!BF) mag = fmaxf(mag, fabsf(x[e]));
+            }
+            if constexpr (!BF) {
+                scl.fit(mag, dq);
+                const float f = scl.factor();
+#pragma unroll
+                for (int e = 0; e < 8; e++) x[e] *= f;
             }
             split16<BF>(x, sh, sl);
             const short *kp[2];
@@ -434,7 +444,7 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
     if (!on) return;
     const float zinv = 1.f / col_sum(zsum), shift = col_sum(esum) * zinv;
 #pragma unroll
-    for (int t = 0; t < G::DT; t++) dq[t] -= shift * pk[t];
+    for (int t = 0; t < G::DT; t++) dq[t] = dq[t] * scl.inverse() - shift * pk[t];
     unsigned bad = bad_columns(dq, zinv);
     const bool here = w0 + n < T && !(bad >> n & 1);
     store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dq) + a.grad_at(tl.bb, tl.nn, 0, qt), g,
@@ -475,13 +485,16 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
 // The tile is 64 keys, 16 per wave (columns), and the walk is over the queries
 // that see any of them, the inverse neighbourhood (e_natten/pytorch.py:13-23), a block at a time: Q
 // and dO rows, the log-sum-exp, delta and 1 / Z of a block in LDS.  dV^T += dO^T P, dK^T += Q^T dS.
+// kPScale: float16 probabilities come out of 1 / Z times 2^14 (see DsScale).
+template <bool BF>
+constexpr float kPScale = BF ? 1.f : 16384.f;
 template <bool BF, int D, bool NARROW>
 __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tiles_t, int ntiles) {
     constexpr int KB = kRowsK<D>;
     using G = BGeo<D, KB>;
     __shared__ __attribute__((aligned(16))) short lds_q[2][KB * G::PITCH];
     __shared__ __attribute__((aligned(16))) short lds_g[2][KB * G::PITCH];
-    __shared__ __attribute__((aligned(16))) float lds_stat[2][3][KB];  // lse * log2e, delta, 1 / Z
+    __shared__ __attribute__((aligned(16))) float lds_stat[2][3][KB];  // lse * log2e, delta, kPScale / Z
     const Shape &s = a.s;
     const int T = s.W, k = s.kw, causal = s.cw, dlim = NARROW ? s.D : D;
     BTile tl;
@@ -501,7 +514,7 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
             const int64_t at = tok0 + min(p0 + (int)threadIdx.x, T - 1);
             sst[0] = a.lse[at] * kLog2e;
             sst[1] = a.delta[at];
-            sst[2] = a.zinv[at];
+            sst[2] = a.zinv[at] * kPScale<BF>;
         }
     };
     auto commit = [&](int buf) __attribute__((always_inline)) {
@@ -519,6 +532,7 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
     const int wa = axis_inv_lo(min(w0, T - 1), k, causal), wb = axis_inv_hi(min(w0 + 16, T) - 1, T, k, causal);
     s16x8 kreg[G::DS], vreg[G::DS];
     f32x4 dk[G::DT], dv[G::DT];
+    DsScale<BF> scl;
     const int kt = min(w0 + n, T - 1);  // this lane's key
     load_row<G::DS, NARROW>(kreg, bseq(a.k, tl) + kt * a.k.sw, g, dlim);
     load_row<G::DS, NARROW>(vreg, bseq(a.v, tl) + kt * a.v.sw, g, dlim);
@@ -561,7 +575,7 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
             // the keys that all 32 queries of the step see
             const int in_lo = band_lo(min(qq + 31, T - 1), T, k, causal), in_hi = band_hi(qq, T, k, causal);
             s16x8 ph, pl, sh, sl;
-            float x[8], y[8];
+            float x[8], y[8], mag = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; e++) x[e] = c[e >> 2][e & 3] * sc2 - sv[0][e >> 2][e & 3];
             if (w0 < in_lo || w0 + 16 > in_hi || qq + 32 > T) {
@@ -577,6 +591,13 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
             for (int e = 0; e < 8; e++) {
                 x[e] = __builtin_amdgcn_exp2f(x[e]) * sv[2][e >> 2][e & 3];
                 y[e] = x[e] * (cp[e >> 2][e & 3] - sv[1][e >> 2][e & 3]);
+                if (!BF) mag = fmaxf(mag, fabsf(y[e]));
+            }
+            if constexpr (!BF) {
+                scl.fit(mag, dk);
+                const float f = scl.factor();
+#pragma unroll
+                for (int e = 0; e < 8; e++) y[e] *= f;
             }
             split16<BF>(x, ph, pl);
             split16<BF>(y, sh, sl);
@@ -601,11 +622,14 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
         __syncthreads();
     }
     if (!on) return;
+    const float unscale = scl.inverse() / kPScale<BF>;  // (powers of two)
+#pragma unroll
+    for (int t = 0; t < G::DT; t++) dk[t] *= unscale;
     unsigned bad = bad_columns(dk) | bad_columns(dv);
     const bool live = w0 + n < T && !(bad >> n & 1);
     const int64_t at = a.grad_at(tl.bb, tl.nn, 0, kt);
     store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dk) + at, g, dk, s.scale, live, dlim);
-    store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dv) + at, g, dv, 1.f, live, dlim);
+    store_token<BF, D, (D >= 64 && !NARROW)>(static_cast<short *>(a.dv) + at, g, dv, 1.f / kPScale<BF>, live, dlim);
     for (; bad; bad &= bad - 1) {
         const int key = w0 + __builtin_ctz(bad);
         if (key >= T) break;

@@ -85,6 +85,35 @@ __device__ __forceinline__ float wave_sum(float x) {
     return x;
 }
 
+// Two 16-bit terms of a float16 value end at 2^-25 absolute (below 2^-14 the rounded value is
+// subnormal, and so is what the rounding left), and values beyond 65504 have none at all.  dS goes
+// with the upstream gradient, whose magnitude is the caller's affair (loss scaling), so float16 dS
+// are multiplied by a power of two per column of the second product that brings the largest so far
+// to between 2^9 and 2^15; the column's sums follow when it has to change, and are divided by it in
+// the end.  bfloat16 has the exponents of float32 and needs none of it.
+template <bool BF>
+struct DsScale {
+    int e = -100;     // the column's dS are multiplied by 2^(10 - e)
+    float top = 0.f;  // largest magnitude that this allows for
+    // `mag`: this lane's largest |dS|; acc: the column's sums
+    template <int DT>
+    __device__ __forceinline__ void fit(float mag, f32x4 (&acc)[DT]) {
+        if constexpr (!BF) {
+            if (__any(mag > top)) {
+                const float m = col_max(mag);
+                const int en = m > top ? max(__builtin_amdgcn_frexp_expf(m), -100) : e;
+                const float corr = __builtin_ldexpf(1.f, max(e - en, -126));
+                top = m > top ? __builtin_ldexpf(1.f, en + 5) : top;
+                e = en;
+#pragma unroll
+                for (int t = 0; t < DT; t++) acc[t] *= corr;
+            }
+        }
+    }
+    __device__ __forceinline__ float factor() const { return BF ? 1.f : __builtin_ldexpf(1.f, 10 - e); }
+    __device__ __forceinline__ float inverse() const { return BF ? 1.f : __builtin_ldexpf(1.f, e - 10); }
+};
+
 // dO . O over the 8 channels of one 16-byte chunk: four two-element dot products that
 // accumulate in float32 (v_dot2c_f32_bf16 / v_dot2c_f32_f16), one instruction per dword where
 // taking the halves apart and multiplying them took six.

@@ -133,3 +133,17 @@ def test_keys_and_values_with_a_common_component(shape, ks, causal, dtype):
         norm = ((x - r).norm() / r.norm()).item()
         print("   ", name, "2-norm %.2e" % norm, flush=True)
         assert norm <= (4e-3 if dtype == BF16 else 5e-4), (name, norm)  # (as in test_band_windows)
+
+
+@pytest.mark.parametrize("shape,ks", [((1, 2, 600, 64), 128), ((1, 2, 400, 128), 300), ((1, 2, 200, 32), 5)])
+def test_float16_with_small_upstream_gradients(shape, ks):
+    # dS of 1e-6 and less, which two float16 terms alone do not hold
+    ensure_built()
+    print("case small gradients", shape, ks, flush=True)
+    q, k, v, g = make_inputs(shape, torch.float32, seed=59)
+    got, ref = _against_oracle([t.to(F16) for t in (q, k, v, g * 1e-4)], ks, True, shape[-1] ** -0.5)
+    for name, x, r in zip(("dQ", "dK", "dV"), got[1:], ref[1:]):
+        norm = ((x - r).norm() / r.norm()).item()
+        rounding = ((r.to(F16).double() - r).norm() / r.norm()).item()
+        print("   ", name, "2-norm %.2e, of the result's rounding alone %.2e" % (norm, rounding), flush=True)
+        assert norm <= 1.05 * rounding, (name, norm, rounding)
