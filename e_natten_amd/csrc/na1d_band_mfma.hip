@@ -135,6 +135,11 @@ __device__ __forceinline__ void load_row(s16x8 (&reg)[DS], const short *row, int
 // instruction per value, once a tile) and computes the tokens with a value that is not finite
 // again, one after the other, from the rows in their windows alone, in float32.  A lane then holds
 // channels lane and lane + 64.
+// Queries whose logits lie beyond kFar take the same way: log2 and natural units do not convert
+// into each other closely enough there for probabilities out of a log-sum-exp, so these are computed in
+// natural units throughout, as by the general kernels.
+constexpr float kFar = 1048576.f;
+__device__ __forceinline__ bool far(float lse) { return !(fabsf(lse) <= kFar); }  // (also NaN)
 __device__ __forceinline__ float exp_neg(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 struct Chan2 {
     float a, b;
@@ -199,7 +204,7 @@ __global__ __launch_bounds__(256, 2) void fwd_band_mfma(FwdArgs a, int tiles_t, 
         in_hi[u] = band_hi(min(w0 + u * 16, T - 1), T, k, causal);
 #pragma unroll
         for (int t = 0; t < G::DT; t++) o[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        m[u] = -1e30f;
+        m[u] = -__FLT_MAX__;
         sum[u] = 0.f;
     }
     kst.commit(lds_k[0]);
@@ -286,7 +291,7 @@ __global__ __launch_bounds__(256, 2) void fwd_band_mfma(FwdArgs a, int tiles_t, 
         const int q0 = w0 + u * 16 + n, qt = min(q0, T - 1);
         const bool live = q0 < T;
         const float total = col_sum(sum[u]);
-        unsigned bad = bad_columns(o[u], total);
+        unsigned bad = bad_columns(o[u], far(m[u]) ? INFINITY : total);
         const bool here = live && !(bad >> n & 1);
         store_token<BF, D, (D >= 64 && !NARROW)>(oseq + qt * a.o.sw, g, o[u], 1.f / total, here, dlim);
         if (a.lse && here && g == 0)
@@ -296,7 +301,7 @@ __global__ __launch_bounds__(256, 2) void fwd_band_mfma(FwdArgs a, int tiles_t, 
             if (t >= T) break;
             const Chan2 q = chan_load<BF>(qseq + t * a.q.sw, dlim);
             Chan2 acc{0.f, 0.f};
-            float mx = -1e30f, z = 0.f;
+            float mx = -INFINITY, z = 0.f;
             for (int key = band_lo(t, T, k, causal); key < band_hi(t, T, k, causal); key++) {
                 const float x = chan_dot(q, chan_load<BF>(kseq + key * a.k.sw, dlim)) * s.scale;
                 const float mn = x > mx ? x : mx, corr = exp_neg(mx - mn), p = exp_neg(x - mn);
@@ -351,7 +356,8 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
     load_row<G::DS, NARROW>(greg, bseq(a.d_o, tl) + qt * a.d_o.sw, g, dlim);
     s16x8 orow[G::DS];
     load_row<G::DS, NARROW>(orow, bseq(a.o, tl) + qt * a.o.sw, g, dlim);
-    lse2 = a.lse[tok0 + qt] * kLog2e;
+    const float lse = a.lse[tok0 + qt];
+    lse2 = far(lse) ? NAN : lse * kLog2e;  // (the whole column is then computed again)
     zsum = esum = 0.f;
     lo = band_lo(qt, T, k, causal);
     cnt = band_hi(qt, T, k, causal) - lo;
@@ -512,7 +518,8 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
         gst.fetch(gseq, a.d_o.sw, p0, T, dlim);
         if (threadIdx.x < KB) {
             const int64_t at = tok0 + min(p0 + (int)threadIdx.x, T - 1);
-            sst[0] = a.lse[at] * kLog2e;
+            const float lse = a.lse[at];
+            sst[0] = far(lse) ? NAN : lse * kLog2e;  // (the keys that this query sees are then computed again)
             sst[1] = a.delta[at];
             sst[2] = a.zinv[at] * kPScale<BF>;
         }

@@ -147,3 +147,22 @@ def test_float16_with_small_upstream_gradients(shape, ks):
         rounding = ((r.to(F16).double() - r).norm() / r.norm()).item()
         print("   ", name, "2-norm %.2e, of the result's rounding alone %.2e" % (norm, rounding), flush=True)
         assert norm <= 1.05 * rounding, (name, norm, rounding)
+
+
+@pytest.mark.parametrize("dtype,size", [(BF16, 1e16), (F16, 4096.0)])
+def test_logits_far_from_zero(dtype, size):
+    # logits of -1e32 (float16: -1.7e7) that are equal over a window: the probabilities are uniform
+    ensure_built()
+    q, k, v, g = make_inputs((1, 2, 150, 64), dtype, seed=61)
+    q, k = torch.zeros_like(q), torch.zeros_like(k)
+    q[..., 0], k[..., 0] = size, -size
+    from e_natten_amd import natten1d
+    x = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    o = natten1d(*x, 40, 1.0, 1, True)
+    dv = torch.autograd.grad(o, x, g.cuda())[2]
+    p = O.axis_window_mask(150, 40, True).double()
+    p = p / p.sum(1, keepdim=True)
+    for name, got, r in (("O", o, p @ v.double()), ("dV", dv, p.T @ g.double())):
+        norm = ((got.detach().cpu().double() - r).norm() / r.norm()).item()
+        print("   ", name, dtype, "2-norm %.2e" % norm, flush=True)
+        assert norm <= (4e-3 if dtype == BF16 else 5e-4), (name, norm)  # (as in test_band_windows)
