@@ -196,7 +196,7 @@ __global__ __launch_bounds__(G::NT, G::WPS) void fwd_small_mfma(FwdArgsSub a, in
         f32x4 o[G::DT];
 #pragma unroll
         for (int t = 0; t < G::DT; t++) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        float m = -1e30f, sum = 0.f;
+        float m = -__FLT_MAX__, sum = 0.f;
         for (int kk = lo & ~15; kk < hi; kk += 32) {
             f32x4 c[2];
             first_product<BF, D>(c, lds_k, kk, n, g, qreg);
@@ -234,11 +234,11 @@ __global__ __launch_bounds__(G::NT, G::WPS) void fwd_small_mfma(FwdArgsSub a, in
             const int t = t0 + __builtin_ctz(bad);
             if (t >= P) break;
             const float q = chan<BF>(qimg + pix(a.q, a.dil, t / s.W, t % s.W), l, s.D);
-            float acc = 0.f, mx = -1e30f, z = 0.f;
+            float acc = 0.f, mx = -INFINITY, z = 0.f;
             for (int j = 0; j < ks * ks; j++) {
                 const int w = lds_win[t], key = ((w & 0xffff) + j / ks) * s.W + (w >> 16) + j % ks;
                 const float x = wave_sum(q * chan<BF>(lds_k + key * G::PITCH, l, D)) * sc2;
-                const float mn = fmaxf(mx, x), corr = __builtin_amdgcn_exp2f(mx - mn);
+                const float mn = x > mx ? x : mx, corr = __builtin_amdgcn_exp2f(mx - mn);
                 const float p = __builtin_amdgcn_exp2f(x - mn);
                 mx = mn;
                 z = z * corr + p;

@@ -102,6 +102,21 @@ def test_keys_and_values_with_a_common_component(shape, ks, dil, dtype):
         assert norm <= (8e-3 if dtype == BF16 else 1e-3), (name, norm)
 
 
+def test_logits_far_from_zero():
+    # images taken whole, logits of -1e32 that are equal over a window: the probabilities are uniform
+    ensure_built()
+    from e_natten_amd import natten2d
+    H, W, ks = 9, 10, 9
+    q, k, v, _ = make_inputs((3, 90, H, W, 32), BF16, seed=61)
+    q, k = torch.zeros_like(q), torch.zeros_like(k)
+    q[..., 0], k[..., 0] = 1e16, -1e16
+    o = natten2d(q.cuda(), k.cuda(), v.cuda(), ks).cpu().double()
+    ref = (O.neighbour_mask(H, W, ks).double() / ks ** 2 @ v.double().flatten(2, 3)).view(v.shape)
+    norm = ((o - ref).norm() / ref.norm()).item()
+    print("    O 2-norm %.2e" % norm, flush=True)
+    assert norm <= 4e-3, norm  # (the rounding of the result, 1.7e-3, and of P)
+
+
 def test_values_that_are_not_finite_stay_in_their_windows():
     # sub-grids that a workgroup takes whole: a NaN in v reaches the queries that see it, and the
     # keys that those see, alone
