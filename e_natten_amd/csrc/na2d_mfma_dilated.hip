@@ -30,7 +30,8 @@ bool sub_layout_ok(const FwdArgsSub &a) {
 bool sub_layout_ok(const BwdArgsSub &a) {
     auto al = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
     return sub_ok(a.q, a.dil) && sub_ok(a.k, a.dil) && sub_ok(a.v, a.dil) && sub_ok(a.o, a.dil) &&
-           sub_ok(a.d_o, a.dil) && al(a.dq) && al(a.dk) && al(a.dv) && a.gsw % 8 == 0 &&
+           sub_ok(a.d_o, a.dil) && al(a.dq) && al(a.dk) && al(a.dv) &&
+           a.gsb % 8 == 0 && a.gsn % 8 == 0 && a.gsh % 8 == 0 && a.gsw % 8 == 0 &&  // 16-byte stores
            a.s.H < 32768 && a.s.W < 32768;  // (the dK/dV pass keeps window starts in 16 bits)
 }
 

@@ -1,4 +1,6 @@
 """Dilated neighborhoods: all sub-grids of one size in one launch, against the dense-mask oracle."""
+import ctypes
+
 import pytest
 import torch
 
@@ -115,6 +117,39 @@ def test_logits_far_from_zero():
     norm = ((o - ref).norm() / ref.norm()).item()
     print("    O 2-norm %.2e" % norm, flush=True)
     assert norm <= 4e-3, norm  # (the rounding of the result, 1.7e-3, and of P)
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_gradient_strides_that_16_byte_stores_do_not_take(axis):
+    # images that would be taken whole; a batch, head or row stride of the gradients that is no
+    # multiple of 8 elements
+    from e_natten_amd import _lib
+    lib = ensure_built()
+    B, N, H, W, D = shape = (2, 65, 14, 14, 32)
+    ks = 7
+    print("case gradient strides", shape, "axis", axis, flush=True)
+    q, k, v, g = (t.cuda() for t in make_inputs(shape, BF16, seed=67))
+    o = torch.empty_like(q)
+    lse = torch.empty(shape[:-1], dtype=torch.float32, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    assert lib.enatten2d_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), B, N, H, W, D,
+                             ks, _lib.BF16, None, None, None, None, 0.2, st) == 0
+    strides = [N * H * W * D, H * W * D, W * D, D]
+    for i in range(axis, -1, -1):  # 4 more elements along `axis`, the outer axes made to fit
+        strides[i] = strides[i + 1] * shape[i + 1] + (4 if i == axis else 0)
+    res = []
+    for gs in (None, strides):
+        views = [torch.zeros(B * (strides[0] if gs else N * H * W * D), dtype=BF16, device="cuda").as_strided(
+            shape, (*(gs or (N * H * W * D, H * W * D, W * D, D)), 1)) for _ in range(3)]
+        ws = torch.empty(lib.enatten2d_bwd_workspace_bytes(B, N, H, W, D, ks, _lib.BF16), dtype=torch.uint8,
+                         device="cuda")
+        assert lib.enatten2d_bwd_into(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), g.data_ptr(), lse.data_ptr(),
+            *(t.data_ptr() for t in views), ws.data_ptr(), B, N, H, W, D, ks, _lib.BF16, None, None, None, None,
+            None, (ctypes.c_int64 * 4)(*gs) if gs else None, 0.2, st) == 0
+        res.append(views)
+    torch.cuda.synchronize()
+    assert_close([t.cpu() for t in (o, *res[1])], [t.cpu() for t in (o, *res[0])], BF16, "axis %d" % axis)
 
 
 def test_values_that_are_not_finite_stay_in_their_windows():
