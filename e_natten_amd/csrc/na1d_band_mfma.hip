@@ -706,7 +706,7 @@ bool band_layout_ok(const View &v) {
 // takes the two sums in one order, as in the general kernels)
 bool band_shape_ok(const Shape &s, int dtype) {
     return s.kw > 1 && (dtype == ENATTEN_BF16 || dtype == ENATTEN_F16) && s.D >= 8 && s.D <= 128 && s.D % 8 == 0 &&
-           s.H == 1 && s.kh == 1 && (int64_t)s.B * s.N * ((s.W + 63) / 64) < ((int64_t)1 << 31) - 8;
+           s.H == 1 && s.kh == 1 && (int64_t)s.B * s.N * ((s.W + 63) / 64) <= ((int64_t)1 << 32) / 256 - 8;  // (threads of a launch)
 }
 
 }  // namespace

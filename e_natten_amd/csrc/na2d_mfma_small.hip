@@ -440,10 +440,18 @@ int bwd_go(const BwdArgsSub &a, hipStream_t st) {
     }
     return check_launch("bwd_small_mfma");
 }
-bool size_ok(const Shape &s, int64_t nimages, int max_tokens) {
-    return s.D <= 64 && (int64_t)s.H * s.W <= max_tokens && nimages < ((int64_t)1 << 31) - 8;
+// (a launch holds fewer than 2^32 threads: more images are left to the tiled kernels, whose grid does
+// not grow with them)
+bool size_ok(const Shape &s, int64_t nimages, int max_tokens, int threads) {
+    return s.D <= 64 && (int64_t)s.H * s.W <= max_tokens && nimages <= ((int64_t)1 << 32) / threads - 8;
 }
 
+// threads of the workgroups that fwd_size and bwd_size choose
+int fwd_threads(const Shape &s) { return s.H * s.W <= 96 ? 256 : 512; }
+int bwd_threads(const Shape &s) {
+    const int P = s.H * s.W;
+    return P <= 96 ? 256 : P <= 208 || s.D > 32 ? 512 : 1024;
+}
 template <bool BF, int D>
 int fwd_size(const FwdArgsSub &a, hipStream_t st) {
     return a.s.H * a.s.W <= 96 ? fwd_go<BF, SGeo<D, 96, 4>>(a, st) : fwd_go<BF, SGeo<D, 208, 8>>(a, st);
@@ -471,11 +479,11 @@ int bwd_size(const BwdArgsSub &a, hipStream_t st) {
 // images 103 / 30); at k = 3 and 5 the other passes have little border to walk (14x14 d64 k3, 128
 // images 10.8 / 14.5).  Their forward from the second tile on (8x8 d32, 1024 images 7.1 / 7.5).
 bool small_fwd_supported(const FwdArgsSub &a) {
-    return size_ok(a.s, images_of(a), 208) && images_of(a) > 256 && (a.dil > 1 || (a.s.kh >= 7 && a.s.H * a.s.W > 64));
+    return size_ok(a.s, images_of(a), 208, fwd_threads(a.s)) && images_of(a) > 256 && (a.dil > 1 || (a.s.kh >= 7 && a.s.H * a.s.W > 64));
 }
 bool small_bwd_supported(const BwdArgsSub &a) {
     const int64_t ni = images_of(a);
-    return size_ok(a.s, ni, a.s.D > 32 && ni < 64 ? 208 : 256) && (a.dil > 1 || (a.s.kh >= 7 && ni >= 128));
+    return size_ok(a.s, ni, a.s.D > 32 && ni < 64 ? 208 : 256, bwd_threads(a.s)) && (a.dil > 1 || (a.s.kh >= 7 && ni >= 128));
 }
 int launch_fwd_small(const FwdArgsSub &a, int dtype, hipStream_t st) {
     if (dtype == ENATTEN_BF16) return a.s.D <= 32 ? fwd_size<true, 32>(a, st) : fwd_size<true, 64>(a, st);

@@ -152,6 +152,27 @@ def test_gradient_strides_that_16_byte_stores_do_not_take(axis):
     assert_close([t.cpu() for t in (o, *res[1])], [t.cpu() for t in (o, *res[0])], BF16, "axis %d" % axis)
 
 
+def test_more_images_than_a_launch_of_one_workgroup_each_holds():
+    # 8.4e6 images of 98 pixels: 512 threads for each would be more than the 2^32 of a launch.  q, k, v and
+    # dO are one image, expanded: every image's results are those of the first
+    ensure_built()
+    shape, ks = ((1 << 23) + 8, 1, 7, 14, 8), 7
+    print("case many images", shape, flush=True)
+    one = make_inputs((1, *shape[1:]), BF16, seed=71)
+    q, k, v, g = (t.cuda().expand(shape) for t in one)
+    o, lse = torch.ops.enatten.na2d_fwd(q, k, v, ks, 0.3)
+    x = [t.double().requires_grad_(True) for t in one[:3]]
+    o_ref = O.natten2d_dense_mask(*x, ks, 0.3)
+    ref = (o_ref.detach(), *torch.autograd.grad(o_ref, x, one[3].double()))
+    got = (o, *torch.ops.enatten.na2d_bwd(q, k, v, o, lse, g, ks, 0.3))
+    assert_close([t[:1].cpu() for t in got], ref, BF16, "first image")
+    for t in got:
+        for part in t.split(1 << 20):
+            assert (part == t[:1]).all()
+    del o, lse, got, t, part
+    torch.cuda.empty_cache()
+
+
 def test_values_that_are_not_finite_stay_in_their_windows():
     # sub-grids that a workgroup takes whole: a NaN in v reaches the queries that see it, and the
     # keys that those see, alone
