@@ -138,6 +138,32 @@ __device__ __forceinline__ LaneQ lane_at(const ARGS &a, const TL &tl, int wave, 
     return q;
 }
 
+// ------------------------------------------------------------------ units of the logits
+// Units of log2: one multiply less per logit.  With a bias natural units, as in the general kernels:
+// a bias may be as low as its type goes (entries that are masked out), and there a log-sum-exp that goes
+// through log2 and back is another number than the logits that it came from.
+constexpr float kUnit = kBias ? 1.f : kLog2e;
+__device__ __forceinline__ float exp_unit(float x) { return __builtin_amdgcn_exp2f(kBias ? x * kLog2e : x); }
+__device__ __forceinline__ float lse_of(float mx, float sum) {
+    if constexpr (kBias) return mx + __builtin_amdgcn_logf(sum) * kLn2;
+    else return (mx + __builtin_amdgcn_logf(sum)) * kLn2;
+}
+// With a bias the backward is renormalised as in the general kernels: 1 / sum p of the recomputed
+// probabilities per query, left by the dQ pass behind the block that holds its counter (a.zinv).
+template <typename ARGS>
+__device__ __forceinline__ float *row_zinv(const ARGS &a) {
+    return a.zinv + (int64_t)a.s.B * a.s.N * a.s.H * a.s.W;
+}
+// what the dK/dV pass stages per query: the log-sum-exp in the logits' unit, delta, 1 / Z
+using QStat = std::conditional_t<kBias, float4, float2>;
+template <bool BF, bool BIAS = kBias>
+__device__ __forceinline__ std::conditional_t<BIAS, float4, float2> load_qstat(const BArgs &a, int64_t qt) {
+    if constexpr (BIAS) return make_float4(a.lse[qt], a.delta[qt], row_zinv(a)[qt], 0.f);
+    else return make_float2(a.lse[qt] * kLog2e, a.delta[qt]);
+}
+__device__ __forceinline__ float zinv_of(const float4 &st) { return st.z; }
+__device__ __forceinline__ float zinv_of(const float2 &) { return 1.f; }
+
 // ------------------------------------------------------------------ operands of the second products
 // Eight probabilities (or dS) of a lane as an operand: rounded to 16 bits, or, with a bias, as the
 // sum of two 16-bit terms (the value rounded, and what that left).  Calls with a bias used to run
@@ -168,8 +194,7 @@ __device__ __forceinline__ f32x4 mfma_op(s16x8 a, const OP &b, f32x4 c) {
 }
 
 // ------------------------------------------------------------------ relative position bias
-// The head's [2k-1, 2k-1] table in LDS, times log2(e), in float32, with a margin of 3 rows and
-// columns: entry (key - query + k - 1) per axis lies at (.. + 3), so that every (token of a 4x4
+// The head's [2k-1, 2k-1] table in LDS, in float32, with a margin of 3 rows and columns: entry (key - query + k - 1) per axis lies at (.. + 3), so that every (token of a 4x4
 // block's halo, pixel of the block) pair has an entry, in its window or not, and the place of a
 // token's entry is a lane constant plus (token row) * TB + (token column), which folds into the
 // LDS read's offset.
@@ -209,7 +234,7 @@ struct BiasRegs {
 #pragma unroll
         for (int i = 0; i < NB; i++) {
             const int e = min((int)threadIdx.x + i * NT, T::E - 1);  // (the same value twice at the end)
-            lds[(e / T::SPAN + 3) * T::TB + e % T::SPAN + 3] = cvt32<BF>(v[i]) * kLog2e;
+            lds[(e / T::SPAN + 3) * T::TB + e % T::SPAN + 3] = cvt32<BF>(v[i]);
         }
     }
 };
@@ -356,7 +381,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
 
     const int wave = FULL ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const int l = threadIdx.x & 63, n = l & 15, g = l >> 4;
-    const float sc2 = s.scale * kLog2e;
+    const float sc2 = s.scale * kUnit;
 
     // registers that carry the next tile while the current one is computed
     const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim);
@@ -429,7 +454,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
         };
 
         if (FULL || lq.wave_on) {
-            // logits^T [halo token][query], masked, in units of log2
+            // logits^T [halo token][query], masked
             const int bq = kBias ? Bias<KS>::query(lq) : 0;
             f32x4 acc[G::MT];
             float mx = -INFINITY;
@@ -457,7 +482,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
             for (int mt = 0; mt < G::MT; mt++) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float p = __builtin_amdgcn_exp2f(acc[mt][i] - mx);
+                    const float p = exp_unit(acc[mt][i] - mx);
                     sum += p;
                     put<BF>(pb[mt >> 1], (mt & 1) * 4 + i, p);
                 }
@@ -485,7 +510,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
             // (FULL: all four lanes of a token write its log-sum-exp, the same value, so that
             // this store is not predicated either)
             if (a.lse && (FULL || (lq.live && g == 0)))
-                a.lse[lq.tok] = (mx + __builtin_amdgcn_logf(sum)) * kLn2;
+                a.lse[lq.tok] = lse_of(mx, sum);
         }
 
         if (!more) {
@@ -534,7 +559,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
 
     const int wave = FULL ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const int l = threadIdx.x & 63, n = l & 15, g = l >> 4;
-    const float sc2 = s.scale * kLog2e;
+    const float sc2 = s.scale * kUnit;
     const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim);
     HaloRegs<D, KS, NW> st;
     s16x8 qnext[G::DS];
@@ -592,7 +617,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
             for (int mt = 0; mt < G::MT; mt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float p = __builtin_amdgcn_exp2f(acc[mt][i] - mx);
+                    const float p = exp_unit(acc[mt][i] - mx);
                     sum += p;
                     put<BF>(pb[mt >> 1], (mt & 1) * 4 + i, p);
                 }
@@ -632,7 +657,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
             store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(const_cast<short *>(image_at(a, a.o, cur)) + lq.qr * row_step(a, a.o) + lq.qc * col_step(a, a.o),
                                g, o, 1.f / sum, lq.live, dlim);
             if (a.lse && (FULL || (lq.live && g == 0)))
-                a.lse[lq.tok] = (mx + __builtin_amdgcn_logf(sum)) * kLn2;
+                a.lse[lq.tok] = lse_of(mx, sum);
         }
         if (!more) {
             if constexpr (FULL) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), see fwd_mfma
@@ -682,7 +707,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
 
     const int wave = FULL ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const int l = threadIdx.x & 63, n = l & 15, g = l >> 4;
-    const float sc2 = s.scale * kLog2e;
+    const float sc2 = s.scale * kUnit;
     auto pick = [&](int t) __attribute__((always_inline)) {
         if constexpr (FRAME) return in_sub(frame_tile(t, ts, s.N), a);
         else if constexpr (ROLL) return in_sub(tile_of_cm(t, ts.tiles_r, ts.tiles_c, s.N), a);
@@ -730,7 +755,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             qreg[ds] = qnext[ds];
             greg[ds] = gnext[ds];
         }
-        lse2 = lse_next * kLog2e;
+        lse2 = lse_next * kUnit;
         if constexpr (kBias) bst.commit(lds_bias);
     };
     if constexpr (FULL) commit();
@@ -771,7 +796,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             constexpr bool kKeepDp = !(G::WAVES == 1 && G::MT >= 16);
             f32x4 dp[kKeepDp ? G::MT : 1];
             Op8 dsb[G::KSTEPS];
-            float dpart = 0.f;
+            float dpart = 0.f, zsum = 0.f;
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
                 const int row = trow(mt, n);
@@ -785,15 +810,17 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, lq.dr, lq.dc);
-                    float x = cs[i] * sc2 - lse2;
-                    if constexpr (kBias) x += lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)];
-                    cs[i] = __builtin_amdgcn_exp2f(ok ? x : -INFINITY);
+                    float x;
+                    if constexpr (kBias) x = cs[i] * sc2 + lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)] - lse2;
+                    else x = cs[i] * sc2 - lse2;
+                    cs[i] = exp_unit(ok ? x : -INFINITY);
+                    if constexpr (kBias) zsum += cs[i];
                     dpart = fmaf(cs[i], cp[i], dpart);
                     put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, cs[i]);
                 }
                 if constexpr (kKeepDp) dp[mt] = cp;
             }
-            const float delta = col_sum(dpart);
+            const float zinv = kBias ? 1.f / col_sum(zsum) : 1.f, delta = col_sum(dpart) * zinv;
             f32x4 ds_all[kBias ? Bias<KS>::USED : 1];
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
@@ -813,7 +840,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                     const float ds = p * (cp[i] - delta);
                     put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
                     if constexpr (kBias)
-                        if (mt < Bias<KS>::USED) ds_all[mt][i] = lq.live ? ds : 0.f;
+                        if (mt < Bias<KS>::USED) ds_all[mt][i] = lq.live ? ds * zinv : 0.f;
                 }
             }
 
@@ -833,8 +860,11 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                         dq[mt]);
             }
 
-            store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale, lq.live, dlim);
-            if (FULL || (lq.live && g == 0)) a.delta[lq.tok] = delta;
+            store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * zinv, lq.live, dlim);
+            if (FULL || (lq.live && g == 0)) {
+                a.delta[lq.tok] = delta;
+                if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
+            }
         }
         if constexpr (kBias) {
             __syncthreads();
@@ -887,7 +917,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
 
     const int wave = FULL ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const int l = threadIdx.x & 63, n = l & 15, g = l >> 4;
-    const float sc2 = s.scale * kLog2e;
+    const float sc2 = s.scale * kUnit;
     const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim);
     HaloRegs<D, KS, NW> st;
     // This lane's dO row is loaded a phase ahead of phase 1, its q row and log-sum-exp a
@@ -966,11 +996,11 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
         } else {
             if constexpr (FULL) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the last tile, nothing is loaded (see fwd_mfma)
         }
-        const float lse2 = lse_cur * kLog2e;
+        const float lse2 = lse_cur * kUnit;
         if (FULL || lq.wave_on) {
             const int bq = kBias ? Bias<KS>::query(lq) : 0;
             Op8 dsb[G::KSTEPS];
-            float dpart = 0.f;
+            float dpart = 0.f, zsum = 0.f;
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
                 const typename G::ARow kp = G::a_row(lds_x, trow(mt, n), g);
@@ -981,14 +1011,16 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, lq.dr, lq.dc);
-                    float x = cs[i] * sc2 - lse2;
-                    if constexpr (kBias) x += lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)];
-                    const float p = __builtin_amdgcn_exp2f(ok ? x : -INFINITY);
+                    float x;
+                    if constexpr (kBias) x = cs[i] * sc2 + lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)] - lse2;
+                    else x = cs[i] * sc2 - lse2;
+                    const float p = exp_unit(ok ? x : -INFINITY);
+                    if constexpr (kBias) zsum += p;
                     dpart = fmaf(p, dp[mt][i], dpart);
                     put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, p);
                 }
             }
-            const float delta = col_sum(dpart);
+            const float zinv = kBias ? 1.f / col_sum(zsum) : 1.f, delta = col_sum(dpart) * zinv;
             f32x4 ds_all[kBias ? Bias<KS>::USED : 1];
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++)
@@ -998,7 +1030,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                     const float ds = p * (dp[mt][i] - delta);
                     put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
                     if constexpr (kBias)
-                        if (mt < Bias<KS>::USED) ds_all[mt][i] = lq.live ? ds : 0.f;
+                        if (mt < Bias<KS>::USED) ds_all[mt][i] = lq.live ? ds * zinv : 0.f;
                 }
             if constexpr (kBias) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
             f32x4 dq[G::DT];
@@ -1015,8 +1047,11 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                     dq[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(kp[0], mt)), lds_read_tr(G::t_at(kp[1], mt))), dsb[ks],
                         dq[mt]);
             }
-            store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale, lq.live, dlim);
-            if (FULL || (lq.live && g == 0)) a.delta[lq.tok] = delta;
+            store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * zinv, lq.live, dlim);
+            if (FULL || (lq.live && g == 0)) {
+                a.delta[lq.tok] = delta;
+                if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
+            }
         }
         if constexpr (kBias) {
             __syncthreads();
@@ -1077,7 +1112,7 @@ __device__ __forceinline__ bool next_block(KeyBlock &b) {
 template <bool BF, int D, int KS, bool ROLL, int SP, int PART>
 __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, int ntiles, Runs rp,
                                            int block, int nblocks, short *lds_q, short *lds_g,
-                                           float2 *lds_stat, f32x4 *lds_red, float *lds_bias) {
+                                           QStat *lds_stat, f32x4 *lds_red, float *lds_bias) {
     using G = Geo<D, KS, 4, SP>;
     const Shape &s = a.s;
     const int dlim = kNarrow ? s.D : D;  // head dim of the tensors: D, or less in the build for narrow dims
@@ -1085,7 +1120,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
     if (sc.t >= sc.t_end) return;
     zero_row<D, KS, 4, SP>(lds_q, dlim);
     zero_row<D, KS, 4, SP>(lds_g, dlim);
-    if (threadIdx.x == 0) lds_stat[G::ZROW] = make_float2(0.f, 0.f);
+    if (threadIdx.x == 0) lds_stat[G::ZROW] = QStat{};
 
     // wave = block of 4x4 keys (0..3) + 4 * PART; part p takes reduction steps
     // K0 = p * CH .. K1 - 1 (compile-time, so that every token's place in the halo and its
@@ -1095,7 +1130,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
     constexpr int CH = (G::KSTEPS + SP - 1) / SP;
     constexpr int K0 = PART * CH, K1 = K0 + CH < G::KSTEPS ? K0 + CH : G::KSTEPS;
     const int l = threadIdx.x & 63, n = l & 15, g = l >> 4;
-    const float sc2 = s.scale * kLog2e;
+    const float sc2 = s.scale * kUnit;
     const int orow = (wave >> 1) * 4, ocol = (wave & 1) * 4;
     int rot = 0;  // ROLL: (first image row of the staged block) % HR
     auto row_of = [&](int tile, int x) __attribute__((always_inline)) {
@@ -1107,7 +1142,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
 
     const HaloPlan<D, KS, 4, SP> plan = make_plan<D, KS, 4, SP>(dlim);
     HaloRegs<D, KS, 4, SP> qst, gst;
-    float2 sst[G::NST];
+    QStat sst[G::NST];
     BiasRegs<BF, KS, G::NT> bst;
     // ROLL: rows [y0, y0 + nr) of the block are what LDS does not hold yet
     auto prefetch = [&](const ATile &tl, int y0, int nr) __attribute__((always_inline)) {
@@ -1126,7 +1161,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
             const int pr = id / G::HC, pc = id % G::HC;
             if (!ROLL || pr < nr) {
                 const int64_t qt = img_tok + (int64_t)((ROLL ? y0 : br) + pr) * s.W + bc + pc;
-                sst[i] = make_float2(a.lse[qt] * kLog2e, a.delta[qt]);
+                sst[i] = load_qstat<BF>(a, qt);
             }
         }
         if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
@@ -1215,11 +1250,13 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
                 }
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float2 st = lds_stat[row_of(mt, g * 4 + i)];  // query of accumulator row g*4+i
+                    const QStat st = lds_stat[row_of(mt, g * 4 + i)];  // query of accumulator row g*4+i
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, n >> 2, n & 3);
-                    float x = cs[i] * sc2 - st.x;
-                    if constexpr (kBias) x += lds_bias[ok ? bk - Bias<KS>::token(mt, g * 4 + i) : 0];
-                    const float p = __builtin_amdgcn_exp2f(ok ? x : -INFINITY);
+                    float x;
+                    if constexpr (kBias) x = cs[i] * sc2 + lds_bias[ok ? bk - Bias<KS>::token(mt, g * 4 + i) : 0] - st.x;
+                    else x = cs[i] * sc2 - st.x;
+                    float p = exp_unit(ok ? x : -INFINITY);
+                    if constexpr (kBias) p *= zinv_of(st);
                     put<BF>(pb, m2 * 4 + i, p);
                     put<BF>(dsb, m2 * 4 + i, p * (cp[i] - st.y));
                 }
@@ -1316,11 +1353,11 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
     // wave = block of 4x4 keys (0..3) + 4 * (its part of the block's queries)
     const int wave = (threadIdx.x >> 6) & 3, part = threadIdx.x >> 8;
     const int l = threadIdx.x & 63, n = l & 15, g = l >> 4;
-    const float sc2 = s.scale * kLog2e;
+    const float sc2 = s.scale * kUnit;
 
     const HaloPlan<D, KSG, 4, SP> plan = make_plan<D, KSG, 4, SP>(dlim);
     HaloRegs<D, KSG, 4, SP> qst, gst;
-    float2 sst[G::NST];
+    QStat sst[G::NST];
     BiasRegs<BF, KS, G::NT> bst;
     // the wave's 4x4 keys of a tile: this lane's key pixel (clamped into the image)
     auto key_of = [&](const ATile &tl, int &kr, int &kc) __attribute__((always_inline)) {
@@ -1336,7 +1373,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
             const int id = threadIdx.x + i * G::NT;
             const int r = min(b.br + id / G::HC, b.qb - 1), c = min(b.bc + id % G::HC, b.cb - 1);
             const int64_t qt = img_tok + (int64_t)r * s.W + c;
-            sst[i] = make_float2(a.lse[qt] * kLog2e, a.delta[qt]);
+            sst[i] = load_qstat<BF>(a, qt);
         }
         if constexpr (kBias) bst.fetch(a.rpb, b.tl.nn);
     };
@@ -1385,10 +1422,18 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
             // differences; the padding row's window is nowhere
             const int r = min(cur.br + id / G::HC, cur.qb - 1), c = min(cur.bc + id % G::HC, cur.cb - 1);
             const int ws = win_start(r, s.H, KS) | (win_start(c, s.W, KS) << 16);
-            // (with a bias also the query's place in a table with TB columns, from the block's origin)
-            const int at = kBias ? (id / G::HC) * Bias<KS>::TB + id % G::HC : 0;
-            if (id < G::ZROW) lds_stat[id] = make_float4(sst[i].x, sst[i].y, __int_as_float(ws), __int_as_float(at));
-            else if (id == G::ZROW) lds_stat[id] = make_float4(0.f, 0.f, __int_as_float(0x7fff7fff), 0.f);
+            if constexpr (kBias) {
+                // (1 / Z too, and in the word of the window the query's place in a table with TB columns,
+                // all from the block's origin: a window starts at most 12 rows before it)
+                const int at = (id / G::HC) * Bias<KS>::TB + id % G::HC;
+                const unsigned w = (unsigned)at | (unsigned)((ws & 0xffff) - cur.br + 64) << 16 |
+                                   (unsigned)((ws >> 16) - cur.bc + 64) << 24;
+                if (id < G::ZROW) lds_stat[id] = make_float4(sst[i].x, sst[i].y, __uint_as_float(w), zinv_of(sst[i]));
+                else if (id == G::ZROW) lds_stat[id] = make_float4(0.f, 0.f, __uint_as_float(0xffff0000u), 0.f);
+            } else {
+                if (id < G::ZROW) lds_stat[id] = make_float4(sst[i].x, sst[i].y, __int_as_float(ws), 0.f);
+                else if (id == G::ZROW) lds_stat[id] = make_float4(0.f, 0.f, __int_as_float(0x7fff7fff), 0.f);
+            }
         }
         if constexpr (kBias) bst.commit(lds_bias);
         if (cur.first) {
@@ -1447,12 +1492,20 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
                     for (int i = 0; i < 4; i++) {
                         const int qi = q0 + m2 * 16 + g * 4 + i;
                         const float4 st = lds_stat[row_of(qi)];
-                        const int ws = __float_as_int(st.z);
-                        const bool ok = ((unsigned)(kr - (ws & 0xffff)) < (unsigned)KS) &
-                                        ((unsigned)(kc - (ws >> 16)) < (unsigned)KS);
-                        float x = cs[i] * sc2 - st.x;
-                        if constexpr (kBias) x += lds_bias[ok ? bk - __float_as_int(st.w) : 0];
-                        const float p = __builtin_amdgcn_exp2f(ok ? x : -INFINITY);
+                        float x, p;
+                        if constexpr (kBias) {
+                            const unsigned w = __float_as_uint(st.z);
+                            const bool ok = ((unsigned)(kr - cur.br + 64) - (w >> 16 & 0xffu) < (unsigned)KS) &
+                                            ((unsigned)(kc - cur.bc + 64) - (w >> 24) < (unsigned)KS);
+                            x = cs[i] * sc2 + lds_bias[ok ? bk - (int)(w & 0xffffu) : 0] - st.x;
+                            p = exp_unit(ok ? x : -INFINITY) * st.w;
+                        } else {
+                            const int ws = __float_as_int(st.z);
+                            const bool ok = ((unsigned)(kr - (ws & 0xffff)) < (unsigned)KS) &
+                                            ((unsigned)(kc - (ws >> 16)) < (unsigned)KS);
+                            x = cs[i] * sc2 - st.x;
+                            p = exp_unit(ok ? x : -INFINITY);
+                        }
                         put<BF>(pb, m2 * 4 + i, p);
                         put<BF>(dsb, m2 * 4 + i, p * (cp[i] - st.y));
                     }
@@ -1553,7 +1606,7 @@ __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) v
     constexpr size_t RED = SP > 1 ? (size_t)2 * G::DT * 256 * sizeof(f32x4) : 0;
     constexpr size_t I_ROWS = FRAME_ONLY ? 0 : (size_t)G::ROWS * G::PITCH * sizeof(short);
     constexpr size_t F_ROWS = (size_t)FG::ROWS * FG::PITCH * sizeof(short);
-    constexpr size_t I_STAT = FRAME_ONLY ? 0 : (G::ROWS * sizeof(float2) + 15) / 16 * 16;
+    constexpr size_t I_STAT = FRAME_ONLY ? 0 : (G::ROWS * sizeof(QStat) + 15) / 16 * 16;
     constexpr size_t F_STAT = FG::ROWS * sizeof(float4);
     constexpr size_t I_ALL = 2 * I_ROWS + I_STAT + RED;
     constexpr size_t F_ALL = 2 * F_ROWS + F_STAT + (RED_OVER ? 0 : RED);
@@ -1570,7 +1623,7 @@ __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) v
         if ((int)blockIdx.x < inner_blocks) {
             short *lds_q = reinterpret_cast<short *>(lds_raw);
             short *lds_g = reinterpret_cast<short *>(lds_raw + I_ROWS);
-            float2 *lds_stat = reinterpret_cast<float2 *>(lds_raw + 2 * I_ROWS);
+            QStat *lds_stat = reinterpret_cast<QStat *>(lds_raw + 2 * I_ROWS);
             f32x4 *lds_red = reinterpret_cast<f32x4 *>(lds_raw + 2 * I_ROWS + I_STAT);
             if (SP == 1 || threadIdx.x < 256)
                 dkdv_inner<BF, D, KS, ROLL, SP, 0>(a, ts, n_inner, rp, blockIdx.x, inner_blocks, lds_q,

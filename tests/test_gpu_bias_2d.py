@@ -55,3 +55,58 @@ def test_bias(shape, ks, dtype, layout):
         assert norm <= (4e-3 if dtype == BF16 else 5e-4), (name, norm)
     again = torch.autograd.grad(natten2d(qg, kg, vg, ks, scale, rpb=bg), (qg, kg, vg, bg), g.cuda())
     assert all(torch.equal(a, b) for a, b in zip(again, got[1:])), "not bit-reproducible"
+
+
+def _dense(q, k, v, rpb, ks, scale):
+    """O in float64 through an explicit softmax (a fused one may not hold a log-sum-exp of -1e38)."""
+    B, N, H, W, D = q.shape
+    at = torch.arange(H * W)
+    dy = at[None] // W - at[:, None] // W + ks - 1
+    dx = at[None] % W - at[:, None] % W + ks - 1
+    s = q.flatten(2, 3) @ k.flatten(2, 3).transpose(-1, -2) * scale
+    s = s + rpb[:, dy.clamp(0, 2 * ks - 2), dx.clamp(0, 2 * ks - 2)]
+    p = s.masked_fill(~O.neighbour_mask(H, W, ks), float("-inf")).softmax(-1)
+    return (p @ v.flatten(2, 3)).view(q.shape)
+
+
+def _both(x, ks, scale):
+    """(O, dQ, dK, dV, dRPB) of the kernels and of the reference; x = (q, k, v, rpb, dO)."""
+    from e_natten_amd import natten2d
+    xg = [t.cuda().requires_grad_(True) for t in x[:4]]
+    o = natten2d(*xg[:3], ks, scale, rpb=xg[3])
+    got = [t.detach().cpu().double() for t in (o, *torch.autograd.grad(o, xg, x[4].cuda()))]
+    xr = [t.double().requires_grad_(True) for t in x[:4]]
+    o_ref = _dense(*xr, ks, scale)
+    return got, [t.detach() for t in (o_ref, *torch.autograd.grad(o_ref, xr, x[4].double()))]
+
+
+def _rpb(heads, ks, seed=5):
+    return torch.randn(heads, 2 * ks - 1, 2 * ks - 1, generator=torch.Generator().manual_seed(seed))
+
+
+NAMES = ("O", "dQ", "dK", "dV", "dRPB")
+
+
+@pytest.mark.parametrize("shape,ks,dtype", [
+    ((1, 2, 26, 24, 32), 5, BF16),
+    ((1, 2, 20, 21, 128), 9, BF16),
+    ((1, 2, 26, 29, 64), 11, BF16),
+    ((1, 2, 24, 24, 32), 7, F16),
+])
+def test_bias_of_the_lowest_value(shape, ks, dtype):
+    # head 0: every entry is the lowest finite value, which absorbs the logits: uniform probabilities.
+    # head 1: the query itself and what follows it are masked out that way; the first query then
+    # has nothing else
+    ensure_built()
+    print("case lowest bias", shape, dtype, "k=%d" % ks, flush=True)
+    q, k, v, g = make_inputs(shape, dtype, seed=73)
+    rpb = _rpb(2, ks).to(dtype)
+    rpb[0] = torch.finfo(dtype).min
+    rpb.view(2, -1)[1, (2 * ks - 1) ** 2 // 2:] = torch.finfo(dtype).min
+    got, ref = _both((q, k, v, rpb, g), ks, shape[-1] ** -0.5)
+    for name, x, r in zip(NAMES, got, ref):
+        norm = ((x - r).norm() / r.norm()).item()
+        print("   ", name, "2-norm %.2e" % norm, flush=True)
+        # (bfloat16 as in test_bias.  Float16's lowest value leaves logits of -65504 their last 8 bits:
+        # in float32 they are rounded to 2^-8, a probability by 1.1e-3 in the mean)
+        assert norm <= (4e-3 if dtype == BF16 else 2e-3), (name, norm)
