@@ -491,9 +491,6 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
 // The tile is 64 keys, 16 per wave (columns), and the walk is over the queries
 // that see any of them, the inverse neighbourhood (e_natten/pytorch.py:13-23), a block at a time: Q
 // and dO rows, the log-sum-exp, delta and 1 / Z of a block in LDS.  dV^T += dO^T P, dK^T += Q^T dS.
-// kPScale: float16 probabilities come out of 1 / Z times 2^14 (see DsScale).
-template <bool BF>
-constexpr float kPScale = BF ? 1.f : 16384.f;
 template <bool BF, int D, bool NARROW>
 __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tiles_t, int ntiles) {
     constexpr int KB = kRowsK<D>;

@@ -110,9 +110,18 @@ struct DsScale {
             }
         }
     }
+    // the same where all dS are known before the first product
+    __device__ __forceinline__ void set(float mag) {
+        const float m = col_max(mag);
+        e = m > 0.f ? max(__builtin_amdgcn_frexp_expf(m), -100) : -100;
+    }
     __device__ __forceinline__ float factor() const { return BF ? 1.f : __builtin_ldexpf(1.f, 10 - e); }
     __device__ __forceinline__ float inverse() const { return BF ? 1.f : __builtin_ldexpf(1.f, e - 10); }
 };
+
+// Normalised float16 probabilities as two terms, times 2^14 for the same reason.
+template <bool BF>
+constexpr float kPScale = BF ? 1.f : 16384.f;
 
 // dO . O over the 8 channels of one 16-byte chunk: four two-element dot products that
 // accumulate in float32 (v_dot2c_f32_bf16 / v_dot2c_f32_f16), one instruction per dword where

@@ -154,11 +154,14 @@ template <typename ARGS>
 __device__ __forceinline__ float *row_zinv(const ARGS &a) {
     return a.zinv + (int64_t)a.s.B * a.s.N * a.s.H * a.s.W;
 }
-// what the dK/dV pass stages per query: the log-sum-exp in the logits' unit, delta, 1 / Z
+// (P in the float16 dK/dV pass, which 1 / Z brings along, as in na1d_band_mfma.hip: see DsScale)
+template <bool BF>
+constexpr float kPUnit = kBias ? kPScale<BF> : 1.f;
+// what the dK/dV pass stages per query: the log-sum-exp in the logits' unit, delta, kPUnit / Z
 using QStat = std::conditional_t<kBias, float4, float2>;
 template <bool BF, bool BIAS = kBias>
 __device__ __forceinline__ std::conditional_t<BIAS, float4, float2> load_qstat(const BArgs &a, int64_t qt) {
-    if constexpr (BIAS) return make_float4(a.lse[qt], a.delta[qt], row_zinv(a)[qt], 0.f);
+    if constexpr (BIAS) return make_float4(a.lse[qt], a.delta[qt], row_zinv(a)[qt] * kPUnit<BF>, 0.f);
     else return make_float2(a.lse[qt] * kLog2e, a.delta[qt]);
 }
 __device__ __forceinline__ float zinv_of(const float4 &st) { return st.z; }
@@ -191,6 +194,27 @@ template <bool BF, typename OP>
 __device__ __forceinline__ f32x4 mfma_op(s16x8 a, const OP &b, f32x4 c) {
     if constexpr (std::is_same_v<OP, TwoTerms>) return mfma16<BF>(a, b.lo, mfma16<BF>(a, b.hi, c));
     else return mfma16<BF>(a, b, c);
+}
+
+// eight dS of a lane, the largest magnitude of which is `mag`, as an operand; acc: the sums they go into
+template <bool BF, int DT>
+__device__ __forceinline__ void put_scaled(Op8 &o, const float (&y)[8], float mag, DsScale<BF> &scl, f32x4 (&acc)[DT]) {
+    scl.fit(mag, acc);
+    const float f = scl.factor();
+#pragma unroll
+    for (int e = 0; e < 8; e++) put<BF>(o, e, y[e] * f);
+}
+// dK and dV of a tile in their own units again
+template <bool BF, int DT>
+__device__ __forceinline__ void unscale(f32x4 (&dk)[DT], f32x4 (&dv)[DT], const DsScale<BF> &scl) {
+    if constexpr (!BF) {
+        const float f = scl.inverse() / kPUnit<BF>;
+#pragma unroll
+        for (int t = 0; t < DT; t++) {
+            dk[t] *= f;
+            dv[t] *= 1.f / kPUnit<BF>;
+        }
+    }
 }
 
 // ------------------------------------------------------------------ relative position bias
@@ -331,6 +355,28 @@ struct BiasGrad {
         }
     }
 };
+// dS of a lane's halo tokens as operands of dQ's product (tiles without tokens hold zeros already),
+// and, times 1 / Z (0 for a lane without a query), as terms of the bias gradient
+template <bool BF, int KS, int STEPS>
+__device__ __forceinline__ void operand_and_sums(Op8 (&dsb)[STEPS], f32x4 (&ds)[Bias<KS>::USED], DsScale<BF> &scl,
+                                                 float zinv) {
+    if constexpr (!BF) {
+        float mag = 0.f;
+#pragma unroll
+        for (int mt = 0; mt < Bias<KS>::USED; mt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) mag = fmaxf(mag, fabsf(ds[mt][i]));
+        scl.set(mag);
+    }
+    const float f = scl.factor();
+#pragma unroll
+    for (int mt = 0; mt < Bias<KS>::USED; mt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds[mt][i] * f);
+            ds[mt][i] = zinv != 0.f ? ds[mt][i] * zinv : 0.f;
+        }
+}
 // d_rpb[head][entry] = the sum over batch entries and tiles of the rows that the dQ pass left, in a
 // fixed order: a workgroup takes 16 entries of a head, 64 threads a strided share of the rows each.
 template <bool BIAS>
@@ -838,13 +884,16 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                 for (int i = 0; i < 4; i++) {
                     const float p = get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i);
                     const float ds = p * (cp[i] - delta);
-                    put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
-                    if constexpr (kBias)
-                        if (mt < Bias<KS>::USED) ds_all[mt][i] = lq.live ? ds * zinv : 0.f;
+                    if constexpr (!kBias) put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
+                    else if (mt < Bias<KS>::USED) ds_all[mt][i] = ds;
                 }
             }
 
-            if constexpr (kBias) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
+            DsScale<BF> scl;
+            if constexpr (kBias) {
+                operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live ? zinv : 0.f);
+                BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
+            }
             f32x4 dq[G::DT];
 #pragma unroll
             for (int mt = 0; mt < G::DT; mt++) dq[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -860,7 +909,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                         dq[mt]);
             }
 
-            store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * zinv, lq.live, dlim);
+            store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * (kBias ? zinv * scl.inverse() : 1.f), lq.live, dlim);
             if (FULL || (lq.live && g == 0)) {
                 a.delta[lq.tok] = delta;
                 if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
@@ -1028,11 +1077,14 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                 for (int i = 0; i < 4; i++) {
                     const float p = get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i);
                     const float ds = p * (dp[mt][i] - delta);
-                    put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
-                    if constexpr (kBias)
-                        if (mt < Bias<KS>::USED) ds_all[mt][i] = lq.live ? ds * zinv : 0.f;
+                    if constexpr (!kBias) put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
+                    else if (mt < Bias<KS>::USED) ds_all[mt][i] = ds;
                 }
-            if constexpr (kBias) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
+            DsScale<BF> scl;
+            if constexpr (kBias) {
+                operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live ? zinv : 0.f);
+                BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
+            }
             f32x4 dq[G::DT];
 #pragma unroll
             for (int mt = 0; mt < G::DT; mt++) dq[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1047,7 +1099,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                     dq[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(kp[0], mt)), lds_read_tr(G::t_at(kp[1], mt))), dsb[ks],
                         dq[mt]);
             }
-            store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * zinv, lq.live, dlim);
+            store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * (kBias ? zinv * scl.inverse() : 1.f), lq.live, dlim);
             if (FULL || (lq.live && g == 0)) {
                 a.delta[lq.tok] = delta;
                 if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
@@ -1229,6 +1281,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
         }
 
         f32x4 dk[G::DT], dv[G::DT];
+        DsScale<BF> scl;
 #pragma unroll
         for (int mt = 0; mt < G::DT; mt++) {
             dk[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1237,6 +1290,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
 #pragma unroll
         for (int ks = K0; ks < K1; ks++) {
             Op8 pb, dsb;
+            float dsv[8], mag = 0.f;  // (float16 with a bias)
 #pragma unroll
             for (int m2 = 0; m2 < 2; m2++) {
                 const int mt = ks * 2 + m2;
@@ -1258,9 +1312,15 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
                     float p = exp_unit(ok ? x : -INFINITY);
                     if constexpr (kBias) p *= zinv_of(st);
                     put<BF>(pb, m2 * 4 + i, p);
-                    put<BF>(dsb, m2 * 4 + i, p * (cp[i] - st.y));
+                    if constexpr (kBias && !BF) {
+                        dsv[m2 * 4 + i] = p * (cp[i] - st.y);
+                        mag = fmaxf(mag, fabsf(dsv[m2 * 4 + i]));
+                    } else {
+                        put<BF>(dsb, m2 * 4 + i, p * (cp[i] - st.y));
+                    }
                 }
             }
+            if constexpr (kBias && !BF) put_scaled<BF>(dsb, dsv, mag, scl, dk);
             typename G::TRow qt[2], gt[2];
 #pragma unroll
             for (int h = 0; h < 2; h++) {
@@ -1277,6 +1337,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
             }
         }
 
+        if constexpr (kBias) unscale<BF>(dk, dv, scl);
         const int kr = cur.r0 + orow + (n >> 2), kc = cur.c0 + ocol + (n & 3);
         const int64_t goff = grad_of(a, cur, kr, kc);
         if constexpr (SP == 1) {
@@ -1401,6 +1462,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
     };
 
     f32x4 dk[G::DT], dv[G::DT];
+    DsScale<BF> scl;
     KeyBlock cur = first_of(sc.t);
     // With one part per block (SP == 1) the loads of a block are issued when the previous
     // block's math is over and the other workgroup on the CU covers their latency
@@ -1442,6 +1504,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
                 dk[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
                 dv[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
+            scl = DsScale<BF>();
         }
         __syncthreads();
 
@@ -1478,6 +1541,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
             };
             for (int q0 = part * 32; q0 < nq; q0 += 32 * SP) {
                 Op8 pb, dsb;
+                float dsv[8], mag = 0.f;  // (float16 with a bias)
 #pragma unroll
                 for (int m2 = 0; m2 < 2; m2++) {
                     const int row = row_of(q0 + m2 * 16 + n);
@@ -1507,9 +1571,15 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
                             p = exp_unit(ok ? x : -INFINITY);
                         }
                         put<BF>(pb, m2 * 4 + i, p);
-                        put<BF>(dsb, m2 * 4 + i, p * (cp[i] - st.y));
+                        if constexpr (kBias && !BF) {
+                            dsv[m2 * 4 + i] = p * (cp[i] - st.y);
+                            mag = fmaxf(mag, fabsf(dsv[m2 * 4 + i]));
+                        } else {
+                            put<BF>(dsb, m2 * 4 + i, p * (cp[i] - st.y));
+                        }
                     }
                 }
+                if constexpr (kBias && !BF) put_scaled<BF>(dsb, dsv, mag, scl, dk);
                 typename G::TRow qt[2], gt[2];
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
@@ -1529,6 +1599,8 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
         // writes it again behind the barrier that opens its arithmetic)
         if (dyn && cur.first && threadIdx.x == 0) lds_tile[0] = fetched;
         const bool live = (wr0 + (n >> 2) < s.H) && (wc0 + (n & 3) < s.W);
+        if constexpr (kBias)
+            if (cur.last) unscale<BF>(dk, dv, scl);
         auto store = [&]() __attribute__((always_inline)) {
             const int64_t goff = grad_of(a, cur.tl, kr, kc);
             store_token<BF, D, kLineStores<D, KS, fits<D, KS>() ? Geo<D, KS, 4, SP>::WAVES : 1>>(static_cast<short *>(a.dk) + goff, g, dk, s.scale, live, dlim);

@@ -110,3 +110,30 @@ def test_bias_of_the_lowest_value(shape, ks, dtype):
         # (bfloat16 as in test_bias.  Float16's lowest value leaves logits of -65504 their last 8 bits:
         # in float32 they are rounded to 2^-8, a probability by 1.1e-3 in the mean)
         assert norm <= (4e-3 if dtype == BF16 else 2e-3), (name, norm)
+
+
+def test_gradients_beyond_float16():
+    # dS of some 1e5, whose 16-bit terms would be an infinity and its negative, under a small softmax
+    # scale: the gradients of q and k themselves are in range (that of the bias is not)
+    ensure_built()
+    q, k, v, g = make_inputs((1, 2, 24, 20, 64), F16, seed=43)
+    got, ref = _both((q, k, v * 200, _rpb(2, 3).to(F16), g * 200), 3, 2.0 ** -10)
+    for name, x, r in zip(NAMES[:4], got, ref):
+        norm = ((x - r).norm() / r.norm()).item()
+        print("   ", name, "2-norm %.2e" % norm, flush=True)
+        assert norm <= 5e-4, (name, norm)  # (as in test_bias)
+
+
+@pytest.mark.parametrize("shape,ks", [((1, 2, 28, 24, 32), 7), ((1, 1, 26, 28, 64), 13), ((1, 1, 20, 24, 128), 9)])
+def test_float16_with_small_upstream_gradients(shape, ks):
+    # dS of 1e-6 and less, which two float16 terms alone do not hold
+    ensure_built()
+    print("case small gradients", shape, ks, flush=True)
+    q, k, v, g = make_inputs(shape, torch.float32, seed=59)
+    x = [t.to(F16) for t in (q, k, v, _rpb(shape[1], ks), g * 1e-4)]
+    got, ref = _both(x, ks, shape[-1] ** -0.5)
+    for name, x, r in list(zip(NAMES, got, ref))[1:4]:
+        norm = ((x - r).norm() / r.norm()).item()
+        rounding = ((r.to(F16).double() - r).norm() / r.norm()).item()
+        print("   ", name, "2-norm %.2e, of the result's rounding alone %.2e" % (norm, rounding), flush=True)
+        assert norm <= 1.05 * rounding, (name, norm, rounding)
