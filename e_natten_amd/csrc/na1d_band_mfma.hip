@@ -133,39 +133,13 @@ __device__ __forceinline__ void load_row(s16x8 (&reg)[DS], const short *row, int
 // sequence) would reach the query's result through its zero probability, and a dS beyond float16
 // would as infinity minus infinity.  So each wave looks at its results before it stores them (one
 // instruction per value, once a tile) and computes the tokens with a value that is not finite
-// again, one after the other, from the rows in their windows alone, in float32.  A lane then holds
-// channels lane and lane + 64.
+// again, one after the other, from the rows in their windows alone, in float32.
 // Queries whose logits lie beyond kFar take the same way: log2 and natural units do not convert
 // into each other closely enough there for probabilities out of a log-sum-exp, so these are computed in
 // natural units throughout, as by the general kernels.
 constexpr float kFar = 1048576.f;
 __device__ __forceinline__ bool far(float lse) { return !(fabsf(lse) <= kFar); }  // (also NaN)
 __device__ __forceinline__ float exp_neg(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
-struct Chan2 {
-    float a, b;
-};
-template <bool BF>
-__device__ __forceinline__ Chan2 chan_load(const short *row, int dlim) {
-    const int c = threadIdx.x & 63;
-    Chan2 r{0.f, 0.f};
-    if (c < dlim) r.a = cvt32<BF>(row[c]);
-    if (c + 64 < dlim) r.b = cvt32<BF>(row[c + 64]);
-    return r;
-}
-template <bool BF>
-__device__ __forceinline__ void chan_store(short *row, int dlim, const Chan2 &x, float mul) {
-    const int c = threadIdx.x & 63;
-    if (c < dlim) row[c] = cvt16<BF>(x.a * mul);
-    if (c + 64 < dlim) row[c + 64] = cvt16<BF>(x.b * mul);
-}
-__device__ __forceinline__ float chan_dot(const Chan2 &x, const Chan2 &y) {
-    return wave_sum(x.a * y.a + x.b * y.b);
-}
-__device__ __forceinline__ void chan_add(Chan2 &acc, float w, const Chan2 &x) {
-    acc.a += w * x.a;
-    acc.b += w * x.b;
-}
-
 // ------------------------------------------------------------------ forward
 template <bool BF, int D, int NQ, bool NARROW>
 __global__ __launch_bounds__(256, 2) void fwd_band_mfma(FwdArgs a, int tiles_t, int ntiles) {

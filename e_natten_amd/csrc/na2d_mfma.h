@@ -123,6 +123,33 @@ struct DsScale {
 template <bool BF>
 constexpr float kPScale = BF ? 1.f : 16384.f;
 
+// One token's channels spread over the wave, for results that are computed again one token after the other:
+// a lane holds channels lane and lane + 64.
+struct Chan2 {
+    float a, b;
+};
+template <bool BF>
+__device__ __forceinline__ Chan2 chan_load(const short *row, int dlim) {
+    const int c = threadIdx.x & 63;
+    Chan2 r{0.f, 0.f};
+    if (c < dlim) r.a = cvt32<BF>(row[c]);
+    if (c + 64 < dlim) r.b = cvt32<BF>(row[c + 64]);
+    return r;
+}
+template <bool BF>
+__device__ __forceinline__ void chan_store(short *row, int dlim, const Chan2 &x, float mul) {
+    const int c = threadIdx.x & 63;
+    if (c < dlim) row[c] = cvt16<BF>(x.a * mul);
+    if (c + 64 < dlim) row[c + 64] = cvt16<BF>(x.b * mul);
+}
+__device__ __forceinline__ float chan_dot(const Chan2 &x, const Chan2 &y) {
+    return wave_sum(x.a * y.a + x.b * y.b);
+}
+__device__ __forceinline__ void chan_add(Chan2 &acc, float w, const Chan2 &x) {
+    acc.a += w * x.a;
+    acc.b += w * x.b;
+}
+
 // dO . O over the 8 channels of one 16-byte chunk: four two-element dot products that
 // accumulate in float32 (v_dot2c_f32_bf16 / v_dot2c_f32_f16), one instruction per dword where
 // taking the halves apart and multiplying them took six.

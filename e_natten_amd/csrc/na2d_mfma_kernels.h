@@ -356,7 +356,8 @@ struct BiasGrad {
     }
 };
 // dS of a lane's halo tokens as operands of dQ's product (tiles without tokens hold zeros already),
-// and, times 1 / Z (0 for a lane without a query), as terms of the bias gradient
+// and, times 1 / Z (0 for a lane without a query, or with one that again_dq computes), as terms of the
+// bias gradient
 template <bool BF, int KS, int STEPS>
 __device__ __forceinline__ void operand_and_sums(Op8 (&dsb)[STEPS], f32x4 (&ds)[Bias<KS>::USED], DsScale<BF> &scl,
                                                  float zinv) {
@@ -397,6 +398,114 @@ __global__ __launch_bounds__(1024) void rpb_tile_reduce(const float *rows, float
     if (threadIdx.x < 16 && e < E) d_rpb[(int64_t)n * E + e] = part[threadIdx.x];
 }
 
+// ------------------------------------------------------------------ results that are not finite
+// With a bias: a result that is not finite is computed again from its window alone, as in
+// na1d_band_mfma.hip (the general kernels, which used to serve these calls, read nothing else).
+// A query's window, with the bias of every key: f(key row, key column, bias) until it returns false
+template <bool BF, int KS, typename F>
+__device__ __forceinline__ void walk_window(const Shape &s, const void *rpb, int head, int qr, int qc, F f) {
+    constexpr int SPAN = 2 * KS - 1;
+    const int r0 = win_start(qr, s.H, KS), c0 = win_start(qc, s.W, KS);
+    const short *b = static_cast<const short *>(rpb) + ((int64_t)head * SPAN + r0 - qr + KS - 1) * SPAN + c0 - qc + KS - 1;
+    for (int i = 0; i < KS * KS; i++)
+        if (!f(r0 + i / KS, c0 + i % KS, cvt32<BF>(b[i / KS * SPAN + i % KS]))) return;
+}
+template <typename ARGS>
+__device__ __forceinline__ const short *pixel(const ARGS &a, const View &v, const ATile &tl, int r, int c) {
+    return image_at(a, v, tl) + r * row_step(a, v) + c * col_step(a, v);
+}
+template <bool BF, int KS>
+__device__ __forceinline__ void again_fwd(const FArgs &a, const ATile &tl, const LaneQ &lq, unsigned bad, int dlim) {
+    const Shape &s = a.s;
+    for (; bad; bad &= bad - 1) {
+        const int col = __builtin_ctz(bad), qr = __shfl(lq.qr, col, 64), qc = __shfl(lq.qc, col, 64);
+        if (!__shfl((int)lq.live, col, 64)) continue;
+        const Chan2 q = chan_load<BF>(pixel(a, a.q, tl, qr, qc), dlim);
+        Chan2 acc{0.f, 0.f};
+        float mx = -INFINITY, z = 0.f;
+        walk_window<BF, KS>(s, a.rpb, tl.nn, qr, qc, [&](int r, int c, float bias) {
+            const float x = chan_dot(q, chan_load<BF>(pixel(a, a.k, tl, r, c), dlim)) * s.scale + bias;
+            const float mn = x > mx ? x : mx, corr = exp_unit(mx - mn), p = exp_unit(x - mn);
+            mx = mn;
+            z = z * corr + p;
+            acc.a *= corr;
+            acc.b *= corr;
+            chan_add(acc, p, chan_load<BF>(pixel(a, a.v, tl, r, c), dlim));
+            return z == z;  // (else nothing finite can come of it)
+        });
+        chan_store<BF>(const_cast<short *>(pixel(a, a.o, tl, qr, qc)), dlim, acc, 1.f / z);
+        if (a.lse && (threadIdx.x & 63) == 0) a.lse[image_token(a, tl) + (int64_t)qr * s.W + qc] = lse_of(mx, z);
+    }
+}
+// sums: the wave's share of the bias gradient, without the queries whose delta is not finite
+template <bool BF, int KS>
+__device__ __forceinline__ void again_dq(const BArgs &a, const ATile &tl, const LaneQ &lq, unsigned bad, float lse,
+                                         float delta, int wave, float *sums, int dlim) {
+    const Shape &s = a.s;
+    const int wr = tl.r0 + (wave >> 1) * 4 - lq.hr0 - lq.orow + 3, wc = tl.c0 + (wave & 1) * 4 - lq.hc0 - lq.ocol + 3;
+    for (; bad; bad &= bad - 1) {
+        const int col = __builtin_ctz(bad), qr = __shfl(lq.qr, col, 64), qc = __shfl(lq.qc, col, 64);
+        if (!__shfl((int)lq.live, col, 64)) continue;
+        const float lse_q = __shfl(lse, col, 64), delta_q = __shfl(delta, col, 64);
+        const Chan2 q = chan_load<BF>(pixel(a, a.q, tl, qr, qc), dlim), go = chan_load<BF>(pixel(a, a.d_o, tl, qr, qc), dlim);
+        float z = 0.f, d = 0.f;
+        walk_window<BF, KS>(s, a.rpb, tl.nn, qr, qc, [&](int r, int c, float bias) {
+            const float p = exp_unit(chan_dot(q, chan_load<BF>(pixel(a, a.k, tl, r, c), dlim)) * s.scale + bias - lse_q);
+            z += p;
+            d += p * chan_dot(go, chan_load<BF>(pixel(a, a.v, tl, r, c), dlim));
+            return z == z;
+        });
+        d /= z;
+        Chan2 acc{0.f, 0.f};
+        walk_window<BF, KS>(s, a.rpb, tl.nn, qr, qc, [&](int r, int c, float bias) {
+            const Chan2 k = chan_load<BF>(pixel(a, a.k, tl, r, c), dlim);
+            const float p = exp_unit(chan_dot(q, k) * s.scale + bias - lse_q) / z;
+            const float ds = p * (chan_dot(go, chan_load<BF>(pixel(a, a.v, tl, r, c), dlim)) - d);
+            chan_add(acc, ds, k);
+            if ((threadIdx.x & 63) == 0 && !(delta_q * 0.f == 0.f))
+                sums[(r - qr + wr) * BiasGrad<KS>::SIDE + c - qc + wc] += ds;
+            return true;
+        });
+        chan_store<BF>(static_cast<short *>(a.dq) + grad_of(a, tl, qr, qc), dlim, acc, s.scale);
+        if ((threadIdx.x & 63) == 0) {
+            const int64_t tok = image_token(a, tl) + (int64_t)qr * s.W + qc;
+            a.delta[tok] = d;
+            row_zinv(a)[tok] = 1.f / z;
+        }
+    }
+}
+// kr, kc: this lane's key
+template <bool BF, int KS>
+__device__ __forceinline__ void again_keys(const BArgs &a, const ATile &tl, int kr_, int kc_, bool live, unsigned bad,
+                                           int dlim) {
+    constexpr int SPAN = 2 * KS - 1;
+    const Shape &s = a.s;
+    for (; bad; bad &= bad - 1) {
+        const int col = __builtin_ctz(bad), kr = __shfl(kr_, col, 64), kc = __shfl(kc_, col, 64);
+        if (!__shfl((int)live, col, 64)) continue;
+        const Chan2 k = chan_load<BF>(pixel(a, a.k, tl, kr, kc), dlim), v = chan_load<BF>(pixel(a, a.v, tl, kr, kc), dlim);
+        Chan2 ak{0.f, 0.f}, av{0.f, 0.f};
+        bool open = true;
+        for (int r = inv_lo(kr, KS); open && r < inv_hi(kr, s.H, KS); r++)
+            for (int c = inv_lo(kc, KS); open && c < inv_hi(kc, s.W, KS); c++) {
+                if ((unsigned)(kr - win_start(r, s.H, KS)) >= (unsigned)KS ||
+                    (unsigned)(kc - win_start(c, s.W, KS)) >= (unsigned)KS)
+                    continue;
+                const int64_t tok = image_token(a, tl) + (int64_t)r * s.W + c;
+                const float bias = cvt32<BF>(
+                    static_cast<const short *>(a.rpb)[((int64_t)tl.nn * SPAN + kr - r + KS - 1) * SPAN + kc - c + KS - 1]);
+                const Chan2 q = chan_load<BF>(pixel(a, a.q, tl, r, c), dlim), go = chan_load<BF>(pixel(a, a.d_o, tl, r, c), dlim);
+                const float p = exp_unit(chan_dot(q, k) * s.scale + bias - a.lse[tok]) * row_zinv(a)[tok];
+                chan_add(av, p, go);
+                chan_add(ak, p * (chan_dot(go, v) - a.delta[tok]), q);
+                open = p == p;
+            }
+        const int64_t to = grad_of(a, tl, kr, kc);
+        chan_store<BF>(static_cast<short *>(a.dk) + to, dlim, ak, s.scale);
+        chan_store<BF>(static_cast<short *>(a.dv) + to, dlim, av, 1.f);
+    }
+}
+
 // ------------------------------------------------------------------ forward
 // ROLL: walk down the columns of an image and keep the halo rows that consecutive
 // tiles share in LDS (see make_runs); otherwise a strided walk over row-major tiles
@@ -408,9 +517,11 @@ __global__ __launch_bounds__(1024) void rpb_tile_reduce(const float *rows, float
 // an explicit wait on its other side, it falls back to waiting for everything outstanding
 // (B4 N4 128x128 d128 k5: 58.8 -> 56.7 us, 256x256: 198.2 -> 189.3, d64 k5: 60.4 -> 58.5).
 // With a bias the head_dim 32 forward takes 169 to 175 registers (k = 7 and 9), one more than three
-// waves per SIMD have: budgeted for three, B8 N8 112x112 k7 114.8 -> 97.8 us.
+// waves per SIMD have: budgeted for three, B8 N8 112x112 k7 114.8 -> 97.8 us.  At k = 5 four (three at
+// head_dim 64) take a register or two too many without a budget (B8 N4 56x56 d64 k5 16.6 us with two).
 template <int D, int KS, int NW>
-constexpr int kFwdWaves = kBias && D == 32 && KS <= 9 ? 3 : Geo<D, KS, NW>::WAVES;
+constexpr int kFwdWaves = kBias && D == 32 && KS == 5 ? 4
+                          : kBias && ((D == 32 && KS <= 9) || (D == 64 && KS == 5)) ? 3 : Geo<D, KS, NW>::WAVES;
 template <bool BF, int D, int KS, bool ROLL, int NW = 4, bool FULL = false>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void fwd_mfma(FArgs a, int tiles_r, int tiles_c, int ntiles, Runs rp) {
     using G = Geo<D, KS, NW>;
@@ -551,12 +662,16 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
                         o[mt]);
             }
 
+            const unsigned bad = kBias ? bad_columns(o, sum) : 0u;
+            const bool here = lq.live && !(bad >> n & 1);
             store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(const_cast<short *>(image_at(a, a.o, cur)) + lq.qr * row_step(a, a.o) + lq.qc * col_step(a, a.o),
-                               g, o, 1.f / sum, lq.live, dlim);
+                               g, o, 1.f / sum, here, dlim);
             // (FULL: all four lanes of a token write its log-sum-exp, the same value, so that
             // this store is not predicated either)
-            if (a.lse && (FULL || (lq.live && g == 0)))
+            if (a.lse && (FULL || (here && g == 0)))
                 a.lse[lq.tok] = lse_of(mx, sum);
+            if constexpr (kBias)
+                if (__builtin_expect(bad != 0, 0)) again_fwd<BF, KS>(a, cur, lq, bad, dlim);
         }
 
         if (!more) {
@@ -700,10 +815,14 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                     o[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(vp[0], mt)), lds_read_tr(G::t_at(vp[1], mt))), pb[ks],
                         o[mt]);
             }
+            const unsigned bad = kBias ? bad_columns(o, sum) : 0u;
+            const bool here = lq.live && !(bad >> n & 1);
             store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(const_cast<short *>(image_at(a, a.o, cur)) + lq.qr * row_step(a, a.o) + lq.qc * col_step(a, a.o),
-                               g, o, 1.f / sum, lq.live, dlim);
-            if (a.lse && (FULL || (lq.live && g == 0)))
+                               g, o, 1.f / sum, here, dlim);
+            if (a.lse && (FULL || (here && g == 0)))
                 a.lse[lq.tok] = lse_of(mx, sum);
+            if constexpr (kBias)
+                if (__builtin_expect(bad != 0, 0)) again_fwd<BF, KS>(a, cur, lq, bad, dlim);
         }
         if (!more) {
             if constexpr (FULL) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), see fwd_mfma
@@ -891,7 +1010,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
 
             DsScale<BF> scl;
             if constexpr (kBias) {
-                operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live ? zinv : 0.f);
+                operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live && delta * 0.f == 0.f ? zinv : 0.f);
                 BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
             }
             f32x4 dq[G::DT];
@@ -909,8 +1028,15 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                         dq[mt]);
             }
 
-            store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * (kBias ? zinv * scl.inverse() : 1.f), lq.live, dlim);
-            if (FULL || (lq.live && g == 0)) {
+            const unsigned bad = kBias ? bad_columns(dq, delta) : 0u;
+            store_token<BF, D, kLineStores<D, KS, G::WAVES>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * (kBias ? zinv * scl.inverse() : 1.f), lq.live && !(bad >> n & 1), dlim);
+            if constexpr (kBias)
+                if (__builtin_expect(bad != 0, 0)) {
+                    BiasGrad<KS>::wave_fence();
+                    again_dq<BF, KS>(a, cur, lq, bad, lse2, delta, wave,
+                                     lds_dbias + wave * BiasGrad<KS>::WORDS + 4 * BiasGrad<KS>::PLANE, dlim);
+                }
+            if (FULL || (lq.live && g == 0 && !(bad >> n & 1))) {
                 a.delta[lq.tok] = delta;
                 if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
             }
@@ -1082,7 +1208,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                 }
             DsScale<BF> scl;
             if constexpr (kBias) {
-                operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live ? zinv : 0.f);
+                operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live && delta * 0.f == 0.f ? zinv : 0.f);
                 BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
             }
             f32x4 dq[G::DT];
@@ -1099,8 +1225,15 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                     dq[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(kp[0], mt)), lds_read_tr(G::t_at(kp[1], mt))), dsb[ks],
                         dq[mt]);
             }
-            store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * (kBias ? zinv * scl.inverse() : 1.f), lq.live, dlim);
-            if (FULL || (lq.live && g == 0)) {
+            const unsigned bad = kBias ? bad_columns(dq, delta) : 0u;
+            store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * (kBias ? zinv * scl.inverse() : 1.f), lq.live && !(bad >> n & 1), dlim);
+            if constexpr (kBias)
+                if (__builtin_expect(bad != 0, 0)) {
+                    BiasGrad<KS>::wave_fence();
+                    again_dq<BF, KS>(a, cur, lq, bad, lse2, delta, wave,
+                                     lds_dbias + wave * BiasGrad<KS>::WORDS + 4 * BiasGrad<KS>::PLANE, dlim);
+                }
+            if (FULL || (lq.live && g == 0 && !(bad >> n & 1))) {
                 a.delta[lq.tok] = delta;
                 if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
             }
@@ -1339,10 +1472,17 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
 
         if constexpr (kBias) unscale<BF>(dk, dv, scl);
         const int kr = cur.r0 + orow + (n >> 2), kc = cur.c0 + ocol + (n & 3);
-        const int64_t goff = grad_of(a, cur, kr, kc);
+        auto store = [&]() __attribute__((always_inline)) {
+            const int64_t goff = grad_of(a, cur, kr, kc);
+            const unsigned bad = kBias ? bad_columns(dk) | bad_columns(dv) : 0u;
+            const bool here = !(bad >> n & 1);
+            store_token<BF, D, kInnerLines<D>, !kBias>(static_cast<short *>(a.dk) + goff, g, dk, s.scale, here, dlim);
+            store_token<BF, D, kInnerLines<D>, !kBias>(static_cast<short *>(a.dv) + goff, g, dv, 1.f, here, dlim);
+            if constexpr (kBias)
+                if (__builtin_expect(bad != 0, 0)) again_keys<BF, KS>(a, cur, kr, kc, true, bad, dlim);
+        };
         if constexpr (SP == 1) {
-            store_token<BF, D, kInnerLines<D>, true>(static_cast<short *>(a.dk) + goff, g, dk, s.scale, true, dlim);
-            store_token<BF, D, kInnerLines<D>, true>(static_cast<short *>(a.dv) + goff, g, dv, 1.f, true, dlim);
+            store();
             if (!more) break;
             load_keys(nxt);
             __syncthreads();
@@ -1367,8 +1507,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
                     dk[mt] += red[mt * 256];
                     dv[mt] += red[(G::DT + mt) * 256];
                 }
-                store_token<BF, D, kInnerLines<D>, true>(static_cast<short *>(a.dk) + goff, g, dk, s.scale, true, dlim);
-                store_token<BF, D, kInnerLines<D>, true>(static_cast<short *>(a.dv) + goff, g, dv, 1.f, true, dlim);
+                store();
             }
             if (!more) break;
         }
@@ -1603,8 +1742,12 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
             if (cur.last) unscale<BF>(dk, dv, scl);
         auto store = [&]() __attribute__((always_inline)) {
             const int64_t goff = grad_of(a, cur.tl, kr, kc);
-            store_token<BF, D, kLineStores<D, KS, fits<D, KS>() ? Geo<D, KS, 4, SP>::WAVES : 1>>(static_cast<short *>(a.dk) + goff, g, dk, s.scale, live, dlim);
-            store_token<BF, D, kLineStores<D, KS, fits<D, KS>() ? Geo<D, KS, 4, SP>::WAVES : 1>>(static_cast<short *>(a.dv) + goff, g, dv, 1.f, live, dlim);
+            const unsigned bad = kBias ? bad_columns(dk) | bad_columns(dv) : 0u;
+            const bool here = live && !(bad >> n & 1);
+            store_token<BF, D, kLineStores<D, KS, fits<D, KS>() ? Geo<D, KS, 4, SP>::WAVES : 1>>(static_cast<short *>(a.dk) + goff, g, dk, s.scale, here, dlim);
+            store_token<BF, D, kLineStores<D, KS, fits<D, KS>() ? Geo<D, KS, 4, SP>::WAVES : 1>>(static_cast<short *>(a.dv) + goff, g, dv, 1.f, here, dlim);
+            if constexpr (kBias)
+                if (__builtin_expect(bad != 0, 0)) again_keys<BF, KS>(a, cur.tl, kr, kc, live, bad, dlim);
         };
         if constexpr (SP == 1) {
             if (cur.last) store();

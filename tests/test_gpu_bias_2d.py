@@ -137,3 +137,43 @@ def test_float16_with_small_upstream_gradients(shape, ks):
         rounding = ((r.to(F16).double() - r).norm() / r.norm()).item()
         print("   ", name, "2-norm %.2e, of the result's rounding alone %.2e" % (norm, rounding), flush=True)
         assert norm <= 1.05 * rounding, (name, norm, rounding)
+
+
+@pytest.mark.parametrize("which", ["k", "v", "dO"])
+@pytest.mark.parametrize("shape,ks,dtype", [
+    ((1, 2, 29, 24, 32), 5, BF16),    # inner tiles and border
+    ((1, 1, 26, 28, 64), 13, F16),    # two waves per block of keys, one halo in LDS at a time
+    ((1, 1, 20, 21, 128), 9, BF16),
+    ((1, 1, 22, 21, 128), 11, F16),   # frame body only
+])
+def test_values_that_are_not_finite_stay_in_their_windows(shape, ks, dtype, which):
+    # a NaN in one pixel of k, v or dO: only what the windows connect with it may be touched, though rows
+    # outside a window are staged beside it
+    ensure_built()
+    print("case not finite", which, shape, dtype, "k=%d" % ks, flush=True)
+    H, W = shape[2:4]
+    at = 12 * W + 9
+    q, k, v, g = make_inputs(shape, dtype, seed=79)
+    rpb, scale = _rpb(shape[1], ks).to(dtype), shape[-1] ** -0.5
+    _, ref = _both((q, k, v, rpb, g), ks, scale)
+    {"k": k, "v": v, "dO": g}[which].flatten(2, 3)[:, :, at] = float("nan")
+    got, _ = _both((q, k, v, rpb, g), ks, scale)
+    mask = O.neighbour_mask(H, W, ks)
+    only = torch.zeros(H * W, dtype=torch.bool)
+    only[at] = True
+    queries = only if which == "dO" else mask[:, at]   # queries with a gradient that is touched
+    keys = mask[queries].any(0)                        # the keys that these see
+    none = torch.zeros_like(only)
+    pairs = (mask & queries[:, None]).nonzero()
+    entries = torch.zeros(2 * ks - 1, 2 * ks - 1, dtype=torch.bool)
+    entries[pairs[:, 1] // W - pairs[:, 0] // W + ks - 1, pairs[:, 1] % W - pairs[:, 0] % W + ks - 1] = True
+    touched = (none if which == "dO" else queries, queries, keys, none if which == "v" else keys, entries.flatten())
+    for name, x, r, t in zip(NAMES, got, ref, touched):
+        x, r = ((y.flatten(2, 3) if name != "dRPB" else y.flatten(1)[None, :, :, None]) for y in (x, r))
+        assert x[:, :, t].isnan().all(), name
+        x, r = x[:, :, ~t], r[:, :, ~t]
+        if r.numel() == 0:
+            continue
+        norm = ((x - r).norm() / r.norm()).item()
+        print("   ", name, "2-norm %.2e" % norm, flush=True)
+        assert norm <= (4e-3 if dtype == BF16 else 5e-4), (name, norm)  # (as in test_bias)
