@@ -4,6 +4,7 @@
 #include <stdio.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "na2d_common.h"
 
@@ -194,6 +195,36 @@ View one_sub(const View &v, int es, int dil, int i, int j) {
     o.sh = v.sh * dil; o.sw = v.sw * dil;
     return o;
 }
+// Sub-grids that fill the chip on their own run one after the other on the kernels for undilated
+// images: these are built for head dims of exactly 32, 64 and 128 and have the fused backward, which
+// the build for all sub-grids at once has not.  `tiles`: 8x8 tiles of one sub-grid over batch and heads.
+// bf16, views of a projection, us, one after the other / all at once.
+// Backward: d128 from 1024 tiles on (B4 N4 128x128 dilation 2 k3 158 / 188, k5 173 / 220, k9 394 / 414; k13
+// already at 512, 224 / 363), d64 and d32 from 2048 (B8 N8 128x128 dilation 2 d64 k5 353 / 486, d32 k7 308 / 384; at
+// 1024 d32 k7 119 / 99); at 512 and 1024 tiles where the tensors no longer fit the caches (B8 N8 128x128 dilation
+// 4 d32 k7 374 / 419, d64 k9 1061 / 1116, B8 N4 d128 k5 470 / 560); head dims between the built ones from 4096
+// (B4 N8 256x256 d48 k7 1149 / 1231, at 2048 294 / 254).
+// Forward, which has one kernel either way: d32 and d64 at 4096 tiles k9 112 / 135 and 181 / 211, at 1024 k7 39 / 33;
+// small windows only at dilation 2 (d64 k3 56 / 67; dilation 3, 4096 tiles, d32 k3 216 / 202: pixels far apart
+// share lines with other sub-grids); d128 k13 at 1024 tiles 101 / 113, k3 at 1936 267 / 291, k7 at 4096 328 / 301.
+bool exact_dim(int D) { return D == 32 || D == 64 || D == 128; }
+template <typename ARGS>
+bool alone(const ARGS &a) {
+    const Shape &s = a.s;
+    const int64_t subs = (int64_t)a.sub_r * a.sub_c;
+    const int64_t tiles = (int64_t)s.B * s.N * ((s.H + 7) / 8) * ((s.W + 7) / 8);
+    if constexpr (std::is_same_v<ARGS, FwdArgsSub>) {
+        if (!exact_dim(s.D) || small_fwd_supported(a)) return false;
+        if (subs == 1) return true;
+        if (s.D == 128) return s.kh >= 11 ? tiles >= 1024 : s.kh <= 5 && tiles >= 1536;
+        return tiles >= 2048 && (s.kh >= 7 || a.dil == 2);
+    } else {
+        if (small_bwd_supported(a)) return false;
+        if (!exact_dim(s.D)) return tiles >= 4096;
+        return subs == 1 || tiles >= (s.D == 128 ? (s.kh >= 11 ? 512 : 1024) : 2048) ||
+               (tiles >= 512 && tiles * subs >= 8192);
+    }
+}
 void *offset(void *p, int64_t elements, int es) { return static_cast<char *>(p) + elements * es; }
 
 int check_dilation(const char *fn, int H, int W, int ks, int dil) {
@@ -383,7 +414,8 @@ int enatten2d_bwd_static(const void *q, const void *k, const void *v, const void
 
 // ---- dilated neighborhoods --------------------------------------------------
 // Sub-grids of one size run as one batch on the matrix-core kernels (up to four groups, one if
-// the dilation divides both sides), and one after the other on the other kernels.  The
+// the dilation divides both sides), and one after the other where they are large (`alone`) and on the
+// other kernels.  The
 // log-sum-exp and the workspace are laid out by group, within a group one [B, heads, h, w]
 // block per sub-grid, whichever kernels serve the call, so that a backward that is routed
 // differently from its forward (a misaligned upstream gradient) finds what it needs.
@@ -416,7 +448,7 @@ int enatten2d_fwd_dilated(const void *q, const void *k, const void *v, void *o, 
             a.s = Shape{B, heads, r.extent, c.extent, D, kernel_size, kernel_size, scale};
             a.sub_r = r.count; a.sub_c = c.count; a.dil = dilation;
             const int64_t per_sub = (int64_t)B * heads * r.extent * c.extent;
-            if (use_mfma(D, kernel_size, dtype) && sub_layout_ok(a)) {
+            if (use_mfma(D, kernel_size, dtype) && sub_layout_ok(a) && !alone(a)) {
                 if ((rc = launch_fwd_mfma_sub(a, dtype, st))) return rc;
             } else {
                 for (int i = 0; i < r.count; i++)
@@ -487,7 +519,7 @@ int enatten2d_bwd_dilated(const void *q, const void *k, const void *v, const voi
             a.sub_r = r.count; a.sub_c = c.count; a.dil = dilation;
             const int64_t per_sub = (int64_t)B * heads * r.extent * c.extent;
             a.delta = static_cast<float *>(workspace);
-            if (use_mfma(D, kernel_size, dtype) && sub_layout_ok(a)) {
+            if (use_mfma(D, kernel_size, dtype) && sub_layout_ok(a) && !alone(a)) {
                 a.zinv = a.delta + r.count * c.count * per_sub;
                 if ((rc = launch_bwd_mfma_sub(a, dtype, st))) return rc;
             } else {

@@ -73,6 +73,31 @@ def test_column_walk_keeps_rows_of_its_own_sub_grid_only():
             assert_close([t[sub] for t in got], ref, BF16, "sub-grid %d %d" % (i, j))
 
 
+@pytest.mark.parametrize("shape,ks,dtype", [
+    ((9, 38, 41, 35, 32), 7, BF16),   # four sizes of sub-grids, 3078 tiles in each
+    ((9, 40, 40, 36, 64), 3, F16),    # 3240 tiles
+    ((8, 64, 32, 34, 128), 5, BF16),  # 3072 tiles: the backward only
+    ((8, 32, 32, 30, 128), 11, F16),  # 1024 tiles
+    ((19, 37, 40, 36, 48), 5, BF16),  # a head_dim between the built ones: 6327 tiles, the backward only
+])
+def test_large_sub_grids_run_one_after_the_other(shape, ks, dtype):
+    ensure_built()
+    from e_natten_amd import natten2d
+    print("case large sub-grids", shape, dtype, "k=%d dilation=2" % ks, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(83)
+    B, N, H, W, d = shape
+    x = torch.randn((B, H, W, 4, N, d), generator=gen, device="cuda", dtype=dtype)
+    q, k, v, g = (t.permute(0, 3, 1, 2, 4) for t in x.unbind(3))
+    q, k, v = (t.detach().requires_grad_(True) for t in (q, k, v))
+    o = natten2d(q, k, v, ks, d ** -0.5, 2)
+    got = (o, *torch.autograd.grad(o, (q, k, v), g))
+    one = (slice(B - 1, B), slice(N - 2, N))  # (every image is the same computation on other data)
+    xr = [t[one].detach().cpu().double().requires_grad_(True) for t in (q, k, v)]
+    o_ref = O.natten2d_dilated_dense_mask(*xr, ks, 2, d ** -0.5)
+    ref = (o_ref.detach(), *torch.autograd.grad(o_ref, xr, g[one].cpu().double()))
+    assert_close([t.detach()[one].cpu() for t in got], ref, dtype, "large sub-grids")
+
+
 @pytest.mark.parametrize("shape,ks,dil,dtype", [
     ((8, 16, 14, 14, 64), 9, 1, BF16),
     ((2, 64, 14, 14, 32), 7, 1, F16),
