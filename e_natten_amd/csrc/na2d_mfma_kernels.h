@@ -457,15 +457,21 @@ __device__ __forceinline__ void again_dq(const BArgs &a, const ATile &tl, const 
         });
         d /= z;
         Chan2 acc{0.f, 0.f};
-        walk_window<BF, KS>(s, a.rpb, tl.nn, qr, qc, [&](int r, int c, float bias) {
-            const Chan2 k = chan_load<BF>(pixel(a, a.k, tl, r, c), dlim);
-            const float p = exp_unit(chan_dot(q, k) * s.scale + bias - lse_q) / z;
-            const float ds = p * (chan_dot(go, chan_load<BF>(pixel(a, a.v, tl, r, c), dlim)) - d);
-            chan_add(acc, ds, k);
-            if ((threadIdx.x & 63) == 0 && !(delta_q * 0.f == 0.f))
-                sums[(r - qr + wr) * BiasGrad<KS>::SIDE + c - qc + wc] += ds;
-            return true;
-        });
+        if (d != d) {  // every dS of the window is NaN
+            float *at = sums + (win_start(qr, s.H, KS) - qr + wr) * BiasGrad<KS>::SIDE + win_start(qc, s.W, KS) - qc + wc;
+            for (int i = threadIdx.x & 63; i < KS * KS; i += 64) at[i / KS * BiasGrad<KS>::SIDE + i % KS] = d;
+            acc = Chan2{d, d};
+        } else {
+            walk_window<BF, KS>(s, a.rpb, tl.nn, qr, qc, [&](int r, int c, float bias) {
+                const Chan2 k = chan_load<BF>(pixel(a, a.k, tl, r, c), dlim);
+                const float p = exp_unit(chan_dot(q, k) * s.scale + bias - lse_q) / z;
+                const float ds = p * (chan_dot(go, chan_load<BF>(pixel(a, a.v, tl, r, c), dlim)) - d);
+                chan_add(acc, ds, k);
+                if ((threadIdx.x & 63) == 0 && !(delta_q * 0.f == 0.f))
+                    sums[(r - qr + wr) * BiasGrad<KS>::SIDE + c - qc + wc] += ds;
+                return true;
+            });
+        }
         chan_store<BF>(static_cast<short *>(a.dq) + grad_of(a, tl, qr, qc), dlim, acc, s.scale);
         if ((threadIdx.x & 63) == 0) {
             const int64_t tok = image_token(a, tl) + (int64_t)qr * s.W + qc;

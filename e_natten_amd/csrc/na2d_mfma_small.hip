@@ -243,6 +243,7 @@ __global__ __launch_bounds__(G::NT, G::WPS) void fwd_small_mfma(FwdArgsSub a, in
                 mx = mn;
                 z = z * corr + p;
                 acc = acc * corr + p * chan<BF>(lds_v + key * G::PITCH, l, D);
+                if (z != z) break;  // nothing finite can come of it
             }
             if (l < s.D) oimg[pix(a.o, a.dil, t / s.W, t % s.W) + l] = cvt16<BF>(acc / z);
             if (a.lse && l == 0) a.lse[im.tok + t] = (mx + __builtin_amdgcn_logf(z)) * kLn2;
@@ -350,6 +351,7 @@ __global__ __launch_bounds__(G::NT, G::WPS) void bwd_small_mfma(BwdArgsSub a, in
                 res += y;
                 acc += y * kr;
                 accp += p * kr;
+                if (z != z) break;  // nothing finite can come of it
             }
             if (l < s.D) static_cast<short *>(a.dq)[grad_pix(t) + l] = cvt16<BF>((acc - res / z * accp) * s.scale);
             if (l == 0) lds_delta[t] += res / z;
@@ -409,6 +411,7 @@ __global__ __launch_bounds__(G::NT, G::WPS) void bwd_small_mfma(BwdArgsSub a, in
                 const float p = __builtin_amdgcn_exp2f(wave_sum(qr * kr) * sc2 - lds_lse[q]);
                 av += p * gr;
                 ak += p * (wave_sum(gr * vr) - lds_delta[q]) * qr;
+                if (p != p) break;  // nothing finite can come of it
             }
             if (l < s.D) {
                 static_cast<short *>(a.dk)[grad_pix(t) + l] = cvt16<BF>(ak * s.scale);
