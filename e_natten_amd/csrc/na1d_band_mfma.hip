@@ -673,22 +673,34 @@ bool band_layout_ok(const View &v) {
     return reinterpret_cast<uintptr_t>(v.ptr) % 16 == 0 && v.sb % 8 == 0 && v.sn % 8 == 0 && v.sw % 8 == 0 &&
            v.sw < (1 << 22);
 }
-// (not windows of one key, whose probability is 1: dP - delta must cancel to an exact zero, which
-// takes the two sums in one order, as in the general kernels)
-bool band_shape_ok(const Shape &s, int dtype) {
-    return s.kw > 1 && (dtype == ENATTEN_BF16 || dtype == ENATTEN_F16) && s.D >= 8 && s.D <= 128 && s.D % 8 == 0 &&
-           s.H == 1 && s.kh == 1 && (int64_t)s.B * s.N * ((s.W + 63) / 64) <= ((int64_t)1 << 32) / 256 - 8;  // (threads of a launch)
+// The smallest window that is taken here.  A tile walks at least two blocks of 64 keys, however few of them its
+// windows hold, and narrow heads give the matrix instructions little to do.  us, general kernels / here, causal, B4 N8
+// T16384 bf16, forward and backward: d8 k6 34 / 37, 80 / 106, k12 58 / 37, 131 / 104; d16 k4 32 / 36, 81 / 107, k8 46 / 36,
+// 109 / 107; d24 k4 40 / 53, 116 / 141, k8 59 / 53, 163 / 141; d32 k3 36 / 37, 110 / 116, k4 40 / 37, 123 / 117; d48 k2 52 / 77,
+// 193 / 208, k4 70 / 77, 247 / 207, k6 87 / 77; d64 k2 61 / 50, 238 / 158.
+// (Not windows of one key, whose probability is 1: dP - delta must cancel to an exact zero, which
+// takes the two sums in one order, as in the general kernels.)
+int least_window(int D, bool backward) {
+    if (D >= 64) return 2;
+    if (D > 32) return backward ? 3 : 6;
+    if (D == 32) return 4;
+    return D <= 8 ? (backward ? 12 : 8) : D <= 16 ? (backward ? 8 : 6) : 8;
+}
+bool band_shape_ok(const Shape &s, int dtype, bool backward) {
+    return (dtype == ENATTEN_BF16 || dtype == ENATTEN_F16) && s.D >= 8 && s.D <= 128 && s.D % 8 == 0 &&
+           s.kw >= least_window(s.D, backward) && s.H == 1 && s.kh == 1 &&
+           (int64_t)s.B * s.N * ((s.W + 63) / 64) <= ((int64_t)1 << 32) / 256 - 8;  // (threads of a launch)
 }
 
 }  // namespace
 
 bool band_supported(const FwdArgs &a, int dtype) {
-    return band_shape_ok(a.s, dtype) && !a.rpb && band_layout_ok(a.q) && band_layout_ok(a.k) &&
+    return band_shape_ok(a.s, dtype, false) && !a.rpb && band_layout_ok(a.q) && band_layout_ok(a.k) &&
            band_layout_ok(a.v) && band_layout_ok(a.o);
 }
 bool band_supported(const BwdArgs &a, int dtype) {
     auto al = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-    return band_shape_ok(a.s, dtype) && !a.rpb && band_layout_ok(a.q) && band_layout_ok(a.k) &&
+    return band_shape_ok(a.s, dtype, true) && !a.rpb && band_layout_ok(a.q) && band_layout_ok(a.k) &&
            band_layout_ok(a.v) && band_layout_ok(a.o) && band_layout_ok(a.d_o) && al(a.dq) && al(a.dk) &&
            al(a.dv) && a.gsb % 8 == 0 && a.gsn % 8 == 0 && a.gsw % 8 == 0;
 }

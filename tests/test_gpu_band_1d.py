@@ -20,6 +20,16 @@ BF16, F16 = torch.bfloat16, torch.float16
     ((1, 2, 257, 64), 51, False, BF16, "proj"),    # centred: clamped windows at both ends
     ((2, 1, 129, 128), 129, False, F16, "plain"),  # window = sequence: plain attention
     ((8, 64, 160, 64), 97, False, BF16, "plain"),  # two groups per wave
+    # the smallest windows of every head_dim: on the general kernels below these, in the backward or both
+    ((1, 2, 140, 64), 2, True, F16, "proj"),
+    ((1, 2, 140, 48), 5, True, BF16, "plain"),     # only the backward here
+    ((1, 2, 140, 48), 6, True, BF16, "proj"),
+    ((1, 2, 140, 56), 2, True, F16, "plain"),      # neither
+    ((1, 2, 140, 32), 4, True, BF16, "plain"),
+    ((1, 2, 140, 32), 3, True, F16, "proj"),       # neither
+    ((1, 2, 140, 24), 8, True, BF16, "proj"),
+    ((1, 2, 140, 16), 6, True, F16, "plain"),      # only the forward here
+    ((1, 2, 140, 8), 12, True, BF16, "proj"),
 ])
 def test_band_windows(shape, ks, causal, dtype, layout):
     ensure_built()
