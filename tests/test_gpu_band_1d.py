@@ -9,17 +9,20 @@ BF16, F16 = torch.bfloat16, torch.float16
 
 
 @pytest.mark.parametrize("shape,ks,causal,dtype,layout", [
-    ((1, 2, 65, 32), 2, True, BF16, "plain"),      # smallest window with a gradient; one position past a tile
+    ((1, 2, 65, 32), 2, True, BF16, "plain"),      # smallest window with a gradient (on the general kernels)
     ((2, 1, 64, 64), 64, True, F16, "plain"),      # plain causal attention of one tile
     ((1, 3, 200, 128), 33, True, BF16, "proj"),    # band edges inside the steps of 32 keys
     ((1, 2, 300, 128), 300, True, F16, "plain"),   # window = sequence
     ((2, 2, 131, 40), 16, True, BF16, "proj"),     # head_dim below a built one
     ((1, 2, 17, 8), 5, True, F16, "plain"),        # shorter than one step of keys
-    ((4, 128, 130, 32), 70, True, BF16, "plain"),  # two groups of queries per wave, the second cut
+    ((4, 128, 130, 32), 70, True, BF16, "plain"),  # more tiles than workgroups at a time, the last one cut
     ((4, 128, 200, 128), 100, True, F16, "proj"),
+    ((2, 90, 330, 128), 256, True, F16, "plain"),  # two groups of queries per wave in the forward, the last tile cut
+    ((2, 90, 330, 128), 257, False, BF16, "proj"),
+    ((2, 90, 310, 128), 300, True, BF16, "proj"),  # ... its second group of some waves past the end
     ((1, 2, 257, 64), 51, False, BF16, "proj"),    # centred: clamped windows at both ends
     ((2, 1, 129, 128), 129, False, F16, "plain"),  # window = sequence: plain attention
-    ((8, 64, 160, 64), 97, False, BF16, "plain"),  # two groups per wave
+    ((8, 64, 160, 64), 97, False, BF16, "plain"),  # more tiles than workgroups at a time
     # the smallest windows of every head_dim: on the general kernels below these, in the backward or both
     ((1, 2, 140, 64), 2, True, F16, "proj"),
     ((1, 2, 140, 48), 5, True, BF16, "plain"),     # only the backward here
