@@ -471,22 +471,28 @@ int bwd_size(const BwdArgsSub &a, hipStream_t st) {
 // Where an image is taken whole, tiled / whole in us, bf16.  The forward: where there are more
 // images than CUs, since the tiled kernel spreads one over four workgroups (14x14 pixels d32 k7: 8
 // images 5.3 / 8.3, 128 images 6.6 / 8.4, 512 images 14.2 / 11.7), and up to 208 pixels: at 16x16 the
-// tiles are whole and level (8192 images d32 k5 211 / 215).  The backward, one kernel in the place of
-// two whose dK/dV pass walks the border: always (4 images 14x14 d64 20.5 / 17.5, 32 images d32
-// 18.8 / 13.2, 512 images 55.9 / 20.1, 3200 images 8x8 68 / 31, 8192 images 16x16 652 / 415).
-// With one size (208 tokens, eight waves) for all, 3200 images 8x8 took 18.6 + 39.4 instead of
-// 15.9 + 31.3.  Not where a few workgroups hold the largest size with one to a CU (d64 k13 16x16: 4
-// images 25.5 / 27.7, 32 images 25.2 / 24.7).
-// Undilated images: for k >= 7 and from 128 images on (14x14 d32 k7: 128 images 16.4 / 13.3, 1024
-// images 99.7 / 38.4; 14x18 d48 k9: 32 images 23.5 / 24.8, 128 images 36.9 / 25.0; 9x10 d64 k9, 1024
-// images 103 / 30); at k = 3 and 5 the other passes have little border to walk (14x14 d64 k3, 128
-// images 10.8 / 14.5).  Their forward from the second tile on (8x8 d32, 1024 images 7.1 / 7.5).
+// tiles are whole and level (8192 images d32 k5 211 / 215).  Undilated ones for k >= 7 from the second tile on
+// (8x8 d32, 1024 images 7.1 / 7.5).
+// The backward, one kernel in the place of two whose dK/dV pass walks the border: always for the smallest size
+// (8x8 d32 k7, 16 to 256 images 8.4 to 9.0 / 6.3 to 6.8; 9x10 d64 k9, 8 images, dilated 16.0 / 13.0), and where the 8x8
+// tiles are too many for two workgroups per CU (14x14 d32 k7 192 images 22.8 / 16.0, d64 k9 31.8 / 23.8, dilated 256
+// images 44.2 / 26.7; 14x18 d48 k9 96 images 35.3 / 28.8; 16x16 d64 k13 128 dilated images 41.7 / 31.4), at head dims
+// up to 32 a little before (14x14 d32 k7 96 images 15.9 / 15.5) and dilated for k >= 5 always (14x14 d32 k7, 8 images 17.0 /
+// 15.2).  With fewer tiles the tiled kernels have the chip to themselves (64 images 14x14 d32 k7 12.9 / 15.3, d64
+// k9 17.9 / 22.9, dilated 20.4 / 23.0, 14x14 d32 k3 dilated 11.6 / 12.6; 128 images 16x16 d32 k7 13.4 / 15.1).  Undilated
+// images for k >= 7 only: at k = 3 and 5 the other passes have little border to walk (14x14 d64 k3, 128
+// images 10.8 / 14.5).
 bool small_fwd_supported(const FwdArgsSub &a) {
-    return size_ok(a.s, images_of(a), 208, fwd_threads(a.s)) && images_of(a) > 256 && (a.dil > 1 || (a.s.kh >= 7 && a.s.H * a.s.W > 64));
+    return size_ok(a.s, images_of(a), 208, fwd_threads(a.s)) && images_of(a) > 256 &&
+           (a.dil > 1 || (a.s.kh >= 7 && a.s.H * a.s.W > 64));
 }
 bool small_bwd_supported(const BwdArgsSub &a) {
-    const int64_t ni = images_of(a);
-    return size_ok(a.s, ni, a.s.D > 32 && ni < 64 ? 208 : 256, bwd_threads(a.s)) && (a.dil > 1 || (a.s.kh >= 7 && ni >= 128));
+    const Shape &s = a.s;
+    const int64_t ni = images_of(a), tiles = ni * ((s.H + 7) / 8) * ((s.W + 7) / 8);
+    if (!size_ok(s, ni, 256, bwd_threads(s))) return false;
+    if (s.H * s.W <= 96) return a.dil > 1 || s.kh >= 7;
+    if (a.dil > 1) return tiles >= 512 || (s.D <= 32 && s.kh >= 5);
+    return s.kh >= 7 && (tiles > 512 || (s.D <= 32 && s.H * s.W <= 208 && tiles >= 384));
 }
 int launch_fwd_small(const FwdArgsSub &a, int dtype, hipStream_t st) {
     if (dtype == ENATTEN_BF16) return a.s.D <= 32 ? fwd_size<true, 32>(a, st) : fwd_size<true, 64>(a, st);
