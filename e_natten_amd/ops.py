@@ -534,7 +534,7 @@ def natten1d(q, k, v, kernel_size=7, scale=1.0, dilation=1, is_causal=False, rpb
     attends keys max(t - kernel_size + 1, 0) .. t; ``rpb`` is a relative position bias
     ``[heads, 2*kernel_size-1]``."""
     if is_causal or rpb is not None:
-        if type(kernel_size) is not int:
+        if not isinstance(kernel_size, int) or isinstance(kernel_size, bool):
             raise TypeError("kernel_size must be an int")
         if rpb is not None and (not isinstance(rpb, torch.Tensor) or rpb.dim() != 2):
             raise ValueError("rpb must be a [heads, 2*kernel_size-1] tensor")

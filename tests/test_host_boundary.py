@@ -256,6 +256,22 @@ def test_window_calls_refuse_meta_tensors_and_other_types():
             f()
 
 
+def test_causal_sequences_take_every_int_as_kernel_size():
+    # an int by inheritance is an int, as in natten2d: the refusal is about the device then
+    import enum
+
+    from e_natten_amd import natten1d, natten2d
+    Size = enum.IntEnum("Size", {"window": 6})
+    t = torch.zeros(1, 2, 20, 8, dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError, match="GPU"):
+        natten1d(t, t, t, Size.window, 1.0, 1, True)
+    with pytest.raises(RuntimeError, match="GPU"):
+        natten2d(t[:, :, :, None], t[:, :, :, None], t[:, :, :, None], (Size.window, 1), 1.0, 1, (True, False))
+    for bad in (True, 6.0, "6"):
+        with pytest.raises(TypeError):
+            natten1d(t, t, t, bad, 1.0, 1, True)
+
+
 def test_window_entry_points_validate(lib):
     from e_natten_amd import _lib, natten1d, natten2d
     f = lambda kh, kw, ch=0, cw=0, H=8, W=8, q=1, rpb=None: lib.enatten2d_fwd_window(
