@@ -268,6 +268,10 @@ class Natten2dDilated(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, Q, K, V, kernel_size, scale, dilation):
+        _validate(Q, K, V, kernel_size)
+        _require_gpu(Q, "natten2d")
+        _window_operands(Q, K, V)
+        scale = float(scale)
         lib = _lib.load()
         q, k, v = (_kernel_layout(t) for t in (Q, K, V))
         B, N, H, W, D = q.shape

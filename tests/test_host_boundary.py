@@ -256,6 +256,24 @@ def test_window_calls_refuse_meta_tensors_and_other_types():
             f()
 
 
+def test_dilated_function_checks_its_operands():
+    # the autograd function itself, not only natten2d, which checks before it: nothing that is not on
+    # the GPU or does not fit together reaches the library
+    from e_natten_amd.ops import Natten2dDilated
+    q = torch.zeros(1, 2, 16, 16, 32, dtype=torch.bfloat16)
+    f = lambda k=q, ks=3: Natten2dDilated.apply(q, k, q, ks, 1.0, 2)
+    with pytest.raises(RuntimeError, match="GPU"):
+        f()
+    for k in (q[:, :1], q.float(), q[0]):
+        with pytest.raises(ValueError):
+            f(k)
+    with pytest.raises(ValueError):
+        f(ks=4)
+    m = q.to("meta")
+    with pytest.raises(RuntimeError, match="GPU"):
+        Natten2dDilated.apply(m, m, m, 3, 1.0, 2)
+
+
 def test_causal_sequences_take_every_int_as_kernel_size():
     # an int by inheritance is an int, as in natten2d: the refusal is about the device then
     import enum
