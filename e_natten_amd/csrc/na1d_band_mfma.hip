@@ -11,7 +11,8 @@
 // the band's edges cut.  Operand layouts are those of na2d_mfma_kernels.h (tokens as MFMA rows,
 // the second product's other operand through the transposing LDS read).
 //
-// The running maximum is only raised when a logit exceeds it by more than 8 (in units of log2):
+// The running maximum is only raised when a logit exceeds it by more than 8 (in units of log2; the
+// conditional rescaling published with FlashAttention-4):
 // until then the probabilities are at most 2^8 times what they would be, which neither float32
 // sums nor 16-bit operands lose anything by, and no cross-lane maximum is formed.
 //

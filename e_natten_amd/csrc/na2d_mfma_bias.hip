@@ -3,9 +3,9 @@
 // centred windows.
 //
 // B8 N4 56x56 d32 k7 bf16, views of a projection: 68 + 103 + 171 us of general kernels and 61 us for
-// the bias gradient before, 13 + 26 + 24 us here (the unbiased kernels: 10 + 11 + 13).  What the
-// bias costs is LDS work: a table read per logit, 28 plane writes and 48 reads per lane and tile for the
-// gradient; the second terms of P and dS double the second products.
+// the bias gradient before, 16 + 30 + 27 + 5 us here, under the profiler.  What the bias costs is LDS work:
+// a table read per logit, 28 plane writes and 48 reads per lane and tile for the gradient; the second
+// terms of P and dS double the second products.
 #include "na2d_common.h"
 
 namespace enatten {

@@ -13,7 +13,7 @@
 // A result that is not finite is computed again from its window alone, as in na1d_band_mfma.hip.
 // Bound by the latency of the staging loads and the vector work on the logits (half of a step's
 // pairs are inside a window at 14x14, k = 7).  B8 N4 56x56 d32 k7 dilation 4, forward and backward
-// on the device: 70.1 us of three tiled kernels before, 31.8 now (2.2 TB/s of its 71 MB).
+// under the profiler: 70.1 us of three tiled kernels before, 13.4 + 26.1 here (1.8 TB/s of its 71 MB).
 #include "na2d_mfma.h"
 
 namespace enatten {

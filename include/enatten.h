@@ -150,7 +150,8 @@ int enatten2d_bwd_into(const void *q, const void *k, const void *v, const void *
  * comparator, test.py:17).  Arguments as in enatten2d_fwd / enatten2d_bwd; H and W must be at
  * least kernel_size * dilation.  Pixels of one residue class modulo the dilation on each axis
  * form a sub-grid on which the undilated rule holds; all sub-grids of one size run as one
- * batch of images on the matrix-core kernels, read and written in place.
+ * batch of images on the matrix-core kernels, or one after the other where each fills the
+ * GPU, read and written in place.
  *   lse         float32 [B * heads * H * W], in an order of the library's own: pass it on to
  *               enatten2d_bwd_dilated
  *   workspace   enatten2d_bwd_dilated_workspace_bytes() bytes of device memory
