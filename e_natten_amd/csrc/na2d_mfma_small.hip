@@ -291,8 +291,8 @@ __global__ __launch_bounds__(G::NT, G::WPS) void bwd_small_mfma(BwdArgsSub a, in
     };
     // dQ.  delta = dO . O is what O was rounded to away from the sum of P dP, an error that all keys
     // of a window share and that keys or values with a common component multiply.  So the residual
-    // E = sum p (dP - delta) is summed beside the products, dQ = A - E / Z sum p k, and the dK/dV jobs
-    // find delta + E / Z (14x14 d64 k9 bf16, k and v of mean 2: dQ off by 4.4e-2 in 2-norm without, 4.1e-3 with).
+    // E = sum p (dP - delta) is summed beside the products, dQ = A - E sum p k, and the dK/dV jobs
+    // find delta + E (sum p is 1 to what the log-sum-exp was rounded to; 14x14 d64 k9 bf16, k and v of mean 2: dQ off by 4.4e-2 in 2-norm without, 4.1e-3 with).
     for (int t0 = wave * 16; t0 < P; t0 += G::NW * 16) {
         const int own = min(t0 + n, P - 1);
         s16x8 qreg[G::DS], greg[G::DS];
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(G::NT, G::WPS) void bwd_small_mfma(BwdArgsSub a, in
         int lo, hi;
         key_run(t0, P, s, lo, hi);
         f32x4 dq[G::DT], pk[G::DT];
-        float zsum = 0.f, esum = 0.f;
+        float esum = 0.f;
 #pragma unroll
         for (int t = 0; t < G::DT; t++) {
             dq[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -321,14 +321,13 @@ __global__ __launch_bounds__(G::NT, G::WPS) void bwd_small_mfma(BwdArgsSub a, in
                 const float x = c[e >> 2][e & 3] * sc2 - lse2;
                 const float p = __builtin_amdgcn_exp2f(inside(pos[e], win, ks) ? x : -INFINITY);
                 const float y = p * (cp[e >> 2][e & 3] - delta);
-                zsum += p;
                 esum += y;
                 ph[e] = cvt16<BF>(p);
                 ds[e] = cvt16<BF>(y);
             }
             second_product<BF, D>(dq, lds_k, kk, n, g, ds, pk, ph);
         }
-        const float shift = col_sum(esum) / col_sum(zsum);
+        const float shift = col_sum(esum);
 #pragma unroll
         for (int t = 0; t < G::DT; t++) dq[t] -= shift * pk[t];
         unsigned bad = bad_columns(dq);
