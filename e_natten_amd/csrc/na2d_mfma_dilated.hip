@@ -6,7 +6,8 @@
 // calls through Python bounded the call.  One launch for all of one size: B8 N4 56x56 d32 k7
 // dilation 4, views of a projection, forward and backward 1060 -> 70 us (16 launches each of 5 +
 // 14 us of kernels and 1100 us of host time before; three kernels of 14 + 25 + 31 us).  Sub-grids
-// that fit one workgroup's LDS go to na2d_mfma_small.hip.
+// that fit one workgroup's LDS go to na2d_mfma_small.hip, and those that fill the chip on their own to
+// the kernels for undilated images (`alone` in enatten_capi.hip).
 #include "na2d_common.h"
 
 namespace enatten {
