@@ -1596,7 +1596,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
     auto first_of = [&](int t) __attribute__((always_inline)) {
         KeyBlock b;
         b.t = t;
-        b.tl = in_sub(frame_tile(t, ts, s.N), a);
+        b.tl = in_sub(frame_tile(t, ts, s.N, sc.step), a);
         b.qa = inv_lo(b.tl.r0, KS);
         b.qb = inv_hi(min(b.tl.r0 + 8, s.H) - 1, s.H, KS);
         b.ca = inv_lo(b.tl.c0, KS);
