@@ -1295,6 +1295,121 @@ __device__ __forceinline__ bool next_block(KeyBlock &b) {
 }
 
 
+// One step of the dK/dV pass: 32 queries (two 16-token tiles) against the wave's 16 keys.
+// AHEAD says how the reads are ordered, with scheduling barriers: 0 as the compiler likes, 1 all
+// operands and statistics of a tile before its matrix instructions, 2 those of both tiles.  Left
+// alone in the frame body's rolled loop the compiler reads the statistics of one query after the
+// other, each behind a wait of its own for LDS, 16 round trips in a row per step at 2 waves per
+// SIMD; the inner body is unrolled and has the next step's arithmetic to put between, so there 1
+// and 2 only cost registers (d128 k5 with its column walk spills with them, 107 -> 222 us), but for
+// head_dim 32, where 2 is ahead (B4 N4 128x128 k9 51.6 -> 48.8 us).
+//   a_of(h), t_of(h): this lane's row of tile h for the direct and for the transposing reads
+//   stat(h, i), at(h, i, st), in(h, i, st): statistics of query 4 g + i of tile h, the place of its
+//   bias in the table, and whether it attends to this lane's key
+template <int D>
+constexpr int kInnerAhead = D == 32 && !kBias ? 2 : 0;
+constexpr int kFrameAhead = 1;
+template <bool BF, typename G, int AHEAD, typename AROW, typename TROW, typename STAT, typename AT, typename IN>
+__device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g, const float *lds_bias, int n, int g,
+                                          float sc2, const s16x8 (&kreg)[G::DS], const s16x8 (&vreg)[G::DS],
+                                          f32x4 (&dk)[G::DT], f32x4 (&dv)[G::DT], DsScale<BF> &scl, AROW a_of,
+                                          TROW t_of, STAT stat, AT at, IN in) {
+    using ST = decltype(stat(0, 0));
+    Op8 pb, dsb;
+    float dsv[8], mag = 0.f;  // (float16 with a bias)
+    s16x8 qa[2][G::DS], ga[2][G::DS];
+    ST st[2][4];
+    auto read = [&](int h) __attribute__((always_inline)) {
+        const int row = a_of(h);
+        const typename G::ARow qp = G::a_row(lds_q, row, g), gp = G::a_row(lds_g, row, g);
+#pragma unroll
+        for (int ds = 0; ds < G::DS; ds++) {
+            qa[h][ds] = *reinterpret_cast<const s16x8 *>(G::a_at(qp, ds));
+            ga[h][ds] = *reinterpret_cast<const s16x8 *>(G::a_at(gp, ds));
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) st[h][i] = stat(h, i);
+    };
+    f32x4 cs[2], cp[2];
+    auto first = [&](int h) __attribute__((always_inline)) {
+        cs[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        cp[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ds = 0; ds < G::DS; ds++) {
+            cs[h] = mfma16<BF>(qa[h][ds], kreg[ds], cs[h]);
+            cp[h] = mfma16<BF>(ga[h][ds], vreg[ds], cp[h]);
+        }
+    };
+    auto weights = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const ST &q = st[h][i];
+            const bool ok = in(h, i, q);
+            float x;
+            if constexpr (kBias) x = cs[h][i] * sc2 + lds_bias[ok ? at(h, i, q) : 0] - q.x;
+            else x = cs[h][i] * sc2 - q.x;
+            float p = exp_unit(ok ? x : -INFINITY);
+            if constexpr (kBias) p *= zinv_of(q);
+            put<BF>(pb, h * 4 + i, p);
+            if constexpr (kBias && !BF) {
+                dsv[h * 4 + i] = p * (cp[h][i] - q.y);
+                mag = fmaxf(mag, fabsf(dsv[h * 4 + i]));
+            } else {
+                put<BF>(dsb, h * 4 + i, p * (cp[h][i] - q.y));
+            }
+        }
+    };
+    typename G::TRow qt[2], gt[2];
+    auto turn_rows = [&](int h) __attribute__((always_inline)) {
+        const int row = t_of(h);
+        qt[h] = G::t_row(lds_q, row, n);
+        gt[h] = G::t_row(lds_g, row, n);
+    };
+    auto fence = [&]() __attribute__((always_inline)) {
+        if constexpr (AHEAD > 0) __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (AHEAD >= 2) {
+        read(0);
+        read(1);
+        fence();
+        first(0);
+        first(1);
+        turn_rows(0);
+        turn_rows(1);
+        fence();
+        weights(0);
+        weights(1);
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            read(h);
+            fence();
+            first(h);
+            turn_rows(h);
+            fence();
+            weights(h);
+        }
+    }
+    if constexpr (kBias) {  // (no registers for more rows than the next product needs)
+        if constexpr (!BF) put_scaled<BF>(dsb, dsv, mag, scl, dk);
+#pragma unroll
+        for (int mt = 0; mt < G::DT; mt++) {
+            dv[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(gt[0], mt)), lds_read_tr(G::t_at(gt[1], mt))), pb, dv[mt]);
+            dk[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(qt[0], mt)), lds_read_tr(G::t_at(qt[1], mt))), dsb, dk[mt]);
+        }
+    } else {
+        s16x8 gr[G::DT], qr[G::DT];
+#pragma unroll
+        for (int mt = 0; mt < G::DT; mt++) gr[mt] = cat(lds_read_tr(G::t_at(gt[0], mt)), lds_read_tr(G::t_at(gt[1], mt)));
+#pragma unroll
+        for (int mt = 0; mt < G::DT; mt++) qr[mt] = cat(lds_read_tr(G::t_at(qt[0], mt)), lds_read_tr(G::t_at(qt[1], mt)));
+#pragma unroll
+        for (int mt = 0; mt < G::DT; mt++) dv[mt] = mfma_op<BF>(gr[mt], pb, dv[mt]);
+#pragma unroll
+        for (int mt = 0; mt < G::DT; mt++) dk[mt] = mfma_op<BF>(qr[mt], dsb, dk[mt]);
+    }
+}
+
 // Inner tiles.  Every key is attended by exactly the queries within k//2 of it
 // and all windows are centred, so the picture is the forward's with the roles of
 // queries and keys exchanged: the staged block is the tile's (8+k-1)^2 halo of
@@ -1427,54 +1542,19 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
             dv[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
 #pragma unroll
-        for (int ks = K0; ks < K1; ks++) {
-            Op8 pb, dsb;
-            float dsv[8], mag = 0.f;  // (float16 with a bias)
-#pragma unroll
-            for (int m2 = 0; m2 < 2; m2++) {
-                const int mt = ks * 2 + m2;
-                const int row = row_of(mt, n);
-                const typename G::ARow qp = G::a_row(lds_q, row, g), gp = G::a_row(lds_g, row, g);
-                f32x4 cs = {0.f, 0.f, 0.f, 0.f}, cp = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int ds = 0; ds < G::DS; ds++) {
-                    cs = mfma16<BF>(*reinterpret_cast<const s16x8 *>(G::a_at(qp, ds)), kreg[ds], cs);
-                    cp = mfma16<BF>(*reinterpret_cast<const s16x8 *>(G::a_at(gp, ds)), vreg[ds], cp);
-                }
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const QStat st = lds_stat[row_of(mt, g * 4 + i)];  // query of accumulator row g*4+i
-                    const bool ok = G::template tok_in<KS>(mt, g * 4 + i, n >> 2, n & 3);
-                    float x;
-                    if constexpr (kBias) x = cs[i] * sc2 + lds_bias[ok ? bk - Bias<KS>::token(mt, g * 4 + i) : 0] - st.x;
-                    else x = cs[i] * sc2 - st.x;
-                    float p = exp_unit(ok ? x : -INFINITY);
-                    if constexpr (kBias) p *= zinv_of(st);
-                    put<BF>(pb, m2 * 4 + i, p);
-                    if constexpr (kBias && !BF) {
-                        dsv[m2 * 4 + i] = p * (cp[i] - st.y);
-                        mag = fmaxf(mag, fabsf(dsv[m2 * 4 + i]));
-                    } else {
-                        put<BF>(dsb, m2 * 4 + i, p * (cp[i] - st.y));
-                    }
-                }
-            }
-            if constexpr (kBias && !BF) put_scaled<BF>(dsb, dsv, mag, scl, dk);
-            typename G::TRow qt[2], gt[2];
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int row = row_of(ks * 2 + h, g * 4 + (n >> 2));
-                qt[h] = G::t_row(lds_q, row, n);
-                gt[h] = G::t_row(lds_g, row, n);
-            }
-#pragma unroll
-            for (int mt = 0; mt < G::DT; mt++) {
-                dv[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(gt[0], mt)), lds_read_tr(G::t_at(gt[1], mt))),
-                                    pb, dv[mt]);
-                dk[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(qt[0], mt)), lds_read_tr(G::t_at(qt[1], mt))),
-                                    dsb, dk[mt]);
-            }
-        }
+        for (int ks = K0; ks < K1; ks++)
+            dkdv_step<BF, G, kInnerAhead<D>>(
+                lds_q, lds_g, lds_bias, n, g, sc2, kreg, vreg, dk, dv, scl,
+                [&](int h) __attribute__((always_inline)) { return row_of(ks * 2 + h, n); },
+                [&](int h) __attribute__((always_inline)) { return row_of(ks * 2 + h, g * 4 + (n >> 2)); },
+                // query of accumulator row g*4+i
+                [&](int h, int i) __attribute__((always_inline)) { return lds_stat[row_of(ks * 2 + h, g * 4 + i)]; },
+                [&](int h, int i, const QStat &) __attribute__((always_inline)) {
+                    return bk - Bias<KS>::token(ks * 2 + h, g * 4 + i);
+                },
+                [&](int h, int i, const QStat &) __attribute__((always_inline)) {
+                    return G::template tok_in<KS>(ks * 2 + h, g * 4 + i, n >> 2, n & 3);
+                });
 
         if constexpr (kBias) unscale<BF>(dk, dv, scl);
         const int kr = cur.r0 + orow + (n >> 2), kc = cur.c0 + ocol + (n & 3);
@@ -1527,6 +1607,10 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
 // tile in the second ring from the border, up to 16 + k/2 rows and columns of them, are
 // one block instead of up to four.  `lds_red` then lies over the staged rows (RED_OVER):
 // the partial sums are exchanged when a tile's last block has been read by every wave.
+template <typename G>
+struct FrameStat {
+    static constexpr int PITCH = G::HC + 3, NONE = G::HR * PITCH, WORDS = NONE + 4;
+};
 template <bool BF, int D, int KS, int SP, int KSG, bool RED_OVER>
 __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, int ntiles,
                                            int block, int nblocks, short *lds_q, short *lds_g,
@@ -1555,6 +1639,14 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
     if (sc.t >= sc.t_end) return;
     zero_row<D, KSG, 4, SP>(lds_q, dlim);
     zero_row<D, KSG, 4, SP>(lds_g, dlim);
+    // The statistics' rows are STP apart: a run of four may reach up to three columns past the
+    // block, and a run past the end of the rectangle reads the four from STNO on.  The windows of
+    // those are nowhere, so no key is in them.
+    constexpr int STP = FrameStat<G>::PITCH, STNO = FrameStat<G>::NONE;
+    for (int id = threadIdx.x; id < G::HR * 3 + 4; id += G::NT)
+        lds_stat[id < G::HR * 3 ? id / 3 * STP + G::HC + id % 3 : STNO + id - G::HR * 3] =
+            kBias ? make_float4(0.f, 0.f, 0.f, __int_as_float(0xffff0000))
+                  : make_float4(0.f, 0.f, __int_as_float(0x7fff7fff), 0.f);
 
     // wave = block of 4x4 keys (0..3) + 4 * (its part of the block's queries)
     const int wave = (threadIdx.x >> 6) & 3, part = threadIdx.x >> 8;
@@ -1627,21 +1719,22 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
         for (int i = 0; i < G::NST; i++) {
             const int id = threadIdx.x + i * G::NT;
             // per staged query: lse * log2e, delta, and where its window starts (row in the low,
-            // column in the high half of a word), so that the mask of a logit is two
-            // differences; the padding row's window is nowhere
+            // column in the high half of a word), so that the mask of a logit is two differences
             const int r = min(cur.br + id / G::HC, cur.qb - 1), c = min(cur.bc + id % G::HC, cur.cb - 1);
-            const int ws = win_start(r, s.H, KS) | (win_start(c, s.W, KS) << 16);
+            // (columns past the tile's queries are copies of the last one: nowhere, like what lies past the block)
+            const bool none = cur.bc + id % G::HC >= cur.cb;
+            const int ws = none ? 0x7fff7fff : win_start(r, s.H, KS) | (win_start(c, s.W, KS) << 16);
+            const int to = id / G::HC * STP + id % G::HC;
             if constexpr (kBias) {
                 // (1 / Z too, and in the word of the window the query's place in a table with TB columns,
                 // all from the block's origin: a window starts at most 12 rows before it)
                 const int at = (id / G::HC) * Bias<KS>::TB + id % G::HC;
-                const unsigned w = (unsigned)at | (unsigned)((ws & 0xffff) - cur.br + 64) << 16 |
-                                   (unsigned)((ws >> 16) - cur.bc + 64) << 24;
-                if (id < G::ZROW) lds_stat[id] = make_float4(sst[i].x, sst[i].y, __uint_as_float(w), zinv_of(sst[i]));
-                else if (id == G::ZROW) lds_stat[id] = make_float4(0.f, 0.f, __uint_as_float(0xffff0000u), 0.f);
+                const unsigned w = none ? 0xffff0000u
+                                        : (unsigned)at | (unsigned)((ws & 0xffff) - cur.br + 64) << 16 |
+                                              (unsigned)((ws >> 16) - cur.bc + 64) << 24;
+                if (id < G::ZROW) lds_stat[to] = make_float4(sst[i].x, sst[i].y, zinv_of(sst[i]), __uint_as_float(w));
             } else {
-                if (id < G::ZROW) lds_stat[id] = make_float4(sst[i].x, sst[i].y, __int_as_float(ws), 0.f);
-                else if (id == G::ZROW) lds_stat[id] = make_float4(0.f, 0.f, __int_as_float(0x7fff7fff), 0.f);
+                if (id < G::ZROW) lds_stat[to] = make_float4(sst[i].x, sst[i].y, __int_as_float(ws), 0.f);
             }
         }
         if constexpr (kBias) bst.commit(lds_bias);
@@ -1676,69 +1769,45 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
             const int rb = min(inv_hi(min(wr0 + 4, s.H) - 1, s.H, KS), cur.br + G::HR);
             const int cc = max(inv_lo(wc0, KS), cur.bc);
             const int cd = min(inv_hi(min(wc0 + 4, s.W) - 1, s.W, KS), cur.bc + G::HC);
-            const int wcols = cd - cc;
-            const int nq = (rb > ra && cd > cc) ? (rb - ra) * wcols : 0;
-            // qi * magic >> 16 == qi / wcols for qi < 2048, wcols <= 32
-            const int magic = wcols > 0 ? (65536 + wcols - 1) / wcols : 0;
-            // staged row of query qi (zero row past the end), branch-free
-            auto row_of = [&](int qi) __attribute__((always_inline)) {
-                const int dvd = (qi * magic) >> 16;
-                const int row = (ra + dvd - cur.br) * G::HC + (cc + qi - dvd * wcols - cur.bc);
-                return qi < nq ? row : (int)G::ZROW;
+            // The rectangle is walked in runs of four queries side by side, `runs` of them per row,
+            // 8 runs per step: a run has one row, so its four statistics lie side by side in LDS
+            // and share the row of their windows, and one division serves all of it.
+            const int wcols = cd - cc, runs = (wcols + 3) >> 2;
+            const int nu = (rb > ra && cd > cc) ? (rb - ra) * runs : 0;
+            // u * magic >> 16 == u / runs for u < 2048, runs <= 8
+            const int magic = wcols > 0 ? (65536 + runs - 1) / runs : 0;
+            const int row0 = (ra - cur.br) * G::HC + cc - cur.bc, stat0 = (ra - cur.br) * STP + cc - cur.bc;
+            // staged row of query x of run u (the zero row past the end of the rectangle)
+            auto row_of = [&](int u, int x) __attribute__((always_inline)) {
+                const int r = (u * magic) >> 16, c = (u - r * runs) * 4 + x;
+                return ((u < nu) & (c < wcols)) ? row0 + r * G::HC + c : (int)G::ZROW;
             };
-            for (int q0 = part * 32; q0 < nq; q0 += 32 * SP) {
-                Op8 pb, dsb;
-                float dsv[8], mag = 0.f;  // (float16 with a bias)
-#pragma unroll
-                for (int m2 = 0; m2 < 2; m2++) {
-                    const int row = row_of(q0 + m2 * 16 + n);
-                    const typename G::ARow qp = G::a_row(lds_q, row, g), gp = G::a_row(lds_g, row, g);
-                    f32x4 cs = {0.f, 0.f, 0.f, 0.f}, cp = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int ds = 0; ds < G::DS; ds++) {
-                        cs = mfma16<BF>(*reinterpret_cast<const s16x8 *>(G::a_at(qp, ds)), kreg[ds], cs);
-                        cp = mfma16<BF>(*reinterpret_cast<const s16x8 *>(G::a_at(gp, ds)), vreg[ds], cp);
-                    }
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int qi = q0 + m2 * 16 + g * 4 + i;
-                        const float4 st = lds_stat[row_of(qi)];
-                        float x, p;
-                        if constexpr (kBias) {
-                            const unsigned w = __float_as_uint(st.z);
-                            const bool ok = ((unsigned)(kr - cur.br + 64) - (w >> 16 & 0xffu) < (unsigned)KS) &
-                                            ((unsigned)(kc - cur.bc + 64) - (w >> 24) < (unsigned)KS);
-                            x = cs[i] * sc2 + lds_bias[ok ? bk - (int)(w & 0xffffu) : 0] - st.x;
-                            p = exp_unit(ok ? x : -INFINITY) * st.w;
-                        } else {
-                            const int ws = __float_as_int(st.z);
-                            const bool ok = ((unsigned)(kr - (ws & 0xffff)) < (unsigned)KS) &
-                                            ((unsigned)(kc - (ws >> 16)) < (unsigned)KS);
-                            x = cs[i] * sc2 - st.x;
-                            p = exp_unit(ok ? x : -INFINITY);
-                        }
-                        put<BF>(pb, m2 * 4 + i, p);
-                        if constexpr (kBias && !BF) {
-                            dsv[m2 * 4 + i] = p * (cp[i] - st.y);
-                            mag = fmaxf(mag, fabsf(dsv[m2 * 4 + i]));
-                        } else {
-                            put<BF>(dsb, m2 * 4 + i, p * (cp[i] - st.y));
-                        }
-                    }
-                }
-                if constexpr (kBias && !BF) put_scaled<BF>(dsb, dsv, mag, scl, dk);
-                typename G::TRow qt[2], gt[2];
+            for (int u0 = part * 8; u0 < nu; u0 += 8 * SP) {
+                int at_run[2];
+                bool row_in[2];
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    const int row = row_of(q0 + h * 16 + g * 4 + (n >> 2));
-                    qt[h] = G::t_row(lds_q, row, n);
-                    gt[h] = G::t_row(lds_g, row, n);
+                    const int u = u0 + h * 4 + g, r = (u * magic) >> 16;
+                    at_run[h] = u < nu ? stat0 + r * STP + (u - r * runs) * 4 : (int)STNO;
                 }
-#pragma unroll
-                for (int mt = 0; mt < G::DT; mt++) {
-                    dv[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(gt[0], mt)), lds_read_tr(G::t_at(gt[1], mt))), pb, dv[mt]);
-                    dk[mt] = mfma_op<BF>(cat(lds_read_tr(G::t_at(qt[0], mt)), lds_read_tr(G::t_at(qt[1], mt))), dsb, dk[mt]);
-                }
+                dkdv_step<BF, G, kFrameAhead>(
+                    lds_q, lds_g, lds_bias, n, g, sc2, kreg, vreg, dk, dv, scl,
+                    [&](int h) __attribute__((always_inline)) { return row_of(u0 + h * 4 + (n >> 2), n & 3); },
+                    [&](int h) __attribute__((always_inline)) { return row_of(u0 + h * 4 + g, n >> 2); },
+                    [&](int h, int i) __attribute__((always_inline)) { return lds_stat[at_run[h] + i]; },
+                    [&](int, int, const float4 &st) __attribute__((always_inline)) {
+                        return bk - (int)(__float_as_uint(st.w) & 0xffffu);
+                    },
+                    [&](int h, int i, const float4 &st) __attribute__((always_inline)) {
+                        const unsigned w = __float_as_uint(kBias ? st.w : st.z);
+                        if constexpr (kBias) {
+                            if (i == 0) row_in[h] = (unsigned)(kr - cur.br + 64) - (w >> 16 & 0xffu) < (unsigned)KS;
+                            return row_in[h] & ((unsigned)(kc - cur.bc + 64) - (w >> 24) < (unsigned)KS);
+                        } else {
+                            if (i == 0) row_in[h] = (unsigned)(kr - (int)(w & 0xffffu)) < (unsigned)KS;
+                            return row_in[h] & ((unsigned)(kc - ((int)w >> 16)) < (unsigned)KS);
+                        }
+                    });
             }
         }
 
@@ -1801,7 +1870,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
 // three workgroups per CU (head_dim <= 64 with small halos; it fits 168 registers there,
 // measured 35 -> 32 us at B8 N2 112x112 d32 k7 and 67 -> 60 us at B4 N4 128x128 d32 k9;
 // the forward and the dQ pass spill under that budget and get slower; with a bias so does this
-// one at head_dim 64: B8 N8 64x64 k5 60 us with two waves, 84 with three).
+// one: B8 N8 64x64 d64 k5 60 us with two waves, 84 with three, B8 N4 56x56 d32 k7 28.2 and 33.9).
 // Size of the frame body's blocks as a kernel size (see dkdv_frame): larger than KS where the
 // pass has one workgroup per CU anyway (two parts per block) and LDS has the room.
 // Where not even one workgroup's Q and dO halos fit LDS (head_dim 128 with kernel_size 11 and
@@ -1814,7 +1883,7 @@ constexpr int kFrameKS = kDkdvFrameOnly<D, KS> ? 5 : SP == 2 && KS >= 9 ? 9 + KS
 template <int D, int KS, int SP>
 constexpr int kDkdvWaves =
     kDkdvFrameOnly<D, KS> ? 2 :
-    SP == 1 && D <= (kBias ? 32 : 64) && 3 * (Geo<D, KS>::LDS_BYTES + 2048) <= 160 * 1024 ? 3 : Geo<D, KS, 4, SP>::WAVES;
+    SP == 1 && !kBias && D <= 64 && 3 * (Geo<D, KS>::LDS_BYTES + 2048) <= 160 * 1024 ? 3 : Geo<D, KS, 4, SP>::WAVES;
 template <bool BF, int D, int KS, bool ROLL, int SP = 1>
 __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) void bwd_dkdv_mfma(
     BArgs a, TileSet ts, int n_inner, int n_frame, int inner_blocks, Runs rp, int dyn) {
@@ -1830,7 +1899,7 @@ __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) v
     constexpr size_t I_ROWS = FRAME_ONLY ? 0 : (size_t)G::ROWS * G::PITCH * sizeof(short);
     constexpr size_t F_ROWS = (size_t)FG::ROWS * FG::PITCH * sizeof(short);
     constexpr size_t I_STAT = FRAME_ONLY ? 0 : (G::ROWS * sizeof(QStat) + 15) / 16 * 16;
-    constexpr size_t F_STAT = FG::ROWS * sizeof(float4);
+    constexpr size_t F_STAT = FrameStat<FG>::WORDS * sizeof(float4);
     constexpr size_t I_ALL = 2 * I_ROWS + I_STAT + RED;
     constexpr size_t F_ALL = 2 * F_ROWS + F_STAT + (RED_OVER ? 0 : RED);
     static_assert(RED <= F_ROWS || !RED_OVER, "the partial sums lie over the staged Q rows");
