@@ -88,6 +88,15 @@ int make_view(const char *fn, const char *name, const void *p, const int64_t *st
 bool use_mfma(int D, int ks, int dtype) {
     return g_path.load() != ENATTEN_PATH_SIMT && mfma_supported(D, ks, dtype);
 }
+// Head dims between 32 and 64 with kernel_size 11 and 13: the kernels for a relative position bias,
+// with a table of zeros where there is none (two terms for P and dS, 1 / Z, values that are not finite
+// stay in their windows: as close to float64 as the general kernels).  bf16, forward and backward, us, general
+// -> these: B1 N16 162x174 d48 k11 4200 -> 923, B2 N8 128x128 d48 k13 3160 -> 449,
+// B1 N2 32x32 d48 k13 401 -> 43.
+bool use_two_terms(int D, int ks, int dtype) {
+    return g_path.load() != ENATTEN_PATH_SIMT && (dtype == ENATTEN_BF16 || dtype == ENATTEN_F16) && D > 32 && D < 64 &&
+           D % 8 == 0 && (ks == 11 || ks == 13);
+}
 bool use_mfma_f32(int D, int ks, int dtype) {
     return g_path.load() != ENATTEN_PATH_SIMT && mfma_f32_supported(D, ks, dtype);
 }
@@ -149,6 +158,7 @@ int run_fwd(const FwdArgs &a, int dtype, hipStream_t st) {
         return launch_fwd_mfma(a, dtype, st);
     }
     if (use_mfma_f32(D, ks, dtype)) return launch_fwd_mfma_f32(a, st);
+    if (use_two_terms(D, ks, dtype)) return launch_fwd_mfma_bias(a, dtype, st);
     return launch_fwd_simt(a, dtype, st);
 }
 int run_bwd(const char *fn, const BwdArgs &a, int dtype, size_t ws_floats, hipStream_t st) {
@@ -165,6 +175,7 @@ int run_bwd(const char *fn, const BwdArgs &a, int dtype, size_t ws_floats, hipSt
     if (use_mfma_f32(D, ks, dtype) && a.grads_contiguous() &&
         ws_floats >= (size_t)a.s.B * a.s.N * a.s.H * a.s.W * mfma_f32_workspace_floats(ks))
         return launch_bwd_mfma_f32(a, st);
+    if (use_two_terms(D, ks, dtype)) return launch_bwd_mfma_bias(a, dtype, st);
     return launch_bwd_simt(a, dtype, st);
 }
 
@@ -588,7 +599,7 @@ int enatten2d_fwd_window(const void *q, const void *k, const void *v, const void
     a.rpb = rpb;
     if (dtype == ENATTEN_F64) return launch_fwd_f64(a, static_cast<hipStream_t>(stream));
     if (use_band(a, dtype)) return launch_fwd_band(a, dtype, static_cast<hipStream_t>(stream));
-    if (rpb && kernel_h == kernel_w && use_mfma(D, kernel_h, dtype))
+    if (rpb && kernel_h == kernel_w && (use_mfma(D, kernel_h, dtype) || use_two_terms(D, kernel_h, dtype)))
         return launch_fwd_mfma_bias(a, dtype, static_cast<hipStream_t>(stream));
     return launch_fwd_simt(a, dtype, static_cast<hipStream_t>(stream));
 }
@@ -652,7 +663,7 @@ int enatten2d_bwd_window(const void *q, const void *k, const void *v, const void
     a.ds_pairs = rpb ? a.delta + (size_t)4 * B * heads * H * W : nullptr;
     if (dtype == ENATTEN_F64) return bwd_f64(fn, a, ws_floats, static_cast<hipStream_t>(stream));
     if (use_band(a, dtype)) return launch_bwd_band(a, dtype, static_cast<hipStream_t>(stream));
-    if (rpb && kernel_h == kernel_w && use_mfma(D, kernel_h, dtype))
+    if (rpb && kernel_h == kernel_w && (use_mfma(D, kernel_h, dtype) || use_two_terms(D, kernel_h, dtype)))
         return launch_bwd_mfma_bias(a, dtype, static_cast<hipStream_t>(stream));
     return launch_bwd_simt(a, dtype, static_cast<hipStream_t>(stream));
 }

@@ -23,7 +23,7 @@ bool mfma_supported(int D, int ks, int dtype) {
     if (ks < 3 || ks > 13 || ks % 2 == 0) return false;
     const int DB = built_dim(D);
     // (head dims below 64 with kernel_size 11 and 13: the dK/dV pass of those lays its partial
-    // sums over the staged rows, zeroed channels included)
+    // sums over the staged rows, zeroed channels included; use_two_terms in enatten_capi.hip)
     if (D != DB && DB == 64 && ks >= 11) return false;
     return fits_rt(DB, ks);
 }

@@ -149,10 +149,11 @@ __device__ __forceinline__ float lse_of(float mx, float sum) {
     else return (mx + __builtin_amdgcn_logf(sum)) * kLn2;
 }
 // With a bias the backward is renormalised as in the general kernels: 1 / sum p of the recomputed
-// probabilities per query, left by the dQ pass behind the block that holds its counter (a.zinv).
+// probabilities per query, left by the dQ pass behind the block that holds its counter (a.zinv);
+// without a bias table there is no counter, and the block itself has them.
 template <typename ARGS>
 __device__ __forceinline__ float *row_zinv(const ARGS &a) {
-    return a.zinv + (int64_t)a.s.B * a.s.N * a.s.H * a.s.W;
+    return a.zinv + (a.rpb ? (int64_t)a.s.B * a.s.N * a.s.H * a.s.W : 0);
 }
 // (P in the float16 dK/dV pass, which 1 / Z brings along, as in na1d_band_mfma.hip: see DsScale)
 template <bool BF>
@@ -251,6 +252,11 @@ struct BiasRegs {
     short v[NB];
     __device__ __forceinline__ void fetch(const void *rpb, int head) {
         const short *p = static_cast<const short *>(rpb) + (int64_t)head * T::E;
+        if (!rpb) {  // no bias: a table of zeros
+#pragma unroll
+            for (int i = 0; i < NB; i++) v[i] = 0;
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < NB; i++) v[i] = p[min((int)threadIdx.x + i * NT, T::E - 1)];
     }
@@ -408,7 +414,7 @@ __device__ __forceinline__ void walk_window(const Shape &s, const void *rpb, int
     const int r0 = win_start(qr, s.H, KS), c0 = win_start(qc, s.W, KS);
     const short *b = static_cast<const short *>(rpb) + ((int64_t)head * SPAN + r0 - qr + KS - 1) * SPAN + c0 - qc + KS - 1;
     for (int i = 0; i < KS * KS; i++)
-        if (!f(r0 + i / KS, c0 + i % KS, cvt32<BF>(b[i / KS * SPAN + i % KS]))) return;
+        if (!f(r0 + i / KS, c0 + i % KS, rpb ? cvt32<BF>(b[i / KS * SPAN + i % KS]) : 0.f)) return;
 }
 template <typename ARGS>
 __device__ __forceinline__ const short *pixel(const ARGS &a, const View &v, const ATile &tl, int r, int c) {
@@ -498,8 +504,8 @@ __device__ __forceinline__ void again_keys(const BArgs &a, const ATile &tl, int 
                     (unsigned)(kc - win_start(c, s.W, KS)) >= (unsigned)KS)
                     continue;
                 const int64_t tok = image_token(a, tl) + (int64_t)r * s.W + c;
-                const float bias = cvt32<BF>(
-                    static_cast<const short *>(a.rpb)[((int64_t)tl.nn * SPAN + kr - r + KS - 1) * SPAN + kc - c + KS - 1]);
+                const int64_t at = ((int64_t)tl.nn * SPAN + kr - r + KS - 1) * SPAN + kc - c + KS - 1;
+                const float bias = a.rpb ? cvt32<BF>(static_cast<const short *>(a.rpb)[at]) : 0.f;
                 const Chan2 q = chan_load<BF>(pixel(a, a.q, tl, r, c), dlim), go = chan_load<BF>(pixel(a, a.d_o, tl, r, c), dlim);
                 const float p = exp_unit(chan_dot(q, k) * s.scale + bias - a.lse[tok]) * row_zinv(a)[tok];
                 chan_add(av, p, go);
@@ -861,7 +867,7 @@ constexpr int kDqWaves = D == 32 && (KS == 7 || KS == 9) && NW == 4 && !kBias ? 
 template <bool BF, int D, int KS, bool FRAME, bool ROLL, int NW = 4, bool FULL = false>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void bwd_dq_mfma(BArgs a, TileSet ts, int ntiles, Runs rp) {
     // (the dK/dV pass that follows on the stream counts its frame tiles here, from zero)
-    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv) *reinterpret_cast<int *>(a.zinv) = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv && (!kBias || a.rpb)) *reinterpret_cast<int *>(a.zinv) = 0;
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_k[G::ROWS * G::PITCH];
     __shared__ __attribute__((aligned(16))) short lds_v[G::ROWS * G::PITCH];
@@ -1017,7 +1023,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             DsScale<BF> scl;
             if constexpr (kBias) {
                 operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live && delta * 0.f == 0.f ? zinv : 0.f);
-                BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
+                if (a.d_rpb) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
             }
             f32x4 dq[G::DT];
 #pragma unroll
@@ -1047,7 +1053,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                 if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
             }
         }
-        if constexpr (kBias) {
+        if (kBias && a.d_rpb) {
             __syncthreads();
             BiasGrad<KS>::template flush<NW>(lds_dbias, a.ds_pairs + (int64_t)sc.t * Bias<KS>::E, cur, s);
         }
@@ -1085,7 +1091,7 @@ constexpr int kDq2Tail = D == 128 && NW == 8 ? (KS == 13 ? 15 : KS == 11 ? 13 : 
 template <bool BF, int D, int KS, int NW = 4, bool FULL = false>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS> : 1)) void bwd_dq2_mfma(BArgs a, TileSet ts, int ntiles) {
     // (the dK/dV pass that follows on the stream counts its frame tiles here, from zero)
-    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv) *reinterpret_cast<int *>(a.zinv) = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv && (!kBias || a.rpb)) *reinterpret_cast<int *>(a.zinv) = 0;
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_x[G::ROWS * G::PITCH];
     __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
@@ -1215,7 +1221,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
             DsScale<BF> scl;
             if constexpr (kBias) {
                 operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live && delta * 0.f == 0.f ? zinv : 0.f);
-                BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
+                if (a.d_rpb) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
             }
             f32x4 dq[G::DT];
 #pragma unroll
@@ -1244,7 +1250,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                 if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
             }
         }
-        if constexpr (kBias) {
+        if (kBias && a.d_rpb) {
             __syncthreads();
             BiasGrad<KS>::template flush<NW>(lds_dbias, a.ds_pairs + (int64_t)sc.t * Bias<KS>::E, cur, s);
         }
@@ -1855,6 +1861,8 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
             }
             if (!more) break;
             if (RED_OVER && cur.last) __syncthreads();  // the sums are read: the next block may land
+            // (the channels that the tensors do not have are zero again in the rows the sums lay over)
+            if (kNarrow && RED_OVER && cur.last && dlim < D) zero_row<D, KSG, 4, SP>(lds_q, dlim);
         }
         if (nxt.first) t_next = dyn ? lds_tile[0] : nxt.t + sc.step;  // the tile after the next one
         cur = nxt;
@@ -2258,7 +2266,7 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                 // staircase leaves the static split 7% or more behind (B4 N4 128x128 k7: 154.6 ->
                 // 135.4 us; measured 4-9% slower at k9 and at 256x256 and 96x96 k7, where it is
                 // not taken).
-                if (a.zinv != nullptr) {
+                if (a.zinv != nullptr && (!kBias || a.rpb)) {
                     int all = grid;
                     if (all > per_i * 8) all = (int)(per_i * 8);
                     double walk;
@@ -2281,7 +2289,7 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                 if (inner_blocks > grid - 8) inner_blocks = grid - 8;
                 if (inner_blocks > (n_inner + 7) / 8 * 8) inner_blocks = (int)((n_inner + 7) / 8 * 8);
             }
-            if (path == ENATTEN_PATH_MFMA_SPLIT_QUEUE && a.zinv != nullptr && n_frame > 0 && !dyn) {
+            if (path == ENATTEN_PATH_MFMA_SPLIT_QUEUE && a.zinv != nullptr && (!kBias || a.rpb) && n_frame > 0 && !dyn) {
                 dyn = 1;
                 const int64_t all = (n_inner + 7) / 8 * 8;
                 inner_blocks = all < grid ? (int)all : grid;
@@ -2295,7 +2303,7 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                 hipLaunchKernelGGL((bwd_dkdv_mfma<BF, D, KS, false, SP>), dim3(grid), dim3(NT), 0, st,
                                    a, ts, (int)n_inner, (int)n_frame, inner_blocks, Runs{0, 0}, dyn);
         }
-        if constexpr (kBias)
+        if (kBias && a.d_rpb)
             hipLaunchKernelGGL((rpb_tile_reduce<kBias>), dim3(a.s.N, (Bias<KS>::E + 15) / 16), dim3(1024), 0, st,
                                a.ds_pairs, a.d_rpb, a.s.B, a.s.N, dq_tiles, Bias<KS>::E);
         return check_launch("enatten2d_bwd");

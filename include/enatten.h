@@ -54,7 +54,9 @@ const char *enatten_last_error(void);
 /*
  * Kernel family that would serve (D, kernel_size, dtype): ENATTEN_PATH_MFMA for
  * the matrix-core kernels, ENATTEN_PATH_SIMT for the general fp32-FMA kernels,
- * ENATTEN_PATH_NONE if the call would be rejected.
+ * ENATTEN_PATH_NONE if the call would be rejected.  (bf16 and fp16 head dims between 32 and
+ * 64 with kernel_size 11 or 13 answer ENATTEN_PATH_SIMT: the matrix-core kernels that serve
+ * them are those with the general kernels' precision.)
  */
 int enatten2d_kernel_path(int D, int kernel_size, int dtype);
 
