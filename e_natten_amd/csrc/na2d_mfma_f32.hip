@@ -549,6 +549,10 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x, c
     using G = Geo32<D, KS>;
     constexpr int NRG = (G::SW + KS / 2 + 3) / 4;   // groups of 4 query rows a wave can meet in a block
     constexpr int NC = G::SW + KS / 2;              // query columns likewise
+    // ... but where both ends of an axis clamp the windows of one wave's keys, which a row of 11 or 12
+    // pixels at kernel_size 5 and of 14 at 7 has: there the blocks are NC columns wide
+    constexpr int BOTH = (KS - 1) / 4 * 4 + 3 + KS;
+    static_assert(BOTH <= 4 * NRG, "rows of such a wave");
     __shared__ __attribute__((aligned(16))) float lds[G::ROWS * G::PITCH];
     const int t = tile_of_block(ntiles);
     if (t < 0) return;
@@ -571,12 +575,13 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x, c
 #pragma unroll
     for (int m = 0; m < G::DT; m++) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
     Regs32 st;
+    const int cols = s.W > NC && s.W <= BOTH ? NC : G::HC;
     for (int br = qa; br < qb; br += G::HR) {
-        for (int bc = ca; bc < cb; bc += G::HC) {
+        for (int bc = ca; bc < cb; bc += cols) {
             fetch32<D, KS>(st, ximg, x.sh, x.sw, br, bc, qb, cb);
             // this wave's queries inside the block
             const int ra = max(wqa, br), rb = min(wqb, br + G::HR);
-            const int cc = max(wca, bc), cd = min(wcb, bc + G::HC);
+            const int cc = max(wca, bc), cd = min(wcb, bc + cols);
             // weights of the block's reduction steps: query (ra + 4 rg + g, cc + c), this
             // lane's key; zero if the query is outside the wave's part or does not attend
             float w[NRG * NC];
