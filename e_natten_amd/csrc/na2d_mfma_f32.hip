@@ -83,6 +83,18 @@ struct Geo32 {
 template <int D, int KS>
 constexpr bool kLines32 = 2 * Geo32<D, KS>::LDS_BYTES <= 160 * 1024;
 
+// dV and dK in one launch where the staged rows of both dO and Q admit two workgroups per CU
+// (head_dim 32, and 64 up to kernel_size 5): the places and bounds of the weights are formed once, a
+// weight pair is one 8-byte load, and what a workgroup waits for (rows, weights, two barriers) it
+// waits for once.  P and dS of a window position then lie side by side in the workspace, which makes
+// the dQ pass's scattered stores half as many as well.  Backward, us, two launches -> one: B8 N7 46x46 d32 k7
+// 174 -> 142 (dK/dV 105 -> 77), B2 N8 128x128 d64 k5 258 -> 234, k3 178 -> 164, d32 k3 99 -> 90.  At head_dim 128
+// the same with 64 channels to a workgroup was level at k5 (dQ pass 256 -> 248, dK/dV 210 -> 219).
+template <int D, int KS>
+constexpr bool kPair32 = 4 * (Geo32<D, KS>::LDS_BYTES + 16) <= 160 * 1024;
+// (the caller's workspace is aligned to its floats)
+typedef float f32x2 __attribute__((ext_vector_type(2), aligned(4)));
+
 struct Regs32 {
     // the largest halo served: kernel_size 7 at head_dim 128 is 196 pixels x 32 chunks
     u32x4 v[25];
@@ -501,7 +513,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_mfma_f32(BwdArgs a, float *ws_p
                         dpart = fmaf(ds[mt][e], dp[mt][e], dpart);
                     }
                 const float delta = col_sum(dpart);
-                float *pp = ws_p + lq.tok * G::KK, *dsp = ws_ds + lq.tok * G::KK;
+                float *pp = ws_p + lq.tok * G::KK * (kPair32<D, KS> ? 2 : 1), *dsp = ws_ds + lq.tok * G::KK;
 #pragma unroll
                 for (int mt = 0; mt < G::MT; mt++)
 #pragma unroll
@@ -512,8 +524,12 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_mfma_f32(BwdArgs a, float *ws_p
                         ds[mt][e] = pv * (dp[mt][e] - delta);    // dS
                         if (ok && lq.live) {
                             const int j = (r - lq.dr) * KS + (c - lq.dc);
-                            pp[j] = pv;
-                            dsp[j] = ds[mt][e];
+                            if constexpr (kPair32<D, KS>) {
+                                *reinterpret_cast<f32x2 *>(pp + 2 * j) = f32x2{pv, ds[mt][e]};
+                            } else {
+                                pp[j] = pv;
+                                dsp[j] = ds[mt][e];
+                            }
                         }
                     }
             }
@@ -543,9 +559,9 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_mfma_f32(BwdArgs a, float *ws_p
 // disjoint banks.  The weights W (P for dV, dS for dK) come from the workspace; a query
 // that does not attend to a key contributes an exact zero.
 template <int D, int KS>
-__global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x, const float *ws_w,
-                                                            float *out, float mul, int tiles_r,
-                                                            int tiles_c, int ntiles) {
+__global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, View x1, const float *ws_w,
+                                                            float *out0, float *out1, float mul0, float mul1,
+                                                            int tiles_r, int tiles_c, int ntiles) {
     using G = Geo32<D, KS>;
     constexpr int NRG = (G::SW + KS / 2 + 3) / 4;   // groups of 4 query rows a wave can meet in a block
     constexpr int NC = G::SW + KS / 2;              // query columns likewise
@@ -553,7 +569,8 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x, c
     // pixels at kernel_size 5 and of 14 at 7 has: there the blocks are NC columns wide
     constexpr int BOTH = (KS - 1) / 4 * 4 + 3 + KS;
     static_assert(BOTH <= 4 * NRG, "rows of such a wave");
-    __shared__ __attribute__((aligned(16))) float lds[G::ROWS * G::PITCH];
+    constexpr int NB = kPair32<D, KS> ? 2 : 1;      // results of this launch (one: x0 and out0)
+    __shared__ __attribute__((aligned(16))) float lds[NB][G::ROWS * G::PITCH];
     const int t = tile_of_block(ntiles);
     if (t < 0) return;
     const Shape &s = a.s;
@@ -568,23 +585,25 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x, c
     const int ca = inv_lo(tl.c0, KS), cb = inv_hi(min(tl.c0 + 8, s.W) - 1, s.W, KS);
     const int wqa = inv_lo(min(wr0, s.H - 1), KS), wqb = inv_hi(min(wr0 + 4, s.H) - 1, s.H, KS);
     const int wca = inv_lo(min(wc0, s.W - 1), KS), wcb = inv_hi(min(wc0 + 4, s.W) - 1, s.W, KS);
-    const float *ximg = image32(x, tl);
     const int64_t img_tok = ((int64_t)tl.bb * s.N + tl.nn) * s.H * (int64_t)s.W;
 
-    f32x4 acc[G::DT];
+    f32x4 acc[NB][G::DT];
 #pragma unroll
-    for (int m = 0; m < G::DT; m++) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    Regs32 st;
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int m = 0; m < G::DT; m++) acc[b][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Regs32 st[NB];
     const int cols = s.W > NC && s.W <= BOTH ? NC : G::HC;
     for (int br = qa; br < qb; br += G::HR) {
         for (int bc = ca; bc < cb; bc += cols) {
-            fetch32<D, KS>(st, ximg, x.sh, x.sw, br, bc, qb, cb);
+            fetch32<D, KS>(st[0], image32(x0, tl), x0.sh, x0.sw, br, bc, qb, cb);
+            if constexpr (NB == 2) fetch32<D, KS>(st[1], image32(x1, tl), x1.sh, x1.sw, br, bc, qb, cb);
             // this wave's queries inside the block
             const int ra = max(wqa, br), rb = min(wqb, br + G::HR);
             const int cc = max(wca, bc), cd = min(wcb, bc + cols);
             // weights of the block's reduction steps: query (ra + 4 rg + g, cc + c), this
             // lane's key; zero if the query is outside the wave's part or does not attend
-            float w[NRG * NC];
+            float w[NB][NRG * NC];
 #pragma unroll
             for (int rg = 0; rg < NRG; rg++)
 #pragma unroll
@@ -594,23 +613,34 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x, c
                     const int pc = kc - win_start(min(qc, s.W - 1), s.W, KS);
                     const bool ok = wave_on && qr < rb && qc < cd && (unsigned)pr < (unsigned)KS &&
                                     (unsigned)pc < (unsigned)KS;
-                    w[rg * NC + c] = ok ? ws_w[(img_tok + (int64_t)qr * s.W + qc) * G::KK + pr * KS + pc] : 0.f;
+                    const float *wp = ws_w + ((img_tok + (int64_t)qr * s.W + qc) * G::KK + pr * KS + pc) * NB;
+                    if constexpr (NB == 2) {
+                        const f32x2 pair = ok ? *reinterpret_cast<const f32x2 *>(wp) : f32x2{0.f, 0.f};
+                        w[0][rg * NC + c] = pair[0];
+                        w[1][rg * NC + c] = pair[1];
+                    } else {
+                        w[0][rg * NC + c] = ok ? *wp : 0.f;
+                    }
                 }
             __syncthreads();  // the previous block's rows are no longer read
-            commit32<D, KS>(lds, st);
+#pragma unroll
+            for (int b = 0; b < NB; b++) commit32<D, KS>(lds[b], st[b]);
             __syncthreads();
             if (wave_on) {
                 // A step's DT operands are read from LDS a step ahead of the matrix
                 // instructions that use them.
-                float x[2][G::DT];
-                auto fetch = [&](int rg, int c, float *dst) __attribute__((always_inline)) {
+                float x[2][NB][G::DT];
+                auto fetch = [&](int rg, int c, float (&dst)[NB][G::DT]) __attribute__((always_inline)) {
                     // LDS row of this lane group's query row in the block (clamped: the
                     // weight of a row or column past the end is zero)
                     const int lrow = min(min(ra + 4 * rg + g, qb - 1) - br, G::HR - 1);
                     const int lcol = min(cc + c - bc, G::HC - 1);
-                    const float *xp = lds + (lrow * G::HC + lcol) * G::PITCH + n;
 #pragma unroll
-                    for (int m = 0; m < G::DT; m++) dst[m] = xp[16 * m];
+                    for (int b = 0; b < NB; b++) {
+                        const float *xp = lds[b] + (lrow * G::HC + lcol) * G::PITCH + n;
+#pragma unroll
+                        for (int m = 0; m < G::DT; m++) dst[b][m] = xp[16 * m];
+                    }
                 };
                 fetch(0, 0, x[0]);
 #pragma unroll
@@ -626,9 +656,11 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x, c
                         __builtin_amdgcn_sched_barrier(0);
                         if (cc + c < cd) {
 #pragma unroll
-                            for (int m = 0; m < G::DT; m++)
-                                acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[step & 1][m], w[step],
-                                                                              acc[m], 0, 0, 0);
+                            for (int b = 0; b < NB; b++)
+#pragma unroll
+                                for (int m = 0; m < G::DT; m++)
+                                    acc[b][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[step & 1][b][m], w[b][step],
+                                                                                     acc[b][m], 0, 0, 0);
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     }
@@ -638,7 +670,8 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x, c
     }
     if (!wave_on) return;
     const int64_t tok = img_tok + (int64_t)kr * s.W + kc;
-    store32<D, kLines32<D, KS>>(out + tok * D, g, acc, mul, live);
+    store32<D, kLines32<D, KS>>(out0 + tok * D, g, acc[0], mul0, live);
+    if constexpr (NB == 2) store32<D, kLines32<D, KS>>(out1 + tok * D, g, acc[1], mul1, live);
 }
 
 // ------------------------------------------------------------------ dispatch
@@ -667,12 +700,14 @@ int bwd32_launch(const BwdArgs &a, hipStream_t st) {
                            dim3(256), 0, st, a, ws_p, ws_ds, tiles_r, tiles_c, (int)nt);
     }
     {
-        // dV = P^T dO, then dK = dS^T Q: the same kernel on the other pair of operands
+        // dV = P^T dO and dK = dS^T Q: in one launch, or one after the other
         ProfScope prof(ENATTEN_KERNEL_BWD_DKDV, "bwd_dkdv_mfma_f32", st);
-        hipLaunchKernelGGL((bwd_dkdv_mfma_f32<D, KS>), dim3(grid), dim3(256), 0, st, a, a.d_o, ws_p,
-                           static_cast<float *>(a.dv), 1.f, tiles_r, tiles_c, (int)nt);
-        hipLaunchKernelGGL((bwd_dkdv_mfma_f32<D, KS>), dim3(grid), dim3(256), 0, st, a, a.q, ws_ds,
-                           static_cast<float *>(a.dk), a.s.scale, tiles_r, tiles_c, (int)nt);
+        float *dv = static_cast<float *>(a.dv), *dk = static_cast<float *>(a.dk);
+        hipLaunchKernelGGL((bwd_dkdv_mfma_f32<D, KS>), dim3(grid), dim3(256), 0, st, a, a.d_o, a.q, ws_p, dv, dk, 1.f,
+                           a.s.scale, tiles_r, tiles_c, (int)nt);
+        if (!kPair32<D, KS>)
+            hipLaunchKernelGGL((bwd_dkdv_mfma_f32<D, KS>), dim3(grid), dim3(256), 0, st, a, a.q, a.q, ws_ds, dk, dk,
+                               a.s.scale, 1.f, tiles_r, tiles_c, (int)nt);
     }
     return check_launch("enatten2d_bwd");
 }
