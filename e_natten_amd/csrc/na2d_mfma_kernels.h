@@ -1302,7 +1302,8 @@ __device__ __forceinline__ bool next_block(KeyBlock &b) {
 
 
 // One step of the dK/dV pass: 32 queries (two 16-token tiles) against the wave's 16 keys.
-// AHEAD says how the reads are ordered, with scheduling barriers: 0 as the compiler likes, 1 all
+// AHEAD says how the reads are ordered, with scheduling barriers: -1 and 0 as the compiler likes (-1: each in
+// the place where it is needed, for the bias, whose inner body has no registers to spare), 1 all
 // operands and statistics of a tile before its matrix instructions, 2 those of both tiles.  Left
 // alone in the frame body's rolled loop the compiler reads the statistics of one query after the
 // other, each behind a wait of its own for LDS, 16 round trips in a row per step at 2 waves per
@@ -1313,7 +1314,7 @@ __device__ __forceinline__ bool next_block(KeyBlock &b) {
 //   stat(h, i), at(h, i, st), in(h, i, st): statistics of query 4 g + i of tile h, the place of its
 //   bias in the table, and whether it attends to this lane's key
 template <int D>
-constexpr int kInnerAhead = D == 32 && !kBias ? 2 : 0;
+constexpr int kInnerAhead = kBias ? -1 : D == 32 ? 2 : 0;
 constexpr int kFrameAhead = 1;
 template <bool BF, typename G, int AHEAD, typename AROW, typename TROW, typename STAT, typename AT, typename IN>
 __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g, const float *lds_bias, int n, int g,
@@ -1321,6 +1322,7 @@ __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g
                                           f32x4 (&dk)[G::DT], f32x4 (&dv)[G::DT], DsScale<BF> &scl, AROW a_of,
                                           TROW t_of, STAT stat, AT at, IN in) {
     using ST = decltype(stat(0, 0));
+    constexpr bool LAZY = AHEAD < 0;  // (four floats a query: no registers to hold eight of them)
     Op8 pb, dsb;
     float dsv[8], mag = 0.f;  // (float16 with a bias)
     s16x8 qa[2][G::DS], ga[2][G::DS];
@@ -1334,7 +1336,7 @@ __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g
             ga[h][ds] = *reinterpret_cast<const s16x8 *>(G::a_at(gp, ds));
         }
 #pragma unroll
-        for (int i = 0; i < 4; i++) st[h][i] = stat(h, i);
+        for (int i = 0; i < 4 && !LAZY; i++) st[h][i] = stat(h, i);
     };
     f32x4 cs[2], cp[2];
     auto first = [&](int h) __attribute__((always_inline)) {
@@ -1349,7 +1351,7 @@ __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g
     auto weights = [&](int h) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const ST &q = st[h][i];
+            const ST q = LAZY ? stat(h, i) : st[h][i];
             const bool ok = in(h, i, q);
             float x;
             if constexpr (kBias) x = cs[h][i] * sc2 + lds_bias[ok ? at(h, i, q) : 0] - q.x;
@@ -1385,6 +1387,22 @@ __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g
         fence();
         weights(0);
         weights(1);
+    } else if constexpr (AHEAD < 0) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int row = a_of(h);
+            const typename G::ARow qp = G::a_row(lds_q, row, g), gp = G::a_row(lds_g, row, g);
+            cs[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+            cp[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ds = 0; ds < G::DS; ds++) {
+                cs[h] = mfma16<BF>(*reinterpret_cast<const s16x8 *>(G::a_at(qp, ds)), kreg[ds], cs[h]);
+                cp[h] = mfma16<BF>(*reinterpret_cast<const s16x8 *>(G::a_at(gp, ds)), vreg[ds], cp[h]);
+            }
+            weights(h);
+        }
+        turn_rows(0);
+        turn_rows(1);
     } else {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -1648,9 +1666,9 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
     // The statistics' rows are STP apart: a run of four may reach up to three columns past the
     // block, and a run past the end of the rectangle reads the four from STNO on.  The windows of
     // those are nowhere, so no key is in them.
-    constexpr int STP = FrameStat<G>::PITCH, STNO = FrameStat<G>::NONE;
-    for (int id = threadIdx.x; id < G::HR * 3 + 4; id += G::NT)
-        lds_stat[id < G::HR * 3 ? id / 3 * STP + G::HC + id % 3 : STNO + id - G::HR * 3] =
+    constexpr int STP = FrameStat<G>::PITCH, STNO = FrameStat<G>::NONE, SPARE = G::HR * 3;
+    for (int id = threadIdx.x; id < SPARE + 4; id += G::NT)
+        lds_stat[id < SPARE ? id / 3 * STP + G::HC + id % 3 : STNO + id - SPARE] =
             kBias ? make_float4(0.f, 0.f, 0.f, __int_as_float(0xffff0000))
                   : make_float4(0.f, 0.f, __int_as_float(0x7fff7fff), 0.f);
 
@@ -1694,7 +1712,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
     auto first_of = [&](int t) __attribute__((always_inline)) {
         KeyBlock b;
         b.t = t;
-        b.tl = in_sub(frame_tile(t, ts, s.N, sc.step), a);
+        b.tl = in_sub(frame_tile(t, ts, s.N, sc.step, ntiles), a);
         b.qa = inv_lo(b.tl.r0, KS);
         b.qb = inv_hi(min(b.tl.r0 + 8, s.H) - 1, s.H, KS);
         b.ca = inv_lo(b.tl.c0, KS);
@@ -1878,7 +1896,9 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
 // three workgroups per CU (head_dim <= 64 with small halos; it fits 168 registers there,
 // measured 35 -> 32 us at B8 N2 112x112 d32 k7 and 67 -> 60 us at B4 N4 128x128 d32 k9;
 // the forward and the dQ pass spill under that budget and get slower; with a bias so does this
-// one: B8 N8 64x64 d64 k5 60 us with two waves, 84 with three, B8 N4 56x56 d32 k7 28.2 and 33.9).
+// one
+// from kernel_size 7 on and at head_dim 64: B8 N8 64x64 d64 k5 60 us with two waves, 84 with three, B8 N4 56x56 d32 k7 28.6
+// and 34.4; B8 N2 112x112 d32 k5 34.1 and 27.1).
 // Size of the frame body's blocks as a kernel size (see dkdv_frame): larger than KS where the
 // pass has one workgroup per CU anyway (two parts per block) and LDS has the room.
 // Where not even one workgroup's Q and dO halos fit LDS (head_dim 128 with kernel_size 11 and
@@ -1891,7 +1911,7 @@ constexpr int kFrameKS = kDkdvFrameOnly<D, KS> ? 5 : SP == 2 && KS >= 9 ? 9 + KS
 template <int D, int KS, int SP>
 constexpr int kDkdvWaves =
     kDkdvFrameOnly<D, KS> ? 2 :
-    SP == 1 && !kBias && D <= 64 && 3 * (Geo<D, KS>::LDS_BYTES + 2048) <= 160 * 1024 ? 3 : Geo<D, KS, 4, SP>::WAVES;
+    SP == 1 && D <= (kBias ? KS <= 5 ? 32 : 0 : 64) && 3 * (Geo<D, KS>::LDS_BYTES + 2048) <= 160 * 1024 ? 3 : Geo<D, KS, 4, SP>::WAVES;
 template <bool BF, int D, int KS, bool ROLL, int SP = 1>
 __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) void bwd_dkdv_mfma(
     BArgs a, TileSet ts, int n_inner, int n_frame, int inner_blocks, Runs rp, int dyn) {
