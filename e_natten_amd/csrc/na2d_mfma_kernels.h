@@ -148,21 +148,28 @@ __device__ __forceinline__ float lse_of(float mx, float sum) {
     if constexpr (kBias) return mx + __builtin_amdgcn_logf(sum) * kLn2;
     else return (mx + __builtin_amdgcn_logf(sum)) * kLn2;
 }
+// Calls without a bias table reach the kernels for one at kernel_size 11 and 13 only (use_two_terms in
+// enatten_capi.hip).  The smaller windows are built without that question: a branch around the table's
+// loads cost the forward at B8 N4 56x56 d32 k7 15.7 -> 17.7 us.
+template <int KS>
+__device__ __host__ __forceinline__ bool has_table(const void *table) {
+    return KS < 11 || table != nullptr;
+}
 // With a bias the backward is renormalised as in the general kernels: 1 / sum p of the recomputed
 // probabilities per query, left by the dQ pass behind the block that holds its counter (a.zinv);
 // without a bias table there is no counter, and the block itself has them.
-template <typename ARGS>
+template <int KS, typename ARGS>
 __device__ __forceinline__ float *row_zinv(const ARGS &a) {
-    return a.zinv + (a.rpb ? (int64_t)a.s.B * a.s.N * a.s.H * a.s.W : 0);
+    return a.zinv + (has_table<KS>(a.rpb) ? (int64_t)a.s.B * a.s.N * a.s.H * a.s.W : 0);
 }
 // (P in the float16 dK/dV pass, which 1 / Z brings along, as in na1d_band_mfma.hip: see DsScale)
 template <bool BF>
 constexpr float kPUnit = kBias ? kPScale<BF> : 1.f;
 // what the dK/dV pass stages per query: the log-sum-exp in the logits' unit, delta, kPUnit / Z
 using QStat = std::conditional_t<kBias, float4, float2>;
-template <bool BF, bool BIAS = kBias>
+template <bool BF, int KS, bool BIAS = kBias>
 __device__ __forceinline__ std::conditional_t<BIAS, float4, float2> load_qstat(const BArgs &a, int64_t qt) {
-    if constexpr (BIAS) return make_float4(a.lse[qt], a.delta[qt], row_zinv(a)[qt] * kPUnit<BF>, 0.f);
+    if constexpr (BIAS) return make_float4(a.lse[qt], a.delta[qt], row_zinv<KS>(a)[qt] * kPUnit<BF>, 0.f);
     else return make_float2(a.lse[qt] * kLog2e, a.delta[qt]);
 }
 __device__ __forceinline__ float zinv_of(const float4 &st) { return st.z; }
@@ -252,7 +259,7 @@ struct BiasRegs {
     short v[NB];
     __device__ __forceinline__ void fetch(const void *rpb, int head) {
         const short *p = static_cast<const short *>(rpb) + (int64_t)head * T::E;
-        if (!rpb) {  // no bias: a table of zeros
+        if (!has_table<KS>(rpb)) {  // no bias: a table of zeros
 #pragma unroll
             for (int i = 0; i < NB; i++) v[i] = 0;
             return;
@@ -414,7 +421,7 @@ __device__ __forceinline__ void walk_window(const Shape &s, const void *rpb, int
     const int r0 = win_start(qr, s.H, KS), c0 = win_start(qc, s.W, KS);
     const short *b = static_cast<const short *>(rpb) + ((int64_t)head * SPAN + r0 - qr + KS - 1) * SPAN + c0 - qc + KS - 1;
     for (int i = 0; i < KS * KS; i++)
-        if (!f(r0 + i / KS, c0 + i % KS, rpb ? cvt32<BF>(b[i / KS * SPAN + i % KS]) : 0.f)) return;
+        if (!f(r0 + i / KS, c0 + i % KS, has_table<KS>(rpb) ? cvt32<BF>(b[i / KS * SPAN + i % KS]) : 0.f)) return;
 }
 template <typename ARGS>
 __device__ __forceinline__ const short *pixel(const ARGS &a, const View &v, const ATile &tl, int r, int c) {
@@ -482,7 +489,7 @@ __device__ __forceinline__ void again_dq(const BArgs &a, const ATile &tl, const 
         if ((threadIdx.x & 63) == 0) {
             const int64_t tok = image_token(a, tl) + (int64_t)qr * s.W + qc;
             a.delta[tok] = d;
-            row_zinv(a)[tok] = 1.f / z;
+            row_zinv<KS>(a)[tok] = 1.f / z;
         }
     }
 }
@@ -505,9 +512,9 @@ __device__ __forceinline__ void again_keys(const BArgs &a, const ATile &tl, int 
                     continue;
                 const int64_t tok = image_token(a, tl) + (int64_t)r * s.W + c;
                 const int64_t at = ((int64_t)tl.nn * SPAN + kr - r + KS - 1) * SPAN + kc - c + KS - 1;
-                const float bias = a.rpb ? cvt32<BF>(static_cast<const short *>(a.rpb)[at]) : 0.f;
+                const float bias = has_table<KS>(a.rpb) ? cvt32<BF>(static_cast<const short *>(a.rpb)[at]) : 0.f;
                 const Chan2 q = chan_load<BF>(pixel(a, a.q, tl, r, c), dlim), go = chan_load<BF>(pixel(a, a.d_o, tl, r, c), dlim);
-                const float p = exp_unit(chan_dot(q, k) * s.scale + bias - a.lse[tok]) * row_zinv(a)[tok];
+                const float p = exp_unit(chan_dot(q, k) * s.scale + bias - a.lse[tok]) * row_zinv<KS>(a)[tok];
                 chan_add(av, p, go);
                 chan_add(ak, p * (chan_dot(go, v) - a.delta[tok]), q);
                 open = p == p;
@@ -867,7 +874,7 @@ constexpr int kDqWaves = D == 32 && (KS == 7 || KS == 9) && NW == 4 && !kBias ? 
 template <bool BF, int D, int KS, bool FRAME, bool ROLL, int NW = 4, bool FULL = false>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void bwd_dq_mfma(BArgs a, TileSet ts, int ntiles, Runs rp) {
     // (the dK/dV pass that follows on the stream counts its frame tiles here, from zero)
-    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv && (!kBias || a.rpb)) *reinterpret_cast<int *>(a.zinv) = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv && (!kBias || has_table<KS>(a.rpb))) *reinterpret_cast<int *>(a.zinv) = 0;
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_k[G::ROWS * G::PITCH];
     __shared__ __attribute__((aligned(16))) short lds_v[G::ROWS * G::PITCH];
@@ -1023,7 +1030,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             DsScale<BF> scl;
             if constexpr (kBias) {
                 operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live && delta * 0.f == 0.f ? zinv : 0.f);
-                if (a.d_rpb) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
+                if (has_table<KS>(a.d_rpb)) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
             }
             f32x4 dq[G::DT];
 #pragma unroll
@@ -1050,10 +1057,10 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                 }
             if (FULL || (lq.live && g == 0 && !(bad >> n & 1))) {
                 a.delta[lq.tok] = delta;
-                if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
+                if constexpr (kBias) row_zinv<KS>(a)[lq.tok] = zinv;
             }
         }
-        if (kBias && a.d_rpb) {
+        if (kBias && has_table<KS>(a.d_rpb)) {
             __syncthreads();
             BiasGrad<KS>::template flush<NW>(lds_dbias, a.ds_pairs + (int64_t)sc.t * Bias<KS>::E, cur, s);
         }
@@ -1091,7 +1098,7 @@ constexpr int kDq2Tail = D == 128 && NW == 8 ? (KS == 13 ? 15 : KS == 11 ? 13 : 
 template <bool BF, int D, int KS, int NW = 4, bool FULL = false>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS> : 1)) void bwd_dq2_mfma(BArgs a, TileSet ts, int ntiles) {
     // (the dK/dV pass that follows on the stream counts its frame tiles here, from zero)
-    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv && (!kBias || a.rpb)) *reinterpret_cast<int *>(a.zinv) = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv && (!kBias || has_table<KS>(a.rpb))) *reinterpret_cast<int *>(a.zinv) = 0;
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_x[G::ROWS * G::PITCH];
     __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
@@ -1221,7 +1228,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
             DsScale<BF> scl;
             if constexpr (kBias) {
                 operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live && delta * 0.f == 0.f ? zinv : 0.f);
-                if (a.d_rpb) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
+                if (has_table<KS>(a.d_rpb)) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
             }
             f32x4 dq[G::DT];
 #pragma unroll
@@ -1247,10 +1254,10 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                 }
             if (FULL || (lq.live && g == 0 && !(bad >> n & 1))) {
                 a.delta[lq.tok] = delta;
-                if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
+                if constexpr (kBias) row_zinv<KS>(a)[lq.tok] = zinv;
             }
         }
-        if (kBias && a.d_rpb) {
+        if (kBias && has_table<KS>(a.d_rpb)) {
             __syncthreads();
             BiasGrad<KS>::template flush<NW>(lds_dbias, a.ds_pairs + (int64_t)sc.t * Bias<KS>::E, cur, s);
         }
@@ -1491,7 +1498,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
             const int pr = id / G::HC, pc = id % G::HC;
             if (!ROLL || pr < nr) {
                 const int64_t qt = img_tok + (int64_t)((ROLL ? y0 : br) + pr) * s.W + bc + pc;
-                sst[i] = load_qstat<BF>(a, qt);
+                sst[i] = load_qstat<BF, KS>(a, qt);
             }
         }
         if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
@@ -1697,7 +1704,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
             const int id = threadIdx.x + i * G::NT;
             const int r = min(b.br + id / G::HC, b.qb - 1), c = min(b.bc + id % G::HC, b.cb - 1);
             const int64_t qt = img_tok + (int64_t)r * s.W + c;
-            sst[i] = load_qstat<BF>(a, qt);
+            sst[i] = load_qstat<BF, KS>(a, qt);
         }
         if constexpr (kBias) bst.fetch(a.rpb, b.tl.nn);
     };
