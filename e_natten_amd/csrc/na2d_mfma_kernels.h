@@ -1317,12 +1317,15 @@ __device__ __forceinline__ bool next_block(KeyBlock &b) {
 // SIMD; the inner body is unrolled and has the next step's arithmetic to put between, so there 1
 // and 2 only cost registers (d128 k5 with its column walk spills with them, 107 -> 222 us), but for
 // head_dim 32, where 2 is ahead (B4 N4 128x128 k9 51.6 -> 48.8 us).
+// With a bias at head_dim 32 the 7x7 and 9x9 windows run at two waves per SIMD anyway (kDkdvWaves), which leaves
+// registers for both tiles in both bodies: B8 N4 56x56 d32 k7 28.9 -> 27.6 us, B8 N2 112x112 k9 66.9 -> 66.5.
 //   a_of(h), t_of(h): this lane's row of tile h for the direct and for the transposing reads
 //   stat(h, i), at(h, i, st), in(h, i, st): statistics of query 4 g + i of tile h, the place of its
 //   bias in the table, and whether it attends to this lane's key
-template <int D>
-constexpr int kInnerAhead = kBias ? -1 : D == 32 ? 2 : 0;
-constexpr int kFrameAhead = 1;
+template <int D, int KS>
+constexpr int kInnerAhead = kBias && (D > 32 || KS < 7 || KS > 9) ? -1 : D == 32 ? 2 : 0;
+template <int D, int KS>
+constexpr int kFrameAhead = kBias && D == 32 && (KS == 7 || KS == 9) ? 2 : 1;
 template <bool BF, typename G, int AHEAD, typename AROW, typename TROW, typename STAT, typename AT, typename IN>
 __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g, const float *lds_bias, int n, int g,
                                           float sc2, const s16x8 (&kreg)[G::DS], const s16x8 (&vreg)[G::DS],
@@ -1574,7 +1577,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
         }
 #pragma unroll
         for (int ks = K0; ks < K1; ks++)
-            dkdv_step<BF, G, kInnerAhead<D>>(
+            dkdv_step<BF, G, kInnerAhead<D, KS>>(
                 lds_q, lds_g, lds_bias, n, g, sc2, kreg, vreg, dk, dv, scl,
                 [&](int h) __attribute__((always_inline)) { return row_of(ks * 2 + h, n); },
                 [&](int h) __attribute__((always_inline)) { return row_of(ks * 2 + h, g * 4 + (n >> 2)); },
@@ -1821,7 +1824,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
                     const int u = u0 + h * 4 + g, r = (u * magic) >> 16;
                     at_run[h] = u < nu ? stat0 + r * STP + (u - r * runs) * 4 : (int)STNO;
                 }
-                dkdv_step<BF, G, kFrameAhead>(
+                dkdv_step<BF, G, kFrameAhead<D, KS>>(
                     lds_q, lds_g, lds_bias, n, g, sc2, kreg, vreg, dk, dv, scl,
                     [&](int h) __attribute__((always_inline)) { return row_of(u0 + h * 4 + (n >> 2), n & 3); },
                     [&](int h) __attribute__((always_inline)) { return row_of(u0 + h * 4 + g, n >> 2); },
