@@ -1326,7 +1326,10 @@ template <int D, int KS>
 constexpr int kInnerAhead = kBias && (D > 32 || KS < 7 || KS > 9) ? -1 : D == 32 ? 2 : 0;
 template <int D, int KS>
 constexpr int kFrameAhead = kBias && D == 32 && (KS == 7 || KS == 9) ? 2 : 1;
-template <bool BF, typename G, int AHEAD, typename AROW, typename TROW, typename STAT, typename AT, typename IN>
+// FRAME: a run of four reaches up to three queries past the wave's own, whose delta may be anything: what
+// no window connects with a key is left out of dS, where P = 0 times a delta that is not finite would
+// be NaN.  (With a bias such keys are computed again, again_keys.)
+template <bool BF, typename G, int AHEAD, bool FRAME, typename AROW, typename TROW, typename STAT, typename AT, typename IN>
 __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g, const float *lds_bias, int n, int g,
                                           float sc2, const s16x8 (&kreg)[G::DS], const s16x8 (&vreg)[G::DS],
                                           f32x4 (&dk)[G::DT], f32x4 (&dv)[G::DT], DsScale<BF> &scl, AROW a_of,
@@ -1373,7 +1376,8 @@ __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g
                 dsv[h * 4 + i] = p * (cp[h][i] - q.y);
                 mag = fmaxf(mag, fabsf(dsv[h * 4 + i]));
             } else {
-                put<BF>(dsb, h * 4 + i, p * (cp[h][i] - q.y));
+                const float ds = p * (cp[h][i] - q.y);
+                put<BF>(dsb, h * 4 + i, kBias || !FRAME || ok ? ds : 0.f);
             }
         }
     };
@@ -1577,7 +1581,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
         }
 #pragma unroll
         for (int ks = K0; ks < K1; ks++)
-            dkdv_step<BF, G, kInnerAhead<D, KS>>(
+            dkdv_step<BF, G, kInnerAhead<D, KS>, false>(
                 lds_q, lds_g, lds_bias, n, g, sc2, kreg, vreg, dk, dv, scl,
                 [&](int h) __attribute__((always_inline)) { return row_of(ks * 2 + h, n); },
                 [&](int h) __attribute__((always_inline)) { return row_of(ks * 2 + h, g * 4 + (n >> 2)); },
@@ -1824,7 +1828,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
                     const int u = u0 + h * 4 + g, r = (u * magic) >> 16;
                     at_run[h] = u < nu ? stat0 + r * STP + (u - r * runs) * 4 : (int)STNO;
                 }
-                dkdv_step<BF, G, kFrameAhead<D, KS>>(
+                dkdv_step<BF, G, kFrameAhead<D, KS>, true>(
                     lds_q, lds_g, lds_bias, n, g, sc2, kreg, vreg, dk, dv, scl,
                     [&](int h) __attribute__((always_inline)) { return row_of(u0 + h * 4 + (n >> 2), n & 3); },
                     [&](int h) __attribute__((always_inline)) { return row_of(u0 + h * 4 + g, n >> 2); },

@@ -40,6 +40,30 @@ def test_logits_far_below_zero(hw, ks, D):
         assert O.rel_err(x, r) <= 2e-2
 
 
+@pytest.mark.parametrize("which", ["dO", "q"])
+@pytest.mark.parametrize("hw,D,ks,dtype", [
+    ((26, 23), 64, 7, BF), ((26, 21), 48, 3, BF), ((30, 27), 64, 11, F16), ((22, 23), 128, 3, F16), ((27, 25), 96, 7, BF),
+    ((25, 27), 128, 11, BF)])
+def test_values_that_are_not_finite_stay_in_their_blocks_of_keys(hw, D, ks, dtype, which):
+    """A NaN in one query, another one in each head: dK and dV of the 4x4 blocks of keys that its window
+    does not meet are finite, though the query may stand right beside those that a block's waves walk."""
+    ensure_built()
+    print("case one query not finite", which, hw, D, ks, flush=True)
+    (H, W), heads, row = hw, 16, 9
+    q, k, v, g = make_inputs((1, heads, H, W, D), dtype, seed=23)
+    for h in range(heads):
+        {"dO": g, "q": q}[which][0, h, row, 4 + h] = float("nan")
+    _, _, dk, dv = run_gpu(q, k, v, g, ks, D ** -0.5)
+    for h in range(heads):
+        keys = O.neighbour_mask(H, W, ks)[row * W + 4 + h].reshape(H, W)
+        blocks = torch.nn.functional.max_pool2d(keys.float()[None], 4, ceil_mode=True)[0] > 0
+        blocks = blocks.repeat_interleave(4, 0).repeat_interleave(4, 1)[:H, :W]
+        for name, x in (("dK", dk), ("dV", dv)):
+            nan = ~x[0, h].float().isfinite().all(-1)
+            assert nan[keys].all(), (name, h)
+            assert not (nan & ~blocks).any(), (name, h, (nan & ~blocks).nonzero().tolist())
+
+
 @pytest.mark.parametrize("D,ks,hw,dtype", [
     (40, 11, (43, 38), BF), (48, 13, (50, 44), BF), (56, 13, (13, 28), F16), (48, 11, (24, 120), F16)])
 def test_largest_windows_below_head_dim_64(D, ks, hw, dtype):
