@@ -732,22 +732,11 @@ __device__ __forceinline__ Tile inner_tile_cm(int t, const TileSet &ts, int N) {
     tl.bb = t / N; tl.nn = t % N;
     return tl;
 }
-// Frame tiles are numbered image by image.  Their cost depends on the place in the image (the tiles
-// of the second ring from the border have up to four blocks of queries, those of a corner one), and
-// a workgroup takes every `step`-th tile: where `step` is a multiple of the tiles of an image, as 64 is of
-// 16, it would get the same place in every image, and those with the dearest place end last.  There, or
-// where it is half a multiple, and on walks of eight tiles and more the places of an image are counted from a
-// start that moves on by about 5/8 of them (an odd number) from one of a workgroup's tiles to the next.  dK/dV pass, bf16 d64 k9, 700
-// images of 26x26 (16 tiles): 491 -> 255 us; 32x32 484 -> 325; B8 N16 28x28 k13 224 -> 109.  On other short
-// walks which places meet is luck either way (with a bias B8 N2 112x112 d32 k9, four tiles: 66 us in order, 75 turned).
-__device__ __forceinline__ Tile frame_tile(int t, const TileSet &ts, int N, int step = 1, int ntiles = 0) {
-    const int per_img = ts.tiles_r * ts.tiles_c - ts.ni_r * ts.ni_c;
-    const int slab = t / per_img;
-    int e = t - slab * per_img;
-    if ((ntiles >= 64 * step || 2 * step % per_img == 0) && per_img <= 4096) {  // (the products stay within an int)
-        const int turn = ((per_img * 5 / 8) | 1) + per_img - step % per_img;
-        e = (e + slab * per_img / step % per_img * turn) % per_img;
-    }
+// Frame tiles, in the order of frame_order.h
+__device__ __forceinline__ Tile frame_tile(int t, const TileSet &ts, int N, int step = 1) {
+    const FramePlace at = frame_place(t, ts.tiles_r * ts.tiles_c - ts.ni_r * ts.ni_c, step, ts.turn);
+    const int slab = at.image;
+    int e = at.place;
     const int top = ts.ir0 * ts.tiles_c, side = ts.tiles_c - ts.ni_c;
     int tr, tc;
     if (e < top) {
