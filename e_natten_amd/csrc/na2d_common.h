@@ -104,7 +104,7 @@ struct TileSet {
     int tiles_r, tiles_c;  // 8x8 tiles per image
     int ir0, ni_r;         // first inner tile row, number of inner tile rows
     int ic0, ni_c;         // first inner tile column, number of inner tile columns
-    int turn = 0;          // order of the frame tiles of the dK/dV pass, see frame_order.h
+    FrameOrder order{0, 1};  // of the frame tiles in the dK/dV pass
 };
 
 void set_error(const char *fmt, ...);

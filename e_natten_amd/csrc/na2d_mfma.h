@@ -733,8 +733,8 @@ __device__ __forceinline__ Tile inner_tile_cm(int t, const TileSet &ts, int N) {
     return tl;
 }
 // Frame tiles, in the order of frame_order.h
-__device__ __forceinline__ Tile frame_tile(int t, const TileSet &ts, int N, int step = 1) {
-    const FramePlace at = frame_place(t, ts.tiles_r * ts.tiles_c - ts.ni_r * ts.ni_c, step, ts.turn);
+__device__ __forceinline__ Tile frame_tile(int t, const TileSet &ts, int N) {
+    const FramePlace at = frame_place(t, ts.tiles_r * ts.tiles_c - ts.ni_r * ts.ni_c, ts.order);
     const int slab = at.image;
     int e = at.place;
     const int top = ts.ir0 * ts.tiles_c, side = ts.tiles_c - ts.ni_c;

@@ -1726,7 +1726,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
     auto first_of = [&](int t) __attribute__((always_inline)) {
         KeyBlock b;
         b.t = t;
-        b.tl = in_sub(frame_tile(t, ts, s.N, sc.step), a);
+        b.tl = in_sub(frame_tile(t, ts, s.N), a);
         b.qa = inv_lo(b.tl.r0, KS);
         b.qb = inv_hi(min(b.tl.r0 + 8, s.H) - 1, s.H, KS);
         b.ca = inv_lo(b.tl.c0, KS);
@@ -2329,7 +2329,7 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                 inner_blocks = all < grid ? (int)all : grid;
             }
             // (the counter deals tiles in their plain order)
-            if (n_frame > 0 && !dyn) ts.turn = frame_turn((int)(n_frame / slabs), (grid - inner_blocks) / 8, n_frame);
+            if (n_frame > 0 && !dyn) ts.order = frame_order((int)(n_frame / slabs), (grid - inner_blocks) / 8, n_frame);
             ProfScope prof(ENATTEN_KERNEL_BWD_DKDV, "bwd_dkdv_mfma", st);
             if (inner_blocks > 0 && roll_pays<D>(n_inner, inner_blocks))
                 hipLaunchKernelGGL((bwd_dkdv_mfma<BF, D, KS, kRollBuilt<D>, SP>), dim3(grid), dim3(NT),

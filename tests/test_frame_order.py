@@ -11,13 +11,14 @@ import pytest
 from _util import ROOT
 
 SOURCE = """#include "frame_order.h"
-extern "C" int turn_of(int per_img, int step, int n) { return enatten::frame_turn(per_img, step, n); }
-extern "C" void order(int n, int per_img, int step, int turn, int *image, int *place) {
+extern "C" int order(int n, int per_img, int step, int plain, int *image, int *place) {
+    const enatten::FrameOrder o = plain ? enatten::FrameOrder{0, 1} : enatten::frame_order(per_img, step, n);
     for (int t = 0; t < n; t++) {
-        const enatten::FramePlace p = enatten::frame_place(t, per_img, step, turn);
+        const enatten::FramePlace p = enatten::frame_place(t, per_img, o);
         image[t] = p.image;
         place[t] = p.place;
     }
+    return o.turn;
 }
 """
 
@@ -31,17 +32,18 @@ def lib(tmp_path_factory):
     return ctypes.CDLL(str(d / "order.so"))
 
 
-def walk(lib, n, per_img, step, turn):
+def walk(lib, n, per_img, step, plain=False):
+    """(turn, image of each tile, its place)"""
     image, place = np.empty(n, np.int32), np.empty(n, np.int32)
-    lib.order(n, per_img, step, turn, *(x.ctypes.data_as(ctypes.c_void_p) for x in (image, place)))
-    return image, place
+    turn = lib.order(n, per_img, step, int(plain), *(x.ctypes.data_as(ctypes.c_void_p) for x in (image, place)))
+    return turn, image, place
 
 
 @pytest.mark.parametrize("per_img", [1, 2, 3, 4, 9, 15, 16, 24, 25, 60, 64, 128, 240, 4096, 4097])
 def test_every_tile_once(lib, per_img):
     for step in (1, 5, 7, 32, 45, 64, 96, 120, per_img // 2 or 1, per_img, 2 * per_img):
         n = (200 * step // per_img + 2) * per_img
-        image, place = walk(lib, n, per_img, step, lib.turn_of(per_img, step, n))
+        _, image, place = walk(lib, n, per_img, step)
         assert (image == np.arange(n) // per_img).all() and place.min() >= 0
         assert np.array_equal(np.sort(image.astype(np.int64) * per_img + place), np.arange(n)), (per_img, step)
 
@@ -97,17 +99,18 @@ def test_no_workgroup_has_more_than_in_the_plain_order(lib):
         per_img, n = len(costs), len(costs) * images
         share = n / (n + inner * images / 2)  # (two inner tiles cost about one border tile)
         step = max(1, min(-(-n // 8), round(32 * wgs * share)))
-        turn = lib.turn_of(per_img, step, n)
+        if n > 30000:
+            continue
+        turn, _, place = walk(lib, n, per_img, step)
         period = per_img // np.gcd(per_img, step)
-        assert (turn != 0) == (per_img >= 3 and (period == 1 or period == 2 and n >= 96 * step)), (per_img, step)
-        if turn and n <= 30000:
+        assert (turn != 0) == (per_img >= 3 and (period == 1 or period == 2 and n >= 32 * step)), (per_img, step)
+        if turn:
             turned += 1
-            new, old = (busiest(costs, walk(lib, n, per_img, step, t)[1], step) for t in (turn, 0))
+            new, old = (busiest(costs, x, step) for x in (place, walk(lib, n, per_img, step, plain=True)[2]))
             assert new <= old, (H, W, images, k, step, new, old)
     assert turned >= 20
     for (H, W, images, k), body, gain in (((26, 26, 128, 9), bodies[3], 1.5), ((28, 28, 128, 13), bodies[5], 1.8)):
         costs, _ = frame_costs(H, W, k, *body[1:3])
-        step = 32 * body[3]
-        new, old = (busiest(costs, walk(lib, len(costs) * images, len(costs), step, t)[1], step)
-                    for t in (lib.turn_of(len(costs), step, len(costs) * images), 0))
+        n, step = len(costs) * images, 32 * body[3]
+        new, old = (busiest(costs, walk(lib, n, len(costs), step, plain)[2], step) for plain in (False, True))
         assert gain * new <= old, (H, W, new, old)
