@@ -17,7 +17,7 @@ OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libenatten.so")
 TORCH_LIB = os.path.join(HERE, "libenatten_torch.so")
 SOURCES = ["na2d_mfma.hip", "na2d_mfma_narrow.hip", "na2d_mfma_dilated.hip", "na2d_mfma_bias.hip",
-           "na2d_mfma_small.hip",
+           "na2d_mfma_two_terms.hip", "na2d_mfma_small.hip",
            "enatten_capi.hip", "enatten_prof.cpp", "na2d_simt.hip",
            "na2d_f64.hip", "na2d_mfma_fused.hip", "na2d_mfma_onepass.hip", "na2d_mfma_f32.hip", "na1d_mfma.hip",
            "na1d_mfma_narrow.hip", "na1d_band_mfma.hip"]

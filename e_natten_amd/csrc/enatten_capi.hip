@@ -88,11 +88,10 @@ int make_view(const char *fn, const char *name, const void *p, const int64_t *st
 bool use_mfma(int D, int ks, int dtype) {
     return g_path.load() != ENATTEN_PATH_SIMT && mfma_supported(D, ks, dtype);
 }
-// Head dims between 32 and 64 with kernel_size 11 and 13: the kernels for a relative position bias,
-// with a table of zeros where there is none (two terms for P and dS, 1 / Z, values that are not finite
-// stay in their windows: as close to float64 as the general kernels).  bf16, forward and backward, us, general
-// -> these: B1 N16 162x174 d48 k11 4200 -> 923, B2 N8 128x128 d48 k13 3160 -> 449,
-// B1 N2 32x32 d48 k13 401 -> 43.
+// Head dims between 32 and 64 with kernel_size 11 and 13: the kernels for a relative position bias, and
+// without one their build without a table (two terms for P and dS, 1 / Z, values that are not finite stay in
+// their windows).  bf16, forward and backward, us, general -> these: B1 N16 162x174 d48 k11 4050 -> 592, with a
+// bias 5800 -> 750; B2 N8 128x128 d48 k13 3090 -> 342, with a bias 4570 -> 480.
 bool use_two_terms(int D, int ks, int dtype) {
     return g_path.load() != ENATTEN_PATH_SIMT && (dtype == ENATTEN_BF16 || dtype == ENATTEN_F16) && D > 32 && D < 64 &&
            D % 8 == 0 && (ks == 11 || ks == 13);
@@ -158,7 +157,7 @@ int run_fwd(const FwdArgs &a, int dtype, hipStream_t st) {
         return launch_fwd_mfma(a, dtype, st);
     }
     if (use_mfma_f32(D, ks, dtype)) return launch_fwd_mfma_f32(a, st);
-    if (use_two_terms(D, ks, dtype)) return launch_fwd_mfma_bias(a, dtype, st);
+    if (use_two_terms(D, ks, dtype)) return launch_fwd_two_terms(a, dtype, st);
     return launch_fwd_simt(a, dtype, st);
 }
 int run_bwd(const char *fn, const BwdArgs &a, int dtype, size_t ws_floats, hipStream_t st) {
@@ -175,7 +174,7 @@ int run_bwd(const char *fn, const BwdArgs &a, int dtype, size_t ws_floats, hipSt
     if (use_mfma_f32(D, ks, dtype) && a.grads_contiguous() &&
         ws_floats >= (size_t)a.s.B * a.s.N * a.s.H * a.s.W * mfma_f32_workspace_floats(ks))
         return launch_bwd_mfma_f32(a, st);
-    if (use_two_terms(D, ks, dtype)) return launch_bwd_mfma_bias(a, dtype, st);
+    if (use_two_terms(D, ks, dtype)) return launch_bwd_two_terms(a, dtype, st);
     return launch_bwd_simt(a, dtype, st);
 }
 

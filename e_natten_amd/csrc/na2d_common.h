@@ -166,9 +166,12 @@ int launch_fwd_small(const FwdArgsSub &a, int dtype, hipStream_t st);
 int launch_bwd_small(const BwdArgsSub &a, int dtype, hipStream_t st);
 // the same kernels with a relative position bias (a.rpb, a.d_rpb; a.ds_pairs takes one row of
 // (2k-1)^2 floats per tile): square centred windows that mfma_supported takes, and head dims between 32
-// and 64 with kernel_size 11 and 13, for which they also serve calls without a bias (no a.rpb)
+// and 64 with kernel_size 11 and 13
 int launch_fwd_mfma_bias(const FwdArgs &a, int dtype, hipStream_t st);
 int launch_bwd_mfma_bias(const BwdArgs &a, int dtype, hipStream_t st);
+// ... and those dims and sizes without a bias
+int launch_fwd_two_terms(const FwdArgs &a, int dtype, hipStream_t st);
+int launch_bwd_two_terms(const BwdArgs &a, int dtype, hipStream_t st);
 // matrix-core kernels of the 1D operator (a.s: H = 1, W = T, kh = 1, kw = kernel_size):
 // bf16 / f16, D in {32, 64, 128}, odd kernel_size 3 .. 49
 bool mfma1d_supported(int D, int ks, int dtype);

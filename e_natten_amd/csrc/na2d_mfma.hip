@@ -8,6 +8,7 @@ namespace {
 constexpr bool kNarrow = false;
 constexpr bool kSub = false;
 constexpr bool kBias = false;
+constexpr bool kTable = false;
 }
 }  // namespace enatten
 

@@ -13,6 +13,7 @@ namespace {
 constexpr bool kNarrow = true;
 constexpr bool kSub = false;
 constexpr bool kBias = true;
+constexpr bool kTable = true;
 }
 }  // namespace enatten
 

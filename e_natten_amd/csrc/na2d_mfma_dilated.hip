@@ -15,6 +15,7 @@ namespace {
 constexpr bool kNarrow = true;
 constexpr bool kSub = true;
 constexpr bool kBias = false;
+constexpr bool kTable = false;
 }
 }  // namespace enatten
 

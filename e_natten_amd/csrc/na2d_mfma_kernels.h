@@ -40,6 +40,10 @@
 // column, head.  The heads are innermost because in the layout of a projection they lie side by
 // side in memory: a workgroup and its neighbours then read the same lines.  `kSub` false folds
 // every one of these helpers to what it is without sub-grids.
+//
+// `kBias`: P and dS in two 16-bit terms, 1 / Z, results that are not finite computed again from their
+// windows; with `kTable` (na2d_mfma_bias.hip) there is a relative position bias, without it
+// (na2d_mfma_two_terms.hip) none.
 
 #include <algorithm>
 
@@ -148,28 +152,22 @@ __device__ __forceinline__ float lse_of(float mx, float sum) {
     if constexpr (kBias) return mx + __builtin_amdgcn_logf(sum) * kLn2;
     else return (mx + __builtin_amdgcn_logf(sum)) * kLn2;
 }
-// Calls without a bias table reach the kernels for one at kernel_size 11 and 13 only (use_two_terms in
-// enatten_capi.hip).  The smaller windows are built without that question: a branch around the table's
-// loads cost the forward at B8 N4 56x56 d32 k7 15.7 -> 17.7 us.
-template <int KS>
-__device__ __host__ __forceinline__ bool has_table(const void *table) {
-    return KS < 11 || table != nullptr;
-}
 // With a bias the backward is renormalised as in the general kernels: 1 / sum p of the recomputed
 // probabilities per query, left by the dQ pass behind the block that holds its counter (a.zinv);
-// without a bias table there is no counter, and the block itself has them.
-template <int KS, typename ARGS>
+// without a table there is no counter, and the block itself has them.
+constexpr bool kCounter = !kBias || kTable;
+template <typename ARGS>
 __device__ __forceinline__ float *row_zinv(const ARGS &a) {
-    return a.zinv + (has_table<KS>(a.rpb) ? (int64_t)a.s.B * a.s.N * a.s.H * a.s.W : 0);
+    return a.zinv + (kCounter ? (int64_t)a.s.B * a.s.N * a.s.H * a.s.W : 0);
 }
 // (P in the float16 dK/dV pass, which 1 / Z brings along, as in na1d_band_mfma.hip: see DsScale)
 template <bool BF>
 constexpr float kPUnit = kBias ? kPScale<BF> : 1.f;
 // what the dK/dV pass stages per query: the log-sum-exp in the logits' unit, delta, kPUnit / Z
 using QStat = std::conditional_t<kBias, float4, float2>;
-template <bool BF, int KS, bool BIAS = kBias>
+template <bool BF, bool BIAS = kBias>
 __device__ __forceinline__ std::conditional_t<BIAS, float4, float2> load_qstat(const BArgs &a, int64_t qt) {
-    if constexpr (BIAS) return make_float4(a.lse[qt], a.delta[qt], row_zinv<KS>(a)[qt] * kPUnit<BF>, 0.f);
+    if constexpr (BIAS) return make_float4(a.lse[qt], a.delta[qt], row_zinv(a)[qt] * kPUnit<BF>, 0.f);
     else return make_float2(a.lse[qt] * kLog2e, a.delta[qt]);
 }
 __device__ __forceinline__ float zinv_of(const float4 &st) { return st.z; }
@@ -259,7 +257,10 @@ struct BiasRegs {
     short v[NB];
     __device__ __forceinline__ void fetch(const void *rpb, int head) {
         const short *p = static_cast<const short *>(rpb) + (int64_t)head * T::E;
-        if (!has_table<KS>(rpb)) {  // no bias: a table of zeros
+        // Never taken.  The branch only keeps the compiler from moving these loads' arithmetic through the kernels
+        // of the largest windows, which then spill (forward B2 N8 128x128 d64 k11 90 -> 76 us with it; below 11x11 it
+        // costs: forward B8 N4 56x56 d32 k7 15.7 -> 17.7).
+        if (KS >= 11 && rpb == nullptr) {
 #pragma unroll
             for (int i = 0; i < NB; i++) v[i] = 0;
             return;
@@ -421,7 +422,7 @@ __device__ __forceinline__ void walk_window(const Shape &s, const void *rpb, int
     const int r0 = win_start(qr, s.H, KS), c0 = win_start(qc, s.W, KS);
     const short *b = static_cast<const short *>(rpb) + ((int64_t)head * SPAN + r0 - qr + KS - 1) * SPAN + c0 - qc + KS - 1;
     for (int i = 0; i < KS * KS; i++)
-        if (!f(r0 + i / KS, c0 + i % KS, has_table<KS>(rpb) ? cvt32<BF>(b[i / KS * SPAN + i % KS]) : 0.f)) return;
+        if (!f(r0 + i / KS, c0 + i % KS, kTable ? cvt32<BF>(b[i / KS * SPAN + i % KS]) : 0.f)) return;
 }
 template <typename ARGS>
 __device__ __forceinline__ const short *pixel(const ARGS &a, const View &v, const ATile &tl, int r, int c) {
@@ -472,7 +473,7 @@ __device__ __forceinline__ void again_dq(const BArgs &a, const ATile &tl, const 
         Chan2 acc{0.f, 0.f};
         if (d != d) {  // every dS of the window is NaN
             float *at = sums + (win_start(qr, s.H, KS) - qr + wr) * BiasGrad<KS>::SIDE + win_start(qc, s.W, KS) - qc + wc;
-            for (int i = threadIdx.x & 63; i < KS * KS; i += 64) at[i / KS * BiasGrad<KS>::SIDE + i % KS] = d;
+            for (int i = threadIdx.x & 63; kTable && i < KS * KS; i += 64) at[i / KS * BiasGrad<KS>::SIDE + i % KS] = d;
             acc = Chan2{d, d};
         } else {
             walk_window<BF, KS>(s, a.rpb, tl.nn, qr, qc, [&](int r, int c, float bias) {
@@ -480,7 +481,7 @@ __device__ __forceinline__ void again_dq(const BArgs &a, const ATile &tl, const 
                 const float p = exp_unit(chan_dot(q, k) * s.scale + bias - lse_q) / z;
                 const float ds = p * (chan_dot(go, chan_load<BF>(pixel(a, a.v, tl, r, c), dlim)) - d);
                 chan_add(acc, ds, k);
-                if ((threadIdx.x & 63) == 0 && !(delta_q * 0.f == 0.f))
+                if (kTable && (threadIdx.x & 63) == 0 && !(delta_q * 0.f == 0.f))
                     sums[(r - qr + wr) * BiasGrad<KS>::SIDE + c - qc + wc] += ds;
                 return true;
             });
@@ -489,7 +490,7 @@ __device__ __forceinline__ void again_dq(const BArgs &a, const ATile &tl, const 
         if ((threadIdx.x & 63) == 0) {
             const int64_t tok = image_token(a, tl) + (int64_t)qr * s.W + qc;
             a.delta[tok] = d;
-            row_zinv<KS>(a)[tok] = 1.f / z;
+            row_zinv(a)[tok] = 1.f / z;
         }
     }
 }
@@ -512,9 +513,9 @@ __device__ __forceinline__ void again_keys(const BArgs &a, const ATile &tl, int 
                     continue;
                 const int64_t tok = image_token(a, tl) + (int64_t)r * s.W + c;
                 const int64_t at = ((int64_t)tl.nn * SPAN + kr - r + KS - 1) * SPAN + kc - c + KS - 1;
-                const float bias = has_table<KS>(a.rpb) ? cvt32<BF>(static_cast<const short *>(a.rpb)[at]) : 0.f;
+                const float bias = kTable ? cvt32<BF>(static_cast<const short *>(a.rpb)[at]) : 0.f;
                 const Chan2 q = chan_load<BF>(pixel(a, a.q, tl, r, c), dlim), go = chan_load<BF>(pixel(a, a.d_o, tl, r, c), dlim);
-                const float p = exp_unit(chan_dot(q, k) * s.scale + bias - a.lse[tok]) * row_zinv<KS>(a)[tok];
+                const float p = exp_unit(chan_dot(q, k) * s.scale + bias - a.lse[tok]) * row_zinv(a)[tok];
                 chan_add(av, p, go);
                 chan_add(ak, p * (chan_dot(go, v) - a.delta[tok]), q);
                 open = p == p;
@@ -546,7 +547,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_k[G::ROWS * G::PITCH];
     __shared__ __attribute__((aligned(16))) short lds_v[G::ROWS * G::PITCH];
-    __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
+    __shared__ float lds_bias[kTable ? Bias<KS>::WORDS : 1];
 
     const Shape &s = a.s;
     const int dlim = kNarrow ? s.D : D;  // head dim of the tensors: D, or less in the build for narrow dims
@@ -574,7 +575,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
             halo_fetch<D, KS>(vst, plan, image_at(a, a.v, tl), row_step(a, a.v), col_step(a, a.v), lq.hr0, lq.hc0, s.H, s.W);
         }
         load_row_chunks(qnext, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
-        if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
+        if constexpr (kTable) bst.fetch(a.rpb, tl.nn);
     };
 
     auto pick = [&](int t) __attribute__((always_inline)) {
@@ -597,7 +598,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
             halo_commit<D, KS>(lds_k, plan, kst);
             halo_commit<D, KS>(lds_v, plan, vst);
         }
-        if constexpr (kBias) bst.commit(lds_bias);
+        if constexpr (kTable) bst.commit(lds_bias);
 #pragma unroll
         for (int ds = 0; ds < G::DS; ds++) qreg[ds] = qnext[ds];
     };
@@ -631,7 +632,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
 
         if (FULL || lq.wave_on) {
             // logits^T [halo token][query], masked
-            const int bq = kBias ? Bias<KS>::query(lq) : 0;
+            const int bq = kTable ? Bias<KS>::query(lq) : 0;
             f32x4 acc[G::MT];
             float mx = -INFINITY;
 #pragma unroll
@@ -645,7 +646,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
                 for (int i = 0; i < 4; i++) {
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, lq.dr, lq.dc);
                     float x = c[i] * sc2;
-                    if constexpr (kBias) x += lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)];
+                    if constexpr (kTable) x += lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)];
                     c[i] = ok ? x : -INFINITY;
                     mx = fmaxf(mx, c[i]);
                 }
@@ -730,7 +731,7 @@ template <bool BF, int D, int KS, int NW = 4, bool FULL = false>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS> : 1)) void fwd2_mfma(FArgs a, int tiles_r, int tiles_c, int ntiles) {
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_x[G::ROWS * G::PITCH];
-    __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
+    __shared__ float lds_bias[kTable ? Bias<KS>::WORDS : 1];
     const Shape &s = a.s;
     const int dlim = kNarrow ? s.D : D;  // head dim of the tensors: D, or less in the build for narrow dims
     Sched sc = make_sched(ntiles, blockIdx.x, gridDim.x);
@@ -749,7 +750,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     };
     auto fetch_q = [&](const ATile &tl, const LaneQ &lq) __attribute__((always_inline)) {
         load_row_chunks(qnext, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
-        if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
+        if constexpr (kTable) bst.fetch(a.rpb, tl.nn);
     };
     ATile cur = in_sub(tile_of(sc.t, tiles_r, tiles_c, s.N, G::TH), a);
     LaneQ lq = lane_at<KS>(a, cur, wave, n);
@@ -760,7 +761,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     // see fwd_mfma)
     auto commit_k = [&]() __attribute__((always_inline)) {
         halo_commit<D, KS>(lds_x, plan, st);
-        if constexpr (kBias) bst.commit(lds_bias);
+        if constexpr (kTable) bst.commit(lds_bias);
 #pragma unroll
         for (int ds = 0; ds < G::DS; ds++) qreg[ds] = qnext[ds];
     };
@@ -773,7 +774,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
         Op8 pb[G::KSTEPS];
         float mx = -INFINITY, sum = 0.f;
         if (FULL || lq.wave_on) {
-            const int bq = kBias ? Bias<KS>::query(lq) : 0;
+            const int bq = kTable ? Bias<KS>::query(lq) : 0;
             f32x4 acc[G::MT];
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
@@ -786,7 +787,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                 for (int i = 0; i < 4; i++) {
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, lq.dr, lq.dc);
                     float x = c[i] * sc2;
-                    if constexpr (kBias) x += lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)];
+                    if constexpr (kTable) x += lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)];
                     c[i] = ok ? x : -INFINITY;
                     mx = fmaxf(mx, c[i]);
                 }
@@ -874,12 +875,12 @@ constexpr int kDqWaves = D == 32 && (KS == 7 || KS == 9) && NW == 4 && !kBias ? 
 template <bool BF, int D, int KS, bool FRAME, bool ROLL, int NW = 4, bool FULL = false>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void bwd_dq_mfma(BArgs a, TileSet ts, int ntiles, Runs rp) {
     // (the dK/dV pass that follows on the stream counts its frame tiles here, from zero)
-    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv && (!kBias || has_table<KS>(a.rpb))) *reinterpret_cast<int *>(a.zinv) = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv && kCounter) *reinterpret_cast<int *>(a.zinv) = 0;
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_k[G::ROWS * G::PITCH];
     __shared__ __attribute__((aligned(16))) short lds_v[G::ROWS * G::PITCH];
-    __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
-    __shared__ __attribute__((aligned(16))) float lds_dbias[kBias ? NW * BiasGrad<KS>::WORDS : 1];
+    __shared__ float lds_bias[kTable ? Bias<KS>::WORDS : 1];
+    __shared__ __attribute__((aligned(16))) float lds_dbias[kTable ? NW * BiasGrad<KS>::WORDS : 1];
 
     const Shape &s = a.s;
     const int dlim = kNarrow ? s.D : D;  // head dim of the tensors: D, or less in the build for narrow dims
@@ -903,7 +904,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
     s16x8 qnext[G::DS], gnext[G::DS];
     float lse_next = 0.f;
     BiasRegs<BF, KS, G::NT> bst;
-    if constexpr (kBias) BiasGrad<KS>::template clear<G::NT>(lds_dbias);
+    if constexpr (kTable) BiasGrad<KS>::template clear<G::NT>(lds_dbias);
     // rows [y0, y0 + nr) of the halo are what LDS does not hold yet
     auto prefetch = [&](const ATile &tl, const LaneQ &lq, int y0, int nr) __attribute__((always_inline)) {
         if constexpr (ROLL) {
@@ -916,7 +917,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
         load_row_chunks(qnext, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
         load_row_chunks(gnext, image_at(a, a.d_o, tl) + lq.qr * row_step(a, a.d_o) + lq.qc * col_step(a, a.d_o), g, dlim);
         lse_next = a.lse[lq.tok];
-        if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
+        if constexpr (kTable) bst.fetch(a.rpb, tl.nn);
     };
 
     ATile cur = pick(sc.t);
@@ -940,7 +941,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             greg[ds] = gnext[ds];
         }
         lse2 = lse_next * kUnit;
-        if constexpr (kBias) bst.commit(lds_bias);
+        if constexpr (kTable) bst.commit(lds_bias);
     };
     if constexpr (FULL) commit();
     for (;;) {
@@ -976,7 +977,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             // the largest halos it is not kept but formed a second time once delta
             // is known (measured faster there: the matrix cores are idle, the
             // registers are not).
-            const int bq = kBias ? Bias<KS>::query(lq) : 0;
+            const int bq = kTable ? Bias<KS>::query(lq) : 0;
             constexpr bool kKeepDp = !(G::WAVES == 1 && G::MT >= 16);
             f32x4 dp[kKeepDp ? G::MT : 1];
             Op8 dsb[G::KSTEPS];
@@ -995,7 +996,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                 for (int i = 0; i < 4; i++) {
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, lq.dr, lq.dc);
                     float x;
-                    if constexpr (kBias) x = cs[i] * sc2 + lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)] - lse2;
+                    if constexpr (kTable) x = cs[i] * sc2 + lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)] - lse2;
                     else x = cs[i] * sc2 - lse2;
                     cs[i] = exp_unit(ok ? x : -INFINITY);
                     if constexpr (kBias) zsum += cs[i];
@@ -1030,7 +1031,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             DsScale<BF> scl;
             if constexpr (kBias) {
                 operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live && delta * 0.f == 0.f ? zinv : 0.f);
-                if (has_table<KS>(a.d_rpb)) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
+                if constexpr (kTable) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
             }
             f32x4 dq[G::DT];
 #pragma unroll
@@ -1053,14 +1054,14 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                 if (__builtin_expect(bad != 0, 0)) {
                     BiasGrad<KS>::wave_fence();
                     again_dq<BF, KS>(a, cur, lq, bad, lse2, delta, wave,
-                                     lds_dbias + wave * BiasGrad<KS>::WORDS + 4 * BiasGrad<KS>::PLANE, dlim);
+                                     kTable ? lds_dbias + wave * BiasGrad<KS>::WORDS + 4 * BiasGrad<KS>::PLANE : nullptr, dlim);
                 }
             if (FULL || (lq.live && g == 0 && !(bad >> n & 1))) {
                 a.delta[lq.tok] = delta;
-                if constexpr (kBias) row_zinv<KS>(a)[lq.tok] = zinv;
+                if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
             }
         }
-        if (kBias && has_table<KS>(a.d_rpb)) {
+        if constexpr (kTable) {
             __syncthreads();
             BiasGrad<KS>::template flush<NW>(lds_dbias, a.ds_pairs + (int64_t)sc.t * Bias<KS>::E, cur, s);
         }
@@ -1094,15 +1095,20 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
 // spilled; with 8 chunks behind the arithmetic 110.6 us, with 13 107.5.
 template <int D, int KS, int NW>
 constexpr int kDq2Tail = D == 128 && NW == 8 ? (KS == 13 ? 15 : KS == 11 ? 13 : 0) : 0;
+// Workgroups per CU that the registers are budgeted for: one in two terms (and float32 dS beside them),
+// which spills 150 to 340 registers otherwise.  dQ pass with a bias, 16x8 tiles of eight waves, which spill too, -> 8x8
+// tiles: B2 N8 128x128 d64 k11 265 -> 193 us, float16 B3 N5 61x83 91 -> 78.
+template <int D, int KS, int NW>
+constexpr int kDq2Wgs = NW == 4 && !(kBias && D == 64) ? kOneHaloWgs<D, KS> : 1;
 // FULL: as in fwd_mfma.
 template <bool BF, int D, int KS, int NW = 4, bool FULL = false>
-__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS> : 1)) void bwd_dq2_mfma(BArgs a, TileSet ts, int ntiles) {
+__global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDq2Wgs<D, KS, NW>)) void bwd_dq2_mfma(BArgs a, TileSet ts, int ntiles) {
     // (the dK/dV pass that follows on the stream counts its frame tiles here, from zero)
-    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv && (!kBias || has_table<KS>(a.rpb))) *reinterpret_cast<int *>(a.zinv) = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv && kCounter) *reinterpret_cast<int *>(a.zinv) = 0;
     using G = Geo<D, KS, NW>;
     __shared__ __attribute__((aligned(16))) short lds_x[G::ROWS * G::PITCH];
-    __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
-    __shared__ __attribute__((aligned(16))) float lds_dbias[kBias ? NW * BiasGrad<KS>::WORDS : 1];
+    __shared__ float lds_bias[kTable ? Bias<KS>::WORDS : 1];
+    __shared__ __attribute__((aligned(16))) float lds_dbias[kTable ? NW * BiasGrad<KS>::WORDS : 1];
     const Shape &s = a.s;
     const int dlim = kNarrow ? s.D : D;  // head dim of the tensors: D, or less in the build for narrow dims
     Sched sc = make_sched(ntiles, blockIdx.x, gridDim.x);
@@ -1119,7 +1125,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     s16x8 qreg[G::DS], gnext[G::DS];
     float lse_cur = 0.f;
     BiasRegs<BF, KS, G::NT> bst;
-    if constexpr (kBias) BiasGrad<KS>::template clear<G::NT>(lds_dbias);
+    if constexpr (kTable) BiasGrad<KS>::template clear<G::NT>(lds_dbias);
     // The last TAIL chunks of a halo are loaded when the arithmetic of the phase is over
     // (fetch_tail): where the registers do not hold a whole halo beside it.
     constexpr int TAIL = kDq2Tail<D, KS, NW>, HEAD = G::NL - TAIL;
@@ -1136,7 +1142,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     auto fetch_q = [&](const ATile &tl, const LaneQ &lq) __attribute__((always_inline)) {
         load_row_chunks(qreg, image_at(a, a.q, tl) + lq.qr * row_step(a, a.q) + lq.qc * col_step(a, a.q), g, dlim);
         lse_cur = a.lse[lq.tok];
-        if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
+        if constexpr (kTable) bst.fetch(a.rpb, tl.nn);
     };
 
     ATile cur = in_sub(tile_of(sc.t, ts.tiles_r, ts.tiles_c, s.N, G::TH), a);
@@ -1175,7 +1181,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
         fetch_tail(a.k, cur, lq);
         __syncthreads();                      // every wave has read V
         halo_commit<D, KS>(lds_x, plan, st);  // K
-        if constexpr (kBias) bst.commit(lds_bias);
+        if constexpr (kTable) bst.commit(lds_bias);
         __syncthreads();
 
         const int tn = sched_peek(sc);
@@ -1192,7 +1198,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
         }
         const float lse2 = lse_cur * kUnit;
         if (FULL || lq.wave_on) {
-            const int bq = kBias ? Bias<KS>::query(lq) : 0;
+            const int bq = kTable ? Bias<KS>::query(lq) : 0;
             Op8 dsb[G::KSTEPS];
             float dpart = 0.f, zsum = 0.f;
 #pragma unroll
@@ -1206,7 +1212,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                 for (int i = 0; i < 4; i++) {
                     const bool ok = G::template tok_in<KS>(mt, g * 4 + i, lq.dr, lq.dc);
                     float x;
-                    if constexpr (kBias) x = cs[i] * sc2 + lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)] - lse2;
+                    if constexpr (kTable) x = cs[i] * sc2 + lds_bias[bq + Bias<KS>::token(mt, g * 4 + i)] - lse2;
                     else x = cs[i] * sc2 - lse2;
                     const float p = exp_unit(ok ? x : -INFINITY);
                     if constexpr (kBias) zsum += p;
@@ -1228,7 +1234,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
             DsScale<BF> scl;
             if constexpr (kBias) {
                 operand_and_sums<BF, KS>(dsb, ds_all, scl, lq.live && delta * 0.f == 0.f ? zinv : 0.f);
-                if (has_table<KS>(a.d_rpb)) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
+                if constexpr (kTable) BiasGrad<KS>::sum(lds_dbias + wave * BiasGrad<KS>::WORDS, ds_all, n, g);
             }
             f32x4 dq[G::DT];
 #pragma unroll
@@ -1245,19 +1251,19 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
                         dq[mt]);
             }
             const unsigned bad = kBias ? bad_columns(dq, delta) : 0u;
-            store_token<BF, D, kLineStores<D, KS, (NW == 4 ? kOneHaloWgs<D, KS> : 1)>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * (kBias ? zinv * scl.inverse() : 1.f), lq.live && !(bad >> n & 1), dlim);
+            store_token<BF, D, kLineStores<D, KS, kDq2Wgs<D, KS, NW>>, FULL>(static_cast<short *>(a.dq) + grad_of(a, cur, lq.qr, lq.qc), g, dq, s.scale * (kBias ? zinv * scl.inverse() : 1.f), lq.live && !(bad >> n & 1), dlim);
             if constexpr (kBias)
                 if (__builtin_expect(bad != 0, 0)) {
                     BiasGrad<KS>::wave_fence();
                     again_dq<BF, KS>(a, cur, lq, bad, lse2, delta, wave,
-                                     lds_dbias + wave * BiasGrad<KS>::WORDS + 4 * BiasGrad<KS>::PLANE, dlim);
+                                     kTable ? lds_dbias + wave * BiasGrad<KS>::WORDS + 4 * BiasGrad<KS>::PLANE : nullptr, dlim);
                 }
             if (FULL || (lq.live && g == 0 && !(bad >> n & 1))) {
                 a.delta[lq.tok] = delta;
-                if constexpr (kBias) row_zinv<KS>(a)[lq.tok] = zinv;
+                if constexpr (kBias) row_zinv(a)[lq.tok] = zinv;
             }
         }
-        if (kBias && has_table<KS>(a.d_rpb)) {
+        if constexpr (kTable) {
             __syncthreads();
             BiasGrad<KS>::template flush<NW>(lds_dbias, a.ds_pairs + (int64_t)sc.t * Bias<KS>::E, cur, s);
         }
@@ -1367,7 +1373,7 @@ __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g
             const ST q = LAZY ? stat(h, i) : st[h][i];
             const bool ok = in(h, i, q);
             float x;
-            if constexpr (kBias) x = cs[h][i] * sc2 + lds_bias[ok ? at(h, i, q) : 0] - q.x;
+            if constexpr (kTable) x = cs[h][i] * sc2 + lds_bias[ok ? at(h, i, q) : 0] - q.x;
             else x = cs[h][i] * sc2 - q.x;
             float p = exp_unit(ok ? x : -INFINITY);
             if constexpr (kBias) p *= zinv_of(q);
@@ -1505,10 +1511,10 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
             const int pr = id / G::HC, pc = id % G::HC;
             if (!ROLL || pr < nr) {
                 const int64_t qt = img_tok + (int64_t)((ROLL ? y0 : br) + pr) * s.W + bc + pc;
-                sst[i] = load_qstat<BF, KS>(a, qt);
+                sst[i] = load_qstat<BF>(a, qt);
             }
         }
-        if constexpr (kBias) bst.fetch(a.rpb, tl.nn);
+        if constexpr (kTable) bst.fetch(a.rpb, tl.nn);
     };
     auto commit = [&](int y0, int nr) __attribute__((always_inline)) {
         if constexpr (ROLL) {
@@ -1534,10 +1540,10 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
                 if (id < G::ZROW) lds_stat[id] = sst[i];
             }
         }
-        if constexpr (kBias) bst.commit(lds_bias);
+        if constexpr (kTable) bst.commit(lds_bias);
     };
     // (entry of this lane's key and a token of its halo: bk - token, see Bias)
-    const int bk = kBias ? ((n >> 2) + KS / 2 + KS + 2) * Bias<KS>::TB + (n & 3) + KS / 2 + KS + 2 : 0;
+    const int bk = kTable ? ((n >> 2) + KS / 2 + KS + 2) * Bias<KS>::TB + (n & 3) + KS / 2 + KS + 2 : 0;
     // B operands of a tile: this lane's key, channels ds*32 + g*8 ..  Loaded when
     // the previous tile's math is over (they would not fit beside it) and complete
     // before the barrier below, i.e. before any newer load is in flight.
@@ -1711,9 +1717,9 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
             const int id = threadIdx.x + i * G::NT;
             const int r = min(b.br + id / G::HC, b.qb - 1), c = min(b.bc + id % G::HC, b.cb - 1);
             const int64_t qt = img_tok + (int64_t)r * s.W + c;
-            sst[i] = load_qstat<BF, KS>(a, qt);
+            sst[i] = load_qstat<BF>(a, qt);
         }
-        if constexpr (kBias) bst.fetch(a.rpb, b.tl.nn);
+        if constexpr (kTable) bst.fetch(a.rpb, b.tl.nn);
     };
     // B operands of the tile: this lane's key, channels ds*32 + g*8 ..
     s16x8 kreg[G::DS], vreg[G::DS];
@@ -1775,7 +1781,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
                 if (id < G::ZROW) lds_stat[to] = make_float4(sst[i].x, sst[i].y, __int_as_float(ws), 0.f);
             }
         }
-        if constexpr (kBias) bst.commit(lds_bias);
+        if constexpr (kTable) bst.commit(lds_bias);
         if (cur.first) {
 #pragma unroll
             for (int mt = 0; mt < G::DT; mt++) {
@@ -1799,7 +1805,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
         const bool wave_on = wr0 < s.H && wc0 < s.W;
         int kr, kc;
         key_of(cur.tl, kr, kc);
-        const int bk = kBias ? (kr - cur.br + KS + 2) * Bias<KS>::TB + (kc - cur.bc + KS + 2) : 0;
+        const int bk = kTable ? (kr - cur.br + KS + 2) * Bias<KS>::TB + (kc - cur.bc + KS + 2) : 0;
         if (wave_on) {
             // this wave's queries inside the staged block: those that attend to any
             // of its 4x4 keys, numbered row-major over their rectangle
@@ -1951,7 +1957,7 @@ __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) v
     // when their walk is over; the counter lies where the general kernels keep 1 / Z per query,
     // and the dQ pass, which runs before this one on the stream, has cleared it.
     __shared__ int lds_tile[2];
-    __shared__ float lds_bias[kBias ? Bias<KS>::WORDS : 1];
+    __shared__ float lds_bias[kTable ? Bias<KS>::WORDS : 1];
     int *tile_ctr = dyn ? reinterpret_cast<int *>(a.zinv) : nullptr;
     if constexpr (!FRAME_ONLY) {
         if ((int)blockIdx.x < inner_blocks) {
@@ -2006,7 +2012,7 @@ template <int D, int KS>
 constexpr bool kTallBuilt =
     D == 64 && KS >= 7 &&
     (size_t)2 * Geo<D, KS, 8>::ROWS * Geo<D, KS, 8>::PITCH * sizeof(short) +
-            (kBias ? Bias<KS>::WORDS * sizeof(float) : 0) <= 160 * 1024;
+            (kTable ? Bias<KS>::WORDS * sizeof(float) : 0) <= 160 * 1024;
 template <int D, int KS>
 constexpr bool kTallDqBuilt = kTallBuilt<D, KS> && KS <= (kBias ? 7 : 9);  // (a bias's planes take LDS too)
 
@@ -2039,15 +2045,15 @@ constexpr bool kFwd2TallBuilt = D == 128 && kOneHaloWgs<D, KS> == 1 && kOneHaloF
                                 (size_t)Geo<D, KS, 8>::ROWS * Geo<D, KS, 8>::PITCH * 2 + 1024 <= 160 * 1024;
 // At head_dim 64 (kernel_size 11 and 13, where one halo of an 8x8 tile fits LDS twice) the one-halo dQ
 // pass takes the 16x8 tiles too: one workgroup of eight waves instead of two of four, a quarter less halo
-// per pixel.  (With a bias, whose planes take LDS too, only at k11.)  B2 N8 128x128 k13 81.5 -> 76.2 us, B4 N8 256x256 626 -> 606, B4 N4 128x128 k11 77.1 -> 76.3.
+// per pixel.  (Not in two terms: the 8x8 tiles have one workgroup per CU and all its registers there.)  B2 N8 128x128 k13 81.5 -> 76.2 us, B4 N8 256x256 626 -> 606, B4 N4 128x128 k11 77.1 -> 76.3.
 template <int D, int KS>
-constexpr bool kDq2TallBuilt = (kFwd2TallBuilt<D, KS> && !kBias) || (D == 64 && KS >= 11 && !(kBias && KS == 13));
+constexpr bool kDq2TallBuilt = !kBias && (kFwd2TallBuilt<D, KS> || (D == 64 && KS >= 11));
 template <int D, int KS>
 constexpr bool kFwd2Built = D == 128 && Geo<D, KS>::WAVES == 1 && kOneHaloFits<D, KS>;
 // Built at all: two halos fit, or the one-halo kernels serve the forward and the dQ pass and
 // the frame body in small blocks the dK/dV pass
 template <int D, int KS>
-constexpr bool kBuilt = fits<D, KS>() || (kFwd2Built<D, KS> && kDq2Built<D, KS>);
+constexpr bool kBuilt = kBias && !kTable ? D == 64 && KS >= 11 : fits<D, KS>() || (kFwd2Built<D, KS> && kDq2Built<D, KS>);
 
 // A frame tile's time in inner tiles in the dK/dV pass at head_dim 128, as the choice of the
 // split takes it (bwd_launch).  Measured over six image sizes from 64x64 to 256x256 with the
@@ -2300,7 +2306,7 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                 // staircase leaves the static split 7% or more behind (B4 N4 128x128 k7: 154.6 ->
                 // 135.4 us; measured 4-9% slower at k9 and at 256x256 and 96x96 k7, where it is
                 // not taken).
-                if (a.zinv != nullptr && (!kBias || a.rpb)) {
+                if (a.zinv != nullptr && kCounter) {
                     int all = grid;
                     if (all > per_i * 8) all = (int)(per_i * 8);
                     double walk;
@@ -2323,7 +2329,7 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                 if (inner_blocks > grid - 8) inner_blocks = grid - 8;
                 if (inner_blocks > (n_inner + 7) / 8 * 8) inner_blocks = (int)((n_inner + 7) / 8 * 8);
             }
-            if (path == ENATTEN_PATH_MFMA_SPLIT_QUEUE && a.zinv != nullptr && (!kBias || a.rpb) && n_frame > 0 && !dyn) {
+            if (path == ENATTEN_PATH_MFMA_SPLIT_QUEUE && a.zinv != nullptr && kCounter && n_frame > 0 && !dyn) {
                 dyn = 1;
                 const int64_t all = (n_inner + 7) / 8 * 8;
                 inner_blocks = all < grid ? (int)all : grid;
@@ -2339,8 +2345,8 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                 hipLaunchKernelGGL((bwd_dkdv_mfma<BF, D, KS, false, SP>), dim3(grid), dim3(NT), 0, st,
                                    a, ts, (int)n_inner, (int)n_frame, inner_blocks, Runs{0, 0}, dyn);
         }
-        if (kBias && a.d_rpb)
-            hipLaunchKernelGGL((rpb_tile_reduce<kBias>), dim3(a.s.N, (Bias<KS>::E + 15) / 16), dim3(1024), 0, st,
+        if constexpr (kTable)
+            hipLaunchKernelGGL((rpb_tile_reduce<kTable>), dim3(a.s.N, (Bias<KS>::E + 15) / 16), dim3(1024), 0, st,
                                a.ds_pairs, a.d_rpb, a.s.B, a.s.N, dq_tiles, Bias<KS>::E);
         return check_launch("enatten2d_bwd");
     } else {

@@ -10,6 +10,7 @@ namespace {
 constexpr bool kNarrow = true;
 constexpr bool kSub = false;
 constexpr bool kBias = false;
+constexpr bool kTable = false;
 }
 }  // namespace enatten
 
