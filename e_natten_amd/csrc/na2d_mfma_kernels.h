@@ -1095,6 +1095,14 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
 // spilled; with 8 chunks behind the arithmetic 110.6 us, with 13 107.5.
 template <int D, int KS, int NW>
 constexpr int kDq2Tail = D == 128 && NW == 8 ? (KS == 13 ? 15 : KS == 11 ? 13 : 0) : 0;
+// Head dims between 32 and 64 with kernel_size 11 and 13 used to run with float32 P and dS on the general
+// kernels.  A window's dS sum to zero, so what its keys have in common cancels in dQ, but only as far as the terms
+// and delta hold (keys and values of mean 32 and deviation 1: dQ 3.9 times as far from float64 as its rounding in
+// bfloat16, 30 times in float16).  So delta's own rounding error is found from the sum that it leaves (`rest`), and
+// what the terms sum to is taken out of dQ with the query's own pixel in the place of every key: within 1% of the
+// rounding for means up to 32, as the general kernels are.  B2 N8 128x128 d64 k13 with a bias: 200 us, without either 206.
+template <int D, int KS>
+constexpr bool kBalanced = kBias && D == 64 && KS >= 11;
 // Workgroups per CU that the registers are budgeted for: one in two terms (and float32 dS beside them),
 // which spills 150 to 340 registers otherwise.  dQ pass with a bias, 16x8 tiles of eight waves, which spill too, -> 8x8
 // tiles: B2 N8 128x128 d64 k11 265 -> 193 us, float16 B3 N5 61x83 91 -> 78.
@@ -1220,14 +1228,26 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDq2Wgs<D, KS, NW>)) void bw
                     put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, p);
                 }
             }
-            const float zinv = kBias ? 1.f / col_sum(zsum) : 1.f, delta = col_sum(dpart) * zinv;
+            const float zinv = kBias ? 1.f / col_sum(zsum) : 1.f;
+            const float most = col_sum(dpart) * zinv;
+            float rest = 0.f;  // delta = most + rest
+            if constexpr (kBalanced<D, KS>) {
+                float e = 0.f;
+#pragma unroll
+                for (int mt = 0; mt < G::MT; mt++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        e = fmaf(get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i), dp[mt][i] - most, e);
+                rest = col_sum(e) * zinv;
+            }
+            const float delta = kBalanced<D, KS> ? most + rest : most;
             f32x4 ds_all[kBias ? Bias<KS>::USED : 1];
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const float p = get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i);
-                    const float ds = p * (dp[mt][i] - delta);
+                    const float ds = p * (kBalanced<D, KS> ? dp[mt][i] - most - rest : dp[mt][i] - delta);
                     if constexpr (!kBias) put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
                     else if (mt < Bias<KS>::USED) ds_all[mt][i] = ds;
                 }
@@ -1239,6 +1259,21 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDq2Wgs<D, KS, NW>)) void bw
             f32x4 dq[G::DT];
 #pragma unroll
             for (int mt = 0; mt < G::DT; mt++) dq[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (kBalanced<D, KS>) {
+                const short one = cvt16<BF>(1.f);
+                f32x4 sum = {0.f, 0.f, 0.f, 0.f};  // (every row is the column's sum)
+#pragma unroll
+                for (int ks = 0; ks < G::KSTEPS; ks++) sum = mfma_op<BF>(s16x8{one, one, one, one, one, one, one, one}, dsb[ks], sum);
+                // this lane's channels of the query's own pixel
+                const short *own = lds_x + ((lq.qr - lq.hr0) * G::HC + lq.qc - lq.hc0) * G::PITCH + g * (D / 4);
+                static_assert(!G::SWZ);
+#pragma unroll
+                for (int h = 0; h < G::DT / 2; h++) {
+                    const s16x8 k8 = *reinterpret_cast<const s16x8 *>(own + 8 * h);
+#pragma unroll
+                    for (int i = 0; i < 8; i++) dq[2 * h + i / 4][i % 4] = -sum[0] * cvt32<BF>(k8[i]);
+                }
+            }
 #pragma unroll
             for (int ks = 0; ks < G::KSTEPS; ks++) {
                 typename G::TRow kp[2];

@@ -23,6 +23,25 @@ def _both(q, k, v, g, rpb, ks, scale):
     return got, [t.detach() for t in (o_ref, *torch.autograd.grad(o_ref, xr, g.double()))]
 
 
+@pytest.mark.parametrize("biased", [False, True])
+@pytest.mark.parametrize("D,ks,hw,dtype", [(40, 13, (27, 30), BF), (48, 11, (32, 29), BF), (56, 11, (26, 37), F16),
+                                           (48, 13, (32, 32), F16)])
+def test_common_components_cancel(D, ks, hw, dtype, biased):
+    # keys and values far from zero: a window's dS sum to zero, and what they fall short of that reaches dQ 32 times.
+    # Besides the rounding of the results there is what float32 leaves of dO . V of some 1e4 (2^-10 in 1e2, the
+    # deviation): 1% of float16's rounding
+    ensure_built()
+    print("case common components", D, ks, hw, dtype, biased, flush=True)
+    q, k, v, g = make_inputs((1, 2, *hw, D), torch.float32, seed=D + ks)
+    q, k, v, g = q.to(dtype), (k + 32).to(dtype), (v + 32).to(dtype), (g + 8).to(dtype)
+    got, ref = _both(q, k, v, g, _rpb(2, ks).to(dtype) if biased else None, ks, D ** -0.5)
+    for name, x, r in list(zip(NAMES, got, ref))[:4]:
+        norm = ((x - r).norm() / r.norm()).item()
+        rounding = ((r.to(dtype).double() - r).norm() / r.norm()).item()
+        print("   ", name, "2-norm %.2e, of the result's rounding alone %.2e" % (norm, rounding), flush=True)
+        assert norm <= 1.02 * rounding, (name, norm, rounding)
+
+
 @pytest.mark.parametrize("which", ["q", "k", "v", "dO"])
 @pytest.mark.parametrize("D,ks,hw,dtype", [
     (48, 11, (43, 38), BF), (40, 13, (44, 44), F16),   # inner tiles and border
