@@ -1100,7 +1100,8 @@ constexpr int kDq2Tail = D == 128 && NW == 8 ? (KS == 13 ? 15 : KS == 11 ? 13 : 
 // and delta hold (keys and values of mean 32 and deviation 1: dQ 3.9 times as far from float64 as its rounding in
 // bfloat16, 30 times in float16).  So delta's own rounding error is found from the sum that it leaves (`rest`), and
 // what the terms sum to is taken out of dQ with the query's own pixel in the place of every key: within 1% of the
-// rounding for means up to 32, as the general kernels are.  B2 N8 128x128 d64 k13 with a bias: 200 us, without either 206.
+// rounding for means up to 32, as the general kernels are. B2 N8 128x128 d48 k13 118 -> 133 us.
+// (BALANCED; head_dim 64 itself, with a bias, is built without.)
 template <int D, int KS>
 constexpr bool kBalanced = kBias && D == 64 && KS >= 11;
 // Workgroups per CU that the registers are budgeted for: one in two terms (and float32 dS beside them),
@@ -1109,7 +1110,7 @@ constexpr bool kBalanced = kBias && D == 64 && KS >= 11;
 template <int D, int KS, int NW>
 constexpr int kDq2Wgs = NW == 4 && !(kBias && D == 64) ? kOneHaloWgs<D, KS> : 1;
 // FULL: as in fwd_mfma.
-template <bool BF, int D, int KS, int NW = 4, bool FULL = false>
+template <bool BF, int D, int KS, int NW = 4, bool FULL = false, bool BALANCED = kBalanced<D, KS> && !kTable>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDq2Wgs<D, KS, NW>)) void bwd_dq2_mfma(BArgs a, TileSet ts, int ntiles) {
     // (the dK/dV pass that follows on the stream counts its frame tiles here, from zero)
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.zinv && kCounter) *reinterpret_cast<int *>(a.zinv) = 0;
@@ -1231,7 +1232,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDq2Wgs<D, KS, NW>)) void bw
             const float zinv = kBias ? 1.f / col_sum(zsum) : 1.f;
             const float most = col_sum(dpart) * zinv;
             float rest = 0.f;  // delta = most + rest
-            if constexpr (kBalanced<D, KS>) {
+            if constexpr (BALANCED) {
                 float e = 0.f;
 #pragma unroll
                 for (int mt = 0; mt < G::MT; mt++)
@@ -1240,14 +1241,14 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDq2Wgs<D, KS, NW>)) void bw
                         e = fmaf(get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i), dp[mt][i] - most, e);
                 rest = col_sum(e) * zinv;
             }
-            const float delta = kBalanced<D, KS> ? most + rest : most;
+            const float delta = BALANCED ? most + rest : most;
             f32x4 ds_all[kBias ? Bias<KS>::USED : 1];
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const float p = get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i);
-                    const float ds = p * (kBalanced<D, KS> ? dp[mt][i] - most - rest : dp[mt][i] - delta);
+                    const float ds = p * (dp[mt][i] - most - rest);
                     if constexpr (!kBias) put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
                     else if (mt < Bias<KS>::USED) ds_all[mt][i] = ds;
                 }
@@ -1259,7 +1260,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDq2Wgs<D, KS, NW>)) void bw
             f32x4 dq[G::DT];
 #pragma unroll
             for (int mt = 0; mt < G::DT; mt++) dq[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if constexpr (kBalanced<D, KS>) {
+            if constexpr (BALANCED) {
                 const short one = cvt16<BF>(1.f);
                 f32x4 sum = {0.f, 0.f, 0.f, 0.f};  // (every row is the column's sum)
 #pragma unroll
@@ -2252,7 +2253,10 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
         }
         if constexpr (kDq2Built<D, KS>) {
             if (!dq_done) {
-                const int grid = persistent_grid<bwd_dq2_mfma<BF, D, KS>>(nb);
+                constexpr bool BOTH = kBalanced<D, KS> && kTable;  // head_dim 64, or below
+                const bool balanced = BOTH && a.s.D < D;
+                const int grid = balanced ? persistent_grid<bwd_dq2_mfma<BF, D, KS, 4, false, BOTH || (kBalanced<D, KS> && !kTable)>>(nb)
+                                          : persistent_grid<bwd_dq2_mfma<BF, D, KS>>(nb);
                 ProfScope prof(ENATTEN_KERNEL_BWD_DQ, "bwd_dq2_mfma", st);
                 if (kDq2Full<D, KS> && a.s.H % G::TH == 0 && a.s.W % G::TW == 0)
                     hipLaunchKernelGGL((bwd_dq2_mfma<BF, D, KS, 4, kDq2Full<D, KS>>), dim3(grid), dim3(256), 0, st,
@@ -2290,6 +2294,9 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                 else
                     hipLaunchKernelGGL((bwd_dq_mfma<BF, D, KS, false, kRollBuilt<D>>), dim3(grid),
                                        dim3(256), 0, st, a, ts, (int)nb, plan_runs(nb, grid, tiles_r));
+                else if (balanced)
+                    hipLaunchKernelGGL((bwd_dq2_mfma<BF, D, KS, 4, false, BOTH || (kBalanced<D, KS> && !kTable)>), dim3(grid),
+                                       dim3(256), 0, st, a, ts, (int)nb);
             } else if (full) {
                 hipLaunchKernelGGL((bwd_dq_mfma<BF, D, KS, false, false, 4, !kNarrow>), dim3(grid), dim3(256), 0,
                                    st, a, ts, (int)nb, Runs{0, 0});
