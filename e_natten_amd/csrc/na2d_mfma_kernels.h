@@ -2091,13 +2091,46 @@ constexpr bool kFwd2Built = D == 128 && Geo<D, KS>::WAVES == 1 && kOneHaloFits<D
 template <int D, int KS>
 constexpr bool kBuilt = kBias && !kTable ? D == 64 && KS >= 11 : fits<D, KS>() || (kFwd2Built<D, KS> && kDq2Built<D, KS>);
 
-// A frame tile's time in inner tiles in the dK/dV pass at head_dim 128, as the choice of the
-// split takes it (bwd_launch).  Measured over six image sizes from 64x64 to 256x256 with the
-// weights 0.8 to 4.0: 1.3 and 1.6 are within 1% of each other at k = 3, 5 and 7; at k = 9, where
-// the frame is two tiles wide, 2.0 is the best or within 3% of it everywhere (B4 N4 128x128: 227 us
-// with 1.15, 245 with 1.6, 176 with 2.0; B2 N2 256x256: 223, 167, 155).
+// A frame tile's time in inner tiles in the dK/dV pass, as the choice of the split takes it (bwd_launch).  At
+// head_dim 128 the walks of the inner side are a staircase, and so are the times: with weights 1.0 to 2.0 over
+// ten image sizes from 56x56 to 256x256, with a bias and without, these lose no size 3% against any other that gains on most.
+// k9 2.0 -> 1.9: B4 N4 128x128 173 -> 158 us, 112x112 142 -> 120, B4 N8 96x96 215 -> 183, with a bias 277 -> 250, 224 ->
+// 189, 342 -> 293, others level; (1.7 and 1.8 gain there too and lose B1 N4 90x140 20%).  k3 1.3 -> 1.4: B3 N5 61x83 23.3 ->
+// 21.6, with a bias 49 -> 40; k5 1.45 -> 1.5: 75x75 20.2 -> 16.8; others level.
 template <int KS>
-constexpr double kFrameCost128 = KS >= 9 ? 2.0 : KS == 5 ? 1.45 : 1.3;
+constexpr double kFrameCost128 = KS >= 9 ? 1.9 : KS == 7 ? 1.3 : KS == 5 ? 1.5 : 1.4;
+// ... and below that, measured by timing every split at eleven image sizes from 40x40 to 256x256, batch times
+// heads 4 to 64.  Without a bias 2 at head_dim 64 (1.68 with the frame body's larger blocks) and 2.5 at head_dim 32
+// are within 2% of the best weight in the mean.  With a bias an inner tile is dearer against a frame tile: dK/dV pass with the
+// weights below and share_inner against 2, 1.68 and 2.5 in proportion, in the mean over the sizes, bf16 / float16, head_dim
+// 64 k3 -6 / -6%, k5 -3 / -5, k7 -6 / -5, k9 -10 / -11, k11 -5 / -3, k13 -3 / 0, head_dim 32 k3 -2, k5 -2 / -2, k7 -8 / -7,
+// k11 -10 / -10, k13 -13 / -10; the size that loses most 4%.  (k9 at head_dim 32: every other weight loses some size
+// 6 to 13%.)
+template <bool BF, int D, int KS>
+constexpr double kFrameCostBias = D == 64 ? (KS == 13 && (!BF || !kTable) ? 1.75 : 1.5)
+                                          : KS == 3 ? 2.1 : KS == 5 ? 2.3 : KS == 7 ? 2.0 : KS == 9 ? 2.5 : 1.9;
+template <bool BF, int D, int KS, bool LARGE>
+constexpr double kFrameCost = D >= 128 ? kFrameCost128<KS>
+                              : kBias ? kFrameCostBias<BF, D, KS>
+                              : LARGE ? 1.68 : D == 32 ? 2.5 : 2.0;
+// With a bias, of `grid` workgroups those on inner tiles.  A workgroup has whole tiles, so a share in proportion may
+// leave one side a tile longer than the other; whole tiles alone would not count that workgroups which end early
+// leave the CU to the others.  So it is the split whose longer side is the shortest by the mean of both: level with the
+// proportion at head_dim 64, 2% faster in the mean at head_dim 32 (B8 N4 56x56 d32 k7 26.4 -> 21.4 us).
+inline int share_inner(int64_t n_inner, int64_t n_frame, int grid, double cost) {
+    const int64_t per_i = (n_inner + 7) / 8, per_f = (n_frame + 7) / 8;
+    double best = 1e30;
+    int inner = 8;
+    for (int ib = 8; ib <= grid - 8 && ib <= per_i * 8; ib += 8) {
+        auto side = [](int64_t tiles, int64_t slots) { return (double)tiles / slots + (double)((tiles + slots - 1) / slots); };
+        const double i = side(per_i, ib / 8), f = cost * side(per_f, (grid - ib) / 8), t = i > f ? i : f;
+        if (t < best) {
+            best = t;
+            inner = ib;
+        }
+    }
+    return inner;
+}
 template <int D, int KS>
 constexpr int kDkdvSplit = D == 64 && Geo<D, KS>::WAVES == 1 ? 2 : 1;
 
@@ -2261,6 +2294,9 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                 if (kDq2Full<D, KS> && a.s.H % G::TH == 0 && a.s.W % G::TW == 0)
                     hipLaunchKernelGGL((bwd_dq2_mfma<BF, D, KS, 4, kDq2Full<D, KS>>), dim3(grid), dim3(256), 0, st,
                                        a, ts, (int)nb);
+                else if (balanced)
+                    hipLaunchKernelGGL((bwd_dq2_mfma<BF, D, KS, 4, false, BOTH || (kBalanced<D, KS> && !kTable)>), dim3(grid),
+                                       dim3(256), 0, st, a, ts, (int)nb);
                 else
                     hipLaunchKernelGGL((bwd_dq2_mfma<BF, D, KS>), dim3(grid), dim3(256), 0, st, a, ts, (int)nb);
                 dq_done = true;
@@ -2294,9 +2330,6 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                 else
                     hipLaunchKernelGGL((bwd_dq_mfma<BF, D, KS, false, kRollBuilt<D>>), dim3(grid),
                                        dim3(256), 0, st, a, ts, (int)nb, plan_runs(nb, grid, tiles_r));
-                else if (balanced)
-                    hipLaunchKernelGGL((bwd_dq2_mfma<BF, D, KS, 4, false, BOTH || (kBalanced<D, KS> && !kTable)>), dim3(grid),
-                                       dim3(256), 0, st, a, ts, (int)nb);
             } else if (full) {
                 hipLaunchKernelGGL((bwd_dq_mfma<BF, D, KS, false, false, 4, !kNarrow>), dim3(grid), dim3(256), 0,
                                    st, a, ts, (int)nb, Runs{0, 0});
@@ -2307,12 +2340,9 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
         }
         {
             // Share the resident workgroups between the two bodies so that they end together.
-            // `cost` is a frame tile's time in inner tiles (measured): 2 at head_dim 64 (1.68 with
-            // the frame body's larger blocks), 2.5 at head_dim 32 (against 2: B8 N2 112x112 k7
-            // 28.7 -> 27.1 us, B8 N4 56x56 20.8 -> 18.6, B4 N4 128x128 k5 27.1 -> 25.4, k3 23.1 ->
-            // 21.5; 2-4% slower at 96x96 and 256x256 k7), kFrameCost128 at head_dim 128.
+            // `cost` is a frame tile's time in inner tiles (kFrameCost).
             constexpr int SP = kDkdvSplit<D, KS>, NT = Geo<D, KS, 4, SP>::NT;
-            const double cost = D >= 128 ? kFrameCost128<KS> : kFrameKS<D, KS, SP> != KS ? 1.68 : D == 32 ? 2.5 : 2.0;
+            const double cost = kFrameCost<BF, D, KS, kFrameKS<D, KS, SP> != KS>;
             const int grid = persistent_grid<bwd_dkdv_mfma<BF, D, KS, false, SP>>(nb, NT);
             int inner_blocks = 0, dyn = 0;
             if (n_frame == 0) {
@@ -2364,6 +2394,8 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                         inner_blocks = all;
                     }
                 }
+            } else if (n_inner > 0 && kBias && !(D == 32 && KS == 9)) {
+                inner_blocks = share_inner(n_inner, n_frame, grid, cost);
             } else if (n_inner > 0) {
                 const double f = (double)n_inner / ((double)n_inner + cost * (double)n_frame);
                 inner_blocks = (int)(f * grid / 8.0 + 0.5) * 8;
