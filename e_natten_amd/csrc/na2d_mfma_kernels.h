@@ -1357,8 +1357,8 @@ __device__ __forceinline__ bool next_block(KeyBlock &b) {
 // alone in the frame body's rolled loop the compiler reads the statistics of one query after the
 // other, each behind a wait of its own for LDS, 16 round trips in a row per step at 2 waves per
 // SIMD; the inner body is unrolled and has the next step's arithmetic to put between, so there 1
-// and 2 only cost registers (d128 k5 with its column walk spills with them, 107 -> 222 us), but for
-// head_dim 32, where 2 is ahead (B4 N4 128x128 k9 51.6 -> 48.8 us).
+// and 2 only cost registers (d128 k5 with its column walk spills with them, 107 -> 222 us; not tried at
+// head_dim 64), but for head_dim 32, where 2 is ahead (B4 N4 128x128 k9 51.6 -> 48.8 us).
 // With a bias at head_dim 32 the 7x7 and 9x9 windows run at two waves per SIMD anyway (kDkdvWaves), which leaves
 // registers for both tiles in both bodies: B8 N4 56x56 d32 k7 28.9 -> 27.6 us, B8 N2 112x112 k9 66.9 -> 66.5.
 //   a_of(h), t_of(h): this lane's row of tile h for the direct and for the transposing reads
@@ -1382,25 +1382,31 @@ __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g
     float dsv[8], mag = 0.f;  // (float16 with a bias)
     s16x8 qa[2][G::DS], ga[2][G::DS];
     ST st[2][4];
+    auto chunk = [&](const typename G::ARow &row, int ds) __attribute__((always_inline)) {
+        return *reinterpret_cast<const s16x8 *>(G::a_at(row, ds));
+    };
     auto read = [&](int h) __attribute__((always_inline)) {
+        if constexpr (LAZY) return;
         const int row = a_of(h);
         const typename G::ARow qp = G::a_row(lds_q, row, g), gp = G::a_row(lds_g, row, g);
 #pragma unroll
         for (int ds = 0; ds < G::DS; ds++) {
-            qa[h][ds] = *reinterpret_cast<const s16x8 *>(G::a_at(qp, ds));
-            ga[h][ds] = *reinterpret_cast<const s16x8 *>(G::a_at(gp, ds));
+            qa[h][ds] = chunk(qp, ds);
+            ga[h][ds] = chunk(gp, ds);
         }
 #pragma unroll
-        for (int i = 0; i < 4 && !LAZY; i++) st[h][i] = stat(h, i);
+        for (int i = 0; i < 4; i++) st[h][i] = stat(h, i);
     };
     f32x4 cs[2], cp[2];
     auto first = [&](int h) __attribute__((always_inline)) {
+        const int row = LAZY ? a_of(h) : 0;
+        const typename G::ARow qp = G::a_row(lds_q, row, g), gp = G::a_row(lds_g, row, g);
         cs[h] = f32x4{0.f, 0.f, 0.f, 0.f};
         cp[h] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ds = 0; ds < G::DS; ds++) {
-            cs[h] = mfma16<BF>(qa[h][ds], kreg[ds], cs[h]);
-            cp[h] = mfma16<BF>(ga[h][ds], vreg[ds], cp[h]);
+            cs[h] = mfma16<BF>(LAZY ? chunk(qp, ds) : qa[h][ds], kreg[ds], cs[h]);
+            cp[h] = mfma16<BF>(LAZY ? chunk(gp, ds) : ga[h][ds], vreg[ds], cp[h]);
         }
     };
     auto weights = [&](int h) __attribute__((always_inline)) {
@@ -1443,32 +1449,18 @@ __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g
         fence();
         weights(0);
         weights(1);
-    } else if constexpr (AHEAD < 0) {
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int row = a_of(h);
-            const typename G::ARow qp = G::a_row(lds_q, row, g), gp = G::a_row(lds_g, row, g);
-            cs[h] = f32x4{0.f, 0.f, 0.f, 0.f};
-            cp[h] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ds = 0; ds < G::DS; ds++) {
-                cs[h] = mfma16<BF>(*reinterpret_cast<const s16x8 *>(G::a_at(qp, ds)), kreg[ds], cs[h]);
-                cp[h] = mfma16<BF>(*reinterpret_cast<const s16x8 *>(G::a_at(gp, ds)), vreg[ds], cp[h]);
-            }
-            weights(h);
-        }
-        turn_rows(0);
-        turn_rows(1);
     } else {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             read(h);
             fence();
             first(h);
-            turn_rows(h);
+            if constexpr (!LAZY) turn_rows(h);
             fence();
             weights(h);
         }
+#pragma unroll
+        for (int h = 0; h < 2 && LAZY; h++) turn_rows(h);
     }
     if constexpr (kBias) {  // (no registers for more rows than the next product needs)
         if constexpr (!BF) put_scaled<BF>(dsb, dsv, mag, scl, dk);
@@ -1951,10 +1943,9 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
 // Waves per SIMD that the dK/dV pass budgets its registers for: three where LDS admits
 // three workgroups per CU (head_dim <= 64 with small halos; it fits 168 registers there,
 // measured 35 -> 32 us at B8 N2 112x112 d32 k7 and 67 -> 60 us at B4 N4 128x128 d32 k9;
-// the forward and the dQ pass spill under that budget and get slower; with a bias so does this
-// one
-// from kernel_size 7 on and at head_dim 64: B8 N8 64x64 d64 k5 60 us with two waves, 84 with three, B8 N4 56x56 d32 k7 28.6
-// and 34.4; B8 N2 112x112 d32 k5 34.1 and 27.1).
+// the forward and the dQ pass spill under that budget and get slower).  With a bias this pass
+// spills too, at head_dim 64 and from kernel_size 7 on: two and three waves B8 N8 64x64 d64 k5 60
+// us and 84, B8 N4 56x56 d32 k7 28.6 and 34.4, but B8 N2 112x112 d32 k5 34.1 and 27.1.
 // Size of the frame body's blocks as a kernel size (see dkdv_frame): larger than KS where the
 // pass has one workgroup per CU anyway (two parts per block) and LDS has the room.
 // Where not even one workgroup's Q and dO halos fit LDS (head_dim 128 with kernel_size 11 and
