@@ -90,8 +90,8 @@ bool use_mfma(int D, int ks, int dtype) {
 }
 // Head dims between 32 and 64 with kernel_size 11 and 13: the kernels for a relative position bias, and
 // without one their build without a table (two terms for P and dS, 1 / Z, values that are not finite stay in
-// their windows).  bf16, forward and backward, us, general -> these: B1 N16 162x174 d48 k11 4050 -> 592, with a
-// bias 5800 -> 750; B2 N8 128x128 d48 k13 3090 -> 342, with a bias 4570 -> 480.
+// their windows).  bf16, forward and backward, us, general -> these: B1 N16 162x174 d48 k11 4050 -> 614, with a
+// bias 5800 -> 768; B2 N8 128x128 d48 k13 3090 -> 357, with a bias 4570 -> 495.
 bool use_two_terms(int D, int ks, int dtype) {
     return g_path.load() != ENATTEN_PATH_SIMT && (dtype == ENATTEN_BF16 || dtype == ENATTEN_F16) && D > 32 && D < 64 &&
            D % 8 == 0 && (ks == 11 || ks == 13);

@@ -3,7 +3,7 @@
 // centred windows.
 //
 // B8 N4 56x56 d32 k7 bf16, views of a projection: 68 + 103 + 171 us of general kernels and 61 us for
-// the bias gradient before, 16 + 30 + 27 + 5 us here, under the profiler.  What the bias costs is LDS work:
+// the bias gradient before, 16 + 30 + 25 + 5 us here, under the profiler.  What the bias costs is LDS work:
 // a table read per logit, 28 plane writes and 48 reads per lane and tile for the gradient; the second
 // terms of P and dS double the second products.
 #include "na2d_common.h"

@@ -1100,8 +1100,8 @@ constexpr int kDq2Tail = D == 128 && NW == 8 ? (KS == 13 ? 15 : KS == 11 ? 13 : 
 // and delta hold (keys and values of mean 32 and deviation 1: dQ 3.9 times as far from float64 as its rounding in
 // bfloat16, 30 times in float16).  So delta's own rounding error is found from the sum that it leaves (`rest`), and
 // what the terms sum to is taken out of dQ with the query's own pixel in the place of every key: within 1% of the
-// rounding for means up to 32, as the general kernels are. B2 N8 128x128 d48 k13 118 -> 133 us.
-// (BALANCED; head_dim 64 itself, with a bias, is built without.)
+// rounding for means up to 32, as the general kernels are.  B2 N8 128x128 d48 k13 118 -> 131 us.
+// (BALANCED; head_dim 64 itself, with a bias, is built without: float16 k13 214 us, 226 with it.)
 template <int D, int KS>
 constexpr bool kBalanced = kBias && D == 64 && KS >= 11;
 // Workgroups per CU that the registers are budgeted for: one in two terms (and float32 dS beside them),
