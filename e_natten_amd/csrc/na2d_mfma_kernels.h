@@ -2095,7 +2095,7 @@ constexpr double kFrameCost128 = KS >= 9 ? 1.9 : KS == 7 ? 1.3 : KS == 5 ? 1.5 :
 // are within 2% of the best weight in the mean.  With a bias an inner tile is dearer against a frame tile: dK/dV pass with the
 // weights below and share_inner against 2, 1.68 and 2.5 in proportion, in the mean over the sizes, bf16 / float16, head_dim
 // 64 k3 -6 / -6%, k5 -3 / -5, k7 -6 / -5, k9 -10 / -11, k11 -5 / -3, k13 -3 / 0, head_dim 32 k3 -2, k5 -2 / -2, k7 -8 / -7,
-// k11 -10 / -10, k13 -13 / -10; the size that loses most 4%.  (k9 at head_dim 32: every other weight loses some size
+// k11 -10 / -10, k13 -13 / -10; the size that loses most 7% (B4 N4 96x96 d64 k5).  (k9 at head_dim 32: every other weight loses some size
 // 6 to 13%.)
 template <bool BF, int D, int KS>
 constexpr double kFrameCostBias = D == 64 ? (KS == 13 && (!BF || !kTable) ? 1.75 : 1.5)
@@ -2277,16 +2277,16 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
         }
         if constexpr (kDq2Built<D, KS>) {
             if (!dq_done) {
-                constexpr bool BOTH = kBalanced<D, KS> && kTable;  // head_dim 64, or below
-                const bool balanced = BOTH && a.s.D < D;
-                const int grid = balanced ? persistent_grid<bwd_dq2_mfma<BF, D, KS, 4, false, BOTH || (kBalanced<D, KS> && !kTable)>>(nb)
+                // (without a table only dims below D come here, and the default is that)
+                const bool balanced = kBalanced<D, KS> && a.s.D < D;
+                const int grid = balanced ? persistent_grid<bwd_dq2_mfma<BF, D, KS, 4, false, kBalanced<D, KS>>>(nb)
                                           : persistent_grid<bwd_dq2_mfma<BF, D, KS>>(nb);
                 ProfScope prof(ENATTEN_KERNEL_BWD_DQ, "bwd_dq2_mfma", st);
                 if (kDq2Full<D, KS> && a.s.H % G::TH == 0 && a.s.W % G::TW == 0)
                     hipLaunchKernelGGL((bwd_dq2_mfma<BF, D, KS, 4, kDq2Full<D, KS>>), dim3(grid), dim3(256), 0, st,
                                        a, ts, (int)nb);
                 else if (balanced)
-                    hipLaunchKernelGGL((bwd_dq2_mfma<BF, D, KS, 4, false, BOTH || (kBalanced<D, KS> && !kTable)>), dim3(grid),
+                    hipLaunchKernelGGL((bwd_dq2_mfma<BF, D, KS, 4, false, kBalanced<D, KS>>), dim3(grid),
                                        dim3(256), 0, st, a, ts, (int)nb);
                 else
                     hipLaunchKernelGGL((bwd_dq2_mfma<BF, D, KS>), dim3(grid), dim3(256), 0, st, a, ts, (int)nb);
