@@ -8,20 +8,24 @@
 // dO.V, dS.K, P^T.dO, dS^T.Q) with the float32 one, v_mfma_f32_16x16x4_f32: true
 // float32 products, no reduced-precision operands anywhere.
 //
-// Geometry as in the 16-bit kernels: a workgroup of four waves owns an 8x8 tile of
-// pixels, a wave a 4x4 block; the wave's 16 pixels are the N dimension of the matrix
-// instructions, the (4+k-1)^2 pixels of its halo the token dimension.  One tensor's
-// halo at a time is staged in LDS (float32 rows of D + 4 floats), so two workgroups
-// share a CU; the other tensor's halo travels from HBM into registers meanwhile.
+// Geometry.  A workgroup of four waves owns an 8x8 tile of pixels, a wave a 4x4 block of it as four blocks of
+// 2x2.  The matrix instructions are those of four (float64) and sixteen (float32) independent 4x4 products,
+// v_mfma_f64_4x4x4_4b_f64 and v_mfma_f32_4x4x1_16b_f32: each 2x2 block of queries meets the (k+1)^2 pixels that
+// its own windows reach, where a 16-wide instruction has the whole 4x4 block meet (k+3)^2 and more: 36 tokens per
+// query instead of 64 at kernel_size 5 (25 are in its window), 16 instead of 48 at 3, 64 instead of 112 at 7.
+// Both shapes run at the rate of the 16-wide ones (16 and 32 products per cycle and SIMD: measured 17.0 and 9.3
+// cycles against 66.1 and 33.0).  Forward, dQ and dK/dV pass, us, 4x4 blocks on the 16-wide instructions -> 2x2 blocks:
+// B4 N4 128x128 d128 k5 160 + 226 + 188 -> 133 + 181 + 177; 96x96 d64 k3 36 + 48 + 39 -> 25 + 33 + 32, k7 72 + 120 + 95 ->
+// 59 + 90 + 93; B4 N8 96x96 d32 k5 52 + 74 + 63 -> 42 + 61 + 49.  What bounds them: HBM at 4.2 TB/s in the forward and the
+// dQ pass, where a tile's two staging phases issue no matrix instruction.  One tensor's halo at a time is staged in LDS (float32 rows of D + 4 floats), so two
+// workgroups share a CU; the other tensor's halo travels from HBM into registers meanwhile.
 //
-// Token numbering.  The float64 instruction leaves lane (n, g) with rows g, g+4, g+8,
-// g+12 of a 16-row tile, the float32 one with rows 4g .. 4g+3.  Token t of a 16-token
-// tile is the pixel (t & 3, t >> 2) of a 4x4 patch of the halo when the halo side is a
-// multiple of 4 (kernel_size 5, 9, 13), so the four tokens of one reduction step of
-// the second products (g = 0..3) sit in four different halo rows, 12 LDS rows apart,
-// and their operand reads fall into disjoint banks; for other kernel sizes tokens are
-// numbered row by row.  Where a float32 product has to line up with the float64 one
-// (dP with P), its operand rows are fetched in the transposed order t -> 4(t&3) + t>>2.
+// Lanes.  A lane is (g, b, j) = (lane >> 4, lane >> 2 & 3, lane & 3): block b of the wave, pixel j of the
+// block.  The (k+1)^2 tokens of a block are numbered in 2x2 patches: token i of patch t lies at a constant distance
+// from the block's first one, so operand addresses are one register and immediate offsets.
+// The float64 product takes channel g of four as its reduction index and leaves lane (g, b, j) with token g of
+// every patch; the float32 products take g as a quarter of the channels, in the first product as a part of
+// the reduction (summed over the lane groups afterwards), in the second one as rows of the result.
 //
 // Backward.  The dQ pass recomputes the logits once (float64), forms P, dP, dS and dQ,
 // and leaves P and dS of every (query, window position) in the workspace, k*k float32
@@ -33,49 +37,33 @@
 //
 // Per-query math: e_natten/triton.py:242-302 (forward), :383-423 (backward).
 
+#include <numeric>
+#include <utility>
+
 #include "na2d_mfma.h"
 
 namespace enatten {
 namespace {
 
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-
 template <int D, int KS>
 struct Geo32 {
     static constexpr int HR = 8 + KS - 1, HC = HR;   // halo of the 8x8 tile
-    static constexpr int SW = 4 + KS - 1;            // halo side of a wave's 4x4 block
-    static constexpr bool PATCH = SW % 4 == 0;
-    static constexpr int NK = SW * SW;
-    static constexpr int NKP = (NK + 15) / 16 * 16;
-    static constexpr int MT = NKP / 16;              // 16-token tiles
+    static constexpr int PW = (KS + 1) / 2;          // 2x2 patches on a side of a block's halo
+    static constexpr int T = PW * PW;                // patches
     static constexpr int KK = KS * KS;
     static constexpr int PITCH = D + 4;              // floats between LDS rows
-    static constexpr int ROWS = HR * HC + 1;         // + an all-zero row for padding tokens
-    static constexpr int ZROW = HR * HC;
+    static constexpr int ROWS = HR * HC;
     static constexpr int CPR = D / 4;                // 16-byte chunks per row
     static constexpr int NCH = HR * HC * CPR;
     static constexpr int NL = (NCH + 255) / 256;     // chunks per thread
     static constexpr int DQ = D / 4;                 // channels per lane group in the first products
-    static constexpr int DT = D / 16;                // 16-channel tiles of the outputs
+    static constexpr int DT = D / 16;                // 16-channel pieces of the outputs
+    static constexpr int STEPS = T * 4;              // tokens of a block: reduction steps of the second products
     static constexpr size_t LDS_BYTES = (size_t)ROWS * PITCH * sizeof(float);
-    // (row, column) inside the wave's halo of token t of tile mt; false: no such token
-    static __device__ __forceinline__ bool tok_rc(int mt, int t, int &r, int &c) {
-        if constexpr (PATCH) {
-            constexpr int PR = SW / 4;
-            r = 4 * (mt / PR) + (t & 3);
-            c = 4 * (mt % PR) + (t >> 2);
-            return true;
-        } else {
-            const int tk = mt * 16 + t;
-            r = tk / SW;
-            c = tk % SW;
-            return tk < NK;
-        }
-    }
-    static __device__ __forceinline__ int tok_row(int mt, int t, int orow, int ocol) {
-        int r, c;
-        return tok_rc(mt, t, r, c) ? (orow + r) * HC + ocol + c : (int)ZROW;
-    }
+    // floats from a block's first token to token i of patch t, and its row and column there
+    static constexpr int row(int t, int i) { return 2 * (t / PW) + (i >> 1); }
+    static constexpr int col(int t, int i) { return 2 * (t % PW) + (i & 1); }
+    static constexpr int at(int t, int i) { return (row(t, i) * HC + col(t, i)) * PITCH; }
 };
 
 // Whole-line stores (store32's LINES) where LDS admits two workgroups per CU: like the 16-bit
@@ -100,50 +88,43 @@ struct Regs32 {
     u32x4 v[25];
 };
 
-// One tensor's halo (origin (hr0, hc0), pixels at or beyond (rlim, clim) clamped) into
-// registers, then into LDS.
+// Pixel of chunk i of this thread in the halo.  Every PER chunks the threads' pixels are RPER whole rows further
+// down, so a thread has PER columns and as many rows to keep instead of one for every chunk.
 template <int D, int KS>
-__device__ __forceinline__ void fetch32(Regs32 &reg, const float *img, int64_t sh, int64_t sw,
-                                        int hr0, int hc0, int rlim, int clim) {
+__device__ __forceinline__ void chunk_pixel(int i, unsigned &r, unsigned &c) {
+    using G = Geo32<D, KS>;
+    constexpr int STEP = 256 / G::CPR, PER = std::lcm(STEP, G::HC) / STEP, RPER = std::lcm(STEP, G::HC) / G::HC;
+    const unsigned pix = threadIdx.x / G::CPR + i % PER * STEP;
+    r = pix / G::HC + i / PER * RPER;
+    c = pix % G::HC;
+}
+// One tensor's halo (origin (hr0, hc0), pixels at or beyond (rlim, clim) clamped) into
+// registers, then into LDS, in PARTS slices, so that the loads can be issued a few at a time between
+// matrix instructions (a wave that issues a whole halo at once is blocked for
+// microseconds while the CU's memory queue takes the loads, and issues no matrix
+// instruction meanwhile).
+template <int D, int KS, int PARTS>
+__device__ __forceinline__ void fetch32_part(Regs32 &reg, const float *img, int64_t sh, int64_t sw,
+                                             int hr0, int hc0, int rlim, int clim, int part) {
     using G = Geo32<D, KS>;
     static_assert(G::NL <= 25, "staging registers");
     const char *base = reinterpret_cast<const char *>(img + hr0 * sh + hc0 * sw);
     const unsigned sh4 = (unsigned)sh * 4u, sw4 = (unsigned)sw * 4u;
-    const int rmax = rlim - 1 - hr0, cmax = clim - 1 - hc0;
+    const unsigned rmax = rlim - 1 - hr0, cmax = clim - 1 - hc0;
 #pragma unroll
     for (int i = 0; i < G::NL; i++) {
-        int pix = (int)threadIdx.x / G::CPR + i * (256 / G::CPR);
-        pix = pix < G::HR * G::HC ? pix : G::HR * G::HC - 1;
-        const unsigned r = (unsigned)min(pix / G::HC, rmax), c = (unsigned)min(pix % G::HC, cmax);
-        const unsigned off = __umul24(r, sh4) + __umul24(c, sw4) + ((unsigned)threadIdx.x % G::CPR) * 16u;
+        if (i * PARTS / G::NL != part) continue;
+        unsigned r, c;
+        chunk_pixel<D, KS>(i, r, c);  // (beyond the last pixel: a row below the halo, clamped like the others)
+        const unsigned off = __umul24(min(r, min(rmax, G::HR - 1u)), sh4) + __umul24(min(c, cmax), sw4) +
+                             (threadIdx.x % G::CPR) * 16u;
         reg.v[i] = *reinterpret_cast<const u32x4 *>(base + off);
     }
 }
-// The same in PARTS slices, so that the loads can be issued a few at a time between
-// matrix instructions (a wave that issues a whole halo at once is blocked for
-// microseconds while the CU's memory queue takes the loads, and issues no matrix
-// instruction meanwhile).
-// TAIL: the last TAIL chunks of a thread are left out of the slices (part == PARTS loads them):
-// a kernel that has no registers for the whole halo beside its arithmetic loads them when the
-// arithmetic is over, instead of having the compiler spill freshly loaded chunks to scratch
-// memory, each behind a wait for its load.
-template <int D, int KS, int PARTS, int TAIL = 0>
-__device__ __forceinline__ void fetch32_part(Regs32 &reg, const float *img, int64_t sh, int64_t sw,
-                                             int hr0, int hc0, int rlim, int clim, int part) {
-    using G = Geo32<D, KS>;
-    static_assert(TAIL < G::NL, "the tail is a part of the halo");
-    const char *base = reinterpret_cast<const char *>(img + hr0 * sh + hc0 * sw);
-    const unsigned sh4 = (unsigned)sh * 4u, sw4 = (unsigned)sw * 4u;
-    const int rmax = rlim - 1 - hr0, cmax = clim - 1 - hc0;
-#pragma unroll
-    for (int i = 0; i < G::NL; i++) {
-        if ((i >= G::NL - TAIL ? PARTS : i * PARTS / (G::NL - TAIL)) != part) continue;
-        int pix = (int)threadIdx.x / G::CPR + i * (256 / G::CPR);
-        pix = pix < G::HR * G::HC ? pix : G::HR * G::HC - 1;
-        const unsigned r = (unsigned)min(pix / G::HC, rmax), c = (unsigned)min(pix % G::HC, cmax);
-        const unsigned off = __umul24(r, sh4) + __umul24(c, sw4) + ((unsigned)threadIdx.x % G::CPR) * 16u;
-        reg.v[i] = *reinterpret_cast<const u32x4 *>(base + off);
-    }
+template <int D, int KS>
+__device__ __forceinline__ void fetch32(Regs32 &reg, const float *img, int64_t sh, int64_t sw,
+                                        int hr0, int hc0, int rlim, int clim) {
+    fetch32_part<D, KS, 1>(reg, img, sh, sw, hr0, hc0, rlim, clim, 0);
 }
 template <int D, int KS>
 __device__ __forceinline__ void commit32(float *lds, const Regs32 &reg) {
@@ -166,6 +147,25 @@ __device__ __forceinline__ float exp_neg64(double x) {
     return fmaf(e, lo * kLn2, e);
 }
 
+// Odd rows of 16 lanes of a against even rows of b: a = (a0, b0, a2, b2), b = (a1, b1, a3, b3).
+__device__ __forceinline__ void swap_rows(float &a, float &b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+}
+// The upper 32 lanes of a against the lower ones of b.
+__device__ __forceinline__ void swap_halves(float &a, float &b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+}
+// out[i]: row i of x in every row
+__device__ __forceinline__ void spread_rows(float x, float (&out)[4]) {
+    float a = x, b = x;
+    swap_rows(a, b);
+    out[0] = a, out[2] = a, out[1] = b, out[3] = b;
+    swap_halves(out[0], out[2]);
+    swap_halves(out[1], out[3]);
+}
+
 // XCD-aware tile of a workgroup: every XCD takes one contiguous run of tiles.
 __device__ __forceinline__ int tile_of_block(int ntiles) {
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -174,70 +174,189 @@ __device__ __forceinline__ int tile_of_block(int ntiles) {
     return (slot < per && t < ntiles) ? t : -1;
 }
 
-// logits^T [token][query] of the wave's halo in float64: acc[mt][e] is token e*4 + g of
-// tile mt for this lane's query.  `qf` holds the query's channels g*D/4 ..
-// The MT token tiles advance together, four channels at a time: MT independent
-// accumulator chains, and a query channel is converted to float64 once for all of them.
-// `hook(j)` runs before the instructions of channel group j of D/16 (used to issue
-// global loads a few at a time).
-template <int D, int KS, typename Hook>
-__device__ __forceinline__ void logits64(const float *lds_k, const float *qf, int orow, int ocol,
-                                         int n, int g, f64x4 *acc, Hook hook) {
-    using G = Geo32<D, KS>;
-    const float *kp[G::MT];
+// This lane's place: block and pixel of the wave's 4x4 queries (or keys), lane group.
+struct Lane {
+    int g, b, j;
+};
+__device__ __forceinline__ Lane lane_place() {
+    const int l = threadIdx.x & 63;
+    return Lane{l >> 4, (l >> 2) & 3, l & 3};
+}
+// lane_query for these lanes: the halo is that of the lane's 2x2 block, (dr, dc) are 0 or 1.
+template <int KS>
+__device__ __forceinline__ LaneQ block_query(const Tile &tl, const Shape &s, int wave, const Lane &ln) {
+    LaneQ q = lane_query<KS>(tl, s, wave, (2 * (ln.b >> 1) + (ln.j >> 1)) * 4 + 2 * (ln.b & 1) + (ln.j & 1));
+    const int r0 = tl.r0 + (wave >> 1) * 4 + 2 * (ln.b >> 1), c0 = tl.c0 + (wave & 1) * 4 + 2 * (ln.b & 1);
+    const int sr0 = win_start(min(r0, s.H - 1), s.H, KS), sc0 = win_start(min(c0, s.W - 1), s.W, KS);
+    q.dr += q.hr0 + q.orow - sr0;
+    q.dc += q.hc0 + q.ocol - sc0;
+    q.orow = sr0 - q.hr0;
+    q.ocol = sc0 - q.hc0;
+    return q;
+}
+
+// this lane's share of one pixel's channels for the first products, channels 16 s + 4 g .. + 3
+template <int D>
+__device__ __forceinline__ void load_quarter(const float *row, int g, float *out) {
 #pragma unroll
-    for (int mt = 0; mt < G::MT; mt++) {
-        kp[mt] = lds_k + G::tok_row(mt, n, orow, ocol) * G::PITCH + g * G::DQ;
-        acc[mt] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int s = 0; s < D / 16; s++) {
+        const f32x4 x = *reinterpret_cast<const f32x4 *>(row + 16 * s + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; e++) out[4 * s + e] = x[e];
     }
+}
+// LDS address of this lane's rows in the first products: token j of a patch, lane group's channels
+template <int D, int KS>
+__device__ __forceinline__ const float *first_base(const float *lds, const LaneQ &lq, const Lane &ln) {
+    using G = Geo32<D, KS>;
+    return lds + ((lq.orow + (ln.j >> 1)) * G::HC + lq.ocol + (ln.j & 1)) * G::PITCH + 4 * ln.g;
+}
+
+// f(0), f(1), ..: with the unrolling pragma the longest of these loops stay loops
+template <typename F, int... I>
+__device__ __forceinline__ void each_step(F f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+// The steps of a first product: the patches of a group (a row of them; all four at kernel_size 3) against four
+// channels per lane group, mul(t, e, x) for patch t and channel e.  A step's rows are read from LDS a step ahead;
+// independent accumulators lie between two uses of one.  `hook(s)` runs before the instructions of channel
+// group s of D/16 (used to issue global loads a few at a time).
+template <int D, int KS, typename Hook, typename Mul>
+__device__ __forceinline__ void first_steps(const float *base, Hook hook, Mul mul) {
+    using G = Geo32<D, KS>;
+    constexpr int GRP = KS == 3 ? 4 : G::PW, PER = G::T / GRP, STEPS = PER * G::DT;
+    f32x4 x[2][GRP];
+    auto fetch = [&](auto at) __attribute__((always_inline)) {
+        constexpr int step = decltype(at)::value;
 #pragma unroll
-    for (int j = 0; j < G::DQ / 4; j++) {
+        for (int i = 0; i < GRP; i++)
+            x[step & 1][i] = *reinterpret_cast<const f32x4 *>(base + G::at(step % PER * GRP + i, 0) + 16 * (step / PER));
+    };
+    fetch(std::integral_constant<int, 0>{});
+    each_step([&](auto at) __attribute__((always_inline)) {
+        constexpr int step = decltype(at)::value;
+        if constexpr (step + 1 < STEPS) fetch(std::integral_constant<int, step + 1>{});
+        if constexpr (step % PER == 0) hook(step / PER);
         __builtin_amdgcn_sched_barrier(0);
-        hook(j);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int i = 0; i < GRP; i++) mul(step % PER * GRP + i, 4 * (step / PER) + e, x[step & 1][i][e]);
         __builtin_amdgcn_sched_barrier(0);
-        f32x4 k4[G::MT];
+    }, std::make_integer_sequence<int, STEPS>{});
+}
+
+// Logits of this lane's query in float64: acc[t] is that of token g of patch t.  `qf` holds the query's channels
+// (load_quarter).
+template <int D, int KS, typename Hook>
+__device__ __forceinline__ void logits64(const float *base, const float *qf, double *acc, Hook hook) {
+    using G = Geo32<D, KS>;
 #pragma unroll
-        for (int mt = 0; mt < G::MT; mt++) k4[mt] = *reinterpret_cast<const f32x4 *>(kp[mt] + 4 * j);
+    for (int t = 0; t < G::T; t++) acc[t] = 0.0;
+    first_steps<D, KS>(base, hook, [&](int t, int c, float x) __attribute__((always_inline)) {
+        acc[t] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)x, (double)qf[c], acc[t], 0, 0, 0);
+    });
+}
+// The same product in float32 (dP = V dO): out[t] is that of token g of patch t.
+template <int D, int KS, typename Hook>
+__device__ __forceinline__ void first32(const float *base, const float *qf, float *out, Hook hook) {
+    using G = Geo32<D, KS>;
+    f32x4 acc[G::T];  // this lane group's quarter of the channels; element i: token i of the patch
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const double qd = (double)qf[4 * j + e];
+    for (int t = 0; t < G::T; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    first_steps<D, KS>(base, hook, [&](int t, int c, float x) __attribute__((always_inline)) {
+        acc[t] = __builtin_amdgcn_mfma_f32_4x4x1f32(x, qf[c], acc[t], 0, 0, 0);
+    });
 #pragma unroll
-            for (int mt = 0; mt < G::MT; mt++)
-                acc[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)k4[mt][e], qd, acc[mt], 0, 0, 0);
+    for (int t = 0; t < G::T; t++) {  // the lane groups' sums; group g keeps token g
+        float x = acc[t][0], y = acc[t][1], z = acc[t][2], w = acc[t][3];
+        swap_halves(x, z);
+        swap_halves(y, w);
+        x += z;
+        y += w;
+        swap_rows(x, y);
+        out[t] = x + y;
+    }
+}
+
+// One token of the second products: rows x of the 2x2 blocks' tokens (D / 16 values per lane, second_fetch), w the
+// token's weight for this lane's query (or key).
+// Rows of the result are channels: with D >= 64 lane (g, b, j) reads channels 64 h + 16 g + 4 j + 0 .. 3 as one
+// 16-byte word, and element i of acc[4 h + m] is channel 64 h + 16 g + 4 i + m; at head_dim 32 it reads
+// channels 16 m + 4 g + j, and element i of acc[m] is channel 16 m + 4 g + i.  From head_dim 64 on every other
+// block has its lane groups read channels 32 further on or back (second_flip): two neighbouring blocks' rows are
+// two pixels apart, which alone would put half of their words on the same banks.
+template <int D>
+__device__ __forceinline__ int second_flip(const Lane &ln) { return D == 32 ? 0 : (ln.b & 1) * 32; }
+template <int D>
+__device__ __forceinline__ int second_channel(const Lane &ln) {
+    return D == 32 ? 4 * ln.g + ln.j : (16 * ln.g + 4 * ln.j) ^ second_flip<D>(ln);
+}
+template <int D>
+__device__ __forceinline__ void second_fetch(const float *row, float *x) {
+    if constexpr (D == 32) {
+#pragma unroll
+        for (int m = 0; m < 2; m++) x[m] = row[16 * m];
+    } else {
+#pragma unroll
+        for (int h = 0; h < D / 64; h++) {
+            const f32x4 r = *reinterpret_cast<const f32x4 *>(row + 64 * h);
+#pragma unroll
+            for (int m = 0; m < 4; m++) x[4 * h + m] = r[m];
+        }
+    }
+}
+template <int D>
+__device__ __forceinline__ void second_step(const float *x, float w, f32x4 *acc) {
+#pragma unroll
+    for (int m = 0; m < D / 16; m++) acc[m] = __builtin_amdgcn_mfma_f32_4x4x1f32(x[m], w, acc[m], 0, 0, 0);
+}
+// acc[m] -> channels (16 m + 4 g .. + 3) ^ second_flip, as store32 takes them: a 4x4 transpose over elements and lane
+// groups
+template <int D>
+__device__ __forceinline__ void second_pieces(f32x4 *acc) {
+    if constexpr (D > 32) {
+#pragma unroll
+        for (int h = 0; h < D / 64; h++) {
+            float x[4][4];
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[m][i] = acc[4 * h + m][i];
+                swap_rows(x[m][0], x[m][1]);
+                swap_rows(x[m][2], x[m][3]);
+                swap_halves(x[m][0], x[m][2]);
+                swap_halves(x[m][1], x[m][3]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[4 * h + i] = f32x4{x[0][i], x[1][i], x[2][i], x[3][i]};
         }
     }
 }
 
-// out^T [channel][query] += X^T w over the wave's halo tokens, X rows from LDS:
-// acc[m][e] is channel 16 m + 4 g + e of this lane's query.  w[mt][e] belongs to token
-// e*4 + g of tile mt (the layout logits64 leaves).
-// `hook(step)` runs before the instructions of reduction step `step` of MT * 4.
+// out [channel][query] = X^T w over the tokens of the lane's block, X rows from LDS, as second_pieces leaves
+// them.  w[t] belongs to token g of patch t.  `hook(step)` runs before the instructions of token `step` of T * 4.
 template <int D, int KS, typename Hook>
-__device__ __forceinline__ void second32(const float *lds_x, const f32x4 *w, int orow, int ocol,
-                                         int n, int g, f32x4 *acc, Hook hook) {
+__device__ __forceinline__ void second32(const float *lds_x, const float *w, const LaneQ &lq, const Lane &ln, f32x4 *acc,
+                                         Hook hook) {
     using G = Geo32<D, KS>;
 #pragma unroll
     for (int m = 0; m < G::DT; m++) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // One reduction step is DT matrix instructions that share w[mt][e]; their DT operands
-    // are read from LDS a step ahead, so the instructions never wait for LDS.
-    constexpr int STEPS = G::MT * 4;
-    float x[2][G::DT];
-    auto fetch = [&](int step, float *dst) __attribute__((always_inline)) {
-        const float *xp = lds_x + G::tok_row(step >> 2, (step & 3) * 4 + g, orow, ocol) * G::PITCH + n;
-#pragma unroll
-        for (int m = 0; m < G::DT; m++) dst[m] = xp[16 * m];
-    };
-    fetch(0, x[0]);
-#pragma unroll
-    for (int step = 0; step < STEPS; step++) {
-        if (step + 1 < STEPS) fetch(step + 1, x[(step + 1) & 1]);
+    const float *base = lds_x + (lq.orow * G::HC + lq.ocol) * G::PITCH + second_channel<D>(ln);
+    // the operands are read from LDS a token ahead, so the instructions never wait for LDS
+    float x[2][G::DT], wb[4];
+    second_fetch<D>(base, x[0]);
+    each_step([&](auto at) __attribute__((always_inline)) {
+        constexpr int step = decltype(at)::value;
+        if constexpr (step + 1 < G::STEPS) second_fetch<D>(base + G::at((step + 1) >> 2, (step + 1) & 3), x[(step + 1) & 1]);
+        if ((step & 3) == 0) spread_rows(w[step >> 2], wb);
         hook(step);
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int m = 0; m < G::DT; m++)
-            acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[step & 1][m], w[step >> 2][step & 3], acc[m], 0, 0, 0);
+        second_step<D>(x[step & 1], wb[step & 3], acc);
         __builtin_amdgcn_sched_barrier(0);
-    }
+    }, std::make_integer_sequence<int, G::STEPS>{});
+    second_pieces<D>(acc);
 }
 
 // Stores one token's D channels.  Piece m of lane group g is channels 16m + 4g .. +3, so the
@@ -245,9 +364,16 @@ __device__ __forceinline__ void second32(const float *lds_x, const f32x4 *w, int
 // non-temporal half lines reach memory in pieces (1.2-1.4x the bytes, at 3.1 TB/s against 5.3 for
 // whole lines).  With LINES the lanes of tokens n and n^1 (adjacent lanes) exchange every other
 // piece, and the eight lanes of the pair write one token's whole 128-byte line per instruction.
-// Every lane of the wave must call this; `live`: this lane's token exists.
+// Every lane of the wave must call this; `live`: this lane's token exists; `flip`: second_flip.  The values
+// stored are acc * (mul + low) with one rounding of the product by mul.
 template <int D, bool LINES>
-__device__ __forceinline__ void store32(float *token, int g, const f32x4 *acc, float mul, bool live) {
+__device__ __forceinline__ void store32(float *token, int g, const f32x4 *acc, int flip, float mul, float low, bool live) {
+    auto times = [&](const f32x4 &x) __attribute__((always_inline)) {
+        f32x4 y;
+#pragma unroll
+        for (int c = 0; c < 4; c++) y[c] = fmaf(x[c], mul, x[c] * low);
+        return y;
+    };
     if constexpr (LINES) {
         const bool odd = threadIdx.x & 1;
         auto xchg = [](unsigned x) __attribute__((always_inline)) {
@@ -263,7 +389,7 @@ __device__ __forceinline__ void store32(float *token, int g, const f32x4 *acc, f
         const int off = (odd ? 16 : 0) + 4 * g;
 #pragma unroll
         for (int k = 0; k < D / 32; k++) {
-            const f32x4 lo = acc[2 * k] * mul, hi = acc[2 * k + 1] * mul;
+            const f32x4 lo = times(acc[2 * k]), hi = times(acc[2 * k + 1]);
             f32x4 sa, sb;
 #pragma unroll
             for (int c = 0; c < 4; c++) {
@@ -271,31 +397,19 @@ __device__ __forceinline__ void store32(float *token, int g, const f32x4 *acc, f
                 sa[c] = odd ? r : lo[c];
                 sb[c] = odd ? hi[c] : r;
             }
-            if (live_a) __builtin_nontemporal_store(sa, reinterpret_cast<f32x4 *>(tok_a + 32 * k + off));
-            if (live_b) __builtin_nontemporal_store(sb, reinterpret_cast<f32x4 *>(tok_b + 32 * k + off));
+            if (live_a) __builtin_nontemporal_store(sa, reinterpret_cast<f32x4 *>(tok_a + (32 * k ^ flip) + off));
+            if (live_b) __builtin_nontemporal_store(sb, reinterpret_cast<f32x4 *>(tok_b + (32 * k ^ flip) + off));
         }
     } else {
         if (!live) return;
 #pragma unroll
         for (int m = 0; m < D / 16; m++)
-            __builtin_nontemporal_store(acc[m] * mul, reinterpret_cast<f32x4 *>(token + 16 * m + 4 * g));
+            __builtin_nontemporal_store(times(acc[m]), reinterpret_cast<f32x4 *>(token + (16 * m ^ flip) + 4 * g));
     }
 }
 
 __device__ __forceinline__ const float *image32(const View &v, const Tile &tl) {
     return static_cast<const float *>(v.ptr) + tl.bb * v.sb + tl.nn * v.sn;
-}
-
-// this lane's share of one pixel's channels for the first products: channels
-// g*D/4 .. (g+1)*D/4 - 1, as float32
-template <int D>
-__device__ __forceinline__ void load_quarter(const float *row, int g, float *out) {
-#pragma unroll
-    for (int j = 0; j < D / 16; j++) {
-        const f32x4 x = *reinterpret_cast<const f32x4 *>(row + g * (D / 4) + 4 * j);
-#pragma unroll
-        for (int e = 0; e < 4; e++) out[4 * j + e] = x[e];
-    }
 }
 
 // Is halo token (r, c) inside the window of the query whose window starts at (dr, dc)?
@@ -312,16 +426,17 @@ __device__ __forceinline__ bool in_window(int r, int c, int dr, int dc) {
 template <int D, int KS>
 __global__ __launch_bounds__(256, 2) void fwd_mfma_f32(FwdArgs a, int tiles_r, int tiles_c, int ntiles) {
     using G = Geo32<D, KS>;
-    constexpr int STEPS = G::MT * 4;
+    constexpr int STEPS = G::STEPS;
     __shared__ __attribute__((aligned(16))) float lds[G::ROWS * G::PITCH];
     Sched sc = make_sched(ntiles, blockIdx.x, gridDim.x);
     if (sc.t >= sc.t_end) return;
     const Shape &s = a.s;
-    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, n = l & 15, g = l >> 4;
-    if (threadIdx.x < G::PITCH) lds[G::ZROW * G::PITCH + threadIdx.x] = 0.f;
+    const int wave = threadIdx.x >> 6;
+    const Lane ln = lane_place();
+    const int g = ln.g;
 
     Tile cur = tile_of(sc.t, tiles_r, tiles_c, s.N);
-    LaneQ lq = lane_query<KS>(cur, s, wave, n);
+    LaneQ lq = block_query<KS>(cur, s, wave, ln);
     Regs32 st;
     float qf[G::DQ];
     fetch32<D, KS>(st, image32(a.k, cur), a.k.sh, a.k.sw, lq.hr0, lq.hc0, s.H, s.W);
@@ -332,7 +447,7 @@ __global__ __launch_bounds__(256, 2) void fwd_mfma_f32(FwdArgs a, int tiles_r, i
         const int tn = sc.t + sc.step;
         const bool more = tn < sc.t_end;
         const Tile nxt = more ? tile_of(tn, tiles_r, tiles_c, s.N) : cur;
-        const LaneQ lqn = lane_query<KS>(nxt, s, wave, n);
+        const LaneQ lqn = block_query<KS>(nxt, s, wave, ln);
         const float *vimg = image32(a.v, cur), *kimg = image32(a.k, nxt);
         auto load_v = [&](int part) __attribute__((always_inline)) {
             fetch32_part<D, KS, G::DQ / 4>(st, vimg, a.v.sh, a.v.sw, lq.hr0, lq.hc0, s.H, s.W, part);
@@ -345,33 +460,29 @@ __global__ __launch_bounds__(256, 2) void fwd_mfma_f32(FwdArgs a, int tiles_r, i
             }
         };
 
-        f32x4 p[G::MT];
-        float lse = 0.f, inv = 0.f;
+        float p[G::T];
+        float lse = 0.f, inv = 0.f, inv_rest = 0.f;
         if (lq.wave_on) {
-            f64x4 acc[G::MT];
-            logits64<D, KS>(lds, qf, lq.orow, lq.ocol, n, g, acc, load_v);
+            double acc[G::T];
+            logits64<D, KS>(first_base<D, KS>(lds, lq, ln), qf, acc, load_v);
             double mx = -INFINITY;
 #pragma unroll
-            for (int mt = 0; mt < G::MT; mt++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    int r, c;
-                    const bool ok = G::tok_rc(mt, e * 4 + g, r, c) && in_window<KS>(r, c, lq.dr, lq.dc);
-                    acc[mt][e] = ok ? acc[mt][e] * (double)s.scale : -INFINITY;
-                    mx = fmax(mx, acc[mt][e]);
-                }
+            for (int t = 0; t < G::T; t++) {
+                const bool ok = in_window<KS>(G::row(t, 0) + (g >> 1), G::col(t, 0) + (g & 1), lq.dr, lq.dc);
+                acc[t] = ok ? acc[t] * (double)s.scale : -INFINITY;
+                mx = fmax(mx, acc[t]);
+            }
             mx = fmax(mx, __shfl_xor(mx, 16, 64));
             mx = fmax(mx, __shfl_xor(mx, 32, 64));
             float sum = 0.f;
 #pragma unroll
-            for (int mt = 0; mt < G::MT; mt++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    p[mt][e] = exp_neg64(acc[mt][e] - mx);
-                    sum += p[mt][e];
-                }
+            for (int t = 0; t < G::T; t++) {
+                p[t] = exp_neg64(acc[t] - mx);
+                sum += p[t];
+            }
             sum = col_sum(sum);
             inv = 1.f / sum;
+            inv_rest = fmaf(-sum, inv, 1.f);  // what its rounding leaves
             lse = (float)(mx + (double)logf(sum));
         } else {
 #pragma unroll
@@ -382,9 +493,9 @@ __global__ __launch_bounds__(256, 2) void fwd_mfma_f32(FwdArgs a, int tiles_r, i
         __syncthreads();
         if (lq.wave_on) {
             f32x4 o[G::DT];
-            second32<D, KS>(lds, p, lq.orow, lq.ocol, n, g, o, load_next);
+            second32<D, KS>(lds, p, lq, ln, o, load_next);
             float *op = const_cast<float *>(image32(a.o, cur)) + lq.qr * a.o.sh + lq.qc * a.o.sw;
-            store32<D, kLines32<D, KS>>(op, g, o, inv, lq.live);
+            store32<D, kLines32<D, KS>>(op, g, o, second_flip<D>(ln), inv, inv * inv_rest, lq.live);
             if (lq.live && a.lse && g == 0) a.lse[lq.tok] = lse;
         } else {
 #pragma unroll
@@ -405,28 +516,21 @@ __global__ __launch_bounds__(256, 2) void fwd_mfma_f32(FwdArgs a, int tiles_r, i
 // go to the workspace, k*k values per query in window order, for the dK/dV pass.
 // Persistent like the forward: K is loaded between the instructions of dP, the next
 // tile's V between those of dQ.
-// Chunks of a halo that the dQ pass loads behind its arithmetic (fetch32_part's TAIL), where it
-// would spill otherwise.  B4 N4 128x128 d128 k5: 84 -> 12 bytes of scratch per lane and
-// 261 -> 231 us; B4 N8 96x96 d32 k7: 76 -> 0 bytes, 194 -> 164 us; d64 k7: 288 -> 96 bytes,
-// 319 -> 273 us (the whole halo behind the arithmetic: its float64 logits of 13 token tiles
-// leave no registers for any of it).
-template <int D, int KS>
-constexpr int kDqTail = D == 128 && KS == 5 ? 5 : D == 32 && KS == 7 ? 5 : D == 64 && KS == 7 ? 12 : 0;
-
 template <int D, int KS>
 __global__ __launch_bounds__(256, 2) void bwd_dq_mfma_f32(BwdArgs a, float *ws_p, float *ws_ds,
                                                           int tiles_r, int tiles_c, int ntiles) {
     using G = Geo32<D, KS>;
-    constexpr int STEPS = G::MT * 4;
+    constexpr int STEPS = G::STEPS;
     __shared__ __attribute__((aligned(16))) float lds[G::ROWS * G::PITCH];
     Sched sc = make_sched(ntiles, blockIdx.x, gridDim.x);
     if (sc.t >= sc.t_end) return;
     const Shape &s = a.s;
-    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, n = l & 15, g = l >> 4;
-    if (threadIdx.x < G::PITCH) lds[G::ZROW * G::PITCH + threadIdx.x] = 0.f;
+    const int wave = threadIdx.x >> 6;
+    const Lane ln = lane_place();
+    const int g = ln.g;
 
     Tile cur = tile_of(sc.t, tiles_r, tiles_c, s.N);
-    LaneQ lq = lane_query<KS>(cur, s, wave, n);
+    LaneQ lq = block_query<KS>(cur, s, wave, ln);
     Regs32 st;
     float go[G::DQ];
     fetch32<D, KS>(st, image32(a.v, cur), a.v.sh, a.v.sw, lq.hr0, lq.hc0, s.H, s.W);
@@ -437,110 +541,83 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_mfma_f32(BwdArgs a, float *ws_p
         const int tn = sc.t + sc.step;
         const bool more = tn < sc.t_end;
         const Tile nxt = more ? tile_of(tn, tiles_r, tiles_c, s.N) : cur;
-        const LaneQ lqn = lane_query<KS>(nxt, s, wave, n);
+        const LaneQ lqn = block_query<KS>(nxt, s, wave, ln);
         const float *kimg = image32(a.k, cur), *vimg = image32(a.v, nxt);
         // this tile's q and log-sum-exp arrive while dP is formed (their registers are
         // free until then: dO's are needed first, q's afterwards)
         float qf[G::DQ];
         float lse_f = 0.f;
         auto load_k = [&](int part) __attribute__((always_inline)) {
-            fetch32_part<D, KS, G::MT, kDqTail<D, KS>>(st, kimg, a.k.sh, a.k.sw, lq.hr0, lq.hc0, s.H, s.W, part);
-            if (part == G::MT - 1) {
+            fetch32_part<D, KS, G::DT>(st, kimg, a.k.sh, a.k.sw, lq.hr0, lq.hc0, s.H, s.W, part);
+            if (part == G::DT - 1) {
                 load_quarter<D>(image32(a.q, cur) + lq.qr * a.q.sh + lq.qc * a.q.sw, g, qf);
                 lse_f = a.lse[lq.tok];
             }
         };
 
-        // dP^T: the operand rows are fetched in the transposed order, so that accumulator
-        // element e of lane group g is token e*4 + g like in the float64 product
-        f32x4 dp[G::MT];
+        float dp[G::T];
         if (lq.wave_on) {
-            const int nt = ((n & 3) << 2) | (n >> 2);
-#pragma unroll
-            for (int mt = 0; mt < G::MT; mt++) {
-                __builtin_amdgcn_sched_barrier(0);
-                load_k(mt);
-                __builtin_amdgcn_sched_barrier(0);
-                const float *vp = lds + G::tok_row(mt, nt, lq.orow, lq.ocol) * G::PITCH + g * G::DQ;
-                f32x4 c = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int j = 0; j < G::DQ / 4; j++) {
-                    const f32x4 v4 = *reinterpret_cast<const f32x4 *>(vp + 4 * j);
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        c = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[e], go[4 * j + e], c, 0, 0, 0);
-                }
-                dp[mt] = c;
-            }
+            first32<D, KS>(first_base<D, KS>(lds, lq, ln), go, dp, load_k);
         } else {
 #pragma unroll
-            for (int part = 0; part < G::MT; part++) load_k(part);
+            for (int part = 0; part < G::DT; part++) load_k(part);
         }
-        if constexpr (kDqTail<D, KS> > 0) load_k(G::MT);
         const double lse = (double)lse_f;
         __syncthreads();  // every wave is done with V
         commit32<D, KS>(lds, st);
         __syncthreads();
         auto load_next = [&](int part) __attribute__((always_inline)) {
             if (more) {
-                fetch32_part<D, KS, STEPS, kDqTail<D, KS>>(st, vimg, a.v.sh, a.v.sw, lqn.hr0, lqn.hc0, s.H, s.W, part);
+                fetch32_part<D, KS, STEPS>(st, vimg, a.v.sh, a.v.sw, lqn.hr0, lqn.hc0, s.H, s.W, part);
                 if (part == STEPS - 1)
                     load_quarter<D>(image32(a.d_o, nxt) + lqn.qr * a.d_o.sh + lqn.qc * a.d_o.sw, g, go);
             }
         };
         if (lq.wave_on) {
-            f32x4 ds[G::MT];
+            float ds[G::T];
             {
-                f64x4 acc[G::MT];
-                logits64<D, KS>(lds, qf, lq.orow, lq.ocol, n, g, acc, [](int) {});
+                double acc[G::T];
+                logits64<D, KS>(first_base<D, KS>(lds, lq, ln), qf, acc, [](int) {});
                 float z = 0.f;
 #pragma unroll
-                for (int mt = 0; mt < G::MT; mt++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        int r, c;
-                        const bool ok = G::tok_rc(mt, e * 4 + g, r, c) && in_window<KS>(r, c, lq.dr, lq.dc);
-                        ds[mt][e] = ok ? exp_neg64(fmin(acc[mt][e] * (double)s.scale - lse, 0.0)) : 0.f;
-                        z += ds[mt][e];
-                    }
-                const float zinv = 1.f / col_sum(z);
+                for (int t = 0; t < G::T; t++) {
+                    const bool ok = in_window<KS>(G::row(t, 0) + (g >> 1), G::col(t, 0) + (g & 1), lq.dr, lq.dc);
+                    ds[t] = ok ? exp_neg64(fmin(acc[t] * (double)s.scale - lse, 0.0)) : 0.f;
+                    z += ds[t];
+                }
+                z = col_sum(z);
+                const float zinv = 1.f / z, zlow = zinv * fmaf(-z, zinv, 1.f);
                 float dpart = 0.f;
 #pragma unroll
-                for (int mt = 0; mt < G::MT; mt++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        ds[mt][e] *= zinv;                       // P
-                        dpart = fmaf(ds[mt][e], dp[mt][e], dpart);
-                    }
+                for (int t = 0; t < G::T; t++) {
+                    ds[t] = fmaf(ds[t], zinv, ds[t] * zlow);  // P
+                    dpart = fmaf(ds[t], dp[t], dpart);
+                }
                 const float delta = col_sum(dpart);
                 float *pp = ws_p + lq.tok * G::KK * (kPair32<D, KS> ? 2 : 1), *dsp = ws_ds + lq.tok * G::KK;
 #pragma unroll
-                for (int mt = 0; mt < G::MT; mt++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        int r, c;
-                        const bool ok = G::tok_rc(mt, e * 4 + g, r, c) && in_window<KS>(r, c, lq.dr, lq.dc);
-                        const float pv = ds[mt][e];
-                        ds[mt][e] = pv * (dp[mt][e] - delta);    // dS
-                        if (ok && lq.live) {
-                            const int j = (r - lq.dr) * KS + (c - lq.dc);
-                            if constexpr (kPair32<D, KS>) {
-                                *reinterpret_cast<f32x2 *>(pp + 2 * j) = f32x2{pv, ds[mt][e]};
-                            } else {
-                                pp[j] = pv;
-                                dsp[j] = ds[mt][e];
-                            }
+                for (int t = 0; t < G::T; t++) {
+                    const int r = G::row(t, 0) + (g >> 1), c = G::col(t, 0) + (g & 1);
+                    const float pv = ds[t];
+                    ds[t] = pv * (dp[t] - delta);        // dS
+                    if (in_window<KS>(r, c, lq.dr, lq.dc) && lq.live) {
+                        const int at = (r - lq.dr) * KS + (c - lq.dc);
+                        if constexpr (kPair32<D, KS>) {
+                            *reinterpret_cast<f32x2 *>(pp + 2 * at) = f32x2{pv, ds[t]};
+                        } else {
+                            pp[at] = pv;
+                            dsp[at] = ds[t];
                         }
                     }
+                }
             }
             f32x4 dq[G::DT];
-            second32<D, KS>(lds, ds, lq.orow, lq.ocol, n, g, dq, load_next);
-            store32<D, kLines32<D, KS>>(static_cast<float *>(a.dq) + lq.tok * D, g, dq, s.scale, lq.live);
+            second32<D, KS>(lds, ds, lq, ln, dq, load_next);
+            store32<D, kLines32<D, KS>>(static_cast<float *>(a.dq) + lq.tok * D, g, dq, second_flip<D>(ln), s.scale, 0.f, lq.live);
         } else {
 #pragma unroll
             for (int part = 0; part < STEPS; part++) load_next(part);
         }
-        if constexpr (kDqTail<D, KS> > 0) load_next(STEPS);
         if (!more) break;
         __syncthreads();  // every wave is done with K
         cur = nxt;
@@ -550,42 +627,46 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_mfma_f32(BwdArgs a, float *ws_p
 }
 
 // ------------------------------------------------------------------ dK or dV
-// Key-centric: the workgroup owns 8x8 keys, a wave 4x4 of them (the N dimension).  The
+// Key-centric: the workgroup owns 8x8 keys, a wave 4x4 of them in blocks of 2x2.  The
 // queries that attend to any key of the tile form a rectangle (the union of the keys'
 // inverse neighbourhoods, e_natten/pytorch.py:13-23), walked in blocks of at most
-// (8+k-1)^2 queries whose X rows (dO for dV, Q for dK) are staged in LDS.  One
-// reduction step takes the four queries (row r .. r+3, column c) of the wave's part of
-// the block: their LDS rows are a halo row apart, so the operand reads fall into
-// disjoint banks.  The weights W (P for dV, dS for dK) come from the workspace; a query
+// (8+k-1)^2 queries whose X rows (dO for dV, Q for dK) are staged in LDS.  In each, a block of keys meets the
+// patches of 2x2 queries from the first that attends to one of its keys on, as many as the wave's widest
+// block of keys needs.  The weights W (P for dV, dS for dK) come from the workspace; a query
 // that does not attend to a key contributes an exact zero.
 template <int D, int KS>
 __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, View x1, const float *ws_w,
                                                             float *out0, float *out1, float mul0, float mul1,
                                                             int tiles_r, int tiles_c, int ntiles) {
     using G = Geo32<D, KS>;
-    constexpr int NRG = (G::SW + KS / 2 + 3) / 4;   // groups of 4 query rows a wave can meet in a block
-    constexpr int NC = G::SW + KS / 2;              // query columns likewise
-    // ... but where both ends of an axis clamp the windows of one wave's keys, which a row of 11 or 12
-    // pixels at kernel_size 5 and of 14 at 7 has: there the blocks are NC columns wide
-    constexpr int BOTH = (KS - 1) / 4 * 4 + 3 + KS;
-    static_assert(BOTH <= 4 * NRG, "rows of such a wave");
+    // Two neighbouring keys are attended by at most k + k/2 + 1 rows of queries, and by up to 2k where both ends of
+    // the axis clamp their windows, which an axis of at most 2k pixels has: it is walked in shorter blocks.
+    constexpr int NP = (KS + KS / 2 + 2) / 2;       // patches on a side
+    static_assert(2 * NP <= G::HR, "patches of a block of keys stay in the staged rows");
     constexpr int NB = kPair32<D, KS> ? 2 : 1;      // results of this launch (one: x0 and out0)
     __shared__ __attribute__((aligned(16))) float lds[NB][G::ROWS * G::PITCH];
     const int t = tile_of_block(ntiles);
     if (t < 0) return;
     const Shape &s = a.s;
     const Tile tl = tile_of(t, tiles_r, tiles_c, s.N);
-    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, n = l & 15, g = l >> 4;
-    // the tile's and the wave's keys, and the queries that attend to them
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Lane ln = lane_place();
+    const int g = ln.g;
+    // the tile's and the lane's keys, and the queries that attend to them
     const int wr0 = tl.r0 + (wave >> 1) * 4, wc0 = tl.c0 + (wave & 1) * 4;
     const bool wave_on = wr0 < s.H && wc0 < s.W;
-    const int kr = min(wr0 + (n >> 2), s.H - 1), kc = min(wc0 + (n & 3), s.W - 1);
-    const bool live = (wr0 + (n >> 2) < s.H) && (wc0 + (n & 3) < s.W);
+    const int kr0 = wr0 + 2 * (ln.b >> 1) + (ln.j >> 1), kc0 = wc0 + 2 * (ln.b & 1) + (ln.j & 1);
+    const int kr = min(kr0, s.H - 1), kc = min(kc0, s.W - 1);
+    const bool live = kr0 < s.H && kc0 < s.W;
     const int qa = inv_lo(tl.r0, KS), qb = inv_hi(min(tl.r0 + 8, s.H) - 1, s.H, KS);
     const int ca = inv_lo(tl.c0, KS), cb = inv_hi(min(tl.c0 + 8, s.W) - 1, s.W, KS);
-    const int wqa = inv_lo(min(wr0, s.H - 1), KS), wqb = inv_hi(min(wr0 + 4, s.H) - 1, s.H, KS);
-    const int wca = inv_lo(min(wc0, s.W - 1), KS), wcb = inv_hi(min(wc0 + 4, s.W) - 1, s.W, KS);
     const int64_t img_tok = ((int64_t)tl.bb * s.N + tl.nn) * s.H * (int64_t)s.W;
+    // first query of [lo, lo + len) that attends to one of the two keys from k0 on, and how many patches they take
+    auto span = [&](int k0, int L, int lo, int len, int &first) __attribute__((always_inline)) {
+        const int ka = min(k0, L - 1), kb = min(k0 + 1, L - 1);
+        first = max(inv_lo(ka, KS), lo);
+        return (min(inv_hi(kb, L, KS), lo + len) - first + 1) >> 1;
+    };
 
     f32x4 acc[NB][G::DT];
 #pragma unroll
@@ -593,76 +674,67 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, 
 #pragma unroll
         for (int m = 0; m < G::DT; m++) acc[b][m] = f32x4{0.f, 0.f, 0.f, 0.f};
     Regs32 st[NB];
-    const int cols = s.W > NC && s.W <= BOTH ? NC : G::HC;
-    for (int br = qa; br < qb; br += G::HR) {
+    const int rows = s.H > 2 * NP && s.H <= 2 * KS ? 2 * NP : G::HR, cols = s.W > 2 * NP && s.W <= 2 * KS ? 2 * NP : G::HC;
+    for (int br = qa; br < qb; br += rows) {
         for (int bc = ca; bc < cb; bc += cols) {
             fetch32<D, KS>(st[0], image32(x0, tl), x0.sh, x0.sw, br, bc, qb, cb);
             if constexpr (NB == 2) fetch32<D, KS>(st[1], image32(x1, tl), x1.sh, x1.sw, br, bc, qb, cb);
-            // this wave's queries inside the block
-            const int ra = max(wqa, br), rb = min(wqb, br + G::HR);
-            const int cc = max(wca, bc), cd = min(wcb, bc + cols);
-            // weights of the block's reduction steps: query (ra + 4 rg + g, cc + c), this
-            // lane's key; zero if the query is outside the wave's part or does not attend
-            float w[NB][NRG * NC];
+            // patches of the block that the wave's keys need (the same number for its blocks of keys), and this
+            // lane's first query: moved up where its last patch would leave the staged rows
+            const int rend = min(rows, qb - br), cend = min(cols, cb - bc);
+            int r0, r1, c0, c1;
+            const int npr = max(span(wr0, s.H, br, rend, r0), span(wr0 + 2, s.H, br, rend, r1));
+            const int npc = max(span(wc0, s.W, bc, cend, c0), span(wc0 + 2, s.W, bc, cend, c1));
+            const int fr = min(ln.b >> 1 ? r1 : r0, br + G::HR - 2 * max(npr, 0));
+            const int fc = min(ln.b & 1 ? c1 : c0, bc + G::HC - 2 * max(npc, 0));
+            // weights of query g of every patch for this lane's key; zero where it does not attend or is not in the block
+            float w[NB][NP * NP];
 #pragma unroll
-            for (int rg = 0; rg < NRG; rg++)
+            for (int pr = 0; pr < NP; pr++) {
+                const int qr = fr + 2 * pr + (g >> 1);
+                const int kpr = kr - win_start(min(qr, s.H - 1), s.H, KS);
+                const bool rok = wave_on && qr < br + rend && (unsigned)kpr < (unsigned)KS;
 #pragma unroll
-                for (int c = 0; c < NC; c++) {
-                    const int qr = ra + 4 * rg + g, qc = cc + c;
-                    const int pr = kr - win_start(min(qr, s.H - 1), s.H, KS);
-                    const int pc = kc - win_start(min(qc, s.W - 1), s.W, KS);
-                    const bool ok = wave_on && qr < rb && qc < cd && (unsigned)pr < (unsigned)KS &&
-                                    (unsigned)pc < (unsigned)KS;
-                    const float *wp = ws_w + ((img_tok + (int64_t)qr * s.W + qc) * G::KK + pr * KS + pc) * NB;
+                for (int pc = 0; pc < NP; pc++) {
+                    if (pr >= npr || pc >= npc) continue;
+                    const int qc = fc + 2 * pc + (g & 1);
+                    const int kpc = kc - win_start(min(qc, s.W - 1), s.W, KS);
+                    const bool ok = rok && qc < bc + cend && (unsigned)kpc < (unsigned)KS;
+                    const float *wp = ws_w + ((img_tok + (int64_t)qr * s.W + qc) * G::KK + kpr * KS + kpc) * NB;
                     if constexpr (NB == 2) {
                         const f32x2 pair = ok ? *reinterpret_cast<const f32x2 *>(wp) : f32x2{0.f, 0.f};
-                        w[0][rg * NC + c] = pair[0];
-                        w[1][rg * NC + c] = pair[1];
+                        w[0][pr * NP + pc] = pair[0];
+                        w[1][pr * NP + pc] = pair[1];
                     } else {
-                        w[0][rg * NC + c] = ok ? *wp : 0.f;
+                        w[0][pr * NP + pc] = ok ? *wp : 0.f;
                     }
                 }
+            }
             __syncthreads();  // the previous block's rows are no longer read
 #pragma unroll
             for (int b = 0; b < NB; b++) commit32<D, KS>(lds[b], st[b]);
             __syncthreads();
             if (wave_on) {
-                // A step's DT operands are read from LDS a step ahead of the matrix
-                // instructions that use them.
-                float x[2][NB][G::DT];
-                auto fetch = [&](int rg, int c, float (&dst)[NB][G::DT]) __attribute__((always_inline)) {
-                    // LDS row of this lane group's query row in the block (clamped: the
-                    // weight of a row or column past the end is zero)
-                    const int lrow = min(min(ra + 4 * rg + g, qb - 1) - br, G::HR - 1);
-                    const int lcol = min(cc + c - bc, G::HC - 1);
+                const int base = ((fr - br) * G::HC + fc - bc) * G::PITCH + second_channel<D>(ln);
 #pragma unroll
-                    for (int b = 0; b < NB; b++) {
-                        const float *xp = lds[b] + (lrow * G::HC + lcol) * G::PITCH + n;
+                for (int pr = 0; pr < NP; pr++) {
+                    if (pr >= npr) break;
 #pragma unroll
-                        for (int m = 0; m < G::DT; m++) dst[b][m] = xp[16 * m];
-                    }
-                };
-                fetch(0, 0, x[0]);
+                    for (int pc = 0; pc < NP; pc++) {
+                        if (pc >= npc) break;
+                        // A patch's operands are read from LDS ahead of its matrix instructions.
+                        float x[4][NB][G::DT], wb[NB][4];
 #pragma unroll
-                for (int rg = 0; rg < NRG; rg++) {
-                    if (ra + 4 * rg >= rb) break;
-#pragma unroll
-                    for (int c = 0; c < NC; c++) {
-                        const int step = rg * NC + c;
-                        // the step after this one (it may lie past the end of the wave's
-                        // part of the block: then its weight is zero or it is not run)
-                        if (c + 1 < NC) fetch(rg, c + 1, x[(step + 1) & 1]);
-                        else if (rg + 1 < NRG) fetch(rg + 1, 0, x[(step + 1) & 1]);
-                        __builtin_amdgcn_sched_barrier(0);
-                        if (cc + c < cd) {
+                        for (int i = 0; i < 4; i++)
 #pragma unroll
                             for (int b = 0; b < NB; b++)
+                                second_fetch<D>(lds[b] + base + ((2 * pr + (i >> 1)) * G::HC + 2 * pc + (i & 1)) * G::PITCH, x[i][b]);
 #pragma unroll
-                                for (int m = 0; m < G::DT; m++)
-                                    acc[b][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[step & 1][b][m], w[b][step],
-                                                                                     acc[b][m], 0, 0, 0);
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
+                        for (int b = 0; b < NB; b++) spread_rows(w[b][pr * NP + pc], wb[b]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++)
+#pragma unroll
+                            for (int b = 0; b < NB; b++) second_step<D>(x[i][b], wb[b][i], acc[b]);
                     }
                 }
             }
@@ -670,8 +742,10 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, 
     }
     if (!wave_on) return;
     const int64_t tok = img_tok + (int64_t)kr * s.W + kc;
-    store32<D, kLines32<D, KS>>(out0 + tok * D, g, acc[0], mul0, live);
-    if constexpr (NB == 2) store32<D, kLines32<D, KS>>(out1 + tok * D, g, acc[1], mul1, live);
+#pragma unroll
+    for (int b = 0; b < NB; b++) second_pieces<D>(acc[b]);
+    store32<D, kLines32<D, KS>>(out0 + tok * D, g, acc[0], second_flip<D>(ln), mul0, 0.f, live);
+    if constexpr (NB == 2) store32<D, kLines32<D, KS>>(out1 + tok * D, g, acc[1], second_flip<D>(ln), mul1, 0.f, live);
 }
 
 // ------------------------------------------------------------------ dispatch

@@ -34,3 +34,24 @@ def test_backward(D, ks, hw):
     torch.cuda.synchronize()
     ref = oracle_all(q, k, v, g, ks, small=True)
     assert_close((o.cpu(), dq.cpu(), dk.cpu(), dv.cpu()), (ref[0], ref[2], ref[3], ref[4]), torch.float32, "d%d k%d" % (D, ks))
+
+
+@pytest.mark.parametrize("D,ks,hw", [
+    # blocks of 2x2 pixels cut by the image's edge, windows clamped at one end and at both, axes of k .. 2k pixels
+    (32, 3, (3, 5)), (64, 3, (6, 4)), (128, 3, (9, 11)), (32, 5, (5, 6)), (64, 5, (9, 10)), (128, 5, (10, 23)), (128, 5, (8, 8)),
+    (32, 7, (13, 14)), (64, 7, (14, 31)), (128, 7, (7, 8)), (128, 7, (13, 22)), (64, 7, (25, 17))])
+def test_views_of_one_projection(D, ks, hw):
+    from e_natten_amd import kernel_path, natten2d
+    ensure_built()
+    assert kernel_path(D, ks, torch.float32) == "mfma"
+    B, N, (H, W) = 2, 2, hw
+    print("case float32 views", D, ks, hw, flush=True)
+    q, k, v, g = make_inputs((B, N, H, W, D), torch.float32, seed=3 * D + ks, q_scale=D ** -0.5)
+    x = torch.stack([t.permute(0, 2, 3, 1, 4) for t in (q, k, v)], dim=3).cuda().requires_grad_(True)  # [B, H, W, 3, N, D]
+    up = g.permute(0, 2, 3, 1, 4).contiguous().cuda().permute(0, 3, 1, 2, 4)
+    o = natten2d(*(t.movedim(3, 1) for t in x.unbind(3)), ks)
+    o.backward(up)
+    torch.cuda.synchronize()
+    ref = oracle_all(q, k, v, g, ks, small=True)
+    got = [x.grad[:, :, :, i].permute(0, 3, 1, 2, 4).cpu() for i in range(3)]
+    assert_close((o.detach().cpu(), *got), (ref[0], ref[2], ref[3], ref[4]), torch.float32, "d%d k%d" % (D, ks))
