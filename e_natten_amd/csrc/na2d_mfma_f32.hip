@@ -147,6 +147,14 @@ __device__ __forceinline__ float exp_neg64(double x) {
     return fmaf(e, lo * kLn2, e);
 }
 
+// XCD-aware tile of a workgroup: every XCD takes one contiguous run of tiles.
+__device__ __forceinline__ int tile_of_block(int ntiles) {
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int per = (ntiles + 7) >> 3;
+    const int t = xcd * per + slot;
+    return (slot < per && t < ntiles) ? t : -1;
+}
+
 // Odd rows of 16 lanes of a against even rows of b: a = (a0, b0, a2, b2), b = (a1, b1, a3, b3).
 __device__ __forceinline__ void swap_rows(float &a, float &b) {
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
@@ -164,14 +172,6 @@ __device__ __forceinline__ void spread_rows(float x, float (&out)[4]) {
     out[0] = a, out[2] = a, out[1] = b, out[3] = b;
     swap_halves(out[0], out[2]);
     swap_halves(out[1], out[3]);
-}
-
-// XCD-aware tile of a workgroup: every XCD takes one contiguous run of tiles.
-__device__ __forceinline__ int tile_of_block(int ntiles) {
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int per = (ntiles + 7) >> 3;
-    const int t = xcd * per + slot;
-    return (slot < per && t < ntiles) ? t : -1;
 }
 
 // This lane's place: block and pixel of the wave's 4x4 queries (or keys), lane group.
@@ -634,6 +634,8 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_mfma_f32(BwdArgs a, float *ws_p
 // patches of 2x2 queries from the first that attends to one of its keys on, as many as the wave's widest
 // block of keys needs.  The weights W (P for dV, dS for dK) come from the workspace; a query
 // that does not attend to a key contributes an exact zero.
+// One tile per workgroup: as a persistent kernel that loads the next tile's rows between the products of the
+// current one it was slower (d128 k5 149 -> 205 us for the two launches below, d64 k3 33 -> 41).
 template <int D, int KS>
 __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, View x1, const float *ws_w,
                                                             float *out0, float *out1, float mul0, float mul1,
@@ -648,24 +650,76 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, 
     const int t = tile_of_block(ntiles);
     if (t < 0) return;
     const Shape &s = a.s;
-    const Tile tl = tile_of(t, tiles_r, tiles_c, s.N);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Lane ln = lane_place();
     const int g = ln.g;
-    // the tile's and the lane's keys, and the queries that attend to them
+    const int rows = s.H > 2 * NP && s.H <= 2 * KS ? 2 * NP : G::HR, cols = s.W > 2 * NP && s.W <= 2 * KS ? 2 * NP : G::HC;
+
+    // the tile's keys and the queries that attend to them, the wave's keys and this lane's
+    const Tile tl = tile_of(t, tiles_r, tiles_c, s.N);
+    const int qa = inv_lo(tl.r0, KS), qb = inv_hi(min(tl.r0 + 8, s.H) - 1, s.H, KS);
+    const int ca = inv_lo(tl.c0, KS), cb = inv_hi(min(tl.c0 + 8, s.W) - 1, s.W, KS);
     const int wr0 = tl.r0 + (wave >> 1) * 4, wc0 = tl.c0 + (wave & 1) * 4;
-    const bool wave_on = wr0 < s.H && wc0 < s.W;
     const int kr0 = wr0 + 2 * (ln.b >> 1) + (ln.j >> 1), kc0 = wc0 + 2 * (ln.b & 1) + (ln.j & 1);
     const int kr = min(kr0, s.H - 1), kc = min(kc0, s.W - 1);
     const bool live = kr0 < s.H && kc0 < s.W;
-    const int qa = inv_lo(tl.r0, KS), qb = inv_hi(min(tl.r0 + 8, s.H) - 1, s.H, KS);
-    const int ca = inv_lo(tl.c0, KS), cb = inv_hi(min(tl.c0 + 8, s.W) - 1, s.W, KS);
     const int64_t img_tok = ((int64_t)tl.bb * s.N + tl.nn) * s.H * (int64_t)s.W;
-    // first query of [lo, lo + len) that attends to one of the two keys from k0 on, and how many patches they take
-    auto span = [&](int k0, int L, int lo, int len, int &first) __attribute__((always_inline)) {
-        const int ka = min(k0, L - 1), kb = min(k0 + 1, L - 1);
-        first = max(inv_lo(ka, KS), lo);
-        return (min(inv_hi(kb, L, KS), lo + len) - first + 1) >> 1;
+    Regs32 st[NB];
+    auto fetch_rows = [&](int br, int bc) __attribute__((always_inline)) {
+        fetch32<D, KS>(st[0], image32(x0, tl), x0.sh, x0.sw, br, bc, qb, cb);
+        if constexpr (NB == 2) fetch32<D, KS>(st[1], image32(x1, tl), x1.sh, x1.sw, br, bc, qb, cb);
+    };
+    // Patches of a block that the wave's keys need (the same number for its blocks of keys), this lane's first
+    // query there (moved up where its last patch would leave the staged rows), and the weights of query g of every patch
+    // for this lane's key.  Where it does not attend, or is not in the block, the weight's place is beyond the
+    // buffer, which reads as zero: a place is one addition of its row's and its column's, without a mask or a branch
+    // (d128 k5 176 -> 149 us for the two launches).
+    int npr, npc, base;
+    float w[NB][NP * NP];
+    auto weights = [&](int br, int bc) __attribute__((always_inline)) {
+        const int rend = min(br + rows, qb), cend = min(bc + cols, cb);
+        // first query of [lo, end) that attends to one of the two keys from k0 on, and how many patches they take
+        auto span = [&](int k0, int L, int lo, int end, int &first) __attribute__((always_inline)) {
+            const int ka = min(k0, L - 1), kb = min(k0 + 1, L - 1);
+            first = max(inv_lo(ka, KS), lo);
+            return (min(inv_hi(kb, L, KS), end) - first + 1) >> 1;
+        };
+        int r0, r1, c0, c1;
+        npr = max(span(wr0, s.H, br, rend, r0), span(wr0 + 2, s.H, br, rend, r1));
+        npc = max(span(wc0, s.W, bc, cend, c0), span(wc0 + 2, s.W, bc, cend, c1));
+        if (wr0 >= s.H || wc0 >= s.W) npr = 0;
+        const int fr = min(ln.b >> 1 ? r1 : r0, br + G::HR - 2 * max(npr, 0));
+        const int fc = min(ln.b & 1 ? c1 : c0, bc + G::HC - 2 * max(npc, 0));
+        base = ((fr - br) * G::HC + fc - bc) * G::PITCH + second_channel<D>(ln);
+        // (at most 14 rows of an image of at most 2^16 columns: below 2^30 bytes)
+        constexpr unsigned kNone = 0x60000000u;
+        const int64_t row0 = img_tok + (int64_t)br * s.W;
+        const auto buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(ws_w + row0 * (G::KK * NB)), 0,
+                                                           (rend - br) * s.W * (G::KK * NB * 4), 0x00027000);
+        unsigned col[NP];
+#pragma unroll
+        for (int pc = 0; pc < NP; pc++) {
+            const int qc = fc + 2 * pc + (g & 1), at = kc - win_start(qc, s.W, KS);
+            col[pc] = qc < cend && (unsigned)at < (unsigned)KS ? (unsigned)(qc * G::KK + at) * (4u * NB) : kNone;
+        }
+#pragma unroll
+        for (int pr = 0; pr < NP; pr++) {
+            if (pr >= npr) break;
+            const int qr = fr + 2 * pr + (g >> 1), at = kr - win_start(qr, s.H, KS);
+            const unsigned row = qr < rend && (unsigned)at < (unsigned)KS
+                                     ? (unsigned)((qr - br) * s.W * G::KK + at * KS) * (4u * NB) : kNone;
+#pragma unroll
+            for (int pc = 0; pc < NP; pc++) {
+                if (pc >= npc) break;
+                if constexpr (NB == 2) {
+                    const auto pair = __builtin_amdgcn_raw_buffer_load_b64(buf, row + col[pc], 0, 0);
+                    w[0][pr * NP + pc] = __uint_as_float(pair[0]);
+                    w[1][pr * NP + pc] = __uint_as_float(pair[1]);
+                } else {
+                    w[0][pr * NP + pc] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(buf, row + col[pc], 0, 0));
+                }
+            }
+        }
     };
 
     f32x4 acc[NB][G::DT];
@@ -673,79 +727,73 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, 
     for (int b = 0; b < NB; b++)
 #pragma unroll
         for (int m = 0; m < G::DT; m++) acc[b][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    Regs32 st[NB];
-    const int rows = s.H > 2 * NP && s.H <= 2 * KS ? 2 * NP : G::HR, cols = s.W > 2 * NP && s.W <= 2 * KS ? 2 * NP : G::HC;
-    for (int br = qa; br < qb; br += rows) {
-        for (int bc = ca; bc < cb; bc += cols) {
-            fetch32<D, KS>(st[0], image32(x0, tl), x0.sh, x0.sw, br, bc, qb, cb);
-            if constexpr (NB == 2) fetch32<D, KS>(st[1], image32(x1, tl), x1.sh, x1.sw, br, bc, qb, cb);
-            // patches of the block that the wave's keys need (the same number for its blocks of keys), and this
-            // lane's first query: moved up where its last patch would leave the staged rows
-            const int rend = min(rows, qb - br), cend = min(cols, cb - bc);
-            int r0, r1, c0, c1;
-            const int npr = max(span(wr0, s.H, br, rend, r0), span(wr0 + 2, s.H, br, rend, r1));
-            const int npc = max(span(wc0, s.W, bc, cend, c0), span(wc0 + 2, s.W, bc, cend, c1));
-            const int fr = min(ln.b >> 1 ? r1 : r0, br + G::HR - 2 * max(npr, 0));
-            const int fc = min(ln.b & 1 ? c1 : c0, bc + G::HC - 2 * max(npc, 0));
-            // weights of query g of every patch for this lane's key; zero where it does not attend or is not in the block
-            float w[NB][NP * NP];
+    int br = qa, bc = ca;
+    fetch_rows(br, bc);
+    weights(br, bc);
+    for (;;) {
+#pragma unroll
+        for (int b = 0; b < NB; b++) commit32<D, KS>(lds[b], st[b]);
+        __syncthreads();
+        bc += cols;
+        if (bc >= cb) bc = ca, br += rows;
+        const bool more = br < qb;
+        if (more) fetch_rows(br, bc);
+        const float *xrow[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) xrow[b] = lds[b] + base;
+        if ((KS > 3 || D < 128) && npr == G::PW && npc == G::PW) {
+            // The patches of an inner tile, without a branch between them: a token's operands are read a token ahead (B4 N4 96x96
+            // d64 k7 85 -> 70 us, d128 k7 256 -> 181; the four patches of d128 k3 56 -> 62).
+            float x[2][NB][G::DT], wb[NB][4];
+#pragma unroll
+            for (int b = 0; b < NB; b++) second_fetch<D>(xrow[b], x[0][b]);
+            each_step([&](auto at) __attribute__((always_inline)) {
+                constexpr int step = decltype(at)::value, next = step + 1;
+                if constexpr (next < G::STEPS)
+#pragma unroll
+                    for (int b = 0; b < NB; b++) second_fetch<D>(xrow[b] + G::at(next >> 2, next & 3), x[next & 1][b]);
+                if constexpr (step % 4 == 0)
+#pragma unroll
+                    for (int b = 0; b < NB; b++) spread_rows(w[b][step / 4 / G::PW * NP + step / 4 % G::PW], wb[b]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int b = 0; b < NB; b++) second_step<D>(x[step & 1][b], wb[b][step & 3], acc[b]);
+                __builtin_amdgcn_sched_barrier(0);
+            }, std::make_integer_sequence<int, G::STEPS>{});
+        } else {
 #pragma unroll
             for (int pr = 0; pr < NP; pr++) {
-                const int qr = fr + 2 * pr + (g >> 1);
-                const int kpr = kr - win_start(min(qr, s.H - 1), s.H, KS);
-                const bool rok = wave_on && qr < br + rend && (unsigned)kpr < (unsigned)KS;
+                if (pr >= npr) break;
 #pragma unroll
                 for (int pc = 0; pc < NP; pc++) {
-                    if (pr >= npr || pc >= npc) continue;
-                    const int qc = fc + 2 * pc + (g & 1);
-                    const int kpc = kc - win_start(min(qc, s.W - 1), s.W, KS);
-                    const bool ok = rok && qc < bc + cend && (unsigned)kpc < (unsigned)KS;
-                    const float *wp = ws_w + ((img_tok + (int64_t)qr * s.W + qc) * G::KK + kpr * KS + kpc) * NB;
-                    if constexpr (NB == 2) {
-                        const f32x2 pair = ok ? *reinterpret_cast<const f32x2 *>(wp) : f32x2{0.f, 0.f};
-                        w[0][pr * NP + pc] = pair[0];
-                        w[1][pr * NP + pc] = pair[1];
-                    } else {
-                        w[0][pr * NP + pc] = ok ? *wp : 0.f;
-                    }
-                }
-            }
-            __syncthreads();  // the previous block's rows are no longer read
+                    if (pc >= npc) break;
+                    // A patch's operands are read from LDS ahead of its matrix instructions.
+                    float x[4][NB][G::DT], wb[NB][4];
 #pragma unroll
-            for (int b = 0; b < NB; b++) commit32<D, KS>(lds[b], st[b]);
-            __syncthreads();
-            if (wave_on) {
-                const int base = ((fr - br) * G::HC + fc - bc) * G::PITCH + second_channel<D>(ln);
+                    for (int i = 0; i < 4; i++)
 #pragma unroll
-                for (int pr = 0; pr < NP; pr++) {
-                    if (pr >= npr) break;
+                        for (int b = 0; b < NB; b++)
+                            second_fetch<D>(xrow[b] + ((2 * pr + (i >> 1)) * G::HC + 2 * pc + (i & 1)) * G::PITCH, x[i][b]);
 #pragma unroll
-                    for (int pc = 0; pc < NP; pc++) {
-                        if (pc >= npc) break;
-                        // A patch's operands are read from LDS ahead of its matrix instructions.
-                        float x[4][NB][G::DT], wb[NB][4];
+                    for (int b = 0; b < NB; b++) spread_rows(w[b][pr * NP + pc], wb[b]);
 #pragma unroll
-                        for (int i = 0; i < 4; i++)
+                    for (int i = 0; i < 4; i++)
 #pragma unroll
-                            for (int b = 0; b < NB; b++)
-                                second_fetch<D>(lds[b] + base + ((2 * pr + (i >> 1)) * G::HC + 2 * pc + (i & 1)) * G::PITCH, x[i][b]);
-#pragma unroll
-                        for (int b = 0; b < NB; b++) spread_rows(w[b][pr * NP + pc], wb[b]);
-#pragma unroll
-                        for (int i = 0; i < 4; i++)
-#pragma unroll
-                            for (int b = 0; b < NB; b++) second_step<D>(x[i][b], wb[b][i], acc[b]);
-                    }
+                        for (int b = 0; b < NB; b++) second_step<D>(x[i][b], wb[b][i], acc[b]);
                 }
             }
         }
+        if (!more) break;
+        weights(br, bc);
+        __syncthreads();  // every wave is done with these rows
     }
-    if (!wave_on) return;
+    if (wr0 >= s.H || wc0 >= s.W) return;
     const int64_t tok = img_tok + (int64_t)kr * s.W + kc;
 #pragma unroll
-    for (int b = 0; b < NB; b++) second_pieces<D>(acc[b]);
-    store32<D, kLines32<D, KS>>(out0 + tok * D, g, acc[0], second_flip<D>(ln), mul0, 0.f, live);
-    if constexpr (NB == 2) store32<D, kLines32<D, KS>>(out1 + tok * D, g, acc[1], second_flip<D>(ln), mul1, 0.f, live);
+    for (int b = 0; b < NB; b++) {
+        second_pieces<D>(acc[b]);
+        store32<D, kLines32<D, KS>>((b ? out1 : out0) + tok * D, g, acc[b], second_flip<D>(ln), b ? mul1 : mul0, 0.f, live);
+    }
 }
 
 // ------------------------------------------------------------------ dispatch
@@ -827,7 +875,7 @@ int launch_fwd_mfma_f32(const FwdArgs &a, hipStream_t st) {
 int launch_bwd_mfma_f32(const BwdArgs &a, hipStream_t st) {
     auto al = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
     if (!layout32_ok(a.q) || !layout32_ok(a.k) || !layout32_ok(a.v) || !layout32_ok(a.d_o) ||
-        !al(a.dq) || !al(a.dk) || !al(a.dv))
+        !al(a.dq) || !al(a.dk) || !al(a.dv) || a.s.W > 65536)  // (rows that long only with strides of zero)
         return launch_bwd_simt(a, ENATTEN_F32, st);
     ENATTEN_F32_BY_D(bwd32_launch, a, st)
     set_error("no float32 matrix-core kernel for head_dim %d, kernel_size %d", a.s.D, a.s.kh);
