@@ -369,8 +369,7 @@ struct BiasGrad {
         }
     }
 };
-// dS of a lane's halo tokens as operands of dQ's product (tiles without tokens hold zeros already),
-// and, times 1 / Z (0 for a lane without a query, or with one that again_dq computes), as terms of the
+// dS of a lane's halo tokens as operands of dQ's product (zero in tiles without tokens), and, times 1 / Z (0 for a lane without a query, or with one that again_dq computes), as terms of the
 // bias gradient
 template <bool BF, int KS, int STEPS>
 __device__ __forceinline__ void operand_and_sums(Op8 (&dsb)[STEPS], f32x4 (&ds)[Bias<KS>::USED], DsScale<BF> &scl,
@@ -391,6 +390,10 @@ __device__ __forceinline__ void operand_and_sums(Op8 (&dsb)[STEPS], f32x4 (&ds)[
             put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds[mt][i] * f);
             ds[mt][i] = zinv != 0.f ? ds[mt][i] * zinv : 0.f;
         }
+#pragma unroll
+    for (int mt = Bias<KS>::USED; mt < 2 * STEPS; mt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, 0.f);
 }
 // d_rpb[head][entry] = the sum over batch entries and tiles of the rows that the dQ pass left, in a
 // fixed order: a workgroup takes 16 entries of a head, 64 threads a strided share of the rows each.
@@ -981,6 +984,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             constexpr bool kKeepDp = !(G::WAVES == 1 && G::MT >= 16);
             f32x4 dp[kKeepDp ? G::MT : 1];
             Op8 dsb[G::KSTEPS];
+            f32x4 ds_all[kBias ? Bias<KS>::USED : 1];  // with a bias: P, then dS, in float32
             float dpart = 0.f, zsum = 0.f;
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
@@ -1001,12 +1005,13 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                     cs[i] = exp_unit(ok ? x : -INFINITY);
                     if constexpr (kBias) zsum += cs[i];
                     dpart = fmaf(cs[i], cp[i], dpart);
-                    put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, cs[i]);
+                    if constexpr (!kBias) put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, cs[i]);
                 }
+                if constexpr (kBias)
+                    if (mt < Bias<KS>::USED) ds_all[mt] = cs;
                 if constexpr (kKeepDp) dp[mt] = cp;
             }
             const float zinv = kBias ? 1.f / col_sum(zsum) : 1.f, delta = col_sum(dpart) * zinv;
-            f32x4 ds_all[kBias ? Bias<KS>::USED : 1];
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
                 f32x4 cp;
@@ -1021,10 +1026,12 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
                 }
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float p = get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i);
-                    const float ds = p * (cp[i] - delta);
-                    if constexpr (!kBias) put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
-                    else if (mt < Bias<KS>::USED) ds_all[mt][i] = ds;
+                    if constexpr (!kBias) {
+                        const float p = get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i);
+                        put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, p * (cp[i] - delta));
+                    } else if (mt < Bias<KS>::USED) {
+                        ds_all[mt][i] *= cp[i] - delta;
+                    }
                 }
             }
 
@@ -1209,6 +1216,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDq2Wgs<D, KS, NW>)) void bw
         if (FULL || lq.wave_on) {
             const int bq = kTable ? Bias<KS>::query(lq) : 0;
             Op8 dsb[G::KSTEPS];
+            f32x4 ds_all[kBias ? Bias<KS>::USED : 1];  // with a bias: P, then dS, in float32
             float dpart = 0.f, zsum = 0.f;
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++) {
@@ -1226,7 +1234,8 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDq2Wgs<D, KS, NW>)) void bw
                     const float p = exp_unit(ok ? x : -INFINITY);
                     if constexpr (kBias) zsum += p;
                     dpart = fmaf(p, dp[mt][i], dpart);
-                    put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, p);
+                    if constexpr (!kBias) put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, p);
+                    else if (mt < Bias<KS>::USED) ds_all[mt][i] = p;
                 }
             }
             const float zinv = kBias ? 1.f / col_sum(zsum) : 1.f;
@@ -1235,22 +1244,22 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDq2Wgs<D, KS, NW>)) void bw
             if constexpr (BALANCED) {
                 float e = 0.f;
 #pragma unroll
-                for (int mt = 0; mt < G::MT; mt++)
+                for (int mt = 0; mt < Bias<KS>::USED; mt++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        e = fmaf(get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i), dp[mt][i] - most, e);
+                    for (int i = 0; i < 4; i++) e = fmaf(ds_all[mt][i], dp[mt][i] - most, e);
                 rest = col_sum(e) * zinv;
             }
             const float delta = BALANCED ? most + rest : most;
-            f32x4 ds_all[kBias ? Bias<KS>::USED : 1];
 #pragma unroll
             for (int mt = 0; mt < G::MT; mt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float p = get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i);
-                    const float ds = p * (dp[mt][i] - most - rest);
-                    if constexpr (!kBias) put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, ds);
-                    else if (mt < Bias<KS>::USED) ds_all[mt][i] = ds;
+                    if constexpr (!kBias) {
+                        const float p = get<BF>(dsb[mt >> 1], (mt & 1) * 4 + i);
+                        put<BF>(dsb[mt >> 1], (mt & 1) * 4 + i, p * (dp[mt][i] - most));
+                    } else if (mt < Bias<KS>::USED) {
+                        ds_all[mt][i] *= dp[mt][i] - most - rest;
+                    }
                 }
             DsScale<BF> scl;
             if constexpr (kBias) {
