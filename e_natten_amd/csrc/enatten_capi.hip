@@ -611,14 +611,13 @@ size_t enatten2d_bwd_window_workspace_bytes(int B, int heads, int H, int W, int 
     return (size_t)B * heads * H * W * (4 + (with_rpb ? (size_t)kernel_h * kernel_w : 0)) * sizeof(float);
 }
 
-int enatten2d_bwd_window(const void *q, const void *k, const void *v, const void *rpb,
-                         const void *o, const void *d_o, const float *lse, void *dq, void *dk,
-                         void *dv, float *d_rpb, void *workspace, int B, int heads, int H, int W,
-                         int D, int kernel_h, int kernel_w, int causal_h, int causal_w, int dtype,
-                         const int64_t *q_strides, const int64_t *k_strides,
-                         const int64_t *v_strides, const int64_t *o_strides,
-                         const int64_t *do_strides, float scale, void *stream) {
-    const char *fn = "enatten2d_bwd_window";
+static int bwd_window(const char *fn, const void *q, const void *k, const void *v, const void *rpb,
+                      const void *o, const void *d_o, const float *lse, void *dq, void *dk,
+                      void *dv, void *d_rpb, bool rpb_typed, void *workspace, int B, int heads, int H, int W,
+                      int D, int kernel_h, int kernel_w, int causal_h, int causal_w, int dtype,
+                      const int64_t *q_strides, const int64_t *k_strides,
+                      const int64_t *v_strides, const int64_t *o_strides,
+                      const int64_t *do_strides, float scale, void *stream) {
     const bool plain = kernel_h == kernel_w && !causal_h && !causal_w && !rpb;
     int rc = check_shape(fn, B, heads, H, W, D, plain ? kernel_h : 1, dtype);
     if (rc) return rc;
@@ -663,8 +662,32 @@ int enatten2d_bwd_window(const void *q, const void *k, const void *v, const void
     if (dtype == ENATTEN_F64) return bwd_f64(fn, a, ws_floats, static_cast<hipStream_t>(stream));
     if (use_band(a, dtype)) return launch_bwd_band(a, dtype, static_cast<hipStream_t>(stream));
     if (rpb && kernel_h == kernel_w && (use_mfma(D, kernel_h, dtype) || use_two_terms(D, kernel_h, dtype)))
-        return launch_bwd_mfma_bias(a, dtype, static_cast<hipStream_t>(stream));
-    return launch_bwd_simt(a, dtype, static_cast<hipStream_t>(stream));
+        return launch_bwd_mfma_bias(a, dtype, static_cast<hipStream_t>(stream), rpb_typed);
+    return launch_bwd_simt(a, dtype, static_cast<hipStream_t>(stream), rpb_typed);
+}
+
+int enatten2d_bwd_window(const void *q, const void *k, const void *v, const void *rpb,
+                         const void *o, const void *d_o, const float *lse, void *dq, void *dk,
+                         void *dv, float *d_rpb, void *workspace, int B, int heads, int H, int W,
+                         int D, int kernel_h, int kernel_w, int causal_h, int causal_w, int dtype,
+                         const int64_t *q_strides, const int64_t *k_strides,
+                         const int64_t *v_strides, const int64_t *o_strides,
+                         const int64_t *do_strides, float scale, void *stream) {
+    return bwd_window("enatten2d_bwd_window", q, k, v, rpb, o, d_o, lse, dq, dk, dv, d_rpb, false, workspace, B, heads, H,
+                      W, D, kernel_h, kernel_w, causal_h, causal_w, dtype, q_strides, k_strides, v_strides, o_strides,
+                      do_strides, scale, stream);
+}
+
+int enatten2d_bwd_window_typed(const void *q, const void *k, const void *v, const void *rpb,
+                               const void *o, const void *d_o, const float *lse, void *dq, void *dk,
+                               void *dv, void *d_rpb, void *workspace, int B, int heads, int H, int W,
+                               int D, int kernel_h, int kernel_w, int causal_h, int causal_w, int dtype,
+                               const int64_t *q_strides, const int64_t *k_strides,
+                               const int64_t *v_strides, const int64_t *o_strides,
+                               const int64_t *do_strides, float scale, void *stream) {
+    return bwd_window("enatten2d_bwd_window_typed", q, k, v, rpb, o, d_o, lse, dq, dk, dv, d_rpb, true, workspace, B,
+                      heads, H, W, D, kernel_h, kernel_w, causal_h, causal_w, dtype, q_strides, k_strides, v_strides,
+                      o_strides, do_strides, scale, stream);
 }
 
 static int view_1d(const char *fn, const char *name, const void *p, const int64_t *st, int N,

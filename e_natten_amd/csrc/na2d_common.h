@@ -50,7 +50,7 @@ struct BwdArgs {
     float *zinv;         // scratch [B, N, H, W]: 1 / sum_j exp(S_j - lse) (vector-ALU kernels)
     Shape s;
     const void *rpb = nullptr;  // relative position bias [N, 2*kh-1, 2*kw-1] in the tensors' type
-    float *d_rpb = nullptr;     // its gradient, float32, fully overwritten (general kernels)
+    void *d_rpb = nullptr;      // its gradient, fully overwritten; float32 unless the launch is told otherwise
     float *ds_pairs = nullptr;  // scratch [B, N, H, W, kh*kw]: dS of every (query, window position),
                                 // from which d_rpb is summed in a fixed order
 };
@@ -125,7 +125,8 @@ struct ProfScope {
 
 // general fp32-FMA kernels: any D <= 1024, any odd window, f32 / bf16 / f16
 int launch_fwd_simt(const FwdArgs &a, int dtype, hipStream_t st);
-int launch_bwd_simt(const BwdArgs &a, int dtype, hipStream_t st);
+// (rpb_typed: a.d_rpb is of the tensors' type, here and in launch_bwd_mfma_bias)
+int launch_bwd_simt(const BwdArgs &a, int dtype, hipStream_t st, bool rpb_typed = false);
 
 // float64 tensors (plain double arithmetic; windows as the general kernels, no bias).  The
 // backward keeps two doubles per query in a.delta (16-byte aligned).
@@ -168,7 +169,7 @@ int launch_bwd_small(const BwdArgsSub &a, int dtype, hipStream_t st);
 // (2k-1)^2 floats per tile): square centred windows that mfma_supported takes, and head dims between 32
 // and 64 with kernel_size 11 and 13
 int launch_fwd_mfma_bias(const FwdArgs &a, int dtype, hipStream_t st);
-int launch_bwd_mfma_bias(const BwdArgs &a, int dtype, hipStream_t st);
+int launch_bwd_mfma_bias(const BwdArgs &a, int dtype, hipStream_t st, bool rpb_typed);
 // ... and those dims and sizes without a bias
 int launch_fwd_two_terms(const FwdArgs &a, int dtype, hipStream_t st);
 int launch_bwd_two_terms(const BwdArgs &a, int dtype, hipStream_t st);

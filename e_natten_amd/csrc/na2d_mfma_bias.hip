@@ -22,6 +22,8 @@ constexpr bool kTable = true;
 namespace enatten {
 
 int launch_fwd_mfma_bias(const FwdArgs &a, int dtype, hipStream_t st) { return fwd_dispatch(a, dtype, st); }
-int launch_bwd_mfma_bias(const BwdArgs &a, int dtype, hipStream_t st) { return bwd_dispatch(a, dtype, 0, st); }
+int launch_bwd_mfma_bias(const BwdArgs &a, int dtype, hipStream_t st, bool rpb_typed) {
+    return bwd_dispatch(a, dtype, rpb_typed ? kRpbTyped : 0, st);
+}
 
 }  // namespace enatten

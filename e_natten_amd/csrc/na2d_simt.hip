@@ -392,7 +392,8 @@ __global__ __launch_bounds__(256) void bwd_dkdv_simt(BwdArgs a, int tiles_x, int
 // no bias).  One workgroup per entry walks all queries of the head in a fixed order, each
 // thread a strided share, and adds the 256 partial sums in a fixed tree: the same bits on
 // every run, where adding the pairs with atomics as they are formed does not give that.
-__global__ __launch_bounds__(256) void rpb_grad_reduce(const float *ds_pairs, float *d_rpb, Shape s) {
+template <typename T>
+__global__ __launch_bounds__(256) void rpb_grad_reduce(const float *ds_pairs, T *d_rpb, Shape s) {
     __shared__ float part[256];
     const int EW = 2 * s.kw - 1, E = (2 * s.kh - 1) * EW;
     const int n = blockIdx.x / E, e = blockIdx.x % E;
@@ -412,7 +413,7 @@ __global__ __launch_bounds__(256) void rpb_grad_reduce(const float *ds_pairs, fl
         if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) d_rpb[blockIdx.x] = part[0];
+    if (threadIdx.x == 0) cvt_out(part[0], d_rpb[blockIdx.x]);
 }
 
 // ---------------------------------------------------------------- dispatch
@@ -456,7 +457,9 @@ int fwd_cfg(const FwdArgs &a, bool vec, hipStream_t st) {
 }
 
 template <typename T, int G, int CH>
-int bwd_cfg(const BwdArgs &a, bool vec, hipStream_t st) {
+// (how: bit 0 for vector loads and stores, bit 1 for a bias gradient of type T)
+int bwd_cfg(const BwdArgs &a, int how, hipStream_t st) {
+    const bool vec = how & 1;
     int tx, ty;
     const dim3 grid = grid_for<G>(a.s, tx, ty);
     {
@@ -469,9 +472,11 @@ int bwd_cfg(const BwdArgs &a, bool vec, hipStream_t st) {
         if (vec) hipLaunchKernelGGL((bwd_dkdv_simt<T, G, CH, true>), grid, dim3(256), 0, st, a, tx, ty);
         else hipLaunchKernelGGL((bwd_dkdv_simt<T, G, CH, false>), grid, dim3(256), 0, st, a, tx, ty);
     }
-    if (a.d_rpb)
-        hipLaunchKernelGGL(rpb_grad_reduce, dim3((unsigned)(a.s.N * (2 * a.s.kh - 1) * (2 * a.s.kw - 1))),
-                           dim3(256), 0, st, a.ds_pairs, a.d_rpb, a.s);
+    if (a.d_rpb) {
+        const dim3 entries((unsigned)(a.s.N * (2 * a.s.kh - 1) * (2 * a.s.kw - 1)));
+        if (how & 2) hipLaunchKernelGGL((rpb_grad_reduce<T>), entries, dim3(256), 0, st, a.ds_pairs, static_cast<T *>(a.d_rpb), a.s);
+        else hipLaunchKernelGGL((rpb_grad_reduce<float>), entries, dim3(256), 0, st, a.ds_pairs, static_cast<float *>(a.d_rpb), a.s);
+    }
     return check_launch("enatten2d_bwd");
 }
 
@@ -495,11 +500,11 @@ int fwd_t(const FwdArgs &a, hipStream_t st) {
     ENATTEN_BY_D(fwd_cfg, T, a, vec, st);
 }
 template <typename T>
-int bwd_t(const BwdArgs &a, hipStream_t st) {
+int bwd_t(const BwdArgs &a, bool rpb_typed, hipStream_t st) {
     const bool vec = a.s.D % 8 == 0 && vec_ok(a.q) && vec_ok(a.k) && vec_ok(a.v) && vec_ok(a.o) &&
                      vec_ok(a.d_o) && vec_ok(a.dq) && vec_ok(a.dk) && vec_ok(a.dv) && a.gsb % 8 == 0 &&
                      a.gsn % 8 == 0 && a.gsh % 8 == 0 && a.gsw % 8 == 0;
-    ENATTEN_BY_D(bwd_cfg, T, a, vec, st);
+    ENATTEN_BY_D(bwd_cfg, T, a, (vec ? 1 : 0) | (rpb_typed ? 2 : 0), st);
 }
 
 }  // namespace
@@ -518,15 +523,15 @@ int launch_fwd_simt(const FwdArgs &a, int dtype, hipStream_t st) {
     return ENATTEN_EINVAL;
 }
 
-int launch_bwd_simt(const BwdArgs &a, int dtype, hipStream_t st) {
+int launch_bwd_simt(const BwdArgs &a, int dtype, hipStream_t st, bool rpb_typed) {
     if (a.s.D > 1024) {
         set_error("head dim %d exceeds the supported maximum of 1024", a.s.D);
         return ENATTEN_EUNSUPPORTED;
     }
     switch (dtype) {
-        case ENATTEN_F32: return bwd_t<float>(a, st);
-        case ENATTEN_BF16: return bwd_t<bf16_t>(a, st);
-        case ENATTEN_F16: return bwd_t<f16_t>(a, st);
+        case ENATTEN_F32: return bwd_t<float>(a, rpb_typed, st);
+        case ENATTEN_BF16: return bwd_t<bf16_t>(a, rpb_typed, st);
+        case ENATTEN_F16: return bwd_t<f16_t>(a, rpb_typed, st);
     }
     set_error("unknown dtype %d", dtype);
     return ENATTEN_EINVAL;

@@ -414,7 +414,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> na_window_bwd(const Tensor &q_, const
     const c10::DeviceGuard guard(q_.device());
     dq = at::empty(q_.sizes(), q_.options());
     dk = at::empty_like(dq), dv = at::empty_like(dq);
-    d_rpb = at::empty(bias ? rpb_->sizes() : at::IntArrayRef({0}), q_.options().dtype(at::kFloat));
+    d_rpb = at::empty(bias ? rpb_->sizes() : at::IntArrayRef({0}), bias ? q_.options() : q_.options().dtype(at::kFloat));
     if (!q_.is_meta()) {
         const Tensor q = kernel_layout(q_), k = kernel_layout(k_), v = kernel_layout(v_);
         const Tensor o = kernel_layout(o_), d_o = kernel_layout(d_o_), lse = lse_.contiguous();
@@ -423,14 +423,13 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> na_window_bwd(const Tensor &q_, const
         Tensor ws = at::empty({(int64_t)enatten2d_bwd_window_workspace_bytes(im.B, im.N, im.H, im.W, (int)kh,
                                                                              (int)kw, bias)},
                               q.options().dtype(at::kByte));
-        check_rc(enatten2d_bwd_window(
+        check_rc(enatten2d_bwd_window_typed(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), bias ? rpb.data_ptr() : nullptr, o.data_ptr(),
             d_o.data_ptr(), lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-            bias ? d_rpb.data_ptr<float>() : nullptr, ws.data_ptr(), im.B, im.N, im.H, im.W, im.D, (int)kh,
+            bias ? d_rpb.data_ptr() : nullptr, ws.data_ptr(), im.B, im.N, im.H, im.W, im.D, (int)kh,
             (int)kw, ch, cw, dtype_code(q), Strides(q), Strides(k), Strides(v), Strides(o), Strides(d_o),
             (float)scale, c10::hip::getCurrentHIPStream().stream()));
     }
-    if (bias && q_.scalar_type() != at::kFloat) d_rpb = d_rpb.to(q_.scalar_type());
     return {dq, dk, dv, d_rpb};
 }
 // (through the dispatcher, as call_fwd and call_bwd)

@@ -239,6 +239,14 @@ int enatten2d_bwd_window(const void *q, const void *k, const void *v, const void
                          const int64_t *q_strides, const int64_t *k_strides,
                          const int64_t *v_strides, const int64_t *o_strides,
                          const int64_t *do_strides, float scale, void *stream);
+/* The same with d_rpb in the tensors' element type: each sum is formed in float32 and rounded once. */
+int enatten2d_bwd_window_typed(const void *q, const void *k, const void *v, const void *rpb,
+                               const void *o, const void *d_o, const float *lse, void *dq, void *dk,
+                               void *dv, void *d_rpb, void *workspace, int B, int heads, int H, int W,
+                               int D, int kernel_h, int kernel_w, int causal_h, int causal_w, int dtype,
+                               const int64_t *q_strides, const int64_t *k_strides,
+                               const int64_t *v_strides, const int64_t *o_strides,
+                               const int64_t *do_strides, float scale, void *stream);
 
 /*
  * 1D neighborhood attention on [B, heads, T, D] tensors: query t attends the

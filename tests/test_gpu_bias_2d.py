@@ -177,3 +177,26 @@ def test_values_that_are_not_finite_stay_in_their_windows(shape, ks, dtype, whic
         norm = ((x - r).norm() / r.norm()).item()
         print("   ", name, "2-norm %.2e" % norm, flush=True)
         assert norm <= (4e-3 if dtype == BF16 else 5e-4), (name, norm)  # (as in test_bias)
+
+
+@pytest.mark.parametrize("shape,kernel,dtype", [
+    ((5, 3, 17, 21, 32), (7, 7), BF16),     # the tiles' sums, more rows than threads of an entry, and a remainder
+    ((1, 2, 9, 8, 64), (5, 5), F16),        # fewer rows than threads
+    ((2, 2, 12, 13, 20), (5, 5), BF16),     # the general kernels: head_dim
+    ((2, 2, 11, 14, 32), (3, 7), F16),      # ... rectangular windows
+    ((1, 2, 10, 12, 32), (3, 3), torch.float32)])
+def test_gradient_in_the_tensors_type(shape, kernel, dtype):
+    # the native binding has the sums written in the tensors' type, the Python Function converts float32 ones
+    ensure_built()
+    from e_natten_amd import natten2d, ops
+    print("case bias gradient", shape, kernel, dtype, flush=True)
+    assert ops.NATIVE_BINDING
+    q, k, v, g = (t.cuda() for t in make_inputs(shape, dtype, seed=3))
+    rpb = torch.randn(shape[1], 2 * kernel[0] - 1, 2 * kernel[1] - 1, generator=torch.Generator().manual_seed(7)).to(dtype).cuda()
+    scale = shape[-1] ** -0.5
+    both = []
+    for call in (lambda r: natten2d(q, k, v, kernel, scale, rpb=r),
+                 lambda r: ops.Natten2dWindow.apply(q, k, v, r, kernel, (False, False), scale)):
+        r = rpb.clone().requires_grad_(True)
+        both.append(torch.autograd.grad(call(r), r, g)[0])
+    assert both[0].dtype == dtype and torch.equal(*both)
