@@ -553,8 +553,10 @@ __device__ __forceinline__ void again_keys(const BArgs &a, const ATile &tl, int 
 // With a bias the head_dim 32 forward takes 169 to 175 registers (k = 7 and 9), one more than three
 // waves per SIMD have: budgeted for three, B8 N8 112x112 k7 114.8 -> 97.8 us.  At k = 5 four (three at
 // head_dim 64) take a register or two too many without a budget (B8 N4 56x56 d64 k5 16.6 us with two).
+// Without one the compiler left alone takes 146 registers at head_dim 32, k = 7, where four waves per SIMD fit without a
+// spill: B6 N9 91x128 49.4 -> 47.3 us, B1 N16 69x69 8.0 -> 6.8; k = 9 spills there.
 template <int D, int KS, int NW>
-constexpr int kFwdWaves = kBias && D == 32 && KS == 5 ? 4
+constexpr int kFwdWaves = D == 32 && (kBias ? KS == 5 : !kNarrow && KS <= 7) ? 4
                           : kBias && ((D == 32 && KS <= 9) || (D == 64 && KS == 5)) ? 3 : Geo<D, KS, NW>::WAVES;
 template <bool BF, int D, int KS, bool ROLL, int NW = 4, bool FULL = false>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void fwd_mfma(FArgs a, int tiles_r, int tiles_c, int ntiles, Runs rp) {
@@ -882,8 +884,13 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
 // per SIMD (LDS admits three workgroups per CU and more); B8 N2 112x112 k = 7: 27.8 -> 24.4
 // us, B4 N4 128x128 k = 9: 37.1 -> 35.0 (with a bias it spills 55 there).  The forward is as fast or faster compiled for two
 // (it then takes about 150 registers and runs three per SIMD anyway).
+// (not the sub-grids of a dilated call: 80 bytes of scratch in three at k = 7, B8 N4 112x112 dilation 2 67.4 -> 56.3 us in two)
+// k = 3 and 5 took one or two registers more than four waves per SIMD have (head_dim 64, k = 3: one more than
+// three): B8 N16 63x93 d32 k5 54.0 -> 48.6 us, B8 N2 112x112 k3 15.1 -> 13.3, B4 N4 128x128 d64 k3 28.7 -> 27.4.
 template <int D, int KS, int NW>
-constexpr int kDqWaves = D == 32 && (KS == 7 || KS == 9) && NW == 4 && !kBias ? 3 : Geo<D, KS, NW>::WAVES;
+constexpr int kDqWaves = kBias || NW != 4 ? Geo<D, KS, NW>::WAVES
+                         : !kNarrow && D == 32 && KS <= 5 ? 4
+                         : (D == 32 && ((KS == 7 && !kSub) || KS == 9)) || (!kNarrow && D == 64 && KS == 3) ? 3 : Geo<D, KS, NW>::WAVES;
 // FULL: as in fwd_mfma (no wave switched off, no store predicated, the staged rows go to LDS at
 // the end of a tile's pass through the loop).
 template <bool BF, int D, int KS, bool FRAME, bool ROLL, int NW = 4, bool FULL = false>
@@ -1975,9 +1982,15 @@ template <int D, int KS>
 constexpr bool kDkdvFrameOnly = !fits<D, KS>();
 template <int D, int KS, int SP>
 constexpr int kFrameKS = kDkdvFrameOnly<D, KS> ? 5 : SP == 2 && KS >= 9 ? 9 + KS / 2 : KS;
+// head_dim 32, k = 5: four waves per SIMD cost 12 bytes of scratch and gain where a workgroup has many tiles (B8 N16 63x93 66.6 ->
+// 57.9 us, B4 N16 128x128 93.5 -> 87.6, B8 N8 41x77 23.9 -> 21.0), and lose where the same rounds are walked by
+// more workgroups (B8 N2 112x112 16.2 -> 16.9); at k = 7 they spill (B8 N2 112x112 22.4 -> 26.8).  In the builds for narrow heads
+// and sub-grids head_dim 64, k = 3 spills 100 to 148 bytes in three and runs in two: d48 B4 N4 128x128 42.2 -> 35.5 us, 61x83
+// float16 16.9 -> 12.9.
 template <int D, int KS, int SP>
 constexpr int kDkdvWaves =
     kDkdvFrameOnly<D, KS> ? 2 :
+    !kNarrow && D == 32 && KS == 5 ? 4 : kNarrow && !kBias && D == 64 && KS == 3 ? 2 :
     SP == 1 && D <= (kBias ? KS <= 5 ? 32 : 0 : 64) && 3 * (Geo<D, KS>::LDS_BYTES + 2048) <= 160 * 1024 ? 3 : Geo<D, KS, 4, SP>::WAVES;
 template <bool BF, int D, int KS, bool ROLL, int SP = 1>
 __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) void bwd_dkdv_mfma(
