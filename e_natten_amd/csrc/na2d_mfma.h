@@ -5,6 +5,7 @@
 
 #include <math.h>
 
+#include <numeric>
 #include <type_traits>
 
 #include "na2d_common.h"
@@ -553,11 +554,20 @@ __device__ __forceinline__ Tile tile_of(int t, int tiles_r, int tiles_c, int N, 
 // order.  The plan is the same for every tile, so it is computed once.
 template <int D, int KS, int NW = 4, int SP = 1>
 struct HaloPlan {
-    int rc[Geo<D, KS, NW, SP>::NL];  // halo row << 8 | halo column of chunk i
-    int ch8;                 // first channel of the thread's chunks
+    // Every PER chunks a thread's pixels are RPER whole rows further down, so it keeps PER places (halo row << 8 |
+    // halo column) instead of one for every chunk: 5 instead of 25 at head_dim 128, k = 13.
+    using G = Geo<D, KS, NW, SP>;
+    static constexpr int STEP = G::NT / G::CPR, PER = std::lcm(STEP, G::HC) / STEP, RPER = std::lcm(STEP, G::HC) / G::HC;
+    static constexpr int KEEP = PER < G::NL ? PER : G::NL;
+    int rc[KEEP];
+    // halo row and column of chunk i (a chunk behind the last pixel: a row below the halo, or its last pixel)
+    __device__ __forceinline__ int row(int i) const { return (rc[i % PER] >> 8) + i / PER * RPER; }
+    __device__ __forceinline__ int col(int i) const { return rc[i % PER] & 255; }
+    int ch8;                 // first channel of the thread's chunks (0 where the thread is off: it loads and drops them)
     int lds0;                // LDS element offset of chunk 0
-    bool on;                 // false: the tensor has no such channels (head dim below D); the
-                             // thread moves nothing and its LDS columns stay zero (zero_row)
+    bool on;                 // false: the tensor has no such channels (head dim below D); the thread loads others, without a
+                             // branch that would keep its registers from one fetch to the next, and writes nothing: its
+                             // LDS columns stay zero (zero_row)
 };
 template <int D, int KS, int NW = 4, int SP = 1>
 __device__ __forceinline__ HaloPlan<D, KS, NW, SP> make_plan(int dlim = D) {
@@ -566,14 +576,15 @@ __device__ __forceinline__ HaloPlan<D, KS, NW, SP> make_plan(int dlim = D) {
     HaloPlan<D, KS, NW, SP> pl;
     pl.ch8 = (threadIdx.x % G::CPR) * 8;
     pl.on = pl.ch8 < dlim;
+    if (!pl.on) pl.ch8 = 0;
     // the rows of one thread's chunks are NT / CPR apart, a multiple of 16 * RPL, so they
     // share one key and the chunk position is the same for all of them
     static_assert((G::NT / G::CPR) % (16 * G::RPL) == 0, "one chunk position per thread");
     pl.lds0 = G::chunk_at(threadIdx.x / G::CPR, threadIdx.x % G::CPR);
 #pragma unroll
-    for (int i = 0; i < G::NL; i++) {
+    for (int i = 0; i < pl.KEEP; i++) {
         int row = threadIdx.x / G::CPR + i * (G::NT / G::CPR);
-        row = row < G::HR * G::HC ? row : G::HR * G::HC - 1;  // tail: harmless duplicate
+        if (pl.PER >= G::NL) row = row < G::HR * G::HC ? row : G::HR * G::HC - 1;
         pl.rc[i] = ((row / G::HC) << 8) | (row % G::HC);
     }
     return pl;
@@ -598,11 +609,10 @@ __device__ __forceinline__ void halo_fetch(HaloRegs<D, KS, NW, SP> &reg, const H
     const char *base = reinterpret_cast<const char *>(img + hr0 * sh + hc0 * sw);
     const unsigned sh2 = (unsigned)sh * 2u, sw2 = (unsigned)sw * 2u;
     const int rmax = rlim - 1 - hr0, cmax = clim - 1 - hc0;
-    if (!pl.on) return;
 #pragma unroll
     for (int i = I0; i < I1; i++) {
-        const unsigned r = (unsigned)min(pl.rc[i] >> 8, rmax);
-        const unsigned c = (unsigned)min(pl.rc[i] & 255, cmax);
+        const unsigned r = (unsigned)min(pl.row(i), rmax);
+        const unsigned c = (unsigned)min(pl.col(i), cmax);
         const unsigned off = __umul24(r, sh2) + __umul24(c, sw2) + (unsigned)pl.ch8 * 2u;
         reg.v[i] = *reinterpret_cast<const u32x4 *>(base + off);
     }
@@ -633,13 +643,12 @@ __device__ __forceinline__ void halo_fetch_rows(HaloRegs<D, KS, NW, SP> &reg, co
     const char *base = reinterpret_cast<const char *>(img + yb * sh + hc0 * sw);
     const unsigned sh2 = (unsigned)sh * 2u, sw2 = (unsigned)sw * 2u;
     const int rmax = rlim - 1 - yb, cmax = clim - 1 - hc0;
-    if (!pl.on) return;
 #pragma unroll
     for (int i = 0; i < G::NL; i++) {
-        const int r = pl.rc[i] >> 8;
+        const int r = pl.row(i);
         if (r < nrows) {
             const unsigned rr = (unsigned)min(r, rmax);
-            const unsigned c = (unsigned)min(pl.rc[i] & 255, cmax);
+            const unsigned c = (unsigned)min(pl.col(i), cmax);
             const unsigned off = __umul24(rr, sh2) + __umul24(c, sw2) + (unsigned)pl.ch8 * 2u;
             reg.v[i] = *reinterpret_cast<const u32x4 *>(base + off);
         }
@@ -654,11 +663,11 @@ __device__ __forceinline__ void halo_commit_rows(short *lds, const HaloPlan<D, K
 #pragma unroll
     for (int i = 0; i < G::NL; i++) {
         const int pix = threadIdx.x / G::CPR + i * (G::NT / G::CPR);
-        const int r = pl.rc[i] >> 8;
+        const int r = pl.row(i);
         if (pix < G::HR * G::HC && r < nrows) {
             int slot = rot + r;
             slot = slot >= G::HR ? slot - G::HR : slot;
-            *reinterpret_cast<u32x4 *>(lds + G::chunk_at(slot * G::HC + (pl.rc[i] & 255),
+            *reinterpret_cast<u32x4 *>(lds + G::chunk_at(slot * G::HC + pl.col(i),
                                                           threadIdx.x % G::CPR)) = reg.v[i];
         }
     }
