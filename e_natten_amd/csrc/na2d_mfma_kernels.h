@@ -884,13 +884,14 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
 // per SIMD (LDS admits three workgroups per CU and more); B8 N2 112x112 k = 7: 27.8 -> 24.4
 // us, B4 N4 128x128 k = 9: 37.1 -> 35.0 (with a bias it spills 55 there).  The forward is as fast or faster compiled for two
 // (it then takes about 150 registers and runs three per SIMD anyway).
-// (not the sub-grids of a dilated call: 80 bytes of scratch in three at k = 7, B8 N4 112x112 dilation 2 67.4 -> 56.3 us in two)
+// (not the sub-grids of a dilated call: 80 bytes of scratch in three at k = 7, B8 N4 112x112 dilation 2 67.4 -> 56.3 us in two;
+// nor k = 9 there and in the build for narrow heads: B4 N4 128x128 d24 35.8 -> 34.0)
 // k = 3 and 5 took one or two registers more than four waves per SIMD have (head_dim 64, k = 3: one more than
 // three): B8 N16 63x93 d32 k5 54.0 -> 48.6 us, B8 N2 112x112 k3 15.1 -> 13.3, B4 N4 128x128 d64 k3 28.7 -> 27.4.
 template <int D, int KS, int NW>
 constexpr int kDqWaves = kBias || NW != 4 ? Geo<D, KS, NW>::WAVES
                          : !kNarrow && D == 32 && KS <= 5 ? 4
-                         : (D == 32 && ((KS == 7 && !kSub) || KS == 9)) || (!kNarrow && D == 64 && KS == 3) ? 3 : Geo<D, KS, NW>::WAVES;
+                         : (D == 32 && ((KS == 7 && !kSub) || (KS == 9 && !kNarrow))) || (!kNarrow && D == 64 && KS == 3) ? 3 : Geo<D, KS, NW>::WAVES;
 // FULL: as in fwd_mfma (no wave switched off, no store predicated, the staged rows go to LDS at
 // the end of a tile's pass through the loop).
 template <bool BF, int D, int KS, bool FRAME, bool ROLL, int NW = 4, bool FULL = false>
@@ -1388,13 +1389,19 @@ __device__ __forceinline__ bool next_block(KeyBlock &b) {
 // head_dim 64), but for head_dim 32, where 2 is ahead (B4 N4 128x128 k9 51.6 -> 48.8 us).
 // With a bias at head_dim 32 the 7x7 and 9x9 windows run at two waves per SIMD anyway (kDkdvWaves), which leaves
 // registers for both tiles in both bodies: B8 N4 56x56 d32 k7 28.9 -> 27.6 us, B8 N2 112x112 k9 66.9 -> 66.5.
+// In the build for head dims 72 to 120 the bodies with blocks of 5x5 windows (k = 3, 5, and 11 and 13, whose tiles are all
+// walked by such blocks) spill 130 to 200 bytes ahead and 50 to 170 with -1: B4 N2 70x94 d96 k11 78.7 -> 62.8 us, k3 18.6 ->
+// 16.4, B2 N5 128x160 k5 71 -> 60; k = 7 and 9 lose (37.3 -> 42.0).  With a bias the border tiles of d128 k3 alone gain (B8 N4 56x56
+// 49.4 -> 44.0).
 //   a_of(h), t_of(h): this lane's row of tile h for the direct and for the transposing reads
 //   stat(h, i), at(h, i, st), in(h, i, st): statistics of query 4 g + i of tile h, the place of its
 //   bias in the table, and whether it attends to this lane's key
 template <int D, int KS>
-constexpr int kInnerAhead = kBias && (D > 32 || KS < 7 || KS > 9) ? -1 : D == 32 ? 2 : 0;
+constexpr bool kWideNarrow = kNarrow && !kBias && D == 128 && KS != 7 && KS != 9;
 template <int D, int KS>
-constexpr int kFrameAhead = kBias && D == 32 && (KS == 7 || KS == 9) ? 2 : 1;
+constexpr int kInnerAhead = (kBias && (D > 32 || KS < 7 || KS > 9)) || kWideNarrow<D, KS> ? -1 : D == 32 ? 2 : 0;
+template <int D, int KS>
+constexpr int kFrameAhead = kBias && D == 32 && (KS == 7 || KS == 9) ? 2 : kWideNarrow<D, KS> || (kBias && D == 128 && KS == 3) ? -1 : 1;
 // FRAME: a run of four reaches up to three queries past the wave's own, whose delta may be anything: what
 // no window connects with a key is left out of dS, where P = 0 times a delta that is not finite would
 // be NaN.  (With a bias such keys are computed again, again_keys.)
@@ -1765,8 +1772,12 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
         // (image_token without sub-grids, written out: through the function the register allocation of the
         // narrow build comes out another way, 61x83 d48 k9 float16 B3 N5 83.9 us for 83.5)
         const int64_t img_tok = kSub ? image_token(a, b.tl) : ((int64_t)b.tl.bb * s.N + b.tl.nn) * s.H * (int64_t)s.W;
-        halo_fetch<D, KSG>(qst, plan, image_at(a, a.q, b.tl), row_step(a, a.q), col_step(a, a.q), b.br, b.bc, b.qb, b.cb);
-        halo_fetch<D, KSG>(gst, plan, image_at(a, a.d_o, b.tl), row_step(a, a.d_o), col_step(a, a.d_o), b.br, b.bc, b.qb, b.cb);
+        // (the branch around the loads only steers the registers of this one body, which spills 104 bytes without it: biased bf16
+        // d64 k13, B8 N4 56x56 86.7 -> 82.3 us; float16 and k = 11 are level or slower with it)
+        if (!(kTable && BF && SP == 2 && KS == 13) || plan.on) {
+            halo_fetch<D, KSG>(qst, plan, image_at(a, a.q, b.tl), row_step(a, a.q), col_step(a, a.q), b.br, b.bc, b.qb, b.cb);
+            halo_fetch<D, KSG>(gst, plan, image_at(a, a.d_o, b.tl), row_step(a, a.d_o), col_step(a, a.d_o), b.br, b.bc, b.qb, b.cb);
+        }
 #pragma unroll
         for (int i = 0; i < G::NST; i++) {
             const int id = threadIdx.x + i * G::NT;
@@ -1986,11 +1997,11 @@ constexpr int kFrameKS = kDkdvFrameOnly<D, KS> ? 5 : SP == 2 && KS >= 9 ? 9 + KS
 // 57.9 us, B4 N16 128x128 93.5 -> 87.6, B8 N8 41x77 23.9 -> 21.0), and lose where the same rounds are walked by
 // more workgroups (B8 N2 112x112 16.2 -> 16.9); at k = 7 they spill (B8 N2 112x112 22.4 -> 26.8).  In the builds for narrow heads
 // and sub-grids head_dim 64, k = 3 spills 100 to 148 bytes in three and runs in two: d48 B4 N4 128x128 42.2 -> 35.5 us, 61x83
-// float16 16.9 -> 12.9.
+// float16 16.9 -> 12.9; k = 5 (148 bytes) 44.7 -> 36.5 and 22.8 -> 16.1.
 template <int D, int KS, int SP>
 constexpr int kDkdvWaves =
     kDkdvFrameOnly<D, KS> ? 2 :
-    !kNarrow && D == 32 && KS == 5 ? 4 : kNarrow && !kBias && D == 64 && KS == 3 ? 2 :
+    !kNarrow && D == 32 && KS == 5 ? 4 : kNarrow && !kBias && D == 64 && KS <= 5 ? 2 :
     SP == 1 && D <= (kBias ? KS <= 5 ? 32 : 0 : 64) && 3 * (Geo<D, KS>::LDS_BYTES + 2048) <= 160 * 1024 ? 3 : Geo<D, KS, 4, SP>::WAVES;
 template <bool BF, int D, int KS, bool ROLL, int SP = 1>
 __global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) void bwd_dkdv_mfma(
