@@ -557,9 +557,11 @@ struct HaloPlan {
     // Every PER chunks a thread's pixels are RPER whole rows further down, so it keeps PER places (halo row << 8 |
     // halo column) instead of one for every chunk: 5 instead of 25 at head_dim 128, k = 13.
     using G = Geo<D, KS, NW, SP>;
-    static constexpr int STEP = G::NT / G::CPR, PER = std::lcm(STEP, G::HC) / STEP, RPER = std::lcm(STEP, G::HC) / G::HC;
-    static constexpr int KEEP = PER < G::NL ? PER : G::NL;
-    int rc[KEEP];
+    // (up to head_dim 64 not for one or two registers: d64 k5 loses 1.5% by the additions)
+    static constexpr int STEP = G::NT / G::CPR, LCM = std::lcm(STEP, G::HC);
+    static constexpr bool ALL = LCM / STEP >= G::NL - (D <= 64 ? 2 : 0);
+    static constexpr int PER = ALL ? G::NL : LCM / STEP, RPER = ALL ? 0 : LCM / G::HC;
+    int rc[PER];
     // halo row and column of chunk i (a chunk behind the last pixel: a row below the halo, or its last pixel)
     __device__ __forceinline__ int row(int i) const { return (rc[i % PER] >> 8) + i / PER * RPER; }
     __device__ __forceinline__ int col(int i) const { return rc[i % PER] & 255; }
@@ -582,9 +584,9 @@ __device__ __forceinline__ HaloPlan<D, KS, NW, SP> make_plan(int dlim = D) {
     static_assert((G::NT / G::CPR) % (16 * G::RPL) == 0, "one chunk position per thread");
     pl.lds0 = G::chunk_at(threadIdx.x / G::CPR, threadIdx.x % G::CPR);
 #pragma unroll
-    for (int i = 0; i < pl.KEEP; i++) {
+    for (int i = 0; i < pl.PER; i++) {
         int row = threadIdx.x / G::CPR + i * (G::NT / G::CPR);
-        if (pl.PER >= G::NL) row = row < G::HR * G::HC ? row : G::HR * G::HC - 1;
+        if (pl.ALL) row = row < G::HR * G::HC ? row : G::HR * G::HC - 1;
         pl.rc[i] = ((row / G::HC) << 8) | (row % G::HC);
     }
     return pl;
