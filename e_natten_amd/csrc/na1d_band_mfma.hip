@@ -3,7 +3,7 @@
 //
 // The kernels of na1d_mfma_kernels.h stage all keys of a tile at once, which ends at a
 // kernel_size of 49.  Here a workgroup of four waves owns a tile of queries and walks the keys
-// that any of them sees, 64 at a time, with an online softmax: K and V rows of a block are in
+// that any of them sees, 64 (or 32) at a time, with an online softmax: K and V rows of a block are in
 // LDS, the next block's are in flight into registers and go into a second buffer, one barrier
 // per block.  A wave owns 16 queries (the columns of v_mfma_f32_16x16x32), or in the forward of long
 // windows two groups of 16, where every operand that comes out of LDS feeds twice the matrix
@@ -40,9 +40,10 @@ namespace {
 
 // Rows of a staged block: keys in the forward and the dQ pass, queries in the dK/dV pass.  64, and
 // 32 for the dK/dV pass at head_dim 64, where the smaller buffers let a third workgroup share the CU
-// (B4 N16 T8192 k32 causal 101 -> 86 us); not for its forward (54.6 -> 57.1), and not at head_dim
-// 128, where the registers leave room for two (dK/dV B1 N16 T8192 k128 62 -> 68), nor at 32, where
-// 32 rows are fewer than the 64 that a pass of all threads moves.
+// (B4 N16 T8192 k32 causal 101 -> 86 us), and for the forward at 128 (short_blocks); not for the
+// forward at 64 (54.6 -> 57.1), not for the backward at head_dim 128, where the registers leave room for two
+// workgroups (dK/dV B1 N16 T8192 k128 62 -> 68), nor at 32, where 32 rows are fewer than the 64 that a
+// pass of all threads moves.
 constexpr int kRowsQ = 64;
 template <int D>
 constexpr int kRowsK = D == 64 ? 32 : 64;
@@ -142,9 +143,10 @@ constexpr float kFar = 1048576.f;
 __device__ __forceinline__ bool far(float lse) { return !(fabsf(lse) <= kFar); }  // (also NaN)
 __device__ __forceinline__ float exp_neg(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 // ------------------------------------------------------------------ forward
-template <bool BF, int D, int NQ, bool NARROW>
-__global__ __launch_bounds__(256, 2) void fwd_band_mfma(FwdArgs a, int tiles_t, int ntiles) {
-    constexpr int KB = kRowsQ;
+// Blocks of 32 keys: 35 KB of LDS and, with half of the staging registers, 119 to 124 in all, so that four workgroups
+// share a CU instead of two (145 registers, 70 KB).  The steps of 32 keys and their order are the same: so are the results.
+template <bool BF, int D, int NQ, bool NARROW, int KB>
+__global__ __launch_bounds__(256, (KB == 32 ? 4 : 2)) void fwd_band_mfma(FwdArgs a, int tiles_t, int ntiles) {
     using G = BGeo<D, KB>;
     __shared__ __attribute__((aligned(16))) short lds_k[2][KB * G::PITCH];
     __shared__ __attribute__((aligned(16))) short lds_v[2][KB * G::PITCH];
@@ -632,23 +634,29 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tile
 // ------------------------------------------------------------------ dispatch
 // Two groups of 16 queries per wave (forward) where the walk is long, a key row is 256 bytes, and
 // tiles of that size still give every CU its two workgroups: the LDS reads of a step then feed twice the
-// matrix instructions.  One group / two, us, causal: head_dim 128 B2 N8 T4096 k400 40.4 / 35.0, B2 N32
-// T8192 k512 351 / 294; at k = 128 (B1 N16 T8192) level (43.1 / 44.1); head_dim 64 B2 N16 T4096 k256
-// 25.7 / 33.5: there more waves count for more.  Not in the dQ pass: its third product takes the
+// matrix instructions.  One group in blocks of 32 keys / two, us, causal, head_dim 128: B2 N32 T8192 k256 172 / 199, k512
+// 268 / 272, k1024 463 / 441, k2500 956 / 863; B2 N8 T4096 k400 32.5 / 33.3, k512 38.6 / 37.4; B1 N16 T4096 k2000 114 / 103.
+// head_dim 64 B2 N16 T4096 k256 25.7 / 33.5: there more waves count for more.  Not in the dQ pass: its third product takes the
 // registers that a second group needs (with two, B2 N32 T8192 d128 k512 spills and its backward
 // takes 1432 us instead of 1005), nor in the dK/dV pass (head_dim 64: 108 / 151).
 bool two_groups(const Shape &s) {
-    return s.D == 128 && s.kw >= 256 && (int64_t)s.B * s.N * ((s.W + 127) / 128) >= 512;
+    return s.D == 128 && s.kw >= 512 && (int64_t)s.B * s.N * ((s.W + 127) / 128) >= 512;
 }
+// The forward above head_dim 64 in blocks of 32 keys: where there are more tiles than the two workgroups per CU of
+// the blocks of 64 take at once; fewer only pay for the barriers.  Blocks of 64 / 32, us: B1 N16 T8192 d128 k200 causal 46.7 / 42.0, k128 on
+// views of one projection, the call, 42.4 / 36.8, k91 centred 35.9 / 33.1; B1 N16 T3000 k400 (752 tiles) 32.7 / 26.0;
+// B3 N4 T3000 k20 (564) 11.8 / 9.1; B2 N8 T8192 d96 k512 77 / 67, B3 N7 T2500 d80 k20 12.1 / 9.0; B1 N16 T2000 k128 (512) 10.2 / 10.0,
+// B1 N7 T3001 k250 (329) 12.4 / 13.6, B1 N4 T4096 k1024 (256) 26.0 / 27.4.
+bool short_blocks(const Shape &s) { return (int64_t)s.B * s.N * ((s.W + 63) / 64) > 512; }
 int band_grid(int64_t ntiles) { return (int)((ntiles + 7) / 8 * 8); }
 
-template <bool BF, int D, int NQ, bool NARROW>
+template <bool BF, int D, int NQ, bool NARROW, int KB = kRowsQ>
 int fwd_go(const FwdArgs &a, hipStream_t st) {
     const int tiles_t = (a.s.W + 64 * NQ - 1) / (64 * NQ);
     const int64_t nt = (int64_t)a.s.B * a.s.N * tiles_t;
     {
         ProfScope prof(ENATTEN_KERNEL_FWD, "fwd_band_mfma", st);
-        hipLaunchKernelGGL((fwd_band_mfma<BF, D, NQ, NARROW>), dim3(band_grid(nt)), dim3(256), 0, st, a, tiles_t,
+        hipLaunchKernelGGL((fwd_band_mfma<BF, D, NQ, NARROW, KB>), dim3(band_grid(nt)), dim3(256), 0, st, a, tiles_t,
                            (int)nt);
     }
     return check_launch("fwd_band_mfma");
@@ -710,10 +718,13 @@ int fwd_dim(const FwdArgs &a, hipStream_t st) {
     switch (a.s.D) {
         case 32: return fwd_go<BF, 32, 1, false>(a, st);
         case 64: return fwd_go<BF, 64, 1, false>(a, st);
-        case 128: return two_groups(a.s) ? fwd_go<BF, 128, 2, false>(a, st) : fwd_go<BF, 128, 1, false>(a, st);
+        case 128:
+            return two_groups(a.s)    ? fwd_go<BF, 128, 2, false>(a, st)
+                   : short_blocks(a.s) ? fwd_go<BF, 128, 1, false, 32>(a, st) : fwd_go<BF, 128, 1, false>(a, st);
     }
     return a.s.D < 32   ? fwd_go<BF, 32, 1, true>(a, st)
-           : a.s.D < 64 ? fwd_go<BF, 64, 1, true>(a, st) : fwd_go<BF, 128, 1, true>(a, st);
+           : a.s.D < 64 ? fwd_go<BF, 64, 1, true>(a, st)
+           : short_blocks(a.s) ? fwd_go<BF, 128, 1, true, 32>(a, st) : fwd_go<BF, 128, 1, true>(a, st);
 }
 template <bool BF>
 int bwd_dim(const BwdArgs &a, hipStream_t st) {

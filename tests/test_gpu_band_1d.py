@@ -65,6 +65,30 @@ def test_band_windows(shape, ks, causal, dtype, layout):
     assert torch.equal(o, natten1d(qg, kg, vg, ks, scale, 1, causal))
 
 
+@pytest.mark.parametrize("shape,ks,causal,dtype", [
+    ((1, 64, 500, 128), 90, True, BF16),    # 512 tiles: blocks of 64 keys
+    ((1, 57, 560, 128), 90, True, BF16),    # 513: blocks of 32
+    ((1, 57, 513, 128), 31, False, F16),    # ... a last tile of one query
+    ((1, 57, 560, 72), 33, True, F16),
+    ((1, 64, 500, 72), 33, True, F16),
+    ((2, 52, 600, 128), 511, True, F16),
+    ((2, 52, 600, 128), 512, True, F16),    # two groups of queries per wave
+    ((2, 52, 577, 128), 513, False, BF16),  # ... the second group of the last tile past the end
+])
+def test_blocks_of_the_forward(shape, ks, causal, dtype):
+    ensure_built()
+    from e_natten_amd import natten1d
+    print("case blocks", shape, dtype, "k=%d" % ks, flush=True)
+    q, k, v, _ = make_inputs(shape, dtype, seed=37)
+    scale = shape[-1] ** -0.5
+    o = natten1d(q.cuda(), k.cuda(), v.cuda(), ks, scale, 1, causal)[-1:, ::16].cpu()
+    qr, kr, vr = (t[-1:, ::16].double().unsqueeze(2) for t in (q, k, v))
+    ref = O.natten2d_window_dense_mask(qr, kr, vr, (1, ks), (False, causal), scale).squeeze(2)
+    norm = ((o.double() - ref).norm() / ref.norm()).item()
+    print("    O 2-norm %.2e" % norm, flush=True)
+    assert norm <= (4e-3 if dtype == BF16 else 5e-4), norm  # (as in test_band_windows)
+
+
 @pytest.mark.parametrize("ks,causal,d,dtype", [(33, True, 64, BF16), (51, False, 128, F16), (70, True, 40, F16)])
 def test_values_that_are_not_finite_stay_in_their_windows(ks, causal, d, dtype):
     # a NaN in v at one position: only queries that see it, and the keys that such queries see, may
