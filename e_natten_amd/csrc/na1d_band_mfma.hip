@@ -468,8 +468,12 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
 // The tile is 64 keys, 16 per wave (columns), and the walk is over the queries
 // that see any of them, the inverse neighbourhood (e_natten/pytorch.py:13-23), a block at a time: Q
 // and dO rows, the log-sum-exp, delta and 1 / Z of a block in LDS.  dV^T += dO^T P, dK^T += Q^T dS.
+// head_dim 64 takes 128 to 152 registers without a budget, four waves per SIMD have 128 (20 bytes of scratch in float16 below
+// 64): causal, us, float16 B4 N8 T8192 d64 k64 54.3 -> 48.7, B2 N16 T4096 k256 52.1 -> 45.6; B4 N8 T8192 d48 k128 60.5 -> 52.5,
+// float16 64.6 -> 57.3; bf16 d64 level.  The dQ pass spills in four (d48 k128 44.6 -> 54.6) or, in blocks of 32 keys, gains only in bf16
+// on many tiles (43.7 -> 43.0; float16 36.8 -> 40.6).
 template <bool BF, int D, bool NARROW>
-__global__ __launch_bounds__(256, 2) void bwd_band_dkdv_mfma(BwdArgs a, int tiles_t, int ntiles) {
+__global__ __launch_bounds__(256, (D == 64 ? 4 : 2)) void bwd_band_dkdv_mfma(BwdArgs a, int tiles_t, int ntiles) {
     constexpr int KB = kRowsK<D>;
     using G = BGeo<D, KB>;
     __shared__ __attribute__((aligned(16))) short lds_q[2][KB * G::PITCH];
