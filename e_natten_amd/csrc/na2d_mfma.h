@@ -570,15 +570,20 @@ struct HaloPlan {
     bool on;                 // false: the tensor has no such channels (head dim below D); the thread loads others, without a
                              // branch that would keep its registers from one fetch to the next, and writes nothing: its
                              // LDS columns stay zero (zero_row)
+    // (a constant) such a thread loads nothing: for the kernels that have registers for the branch, and would pay for the
+    // loads.  Forward, us, without -> with: B6 N15 71x71 d48 k3 40.2 -> 37.4, k7 65.1 -> 62.7, k9 73.0 -> 70.0, B4 N8 91x91 d96 k5
+    // 54.1 -> 52.2; not with a bias (d24 k7 13.1 -> 14.3), on sub-grids, nor at k = 13.  dQ pass d48 k3 49.9 -> 48.3, d96 k5 61.5 -> 60.4.
+    bool skip;
 };
 template <int D, int KS, int NW = 4, int SP = 1>
-__device__ __forceinline__ HaloPlan<D, KS, NW, SP> make_plan(int dlim = D) {
+__device__ __forceinline__ HaloPlan<D, KS, NW, SP> make_plan(int dlim = D, bool skip = false) {
     using G = Geo<D, KS, NW, SP>;
     static_assert(G::NT % G::CPR == 0, "a thread keeps one channel chunk");
     HaloPlan<D, KS, NW, SP> pl;
     pl.ch8 = (threadIdx.x % G::CPR) * 8;
     pl.on = pl.ch8 < dlim;
     if (!pl.on) pl.ch8 = 0;
+    pl.skip = skip;
     // the rows of one thread's chunks are NT / CPR apart, a multiple of 16 * RPL, so they
     // share one key and the chunk position is the same for all of them
     static_assert((G::NT / G::CPR) % (16 * G::RPL) == 0, "one chunk position per thread");
@@ -611,6 +616,7 @@ __device__ __forceinline__ void halo_fetch(HaloRegs<D, KS, NW, SP> &reg, const H
     const char *base = reinterpret_cast<const char *>(img + hr0 * sh + hc0 * sw);
     const unsigned sh2 = (unsigned)sh * 2u, sw2 = (unsigned)sw * 2u;
     const int rmax = rlim - 1 - hr0, cmax = clim - 1 - hc0;
+    if (pl.skip && !pl.on) return;
 #pragma unroll
     for (int i = I0; i < I1; i++) {
         const unsigned r = (unsigned)min(pl.row(i), rmax);
@@ -645,6 +651,7 @@ __device__ __forceinline__ void halo_fetch_rows(HaloRegs<D, KS, NW, SP> &reg, co
     const char *base = reinterpret_cast<const char *>(img + yb * sh + hc0 * sw);
     const unsigned sh2 = (unsigned)sh * 2u, sw2 = (unsigned)sw * 2u;
     const int rmax = rlim - 1 - yb, cmax = clim - 1 - hc0;
+    if (pl.skip && !pl.on) return;
 #pragma unroll
     for (int i = 0; i < G::NL; i++) {
         const int r = pl.row(i);

@@ -577,7 +577,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
     const float sc2 = s.scale * kUnit;
 
     // registers that carry the next tile while the current one is computed
-    const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim);
+    const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim, !kTable && !kSub && KS <= 11);
     HaloRegs<D, KS, NW> kst, vst;
     s16x8 qnext[G::DS];
     BiasRegs<BF, KS, G::NT> bst;
@@ -921,7 +921,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
         else return in_sub(tile_of(t, ts.tiles_r, ts.tiles_c, s.N, G::TH), a);
     };
 
-    const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim);
+    const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim, !kTable && (KS == 3 || (D != 64 && KS == 5)));
     HaloRegs<D, KS, NW> kst, vst;
     s16x8 qnext[G::DS], gnext[G::DS];
     float lse_next = 0.f;
