@@ -4,9 +4,8 @@
 // (the reference's benchmark inputs, e_natten/triton.py:280 applies no scale) a float32
 // dot product is good to ~1e-5, which exp() turns into a relative error of the
 // probabilities and ~1e-4 absolute error of dQ and dK.  So the logits are formed with
-// the float64 matrix instruction v_mfma_f64_16x16x4_f64 and every other product (P.V,
-// dO.V, dS.K, P^T.dO, dS^T.Q) with the float32 one, v_mfma_f32_16x16x4_f32: true
-// float32 products, no reduced-precision operands anywhere.
+// a float64 matrix instruction and every other product (P.V, dO.V, dS.K, P^T.dO, dS^T.Q)
+// with a float32 one: true float32 products, no reduced-precision operands anywhere.
 //
 // Geometry.  A workgroup of four waves owns an 8x8 tile of pixels, a wave a 4x4 block of it as four blocks of
 // 2x2.  The matrix instructions are those of four (float64) and sixteen (float32) independent 4x4 products,
@@ -15,9 +14,10 @@
 // query instead of 64 at kernel_size 5 (25 are in its window), 16 instead of 48 at 3, 64 instead of 112 at 7.
 // Both shapes run at the rate of the 16-wide ones (16 and 32 products per cycle and SIMD: measured 17.0 and 9.3
 // cycles against 66.1 and 33.0).  Forward, dQ and dK/dV pass, us, 4x4 blocks on the 16-wide instructions -> 2x2 blocks:
-// B4 N4 128x128 d128 k5 160 + 226 + 188 -> 133 + 181 + 177; 96x96 d64 k3 36 + 48 + 39 -> 25 + 33 + 32, k7 72 + 120 + 95 ->
-// 59 + 90 + 93; B4 N8 96x96 d32 k5 52 + 74 + 63 -> 42 + 61 + 49.  What bounds them: HBM at 4.2 TB/s in the forward and the
-// dQ pass, where a tile's two staging phases issue no matrix instruction.  One tensor's halo at a time is staged in LDS (float32 rows of D + 4 floats), so two
+// B4 N4 128x128 d128 k5 160 + 226 + 188 -> 133 + 181 + 149; 96x96 d64 k3 36 + 48 + 39 -> 25 + 33 + 28, k7 72 + 120 + 95 ->
+// 59 + 90 + 71; B4 N8 96x96 d32 k5 52 + 74 + 63 -> 43 + 61 + 42.  What bounds them: HBM at 4.2 TB/s in the forward and the
+// dQ pass, where a tile's two staging phases issue no matrix instruction, and LDS reads of the second products, whose bank
+// conflicts are 40% of the LDS cycles.  One tensor's halo at a time is staged in LDS (float32 rows of D + 4 floats), so two
 // workgroups share a CU; the other tensor's halo travels from HBM into registers meanwhile.
 //
 // Lanes.  A lane is (g, b, j) = (lane >> 4, lane >> 2 & 3, lane & 3): block b of the wave, pixel j of the
@@ -75,7 +75,7 @@ constexpr bool kLines32 = 2 * Geo32<D, KS>::LDS_BYTES <= 160 * 1024;
 // (head_dim 32, and 64 up to kernel_size 5): the places and bounds of the weights are formed once, a
 // weight pair is one 8-byte load, and what a workgroup waits for (rows, weights, two barriers) it
 // waits for once.  P and dS of a window position then lie side by side in the workspace, which makes
-// the dQ pass's scattered stores half as many as well.  Backward, us, two launches -> one: B8 N7 46x46 d32 k7
+// the dQ pass's scattered stores half as many as well.  Backward, us, two launches -> one, measured with 4x4 blocks: B8 N7 46x46 d32 k7
 // 174 -> 142 (dK/dV 105 -> 77), B2 N8 128x128 d64 k5 258 -> 234, k3 178 -> 164, d32 k3 99 -> 90.  At head_dim 128
 // the same with 64 channels to a workgroup was level at k5 (dQ pass 256 -> 248, dK/dV 210 -> 219).
 template <int D, int KS>
