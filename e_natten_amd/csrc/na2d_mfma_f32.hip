@@ -365,13 +365,15 @@ __device__ __forceinline__ void second32(const float *lds_x, const float *w, con
 // whole lines).  With LINES the lanes of tokens n and n^1 (adjacent lanes) exchange every other
 // piece, and the eight lanes of the pair write one token's whole 128-byte line per instruction.
 // Every lane of the wave must call this; `live`: this lane's token exists; `flip`: second_flip.  The values
-// stored are acc * (mul + low) with one rounding of the product by mul.
-template <int D, bool LINES>
-__device__ __forceinline__ void store32(float *token, int g, const f32x4 *acc, int flip, float mul, float low, bool live) {
+// stored are acc * mul, or, with REST, acc * (mul + low) with one rounding of the product by mul; low > 0, so that an
+// infinity stays one.
+template <int D, bool LINES, bool REST = false>
+__device__ __forceinline__ void store32(float *token, int g, const f32x4 *acc, int flip, float mul, bool live, float low = 0.f) {
     auto times = [&](const f32x4 &x) __attribute__((always_inline)) {
         f32x4 y;
 #pragma unroll
-        for (int c = 0; c < 4; c++) y[c] = fmaf(x[c], mul, x[c] * low);
+        for (int c = 0; c < 4; c++)
+            y[c] = REST ? fmaf(x[c], mul, x[c] * low) : x[c] * mul;
         return y;
     };
     if constexpr (LINES) {
@@ -483,6 +485,10 @@ __global__ __launch_bounds__(256, 2) void fwd_mfma_f32(FwdArgs a, int tiles_r, i
             sum = col_sum(sum);
             inv = 1.f / sum;
             inv_rest = fmaf(-sum, inv, 1.f);  // what its rounding leaves
+            if (inv_rest <= 0.f) {            // (from below, store32; not where the sum is NaN or zero)
+                inv = __uint_as_float(__float_as_uint(inv) - 1u);
+                inv_rest = fmaf(-sum, inv, 1.f);
+            }
             lse = (float)(mx + (double)logf(sum));
         } else {
 #pragma unroll
@@ -495,7 +501,7 @@ __global__ __launch_bounds__(256, 2) void fwd_mfma_f32(FwdArgs a, int tiles_r, i
             f32x4 o[G::DT];
             second32<D, KS>(lds, p, lq, ln, o, load_next);
             float *op = const_cast<float *>(image32(a.o, cur)) + lq.qr * a.o.sh + lq.qc * a.o.sw;
-            store32<D, kLines32<D, KS>>(op, g, o, second_flip<D>(ln), inv, inv * inv_rest, lq.live);
+            store32<D, kLines32<D, KS>, true>(op, g, o, second_flip<D>(ln), inv, lq.live, inv * inv_rest);
             if (lq.live && a.lse && g == 0) a.lse[lq.tok] = lse;
         } else {
 #pragma unroll
@@ -613,7 +619,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_mfma_f32(BwdArgs a, float *ws_p
             }
             f32x4 dq[G::DT];
             second32<D, KS>(lds, ds, lq, ln, dq, load_next);
-            store32<D, kLines32<D, KS>>(static_cast<float *>(a.dq) + lq.tok * D, g, dq, second_flip<D>(ln), s.scale, 0.f, lq.live);
+            store32<D, kLines32<D, KS>>(static_cast<float *>(a.dq) + lq.tok * D, g, dq, second_flip<D>(ln), s.scale, lq.live);
         } else {
 #pragma unroll
             for (int part = 0; part < STEPS; part++) load_next(part);
@@ -792,7 +798,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, 
 #pragma unroll
     for (int b = 0; b < NB; b++) {
         second_pieces<D>(acc[b]);
-        store32<D, kLines32<D, KS>>((b ? out1 : out0) + tok * D, g, acc[b], second_flip<D>(ln), b ? mul1 : mul0, 0.f, live);
+        store32<D, kLines32<D, KS>>((b ? out1 : out0) + tok * D, g, acc[b], second_flip<D>(ln), b ? mul1 : mul0, live);
     }
 }
 

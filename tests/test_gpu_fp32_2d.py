@@ -55,3 +55,47 @@ def test_views_of_one_projection(D, ks, hw):
     ref = oracle_all(q, k, v, g, ks, small=True)
     got = [x.grad[:, :, :, i].permute(0, 3, 1, 2, 4).cpu() for i in range(3)]
     assert_close((o.detach().cpu(), *got), (ref[0], ref[2], ref[3], ref[4]), torch.float32, "d%d k%d" % (D, ks))
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("ks", [3, 5, 7])
+def test_infinite_results(D, ks):
+    """Results that are infinite by the operator's arithmetic leave as the infinity, not as NaN.  (A query or key that shares a
+    2x2 block with one that sees the value, but does not see it itself, may get NaN: its weight, zero, meets the infinity.)"""
+    from e_natten_amd import natten2d
+    ensure_built()
+    print("case float32 infinities", D, ks, flush=True)
+    H, W, r, c = 24, 24, 11, 11  # (windows and tiles away from the border)
+    shape, inf = (1, 1, H, W, D), float("inf")
+    near = torch.zeros(H, W, dtype=torch.bool)
+    near[r - ks // 2:r + ks // 2 + 1, c - ks // 2:c + ks // 2 + 1] = True  # sees (r, c), and is seen from there
+
+    def run(q, k, v, g):
+        ins = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+        o = natten2d(*ins, ks)
+        return [t.detach().cpu()[0, 0] for t in (o, *torch.autograd.grad(o, ins, g.cuda()))]
+
+    # one infinite value, one infinite element of the upstream gradient
+    q, k, v, g = make_inputs(shape, torch.float32, seed=D + ks, q_scale=D ** -0.5)
+    plain = run(q, k, v, g)
+    for sign in (1, -1):
+        v2, g2 = v.clone(), g.clone()
+        v2[0, 0, r, c, 5] = g2[0, 0, r, c, D - 3] = sign * inf
+        o, dv = run(q, k, v2, g)[0], run(q, k, v, g2)[3]
+        assert (o[near][:, 5] == sign * inf).all() and (dv[near][:, D - 3] == sign * inf).all()
+        for got, ref, ch in ((o, plain[0], 5), (dv, plain[3], D - 3)):
+            keep = torch.arange(D) != ch
+            assert torch.equal(got[..., keep], ref[..., keep])
+            assert got[..., ch][~near].isnan().sum() <= 2 * ks + 1 and torch.equal(
+                got[..., ch][~near & ~got[..., ch].isnan()], ref[..., ch][~near & ~got[..., ch].isnan()])
+    # finite inputs whose gradients overflow: all logits zero (q has channel 2 only, k channel 1), dP = 1e38 for one pair
+    q, k, v, g = (torch.zeros(shape) for _ in range(4))
+    q[0, 0, r, c, 2] = k[0, 0, r, c, 1] = 1e8
+    v[0, 0, r, c, 0] = g[0, 0, r, c, 0] = 1e19
+    got = run(q, k, v, g)
+    ref = oracle_all(q, k, v, g, ks, small=True)
+    ref = [ref[i][0, 0].float() for i in (0, 2, 3, 4)]  # (float64 until here)
+    assert ref[1].isinf().sum() == 1 and ref[2].isinf().sum() == ks * ks
+    for name, x, y in zip(("O", "dQ", "dK", "dV"), got, ref):
+        assert torch.equal(x.isinf(), y.isinf()) and torch.equal(x[x.isinf()], y[y.isinf()]), name
+        assert torch.allclose(x[x.isfinite()], y[x.isfinite()], rtol=1e-5, atol=0), name
