@@ -632,6 +632,17 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_mfma_f32(BwdArgs a, float *ws_p
     }
 }
 
+// Operands of a query that is not met: zeros, moved there on a branch that few patches take (as a choice between two values
+// they would cost every patch; the empty asm keeps the compiler from making one of the branch).
+template <int N>
+__device__ __forceinline__ void cut(float *x) {
+#pragma unroll
+    for (int m = 0; m < N; m++) {
+        x[m] = 0.f;
+        asm volatile("" : "+v"(x[m]));
+    }
+}
+
 // ------------------------------------------------------------------ dK or dV
 // Key-centric: the workgroup owns 8x8 keys, a wave 4x4 of them in blocks of 2x2.  The
 // queries that attend to any key of the tile form a rectangle (the union of the keys'
@@ -650,9 +661,8 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, 
     // Two neighbouring keys are attended by at most k + k/2 + 1 rows of queries, and by up to 2k where both ends of
     // the axis clamp their windows, which an axis of at most 2k pixels has: it is walked in shorter blocks.
     constexpr int NP = (KS + KS / 2 + 2) / 2;       // patches on a side
-    static_assert(2 * NP <= G::HR, "patches of a block of keys stay in the staged rows");
     constexpr int NB = kPair32<D, KS> ? 2 : 1;      // results of this launch (one: x0 and out0)
-    __shared__ __attribute__((aligned(16))) float lds[NB][G::ROWS * G::PITCH];
+    __shared__ __attribute__((aligned(16))) float lds[NB][(G::ROWS + 1) * G::PITCH];  // (the column behind the last)
     const int t = tile_of_block(ntiles);
     if (t < 0) return;
     const Shape &s = a.s;
@@ -675,27 +685,38 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, 
         fetch32<D, KS>(st[0], image32(x0, tl), x0.sh, x0.sw, br, bc, qb, cb);
         if constexpr (NB == 2) fetch32<D, KS>(st[1], image32(x1, tl), x1.sh, x1.sw, br, bc, qb, cb);
     };
-    // Patches of a block that the wave's keys need (the same number for its blocks of keys), this lane's first
-    // query there (moved up where its last patch would leave the staged rows), and the weights of query g of every patch
+    // Patches of a block that the wave's keys need (the same number for its blocks of keys), the rows and columns of
+    // queries in them, this lane's first query there, and the weights of query g of every patch
     // for this lane's key.  Where it does not attend, or is not in the block, the weight's place is beyond the
     // buffer, which reads as zero: a place is one addition of its row's and its column's, without a mask or a branch
     // (d128 k5 176 -> 149 us for the two launches).
-    int npr, npc, base;
+    // All patches lie within the queries that the wave's keys together need, a block that needs fewer moved up where
+    // its last patch would leave them, and where they are an odd number the last patch is cut: every query is met once
+    // and no other is, so that a value that is not finite reaches no key that does not see it but one beside such keys.
+    int npr, npc, nr, nc, base;
     float w[NB][NP * NP];
     auto weights = [&](int br, int bc) __attribute__((always_inline)) {
         const int rend = min(br + rows, qb), cend = min(bc + cols, cb);
-        // first query of [lo, end) that attends to one of the two keys from k0 on, and how many patches they take
-        auto span = [&](int k0, int L, int lo, int end, int &first) __attribute__((always_inline)) {
-            const int ka = min(k0, L - 1), kb = min(k0 + 1, L - 1);
-            first = max(inv_lo(ka, KS), lo);
-            return (min(inv_hi(kb, L, KS), end) - first + 1) >> 1;
+        // of the queries [lo, end), those that attend to one of the two keys from k0 on, and of the two keys behind them: the
+        // first ones, the patches that the longer of both takes, and how many queries both are together
+        auto span = [&](int k0, int L, int lo, int end, int (&first)[2], int &patches) __attribute__((always_inline)) {
+            int last[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                first[i] = max(inv_lo(min(k0 + 2 * i, L - 1), KS), lo);
+                last[i] = min(inv_hi(min(k0 + 2 * i + 1, L - 1), L, KS), end);
+            }
+            patches = (max(last[0] - first[0], last[1] - first[1]) + 1) >> 1;
+            const int from = min(first[0], first[1]), all = max(last[0], last[1]) - from, most = max(all - 2 * patches, 0);
+#pragma unroll
+            for (int i = 0; i < 2; i++) first[i] = min(first[i], from + most);
+            return min(all, 2 * patches);
         };
-        int r0, r1, c0, c1;
-        npr = max(span(wr0, s.H, br, rend, r0), span(wr0 + 2, s.H, br, rend, r1));
-        npc = max(span(wc0, s.W, bc, cend, c0), span(wc0 + 2, s.W, bc, cend, c1));
-        if (wr0 >= s.H || wc0 >= s.W) npr = 0;
-        const int fr = min(ln.b >> 1 ? r1 : r0, br + G::HR - 2 * max(npr, 0));
-        const int fc = min(ln.b & 1 ? c1 : c0, bc + G::HC - 2 * max(npc, 0));
+        int r0[2], c0[2];
+        nr = span(wr0, s.H, br, rend, r0, npr);
+        nc = span(wc0, s.W, bc, cend, c0, npc);
+        if (wr0 >= s.H || wc0 >= s.W) npr = nr = 0;
+        const int fr = ln.b >> 1 ? r0[1] : r0[0], fc = ln.b & 1 ? c0[1] : c0[0];
         base = ((fr - br) * G::HC + fc - bc) * G::PITCH + second_channel<D>(ln);
         // (at most 14 rows of an image of at most 2^16 columns: below 2^30 bytes)
         constexpr unsigned kNone = 0x60000000u;
@@ -747,7 +768,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, 
         const float *xrow[NB];
 #pragma unroll
         for (int b = 0; b < NB; b++) xrow[b] = lds[b] + base;
-        if ((KS > 3 || D < 128) && npr == G::PW && npc == G::PW) {
+        if ((KS > 3 || D < 128) && nr == KS + 1 && nc == KS + 1) {
             // The patches of an inner tile, without a branch between them: a token's operands are read a token ahead (B4 N4 96x96
             // d64 k7 85 -> 70 us, d128 k7 256 -> 181; the four patches of d128 k3 56 -> 62).
             float x[2][NB][G::DT], wb[NB][4];
@@ -770,6 +791,8 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, 
 #pragma unroll
             for (int pr = 0; pr < NP; pr++) {
                 if (pr >= npr) break;
+                const bool cut_row = 2 * pr + 1 >= nr;
+                const int below = cut_row ? 0 : G::HC * G::PITCH;  // (a row cut off is not in the staged block, perhaps)
 #pragma unroll
                 for (int pc = 0; pc < NP; pc++) {
                     if (pc >= npc) break;
@@ -779,9 +802,15 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, 
                     for (int i = 0; i < 4; i++)
 #pragma unroll
                         for (int b = 0; b < NB; b++)
-                            second_fetch<D>(xrow[b] + ((2 * pr + (i >> 1)) * G::HC + 2 * pc + (i & 1)) * G::PITCH, x[i][b]);
+                            second_fetch<D>(xrow[b] + (i >> 1 ? below : 0) + (2 * pr * G::HC + 2 * pc + (i & 1)) * G::PITCH, x[i][b]);
 #pragma unroll
                     for (int b = 0; b < NB; b++) spread_rows(w[b][pr * NP + pc], wb[b]);
+                    if (cut_row)
+#pragma unroll
+                        for (int b = 0; b < NB; b++) cut<G::DT>(x[2][b]), cut<G::DT>(x[3][b]);
+                    if (2 * pc + 1 >= nc)
+#pragma unroll
+                        for (int b = 0; b < NB; b++) cut<G::DT>(x[1][b]), cut<G::DT>(x[3][b]);
 #pragma unroll
                     for (int i = 0; i < 4; i++)
 #pragma unroll

@@ -99,3 +99,27 @@ def test_infinite_results(D, ks):
     for name, x, y in zip(("O", "dQ", "dK", "dV"), got, ref):
         assert torch.equal(x.isinf(), y.isinf()) and torch.equal(x[x.isinf()], y[y.isinf()]), name
         assert torch.allclose(x[x.isfinite()], y[x.isfinite()], rtol=1e-5, atol=0), name
+
+
+@pytest.mark.parametrize("D,ks,hw", [(32, 3, (9, 10)), (64, 3, (12, 17)), (128, 5, (14, 11)), (32, 5, (10, 16)), (64, 7, (13, 19)), (128, 7, (15, 8))])
+def test_one_infinite_gradient_anywhere(D, ks, hw):
+    """An infinite element of the upstream gradient at every place of an image, one in a head: every key that its query sees
+    has an infinite dV, and of the others none that is 4 or more pixels away from such a key has NaN (the blocks of keys of a
+    wave are walked over the same queries)."""
+    from e_natten_amd import natten2d
+    ensure_built()
+    print("case float32 infinity anywhere", D, ks, hw, flush=True)
+    H, W = hw
+    n = H * W
+    one = torch.arange(n)
+    q, k, v, g = (t.expand(1, n, H, W, D).contiguous() for t in make_inputs((1, 1, H, W, D), torch.float32, seed=D + ks, q_scale=D ** -0.5))
+    g.view(n, n, D)[one, one, 7] = float("inf")
+    ins = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    dv = torch.autograd.grad(natten2d(*ins, ks), ins, g.cuda())[2].cpu()[0, ..., 7]
+    first = lambda i, L: min(max(i - ks // 2, 0), L - ks)
+    for at in range(n):
+        r, c = first(at // W, H), first(at % W, W)
+        assert (dv[at, r:r + ks, c:c + ks] == float("inf")).all(), (at // W, at % W)
+        far = torch.ones(H, W, dtype=torch.bool)
+        far[max(r - 3, 0):r + ks + 3, max(c - 3, 0):c + ks + 3] = False
+        assert dv[at][far].isfinite().all(), (at // W, at % W)
