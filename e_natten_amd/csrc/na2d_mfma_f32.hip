@@ -653,7 +653,9 @@ __device__ __forceinline__ void cut(float *x) {
 // that does not attend to a key contributes an exact zero.
 // One tile per workgroup: as a persistent kernel that loads the next tile's rows between the products of the
 // current one it was slower (d128 k5 149 -> 205 us for the two launches below, d64 k3 33 -> 41).
-template <int D, int KS>
+// WIDE: images wider than 65536 pixels, where a weight's place in the rows of a block takes more than 32 bits: plain loads
+// of the weights that there are; the sums are the same.
+template <int D, int KS, bool WIDE>
 __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, View x1, const float *ws_w,
                                                             float *out0, float *out1, float mul0, float mul1,
                                                             int tiles_r, int tiles_c, int ntiles) {
@@ -718,11 +720,28 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_mfma_f32(BwdArgs a, View x0, 
         if (wr0 >= s.H || wc0 >= s.W) npr = nr = 0;
         const int fr = ln.b >> 1 ? r0[1] : r0[0], fc = ln.b & 1 ? c0[1] : c0[0];
         base = ((fr - br) * G::HC + fc - bc) * G::PITCH + second_channel<D>(ln);
-        // (at most 14 rows of an image of at most 2^16 columns: below 2^30 bytes)
+        // (at most 14 rows of an image of at most 2^16 columns, WIDE: below 2^30 bytes)
         constexpr unsigned kNone = 0x60000000u;
         const int64_t row0 = img_tok + (int64_t)br * s.W;
         const auto buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(ws_w + row0 * (G::KK * NB)), 0,
                                                            (rend - br) * s.W * (G::KK * NB * 4), 0x00027000);
+        if constexpr (WIDE) {
+#pragma unroll
+            for (int pr = 0; pr < NP; pr++) {
+                if (pr >= npr) break;
+                const int qr = fr + 2 * pr + (g >> 1), ar = kr - win_start(qr, s.H, KS);
+#pragma unroll
+                for (int pc = 0; pc < NP; pc++) {
+                    if (pc >= npc) break;
+                    const int qc = fc + 2 * pc + (g & 1), ac = kc - win_start(qc, s.W, KS);
+                    const bool ok = qr < rend && qc < cend && (unsigned)ar < (unsigned)KS && (unsigned)ac < (unsigned)KS;
+                    const float *at = ws_w + ((img_tok + qr * (int64_t)s.W + qc) * G::KK + ar * KS + ac) * NB;
+#pragma unroll
+                    for (int b = 0; b < NB; b++) w[b][pr * NP + pc] = ok ? at[b] : 0.f;
+                }
+            }
+            return;
+        }
         unsigned col[NP];
 #pragma unroll
         for (int pc = 0; pc < NP; pc++) {
@@ -860,11 +879,12 @@ int bwd32_launch(const BwdArgs &a, hipStream_t st) {
         // dV = P^T dO and dK = dS^T Q: in one launch, or one after the other
         ProfScope prof(ENATTEN_KERNEL_BWD_DKDV, "bwd_dkdv_mfma_f32", st);
         float *dv = static_cast<float *>(a.dv), *dk = static_cast<float *>(a.dk);
-        hipLaunchKernelGGL((bwd_dkdv_mfma_f32<D, KS>), dim3(grid), dim3(256), 0, st, a, a.d_o, a.q, ws_p, dv, dk, 1.f,
-                           a.s.scale, tiles_r, tiles_c, (int)nt);
+        const auto kernel = a.s.W > 65536 ? bwd_dkdv_mfma_f32<D, KS, true> : bwd_dkdv_mfma_f32<D, KS, false>;
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, st, a, a.d_o, a.q, ws_p, dv, dk, 1.f, a.s.scale, tiles_r,
+                           tiles_c, (int)nt);
         if (!kPair32<D, KS>)
-            hipLaunchKernelGGL((bwd_dkdv_mfma_f32<D, KS>), dim3(grid), dim3(256), 0, st, a, a.q, a.q, ws_ds, dk, dk,
-                               a.s.scale, 1.f, tiles_r, tiles_c, (int)nt);
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, st, a, a.q, a.q, ws_ds, dk, dk, a.s.scale, 1.f,
+                               tiles_r, tiles_c, (int)nt);
     }
     return check_launch("enatten2d_bwd");
 }
@@ -910,7 +930,7 @@ int launch_fwd_mfma_f32(const FwdArgs &a, hipStream_t st) {
 int launch_bwd_mfma_f32(const BwdArgs &a, hipStream_t st) {
     auto al = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
     if (!layout32_ok(a.q) || !layout32_ok(a.k) || !layout32_ok(a.v) || !layout32_ok(a.d_o) ||
-        !al(a.dq) || !al(a.dk) || !al(a.dv) || a.s.W > 65536)  // (rows that long only with strides of zero)
+        !al(a.dq) || !al(a.dk) || !al(a.dv))
         return launch_bwd_simt(a, ENATTEN_F32, st);
     ENATTEN_F32_BY_D(bwd32_launch, a, st)
     set_error("no float32 matrix-core kernel for head_dim %d, kernel_size %d", a.s.D, a.s.kh);

@@ -123,3 +123,23 @@ def test_one_infinite_gradient_anywhere(D, ks, hw):
         far = torch.ones(H, W, dtype=torch.bool)
         far[max(r - 3, 0):r + ks + 3, max(c - 3, 0):c + ks + 3] = False
         assert dv[at][far].isfinite().all(), (at // W, at % W)
+
+
+@pytest.mark.parametrize("ks,W,D", [(3, 65536, 32), (3, 65537, 32), (5, 65600, 64), (7, 70001, 32), (3, 70001, 128)])
+def test_wide_images(ks, W, D):
+    """Images on both sides of the width from which the dK/dV pass has 64-bit places: views of [.., W, H, D] tensors, whose
+    strides between rows and columns are both small.  Every width is on the matrix-core kernels."""
+    from e_natten_amd import natten2d
+    lib = ensure_built()
+    print("case float32 wide", ks, W, D, flush=True)
+    q, k, v, g = make_inputs((1, 1, ks + 1, W, D), torch.float32, seed=W, q_scale=D ** -0.5)
+    swap = lambda t: t.transpose(2, 3).contiguous().cuda().transpose(2, 3)
+    ins = [swap(t).requires_grad_(True) for t in (q, k, v)]
+    lib.enatten_profile_enable(1)
+    o = natten2d(*ins, ks)
+    got = [t.detach().cpu() for t in (o, *torch.autograd.grad(o, ins, swap(g)))]
+    lib.enatten_profile_enable(0)
+    names = [lib.enatten_profile_kernel_name(i) for i in range(3)]
+    assert names == [b"fwd_mfma_f32", b"bwd_dq_mfma_f32", b"bwd_dkdv_mfma_f32"], names
+    ref = oracle_all(q, k, v, g, ks)
+    assert_close(got, (ref[0], *ref[2:]), torch.float32, "d%d k%d W %d" % (D, ks, W))
