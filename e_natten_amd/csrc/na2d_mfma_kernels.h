@@ -554,9 +554,10 @@ __device__ __forceinline__ void again_keys(const BArgs &a, const ATile &tl, int 
 // waves per SIMD have: budgeted for three, B8 N8 112x112 k7 114.8 -> 97.8 us.  At k = 5 four (three at
 // head_dim 64) take a register or two too many without a budget (B8 N4 56x56 d64 k5 16.6 us with two).
 // Without one the compiler left alone takes 146 registers at head_dim 32, k = 7, where four waves per SIMD fit without a
-// spill: B6 N9 91x128 49.4 -> 47.3 us, B1 N16 69x69 8.0 -> 6.8; k = 9 spills there.
+// spill: B6 N9 91x128 49.4 -> 47.3 us, B1 N16 69x69 8.0 -> 6.8; k = 9 spills there, and k = 5, which runs four without a budget,
+// loses by the order of instructions that one leads to (B2 N12 234x210 67.2 -> 69.5, B5 N5 126x126 21.4 -> 22.4).
 template <int D, int KS, int NW>
-constexpr int kFwdWaves = D == 32 && (kBias ? KS == 5 : !kNarrow && KS <= 7) ? 4
+constexpr int kFwdWaves = D == 32 && (kBias ? KS == 5 : !kNarrow && KS == 7) ? 4
                           : kBias && ((D == 32 && KS <= 9) || (D == 64 && KS == 5)) ? 3 : Geo<D, KS, NW>::WAVES;
 template <bool BF, int D, int KS, bool ROLL, int NW = 4, bool FULL = false>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void fwd_mfma(FArgs a, int tiles_r, int tiles_c, int ntiles, Runs rp) {
