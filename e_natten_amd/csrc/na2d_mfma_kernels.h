@@ -1994,18 +1994,22 @@ template <int D, int KS>
 constexpr bool kDkdvFrameOnly = !fits<D, KS>();
 template <int D, int KS, int SP>
 constexpr int kFrameKS = kDkdvFrameOnly<D, KS> ? 5 : SP == 2 && KS >= 9 ? 9 + KS / 2 : KS;
-// head_dim 32, k = 5: four waves per SIMD cost 12 bytes of scratch and gain where a workgroup has many tiles (B8 N16 63x93 66.6 ->
-// 57.9 us, B4 N16 128x128 93.5 -> 87.6, B8 N8 41x77 23.9 -> 21.0), and lose where the same rounds are walked by
-// more workgroups (B8 N2 112x112 16.2 -> 16.9); at k = 7 they spill (B8 N2 112x112 22.4 -> 26.8).  In the builds for narrow heads
+// In the builds for narrow heads
 // and sub-grids head_dim 64, k = 3 spills 100 to 148 bytes in three and runs in two: d48 B4 N4 128x128 42.2 -> 35.5 us, 61x83
 // float16 16.9 -> 12.9; k = 5 (148 bytes) 44.7 -> 36.5 and 22.8 -> 16.1.
 template <int D, int KS, int SP>
 constexpr int kDkdvWaves =
-    kDkdvFrameOnly<D, KS> ? 2 :
-    !kNarrow && D == 32 && KS == 5 ? 4 : kNarrow && !kBias && D == 64 && KS <= 5 ? 2 :
+    kDkdvFrameOnly<D, KS> ? 2 : kNarrow && !kBias && D == 64 && KS <= 5 ? 2 :
     SP == 1 && D <= (kBias ? KS <= 5 ? 32 : 0 : 64) && 3 * (Geo<D, KS>::LDS_BYTES + 2048) <= 160 * 1024 ? 3 : Geo<D, KS, 4, SP>::WAVES;
-template <bool BF, int D, int KS, bool ROLL, int SP = 1>
-__global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), (kDkdvWaves<D, KS, SP>)) void bwd_dkdv_mfma(
+// head_dim 32, k = 5: a second build for four waves per SIMD (12 bytes of scratch) where there are more tiles than its four workgroups
+// per CU take at once, with the workgroups shared out by share_inner at weight 2.6, from the times of every split of 54 calls:
+// 8% faster in the mean (B8 N16 63x93 66.6 -> 57.9 us, B4 N8 128x128 40.7 -> 36.3, B8 N2 112x112 16.4 -> 16.1).  In proportion they
+// lost where both sides come to whole tiles unevenly (B8 N2 112x112 16.8, B7 N5 127x115 43.5 -> 45.3), and fewer tiles lose to the
+// scratch alone (B3 N16 21x32 6.9 -> 7.2).  At k = 7 they spill (B8 N2 112x112 22.4 -> 26.8).
+template <int D, int KS>
+constexpr bool kFourWaves = !kNarrow && D == 32 && KS == 5;
+template <bool BF, int D, int KS, bool ROLL, int SP = 1, int WAVES = kDkdvWaves<D, KS, SP>>
+__global__ __launch_bounds__((Geo<D, KS, 4, SP>::NT), WAVES) void bwd_dkdv_mfma(
     BArgs a, TileSet ts, int n_inner, int n_frame, int inner_blocks, Runs rp, int dyn) {
     using G = Geo<D, KS, 4, SP>;
     using FG = Geo<D, kFrameKS<D, KS, SP>, 4, SP>;  // blocks of the frame body
@@ -2380,8 +2384,11 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
             // Share the resident workgroups between the two bodies so that they end together.
             // `cost` is a frame tile's time in inner tiles (kFrameCost).
             constexpr int SP = kDkdvSplit<D, KS>, NT = Geo<D, KS, 4, SP>::NT;
-            const double cost = kFrameCost<BF, D, KS, kFrameKS<D, KS, SP> != KS>;
-            const int grid = persistent_grid<bwd_dkdv_mfma<BF, D, KS, false, SP>>(nb, NT);
+            constexpr int MANY = kFourWaves<D, KS> ? 4 : kDkdvWaves<D, KS, SP>;
+            const bool many = kFourWaves<D, KS> && nb > 1024;
+            const double cost = many ? 2.6 : kFrameCost<BF, D, KS, kFrameKS<D, KS, SP> != KS>;
+            const int grid = many ? persistent_grid<bwd_dkdv_mfma<BF, D, KS, false, SP, MANY>>(nb, NT)
+                                  : persistent_grid<bwd_dkdv_mfma<BF, D, KS, false, SP>>(nb, NT);
             int inner_blocks = 0, dyn = 0;
             if (n_frame == 0) {
                 inner_blocks = grid;
@@ -2432,7 +2439,7 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                         inner_blocks = all;
                     }
                 }
-            } else if (n_inner > 0 && kBias && !(D == 32 && KS == 9)) {
+            } else if (n_inner > 0 && (many || (kBias && !(D == 32 && KS == 9)))) {
                 inner_blocks = share_inner(n_inner, n_frame, grid, cost);
             } else if (n_inner > 0) {
                 const double f = (double)n_inner / ((double)n_inner + cost * (double)n_frame);
@@ -2454,8 +2461,9 @@ int bwd_launch(const BArgs &a, int path, hipStream_t st) {
                                    0, st, a, ts, (int)n_inner, (int)n_frame, inner_blocks,
                                    plan_runs(n_inner, inner_blocks, ts.ni_r), dyn);
             else
-                hipLaunchKernelGGL((bwd_dkdv_mfma<BF, D, KS, false, SP>), dim3(grid), dim3(NT), 0, st,
-                                   a, ts, (int)n_inner, (int)n_frame, inner_blocks, Runs{0, 0}, dyn);
+                hipLaunchKernelGGL((many ? bwd_dkdv_mfma<BF, D, KS, false, SP, MANY> : bwd_dkdv_mfma<BF, D, KS, false, SP>),
+                                   dim3(grid), dim3(NT), 0, st, a, ts, (int)n_inner, (int)n_frame, inner_blocks,
+                                   Runs{0, 0}, dyn);
         }
         if constexpr (kTable) {
             const auto reduce = path == kRpbTyped ? rpb_tile_reduce<kTable, BF, true> : rpb_tile_reduce<kTable, BF, false>;

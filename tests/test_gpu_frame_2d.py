@@ -93,3 +93,16 @@ def test_largest_windows_below_head_dim_64(D, ks, hw, dtype):
             sub = [t.detach()[at].contiguous().requires_grad_(True) for t in (qg, kg, vg)]
             want = torch.autograd.grad(natten2d(*sub, ks, scale), sub, gg[at].contiguous())
             assert all(torch.equal(a[at], b) for a, b in zip(grads, want))
+
+
+@pytest.mark.parametrize("shape,dtype", [
+    ((8, 8, 32, 32), BF), ((1, 41, 40, 40), BF), ((1, 41, 40, 40), F16),  # 1024 and 1025 tiles: the build for three waves, and for four
+    ((1, 45, 37, 43), F16), ((2, 1, 166, 252), BF)])                     # ... cut tiles, nearly all tiles inner
+def test_four_waves_at_head_dim_32(shape, dtype):
+    ensure_built()
+    shape = (*shape, 32)
+    print("case four waves", shape, dtype, flush=True)
+    q, k, v, g = make_inputs(shape, dtype, seed=5)
+    o, _, dq, dk, dv = run_capi(q, k, v, g, 5, 32 ** -0.5)
+    ref = oracle_all(q, k, v, g, 5, 32 ** -0.5)
+    assert_close((o, dq, dk, dv), (ref[0], ref[2], ref[3], ref[4]), dtype, "four waves")
