@@ -200,3 +200,12 @@ def test_gradient_in_the_tensors_type(shape, kernel, dtype):
         r = rpb.clone().requires_grad_(True)
         both.append(torch.autograd.grad(call(r), r, g)[0])
     assert both[0].dtype == dtype and torch.equal(*both)
+
+
+@pytest.mark.parametrize("shape,ks,dtype", [
+    ((70, 2, 8, 8, 32), 7, BF16),     # one tile to an image, more images than threads of an entry
+    ((33, 3, 13, 9, 32), 5, F16),     # four
+    ((2, 2, 64, 64, 32), 3, F16),     # as many as threads
+    ((2, 1, 67, 65, 32), 3, BF16)])   # more
+def test_sums_over_the_tiles_of_many_images(shape, ks, dtype):
+    test_bias(shape, ks, dtype, "plain")
