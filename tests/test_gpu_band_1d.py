@@ -203,3 +203,14 @@ def test_logits_far_from_zero(dtype, size):
         norm = ((got.detach().cpu().double() - r).norm() / r.norm()).item()
         print("   ", name, dtype, "2-norm %.2e" % norm, flush=True)
         assert norm <= (4e-3 if dtype == BF16 else 5e-4), (name, norm)  # (as in test_band_windows)
+
+
+@pytest.mark.parametrize("shape,ks,causal,dtype,layout", [
+    ((2, 52, 600, 128), 512, True, F16, "plain"),   # the second group of the last tile cut
+    ((2, 52, 577, 128), 513, False, BF16, "proj"),  # ... past the end, but for one query
+    ((2, 52, 640, 128), 600, True, BF16, "proj"),   # whole tiles
+])
+def test_two_groups_of_queries(shape, ks, causal, dtype, layout):
+    # two groups of queries per wave in the forward, from 512 keys on: the gradients need its log-sum-exp as well (windows of 256 to
+    # 300 keys, above, are walked with one group in blocks of 32 keys)
+    test_band_windows(shape, ks, causal, dtype, layout)
