@@ -1529,6 +1529,11 @@ __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g
 // queries and keys exchanged: the staged block is the tile's (8+k-1)^2 halo of
 // queries, a wave's queries are the (4+k-1)^2 halo of its 4x4 keys at a fixed
 // place in it, and the mask depends on the lane only.
+// A branch around the loads of a thread without channels (HaloPlan::skip) in the dK/dV pass: the bodies of large windows with a bias spill less with the branch, but for
+// float16 in two shares of the queries.  Pass, us, without -> with: d32 k13 B5 N6 103x86 float16 149.3 -> 140.9, B2 N5 74x91 bf16 50.5 ->
+// 49.7; bf16 d64 k11 B8 N4 56x56 69.3 -> 67.3, k13 B2 N5 74x91 80.9 -> 78.1 (float16 77.5 -> 78.9).
+template <bool BF, int D, int KS, int SP>
+constexpr bool kDkdvSkip = kTable && (SP == 2 ? BF : D == 32 && KS == 13);
 template <bool BF, int D, int KS, bool ROLL, int SP, int PART>
 __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, int ntiles, Runs rp,
                                            int block, int nblocks, short *lds_q, short *lds_g,
@@ -1560,7 +1565,7 @@ __device__ __forceinline__ void dkdv_inner(const BArgs &a, const TileSet &ts, in
         return in_sub(ROLL ? inner_tile_cm(t, ts, s.N) : inner_tile(t, ts, s.N), a);
     };
 
-    const HaloPlan<D, KS, 4, SP> plan = make_plan<D, KS, 4, SP>(dlim);
+    const HaloPlan<D, KS, 4, SP> plan = make_plan<D, KS, 4, SP>(dlim, kDkdvSkip<BF, D, KS, SP>);
     HaloRegs<D, KS, 4, SP> qst, gst;
     QStat sst[G::NST];
     BiasRegs<BF, KS, G::NT> bst;
@@ -1780,9 +1785,7 @@ __device__ __forceinline__ void dkdv_frame(const BArgs &a, const TileSet &ts, in
         // (image_token without sub-grids, written out: through the function the register allocation of the
         // narrow build comes out another way, 61x83 d48 k9 float16 B3 N5 83.9 us for 83.5)
         const int64_t img_tok = kSub ? image_token(a, b.tl) : ((int64_t)b.tl.bb * s.N + b.tl.nn) * s.H * (int64_t)s.W;
-        // (the branch around the loads only steers the registers of this one body, which spills 104 bytes without it: biased bf16
-        // d64 k13, B8 N4 56x56 86.7 -> 82.3 us; float16 and k = 11 are level or slower with it)
-        if (!(kTable && BF && SP == 2 && KS == 13) || plan.on) {
+        if (!kDkdvSkip<BF, D, KS, SP> || plan.on) {
             halo_fetch<D, KSG>(qst, plan, image_at(a, a.q, b.tl), row_step(a, a.q), col_step(a, a.q), b.br, b.bc, b.qb, b.cb);
             halo_fetch<D, KSG>(gst, plan, image_at(a, a.d_o, b.tl), row_step(a, a.d_o), col_step(a, a.d_o), b.br, b.bc, b.qb, b.cb);
         }
