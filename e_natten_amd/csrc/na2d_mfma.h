@@ -552,14 +552,14 @@ __device__ __forceinline__ Tile tile_of(int t, int tiles_r, int tiles_c, int N, 
 // Staging plan of one thread: which 16-byte chunks of a halo it moves.  Chunk i of
 // thread t is chunk number t + 256*i of the halo in (row, column, channel-chunk)
 // order.  The plan is the same for every tile, so it is computed once.
-template <int D, int KS, int NW = 4, int SP = 1>
+template <int D, int KS, int NW = 4, int SP = 1, bool KEEP = false>
 struct HaloPlan {
     // Every PER chunks a thread's pixels are RPER whole rows further down, so it keeps PER places (halo row << 8 |
     // halo column) instead of one for every chunk: 5 instead of 25 at head_dim 128, k = 13.
     using G = Geo<D, KS, NW, SP>;
-    // (up to head_dim 64 not for one or two registers: d64 k5 loses 1.5% by the additions)
+    // (up to head_dim 64 not for one or two registers: d64 k5 loses 1.5% by the additions; KEEP: for a kernel that loses more)
     static constexpr int STEP = G::NT / G::CPR, LCM = std::lcm(STEP, G::HC);
-    static constexpr bool ALL = LCM / STEP >= G::NL - (D <= 64 ? 2 : 0);
+    static constexpr bool ALL = KEEP || LCM / STEP >= G::NL - (D <= 64 ? 2 : 0);
     static constexpr int PER = ALL ? G::NL : LCM / STEP, RPER = ALL ? 0 : LCM / G::HC;
     int rc[PER];
     // halo row and column of chunk i (a chunk behind the last pixel: a row below the halo, or its last pixel)
@@ -571,15 +571,14 @@ struct HaloPlan {
                              // branch that would keep its registers from one fetch to the next, and writes nothing: its
                              // LDS columns stay zero (zero_row)
     // (a constant) such a thread loads nothing: for the kernels that have registers for the branch, and would pay for the
-    // loads.  Forward, us, without -> with: B6 N15 71x71 d48 k3 40.2 -> 37.4, k7 65.1 -> 62.7, k9 73.0 -> 70.0, B4 N8 91x91 d96 k5
-    // 54.1 -> 52.2; not with a bias (d24 k7 13.1 -> 14.3), on sub-grids, nor at k = 13.  dQ pass d48 k3 49.9 -> 48.3, d96 k5 61.5 -> 60.4.
+    // loads (kFwdSkip, kDkdvSkip and the dQ pass's in na2d_mfma_kernels.h)
     bool skip;
 };
-template <int D, int KS, int NW = 4, int SP = 1>
-__device__ __forceinline__ HaloPlan<D, KS, NW, SP> make_plan(int dlim = D, bool skip = false) {
+template <int D, int KS, int NW = 4, int SP = 1, bool KEEP = false>
+__device__ __forceinline__ HaloPlan<D, KS, NW, SP, KEEP> make_plan(int dlim = D, bool skip = false) {
     using G = Geo<D, KS, NW, SP>;
     static_assert(G::NT % G::CPR == 0, "a thread keeps one channel chunk");
-    HaloPlan<D, KS, NW, SP> pl;
+    HaloPlan<D, KS, NW, SP, KEEP> pl;
     pl.ch8 = (threadIdx.x % G::CPR) * 8;
     pl.on = pl.ch8 < dlim;
     if (!pl.on) pl.ch8 = 0;
@@ -608,8 +607,8 @@ struct HaloRegs {
 // 24-bit multiplies: strides are below 2^22 elements (checked on the host).
 // (I0, I1: only this thread's chunks I0 .. I1-1, for a kernel that loads the last chunks of a
 // halo behind its arithmetic because it has no registers for them beside it)
-template <int D, int KS, int NW = 4, int SP = 1, int I0 = 0, int I1 = Geo<D, KS, NW, SP>::NL>
-__device__ __forceinline__ void halo_fetch(HaloRegs<D, KS, NW, SP> &reg, const HaloPlan<D, KS, NW, SP> &pl,
+template <int D, int KS, int NW = 4, int SP = 1, int I0 = 0, int I1 = Geo<D, KS, NW, SP>::NL, bool KEEP>
+__device__ __forceinline__ void halo_fetch(HaloRegs<D, KS, NW, SP> &reg, const HaloPlan<D, KS, NW, SP, KEEP> &pl,
                                   const short *img, int64_t sh, int64_t sw, int hr0, int hc0,
                                   int rlim, int clim) {
     using G = Geo<D, KS, NW, SP>;
@@ -626,8 +625,8 @@ __device__ __forceinline__ void halo_fetch(HaloRegs<D, KS, NW, SP> &reg, const H
     }
 }
 // Registers -> LDS, one row of D channels per pixel, chunks permuted (Geo::key).
-template <int D, int KS, int NW = 4, int SP = 1>
-__device__ __forceinline__ void halo_commit(short *lds, const HaloPlan<D, KS, NW, SP> &pl,
+template <int D, int KS, int NW = 4, int SP = 1, bool KEEP>
+__device__ __forceinline__ void halo_commit(short *lds, const HaloPlan<D, KS, NW, SP, KEEP> &pl,
                                    const HaloRegs<D, KS, NW, SP> &reg) {
     using G = Geo<D, KS, NW, SP>;
     if (!pl.on) return;
@@ -642,8 +641,8 @@ __device__ __forceinline__ void halo_commit(short *lds, const HaloPlan<D, KS, NW
 // in row slot y % HR): move only the `nrows` image rows from y0 on, all HC columns
 // from hc0 on.  A tile that follows its upper neighbour thus loads only the rows
 // the neighbour's halo did not hold.
-template <int D, int KS, int NW = 4, int SP = 1>
-__device__ __forceinline__ void halo_fetch_rows(HaloRegs<D, KS, NW, SP> &reg, const HaloPlan<D, KS, NW, SP> &pl,
+template <int D, int KS, int NW = 4, int SP = 1, bool KEEP>
+__device__ __forceinline__ void halo_fetch_rows(HaloRegs<D, KS, NW, SP> &reg, const HaloPlan<D, KS, NW, SP, KEEP> &pl,
                                                 const short *img, int64_t sh, int64_t sw, int y0,
                                                 int hc0, int nrows, int rlim, int clim) {
     using G = Geo<D, KS, NW, SP>;
@@ -663,8 +662,8 @@ __device__ __forceinline__ void halo_fetch_rows(HaloRegs<D, KS, NW, SP> &reg, co
         }
     }
 }
-template <int D, int KS, int NW = 4, int SP = 1>
-__device__ __forceinline__ void halo_commit_rows(short *lds, const HaloPlan<D, KS, NW, SP> &pl,
+template <int D, int KS, int NW = 4, int SP = 1, bool KEEP>
+__device__ __forceinline__ void halo_commit_rows(short *lds, const HaloPlan<D, KS, NW, SP, KEEP> &pl,
                                                  const HaloRegs<D, KS, NW, SP> &reg, int y0, int nrows) {
     using G = Geo<D, KS, NW, SP>;
     const int rot = y0 % G::HR;

@@ -566,6 +566,20 @@ __device__ __forceinline__ void again_keys(const BArgs &a, const ATile &tl, int 
 template <int D, int KS, int NW>
 constexpr int kFwdWaves = D == 32 && (kBias ? KS == 5 : !kNarrow && KS == 7) ? 4
                           : kBias && ((D == 32 && KS <= 9) || (D == 64 && KS == 5)) ? 3 : Geo<D, KS, NW>::WAVES;
+// How the staging threads of the builds for narrow heads, sub-grids and a bias fetch (HaloPlan).  A branch around the loads of a thread
+// without channels (SKIP) keeps them together, ahead of the tile's arithmetic; without one the compiler places them among it,
+// which takes fewer registers.  Where a build has the registers the branch is level or ahead, elsewhere it costs up to 16%;
+// where the places of the chunks are formed anew (not KEEP), the additions cost up to 9% at head_dim 128.  The rules follow the
+// means of 6 to 24 calls of each build and window.  Forward, us, loads among the arithmetic, places of one period -> as here: bias d128 k3
+// B4 N11 118x78 d96 82.9 -> 76.2, k5 B8 N4 56x56 23.7 -> 22.4, k11 58.9 -> 55.3, k13 bf16 65.7 -> 58.4 (float16 91.8, with the
+// branch 95.4), d64 k9 25.3 -> 24.9; dilation 2 d32 k11 +11% -> level, d64 k11 +9% -> level, d128 k3 up to +6% -> level; narrow
+// d120 k7 +4% -> level, d24 k11 +7% -> level.  Without the branch: bias d32 k7 -4%, d128 k9 -8%, dilation 2 d64 k5 -10%, d32 k9 -10%.
+template <int D, int KS>
+constexpr bool kFwdKeep = D == 128 && (kTable ? KS <= 5 || KS == 11 : kSub && KS == 3);
+template <bool BF, int D, int KS>
+constexpr bool kFwdSkip = kFwdKeep<D, KS> ||
+    (kTable ? (D == 64 ? KS >= 9 && (BF || KS != 11) : D == 128 && KS == 13 && BF)
+     : kSub ? D <= 64 && KS == 11 : KS <= 11 || D == 32);
 template <bool BF, int D, int KS, bool ROLL, int NW = 4, bool FULL = false>
 __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void fwd_mfma(FArgs a, int tiles_r, int tiles_c, int ntiles, Runs rp) {
     using G = Geo<D, KS, NW>;
@@ -585,7 +599,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kFwdWaves<D, KS, NW>)) void 
     const float sc2 = s.scale * kUnit;
 
     // registers that carry the next tile while the current one is computed
-    const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim, !kTable && !kSub && KS <= 11);
+    const auto plan = make_plan<D, KS, NW, 1, kFwdKeep<D, KS>>(dlim, kFwdSkip<BF, D, KS>);
     HaloRegs<D, KS, NW> kst, vst;
     s16x8 qnext[G::DS];
     BiasRegs<BF, KS, G::NT> bst;
@@ -765,7 +779,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (NW == 4 ? kOneHaloWgs<D, KS>
     const int wave = FULL ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const int l = threadIdx.x & 63, n = l & 15, g = l >> 4;
     const float sc2 = s.scale * kUnit;
-    const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim);
+    const auto plan = make_plan<D, KS, NW, 1, kFwdKeep<D, KS>>(dlim, kFwdSkip<BF, D, KS>);
     HaloRegs<D, KS, NW> st;
     s16x8 qnext[G::DS];
     BiasRegs<BF, KS, G::NT> bst;
@@ -1529,7 +1543,7 @@ __device__ __forceinline__ void dkdv_step(const short *lds_q, const short *lds_g
 // queries and keys exchanged: the staged block is the tile's (8+k-1)^2 halo of
 // queries, a wave's queries are the (4+k-1)^2 halo of its 4x4 keys at a fixed
 // place in it, and the mask depends on the lane only.
-// A branch around the loads of a thread without channels (HaloPlan::skip) in the dK/dV pass: the bodies of large windows with a bias spill less with the branch, but for
+// SKIP of the dK/dV pass, as in the forward (kFwdSkip): the bodies of large windows with a bias spill less with the branch, but for
 // float16 in two shares of the queries.  Pass, us, without -> with: d32 k13 B5 N6 103x86 float16 149.3 -> 140.9, B2 N5 74x91 bf16 50.5 ->
 // 49.7; bf16 d64 k11 B8 N4 56x56 69.3 -> 67.3, k13 B2 N5 74x91 80.9 -> 78.1 (float16 77.5 -> 78.9).
 template <bool BF, int D, int KS, int SP>
