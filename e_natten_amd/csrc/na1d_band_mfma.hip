@@ -472,8 +472,8 @@ __global__ __launch_bounds__(256, 2) void bwd_band_dq_mfma(BwdArgs a, int tiles_
 // 64): causal, us, float16 B4 N8 T8192 d64 k64 54.3 -> 48.7, B2 N16 T4096 k256 52.1 -> 45.6; B4 N8 T8192 d48 k128 60.5 -> 52.5,
 // float16 64.6 -> 57.3; bf16 d64 level.  The dQ pass spills in four (d48 k128 44.6 -> 54.6) or, in blocks of 32 keys, gains only in bf16
 // on many tiles (43.7 -> 43.0; float16 36.8 -> 40.6).
-template <bool BF, int D, bool NARROW>
-__global__ __launch_bounds__(256, (D == 64 ? 4 : 2)) void bwd_band_dkdv_mfma(BwdArgs a, int tiles_t, int ntiles) {
+template <bool BF, int D, bool NARROW, int WAVES = D == 64 ? 4 : 2>
+__global__ __launch_bounds__(256, WAVES) void bwd_band_dkdv_mfma(BwdArgs a, int tiles_t, int ntiles) {
     constexpr int KB = kRowsK<D>;
     using G = BGeo<D, KB>;
     __shared__ __attribute__((aligned(16))) short lds_q[2][KB * G::PITCH];
@@ -652,6 +652,11 @@ bool two_groups(const Shape &s) {
 // B3 N4 T3000 k20 (564) 11.8 / 9.1; B2 N8 T8192 d96 k512 77 / 67, B3 N7 T2500 d80 k20 12.1 / 9.0; B1 N16 T2000 k128 (512) 10.2 / 10.0,
 // B1 N7 T3001 k250 (329) 12.4 / 13.6, B1 N4 T4096 k1024 (256) 26.0 / 27.4.
 bool short_blocks(const Shape &s) { return (int64_t)s.B * s.N * ((s.W + 63) / 64) > 512; }
+// The dK/dV pass of head dims 40 to 56 in float16, whose build for four waves per SIMD has 20 bytes of scratch: up to as many tiles as
+// three workgroups on each of the 256 CUs take at once there is nothing to run in the fourth, and the build without that budget is
+// ahead by 2% of the backward in the mean of 28 calls each of d40 and d56, 128 to 768 tiles, windows of 16 to 401 (B4 N8 T800 d40 k101
+// 24.6 -> 24.0 us).  With 812 to 2970 tiles four are ahead by 5%.  Bf16 and head_dim 64 are level up to 768.
+constexpr int64_t kThreePerCu = 768;
 int band_grid(int64_t ntiles) { return (int)((ntiles + 7) / 8 * 8); }
 
 template <bool BF, int D, int NQ, bool NARROW, int KB = kRowsQ>
@@ -676,8 +681,9 @@ int bwd_go(const BwdArgs &a, hipStream_t st) {
     }
     {
         ProfScope prof(ENATTEN_KERNEL_BWD_DKDV, "bwd_band_dkdv_mfma", st);
-        hipLaunchKernelGGL((bwd_band_dkdv_mfma<BF, D, NARROW>), dim3(band_grid(nt)), dim3(256), 0, st, a, tiles_t,
-                           (int)nt);
+        const auto kernel = !BF && NARROW && D == 64 && nt <= kThreePerCu ? bwd_band_dkdv_mfma<BF, D, NARROW, 2>
+                                                                          : bwd_band_dkdv_mfma<BF, D, NARROW>;
+        hipLaunchKernelGGL(kernel, dim3(band_grid(nt)), dim3(256), 0, st, a, tiles_t, (int)nt);
     }
     return check_launch("bwd_band_mfma");
 }

@@ -214,3 +214,12 @@ def test_two_groups_of_queries(shape, ks, causal, dtype, layout):
     # two groups of queries per wave in the forward, from 512 keys on: the gradients need its log-sum-exp as well (windows of 256 to
     # 300 keys, above, are walked with one group in blocks of 32 keys)
     test_band_windows(shape, ks, causal, dtype, layout)
+
+
+@pytest.mark.parametrize("shape,ks,causal,dtype,layout", [
+    ((4, 24, 512, 48), 33, True, F16, "plain"),    # 768 tiles: no budget of four waves per SIMD in the dK/dV pass
+    ((1, 71, 700, 48), 101, False, F16, "proj"),   # 781: four
+    ((4, 24, 449, 40), 20, True, F16, "proj"),     # 768, the last of a sequence with one key
+])
+def test_tiles_of_the_key_pass(shape, ks, causal, dtype, layout):
+    test_band_windows(shape, ks, causal, dtype, layout)
