@@ -647,8 +647,8 @@ bool two_groups(const Shape &s) {
     return s.D == 128 && s.kw >= 512 && (int64_t)s.B * s.N * ((s.W + 127) / 128) >= 512;
 }
 // The forward above head_dim 64 in blocks of 32 keys: where there are more tiles than the two workgroups per CU of
-// the blocks of 64 take at once; fewer only pay for the barriers.  Blocks of 64 / 32, us: B1 N16 T8192 d128 k200 causal 46.7 / 42.0, k128 on
-// views of one projection, the call, 42.4 / 36.8, k91 centred 35.9 / 33.1; B1 N16 T3000 k400 (752 tiles) 32.7 / 26.0;
+// the blocks of 64 take at once; fewer only pay for the barriers.  Blocks of 64 / 32, us: B1 N16 T8192 d128 k200 causal
+// 46.7 / 42.0, k128 on views of one projection, the call, 42.4 / 36.8, k91 centred 35.9 / 33.1; B1 N16 T3000 k400 (752 tiles) 32.7 / 26.0;
 // B3 N4 T3000 k20 (564) 11.8 / 9.1; B2 N8 T8192 d96 k512 77 / 67, B3 N7 T2500 d80 k20 12.1 / 9.0; B1 N16 T2000 k128 (512) 10.2 / 10.0,
 // B1 N7 T3001 k250 (329) 12.4 / 13.6, B1 N4 T4096 k1024 (256) 26.0 / 27.4.
 bool short_blocks(const Shape &s) { return (int64_t)s.B * s.N * ((s.W + 63) / 64) > 512; }
@@ -692,7 +692,7 @@ bool band_layout_ok(const View &v) {
     return reinterpret_cast<uintptr_t>(v.ptr) % 16 == 0 && v.sb % 8 == 0 && v.sn % 8 == 0 && v.sw % 8 == 0 &&
            v.sw < (1 << 22);
 }
-// The smallest window that is taken here.  A tile walks at least two blocks of 64 keys, however few of them its
+// The smallest window that is taken here.  A tile walks at least two blocks of 64 keys (three of 32), however few of them its
 // windows hold, and narrow heads give the matrix instructions little to do.  us, general kernels / here, causal, B4 N8
 // T16384 bf16, forward and backward: d8 k6 34 / 37, 80 / 106, k12 58 / 37, 131 / 104; d16 k4 32 / 36, 81 / 107, k8 46 / 36,
 // 109 / 107; d24 k4 40 / 53, 116 / 141, k8 59 / 53, 163 / 141; d32 k3 36 / 37, 110 / 116, k4 40 / 37, 123 / 117; d48 k2 52 / 77,

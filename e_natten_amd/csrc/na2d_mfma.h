@@ -571,7 +571,7 @@ struct HaloPlan {
                              // branch that would keep its registers from one fetch to the next, and writes nothing: its
                              // LDS columns stay zero (zero_row)
     // (a constant) such a thread loads nothing: for the kernels that have registers for the branch, and would pay for the
-    // loads (kFwdSkip, kDkdvSkip and the dQ pass's in na2d_mfma_kernels.h)
+    // loads (kFwdSkip, kDqSkip and kDkdvSkip in na2d_mfma_kernels.h)
     bool skip;
 };
 template <int D, int KS, int NW = 4, int SP = 1, bool KEEP = false>

@@ -224,10 +224,10 @@ __device__ __forceinline__ void unscale(f32x4 (&dk)[DT], f32x4 (&dv)[DT], const 
 }
 
 // ------------------------------------------------------------------ relative position bias
-// The head's [2k-1, 2k-1] table in LDS, in float32, with a margin of 3 rows and columns: entry (key - query + k - 1) per axis lies at (.. + 3), so that every (token of a 4x4
-// block's halo, pixel of the block) pair has an entry, in its window or not, and the place of a
-// token's entry is a lane constant plus (token row) * TB + (token column), which folds into the
-// LDS read's offset.
+// The head's [2k-1, 2k-1] table in LDS, in float32, with a margin of 3 rows and columns: entry (key - query + k - 1)
+// per axis lies at (.. + 3), so that every (token of a 4x4 block's halo, pixel of the block) pair has an entry, in its
+// window or not, and the place of a token's entry is a lane constant plus (token row) * TB + (token column), which folds
+// into the LDS read's offset.
 template <int KS>
 struct Bias {
     using G = Geo<32, KS>;  // (the numbering of the halo tokens depends on KS alone)
@@ -369,8 +369,8 @@ struct BiasGrad {
         }
     }
 };
-// dS of a lane's halo tokens as operands of dQ's product (zero in tiles without tokens), and, times 1 / Z (0 for a lane without a query, or with one that again_dq computes), as terms of the
-// bias gradient
+// dS of a lane's halo tokens as operands of dQ's product (zero in tiles without tokens), and, times 1 / Z (0 for a
+// lane without a query, or with one that again_dq computes), as terms of the bias gradient
 template <bool BF, int KS, int STEPS>
 __device__ __forceinline__ void operand_and_sums(Op8 (&dsb)[STEPS], f32x4 (&ds)[Bias<KS>::USED], DsScale<BF> &scl,
                                                  float zinv) {
@@ -914,6 +914,11 @@ template <int D, int KS, int NW>
 constexpr int kDqWaves = kBias || NW != 4 ? Geo<D, KS, NW>::WAVES
                          : !kNarrow && D == 32 && KS <= 5 ? 4
                          : (D == 32 && ((KS == 7 && !kSub) || (KS == 9 && !kNarrow))) || (!kNarrow && D == 64 && KS == 3) ? 3 : Geo<D, KS, NW>::WAVES;
+// SKIP of the dQ pass (kFwdSkip).  Time without the branch: k = 3 up to 10% more at d48, 9% at d80 and d96, 7% on the
+// sub-grids of d32; k = 5 6% more there, and 3 to 17% less at d48.  From k = 7 on the builds that spill with the branch are
+// up to 48% faster without (d96 k11), the others level.
+template <int D, int KS>
+constexpr bool kDqSkip = !kTable && (KS == 3 || (D != 64 && KS == 5));
 // FULL: as in fwd_mfma (no wave switched off, no store predicated, the staged rows go to LDS at
 // the end of a tile's pass through the loop).
 template <bool BF, int D, int KS, bool FRAME, bool ROLL, int NW = 4, bool FULL = false>
@@ -943,7 +948,7 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
         else return in_sub(tile_of(t, ts.tiles_r, ts.tiles_c, s.N, G::TH), a);
     };
 
-    const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim, !kTable && (KS == 3 || (D != 64 && KS == 5)));
+    const HaloPlan<D, KS, NW> plan = make_plan<D, KS, NW>(dlim, kDqSkip<D, KS>);
     HaloRegs<D, KS, NW> kst, vst;
     s16x8 qnext[G::DS], gnext[G::DS];
     float lse_next = 0.f;
@@ -1017,7 +1022,8 @@ __global__ __launch_bounds__((Geo<D, KS, NW>::NT), (kDqWaves<D, KS, NW>)) void b
             // P^T and dP^T on the halo; delta = sum_j P_j dP_j (= dO . O) comes from
             // the same values that form dS, so sum_j dS_j vanishes to rounding
             // P is kept rounded to 16 bits (it is about to be rounded into dS
-            // anyway) in the registers that will hold dS.  dP stays float32; with
+            // anyway) in the registers that will hold dS; with a bias and in two terms, where
+            // dS is not rounded to 16 bits, in float32.  dP stays float32; with
             // the largest halos it is not kept but formed a second time once delta
             // is known (measured faster there: the matrix cores are idle, the
             // registers are not).
@@ -2145,7 +2151,8 @@ constexpr bool kFwd2TallBuilt = D == 128 && kOneHaloWgs<D, KS> == 1 && kOneHaloF
                                 (size_t)Geo<D, KS, 8>::ROWS * Geo<D, KS, 8>::PITCH * 2 + 1024 <= 160 * 1024;
 // At head_dim 64 (kernel_size 11 and 13, where one halo of an 8x8 tile fits LDS twice) the one-halo dQ
 // pass takes the 16x8 tiles too: one workgroup of eight waves instead of two of four, a quarter less halo
-// per pixel.  (Not in two terms: the 8x8 tiles have one workgroup per CU and all its registers there.)  B2 N8 128x128 k13 81.5 -> 76.2 us, B4 N8 256x256 626 -> 606, B4 N4 128x128 k11 77.1 -> 76.3.
+// per pixel.  (Not in two terms: the 8x8 tiles have one workgroup per CU and all its registers there.)
+// B2 N8 128x128 k13 81.5 -> 76.2 us, B4 N8 256x256 626 -> 606, B4 N4 128x128 k11 77.1 -> 76.3.
 template <int D, int KS>
 constexpr bool kDq2TallBuilt = !kBias && (kFwd2TallBuilt<D, KS> || (D == 64 && KS >= 11));
 template <int D, int KS>

@@ -292,7 +292,8 @@ __global__ __launch_bounds__(G::NT, G::WPS) void bwd_small_mfma(BwdArgsSub a, in
     // dQ.  delta = dO . O is what O was rounded to away from the sum of P dP, an error that all keys
     // of a window share and that keys or values with a common component multiply.  So the residual
     // E = sum p (dP - delta) is summed beside the products, dQ = A - E sum p k, and the dK/dV jobs
-    // find delta + E (sum p is 1 to what the log-sum-exp was rounded to; 14x14 d64 k9 bf16, k and v of mean 2: dQ off by 4.4e-2 in 2-norm without, 4.1e-3 with).
+    // find delta + E (sum p is 1 to what the log-sum-exp was rounded to; 14x14 d64 k9 bf16, k and v of
+    // mean 2: dQ off by 4.4e-2 in 2-norm without, 4.1e-3 with).
     for (int t0 = wave * 16; t0 < P; t0 += G::NW * 16) {
         const int own = min(t0 + n, P - 1);
         s16x8 qreg[G::DS], greg[G::DS];
