@@ -13,11 +13,12 @@
 // its own windows reach, where a 16-wide instruction has the whole 4x4 block meet (k+3)^2 and more: 36 tokens per
 // query instead of 64 at kernel_size 5 (25 are in its window), 16 instead of 48 at 3, 64 instead of 112 at 7.
 // Both shapes run at the rate of the 16-wide ones (16 and 32 products per cycle and SIMD: measured 17.0 and 9.3
-// cycles against 66.1 and 33.0).  Forward, dQ and dK/dV pass, us, 4x4 blocks on the 16-wide instructions -> 2x2 blocks:
-// B4 N4 128x128 d128 k5 160 + 226 + 188 -> 133 + 181 + 149; 96x96 d64 k3 36 + 48 + 39 -> 25 + 33 + 28, k7 72 + 120 + 95 ->
-// 59 + 90 + 71; B4 N8 96x96 d32 k5 52 + 74 + 63 -> 43 + 61 + 42.  What bounds them: HBM at 4.2 TB/s in the forward and the
-// dQ pass, where a tile's two staging phases issue no matrix instruction, and LDS reads of the second products, whose bank
-// conflicts are 40% of the LDS cycles.  One tensor's halo at a time is staged in LDS (float32 rows of D + 4 floats), so two
+// cycles against 66.1 and 33.0).  Forward, dQ and dK/dV pass, us, 4x4 blocks on the 16-wide instructions -> 2x2 blocks,
+// B4 N4 128x128, launches queued behind each other: d128 k5 163 + 226 + 187 -> 137 + 182 + 148, d64 k3 64 + 89 + 66 -> 46 + 64 +
+// 47, k7 132 + 237 + 175 -> 109 + 171 + 130, d32 k5 49 + 64 + 56 -> 40 + 53 + 34.  What bounds them at d128 k5: a tile's two
+// staging phases, which issue no matrix instruction (a fifth of the wave cycles are waits; 3.5 TB/s of the 5.7 that HBM gives
+// the 16-bit forward), and LDS reads of the second products, whose bank conflicts are 40% of the LDS cycles (0 to 14% with
+// the 4x4 blocks).  One tensor's halo at a time is staged in LDS (float32 rows of D + 4 floats), so two
 // workgroups share a CU; the other tensor's halo travels from HBM into registers meanwhile.
 //
 // Lanes.  A lane is (g, b, j) = (lane >> 4, lane >> 2 & 3, lane & 3): block b of the wave, pixel j of the
